@@ -1,0 +1,41 @@
+// Launches of the block-structured kernels (layer_block.hpp, descend_block.hpp). Each family of
+// instantiations is a translation unit of its own, so that they compile in parallel.
+#pragma once
+#include "descend_block.hpp"
+#include "layer_block.hpp"
+
+namespace slos {
+
+// grid, LDS, stream and the plan's device tables of one launch
+struct BlockGrid {
+  dim3 grid;
+  size_t lds;
+  hipStream_t st;
+  const uint64_t* cg;
+  const int* lo;
+  const void* tuples;
+  int me, multiset;
+};
+
+// the stream-slot count instantiated for prefix width d (exact where the big layers live)
+inline int block_maxd(int d) { return d <= 4 ? 4 : d <= 8 ? d : 16; }
+
+// k_layer_block for prefix width d = K - suf (block_kernels.hip, one object per KIND)
+template <int KIND>
+void launch_layer_block(bool comp, int d, int suf, const BlockGrid& g, const float2* par, void* out, const BlockLayer& L);
+
+// k_layer_group for prefix width d = K - 5 in 2..6 (group_kernels.hip)
+void launch_layer_group(int d, int kind, bool comp, const BlockGrid& g, const float2* par, void* out, const BlockLayer& L,
+                        const uint4* items, uint32_t n_items);
+
+// k_layer_block_group for prefix width d = K - 4 (uneven_kernels.hip)
+void launch_layer_block_group(bool comp, int d, uint32_t grid, size_t lds, hipStream_t st, const GroupLaunch& gl);
+
+// k_descend_block and k_adjoint_block with maxd (4, 6 or 8) prefix slots (descend_kernels.hip)
+void launch_descend_block(int maxd, const BlockGrid& g, int K, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
+                          uint64_t S_pre, uint64_t per_wave, float scale, uint32_t xcd_chunk);
+void launch_adjoint_block(int maxd, const BlockGrid& g, int K, int m, int col, const float2* U, const float2* psi,
+                          const float2* gk, uint64_t Sk, float2* gout, uint64_t Sp, uint64_t S_pre, uint64_t per_wave,
+                          uint32_t xcd_chunk, double2* partial);
+
+}  // namespace slos

@@ -24,6 +24,7 @@
 #include "descend_block.hpp"
 #include "layer_f64.hpp"
 #include "pull_index.hpp"
+#include "block_launch.hpp"
 
 namespace {
 
@@ -626,13 +627,10 @@ __global__ __launch_bounds__(64) void k_reduce_gu(const double2* __restrict__ pa
   }
 }
 
-// the stream-slot count instantiated for prefix width d (exact where the big layers live)
-int block_maxd(int d) { return d <= 4 ? 4 : d <= 8 ? d : 16; }
-
 // dynamic LDS of the single-plan block kernel for layer K with suffix length suf, or 0 if it
 // does not fit the GPU's LDS
 size_t block_lds_fit(int K, int me, int suf) {
-  const size_t sh = slos::block_dyn_lds(K, me, block_maxd(K - suf));
+  const size_t sh = slos::block_dyn_lds(K, me, slos::block_maxd(K - suf));
   return sh + slos::kBlockStaticLds <= lds_limit() ? sh : 0;
 }
 
@@ -641,30 +639,6 @@ size_t block_lds_fit(int K, int me, int suf) {
 // n = 11, m = 32: less per-block set-up and fewer part-filled sweep steps), else 4
 int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
   return (dt.tuples5 && K - 5 >= 1 && K - 5 <= 8 && block_lds_fit(K, p->me, 5)) ? 5 : slos::kSuf;
-}
-
-template <int KIND, bool COMP>
-void launch_block_kind(int maxd, int suf, dim3 grid, size_t sh, hipStream_t st, const DevTables& dt,
-                       const slos_plan* p, const float2* par, void* out, const slos::BlockLayer& L) {
-#define SLOS_BLK(D, S, T)                                                                                        \
-  hipLaunchKernelGGL((slos::k_layer_block<KIND, COMP, D, S>), grid, dim3(slos::kBlockThreads), sh, st, dt.cg, dt.lo, \
-                     T, p->me, p->me + 1, p->multiset, par, out, L)
-  // one stream slot per prefix position: exact widths where the big layers live (d = K - suf)
-  if (suf == 5) {
-    if (maxd <= 4) SLOS_BLK(4, 5, dt.tuples5);
-    else if (maxd == 5) SLOS_BLK(5, 5, dt.tuples5);
-    else if (maxd == 6) SLOS_BLK(6, 5, dt.tuples5);
-    else if (maxd == 7) SLOS_BLK(7, 5, dt.tuples5);
-    else SLOS_BLK(8, 5, dt.tuples5);
-  } else {
-    if (maxd <= 4) SLOS_BLK(4, 4, dt.tuples);
-    else if (maxd == 5) SLOS_BLK(5, 4, dt.tuples);
-    else if (maxd == 6) SLOS_BLK(6, 4, dt.tuples);
-    else if (maxd == 7) SLOS_BLK(7, 4, dt.tuples);
-    else if (maxd == 8) SLOS_BLK(8, 4, dt.tuples);
-    else SLOS_BLK(16, 4, dt.tuples);
-  }
-#undef SLOS_BLK
 }
 
 int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, int kind, bool comp, hipStream_t st) {
@@ -695,42 +669,19 @@ int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, in
     const uint64_t gwgs = ((uint64_t)gn + slos::kWaves - 1) / slos::kWaves;
     if (shg + slos::kBlockStaticLds <= lds_limit() && gwgs <= 0x7fffffffull) {
       L.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
-      const dim3 ggrid((unsigned)gwgs, (unsigned)a.B);
-      const int maxd = a.K - suf;
-#define SLOS_GRP2(D, C)                                                                                                \
-  if (grp_last)                                                                                                        \
-    hipLaunchKernelGGL((slos::k_layer_group<D, 1, C>), ggrid, dim3(slos::kBlockThreads), shg, st, dt.cg, dt.lo,          \
-                       dt.tuples5, p->me, p->me + 1, a.par, a.out, L, gitems, gn);                                      \
-  else                                                                                                                 \
-    hipLaunchKernelGGL((slos::k_layer_group<D, 0, C>), ggrid, dim3(slos::kBlockThreads), shg, st, dt.cg, dt.lo,          \
-                       dt.tuples5, p->me, p->me + 1, a.par, a.out, L, gitems, gn)
-#define SLOS_GRP(D)      \
-  if (comp) {            \
-    SLOS_GRP2(D, true);  \
-  } else {               \
-    SLOS_GRP2(D, false); \
-  }
-      if (maxd <= 2) { SLOS_GRP(2); }
-      else if (maxd == 3) { SLOS_GRP(3); }
-      else if (maxd == 4) { SLOS_GRP(4); }
-      else if (maxd == 5) { SLOS_GRP(5); }
-      else { SLOS_GRP(6); }
-#undef SLOS_GRP
-#undef SLOS_GRP2
+      const slos::BlockGrid bg{dim3((unsigned)gwgs, (unsigned)a.B), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
+      slos::launch_layer_group(a.K - suf, grp_last ? 1 : 0, comp, bg, a.par, a.out, L, gitems, gn);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
     }
   }
   const size_t sh = block_lds_fit(a.K, p->me, suf);
   if (!sh) return fail(SLOS_ERANGE, "block kernel LDS exceeds the GPU's LDS");
-  dim3 grid((unsigned)wgs, (unsigned)a.B);
-  const int maxd = a.K - suf;
-  if (kind == 0) comp ? launch_block_kind<0, true>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L)
-                      : launch_block_kind<0, false>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L);
-  else if (kind == 1) comp ? launch_block_kind<1, true>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L)
-                           : launch_block_kind<1, false>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L);
-  else comp ? launch_block_kind<2, true>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L)
-            : launch_block_kind<2, false>(maxd, suf, grid, sh, st, dt, p, a.par, a.out, L);
+  const slos::BlockGrid bg{dim3((unsigned)wgs, (unsigned)a.B), sh, st, dt.cg, dt.lo,
+                           suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
+  if (kind == 0) slos::launch_layer_block<0>(comp, a.K - suf, suf, bg, a.par, a.out, L);
+  else if (kind == 1) slos::launch_layer_block<1>(comp, a.K - suf, suf, bg, a.par, a.out, L);
+  else slos::launch_layer_block<2>(comp, a.K - suf, suf, bg, a.par, a.out, L);
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
 }
@@ -1140,20 +1091,8 @@ bool group_can_block(const slos_group* G, const std::vector<DevTables>& dts, int
       if (!dts[g].tuples) return false;
       off = std::max(off, slos::block_table_offset(K, G->plans[g]->me));
     }
-  const size_t sh = off + (size_t)slos::kWaves * slos::kBlockBatch * slos::block_words(block_maxd(K - slos::kSuf)) * 4;
+  const size_t sh = off + (size_t)slos::kWaves * slos::kBlockBatch * slos::block_words(slos::block_maxd(K - slos::kSuf)) * 4;
   return sh + slos::kBlockStaticLds <= lds_limit();
-}
-
-template <bool COMP>
-void launch_block_group(int maxd, uint32_t grid, size_t sh, hipStream_t st, const slos::GroupLaunch& gl) {
-#define SLOS_BLKG(D) hipLaunchKernelGGL((slos::k_layer_block_group<COMP, D>), dim3(grid), dim3(slos::kBlockThreads), sh, st, gl)
-  if (maxd <= 4) SLOS_BLKG(4);
-  else if (maxd == 5) SLOS_BLKG(5);
-  else if (maxd == 6) SLOS_BLKG(6);
-  else if (maxd == 7) SLOS_BLKG(7);
-  else if (maxd == 8) SLOS_BLKG(8);
-  else SLOS_BLKG(16);
-#undef SLOS_BLKG
 }
 
 // layer K of every plan with n >= K as one launch per plan, through the single-plan path (the
@@ -1241,14 +1180,13 @@ int group_layer(const slos_group* G, int K, const GroupArgs& a, const GroupWs& w
   gl.total = (uint32_t)total;
   if (block) {
     gl.table_off = (uint32_t)sh;
-    sh += (size_t)slos::kWaves * slos::kBlockBatch * slos::block_words(block_maxd(K - slos::kSuf)) * 4;
+    sh += (size_t)slos::kWaves * slos::kBlockBatch * slos::block_words(slos::block_maxd(K - slos::kSuf)) * 4;
   }
   if (sh + (block ? slos::kBlockStaticLds : 0) > lds_limit()) return fail(SLOS_ERANGE, "group layer LDS exceeds the GPU's LDS");
   const uint32_t all = (uint32_t)(8 * ((total + 7) / 8));
   const uint32_t grid = c.grid ? std::min<uint32_t>(std::max<uint32_t>(c.grid & ~7u, 8), all) : all;
   const bool comp = a.flags & SLOS_FLAG_COMPENSATED;
-  if (block) comp ? launch_block_group<true>(K - slos::kSuf, grid, sh, st, gl)
-                  : launch_block_group<false>(K - slos::kSuf, grid, sh, st, gl);
+  if (block) slos::launch_layer_block_group(comp, K - slos::kSuf, grid, sh, st, gl);
   else
     with_km(K, [&](auto km) {
       constexpr int KM = decltype(km)::value;
@@ -1820,17 +1758,8 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   if (L.block && dt.tuples) {
     const dim3 grid((unsigned)L.nblk, (unsigned)batch);
     const uint64_t S_pre = p->size(k - 1 - slos::kSuf);
-#define SLOS_ADJ(D, E)                                                                                                 \
-  hipLaunchKernelGGL((slos::k_adjoint_block<D, E>), grid, dim3(slos::kBlockThreads), L.lds, st, dt.cg, dt.lo, dt.tuples, \
-                     p->me, p->me + 1, k, p->m, col, Uf, psi, gk, Sk, gout, Sp, S_pre, L.per_wave, L.xcd_chunk, part)
-#define SLOS_ADJ_E(D)                   \
-  if (p->me <= 16) SLOS_ADJ(D, 16);     \
-  else SLOS_ADJ(D, 32)
-    if (L.maxd == 4) { SLOS_ADJ_E(4); }
-    else if (L.maxd == 6) { SLOS_ADJ_E(6); }
-    else { SLOS_ADJ_E(8); }
-#undef SLOS_ADJ_E
-#undef SLOS_ADJ
+    const slos::BlockGrid bg{grid, L.lds, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+    slos::launch_adjoint_block(L.maxd, bg, k, p->m, col, Uf, psi, gk, Sk, gout, Sp, S_pre, L.per_wave, L.xcd_chunk, part);
   } else {
     with_km(k - 1, [&](auto km) {
       hipLaunchKernelGGL((k_adjoint_layer<decltype(km)::value>), dim3((unsigned)L.nblk, (unsigned)batch),
@@ -1873,18 +1802,8 @@ int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1,
       const uint32_t xc = (uint32_t)std::max<uint64_t>(1, (1ull << 16) / ((uint64_t)slos::kWaves * pw));
       const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
       const uint64_t S_pre = p->size(dp);
-#define SLOS_DESC(D, E)                                                                                                  \
-  hipLaunchKernelGGL((slos::k_descend_block<D, E>), grid, dim3(slos::kBlockThreads), shb, st, dt.cg, dt.lo, dt.tuples, \
-                     p->me, p->me + 1, k, q_k, Sk, q_km1, Sp, S_pre, pw, (float)scale, xc)
-#define SLOS_DESC_E(D)          \
-  if (p->me <= 16) SLOS_DESC(D, 16); \
-  else if (p->me <= 32) SLOS_DESC(D, 32); \
-  else SLOS_DESC(D, 64)
-      if (maxd == 4) { SLOS_DESC_E(4); }
-      else if (maxd == 6) { SLOS_DESC_E(6); }
-      else { SLOS_DESC_E(8); }
-#undef SLOS_DESC_E
-#undef SLOS_DESC
+      const slos::BlockGrid bg{grid, shb, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+      slos::launch_descend_block(maxd, bg, k, q_k, Sk, q_km1, Sp, S_pre, pw, (float)scale, xc);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
     }
