@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_descend_block(const uint64_t*
   const int64_t b = blockIdx.y;
   const int wv = (int)rfl(threadIdx.x >> 6);
   // work groups in XCD chunks, as the forward block kernel
-  const uint64_t g = uniform_u64(((uint64_t)xcd_chunk_index(blockIdx.x, xcd_chunk) * kWaves + wv) * per_wave);
+  const uint64_t g = uniform_u64(((uint64_t)xcd_chunk_index(blockIdx.x, xcd_chunk, gridDim.x) * kWaves + wv) * per_wave);
   uint32_t* tbl = reinterpret_cast<uint32_t*>(smem + desc_table_offset(K, me)) + (size_t)wv * kBlockBatch * desc_words(MAXD);
   descend_wave<MAXD, ME>(tg, tl, K, qk_all + (size_t)b * Sk, qout_all + (size_t)b * Sp, Sp, S_pre, per_wave, tbl, g, scale);
 }
@@ -421,7 +421,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_adjoint_block(const uint64_t*
   float2 gacc[ME];
 #pragma unroll
   for (int a = 0; a < ME; ++a) gacc[a] = make_float2(0.f, 0.f);
-  const uint64_t g = uniform_u64(((uint64_t)xcd_chunk_index(blockIdx.x, xcd_chunk) * kWaves + wv) * per_wave);
+  const uint64_t g = uniform_u64(((uint64_t)xcd_chunk_index(blockIdx.x, xcd_chunk, gridDim.x) * kWaves + wv) * per_wave);
   uint32_t* tbl = reinterpret_cast<uint32_t*>(smem + desc_table_offset(K, me)) + (size_t)wv * kBlockBatch * desc_words(MAXD);
   desc_block_walk<MAXD>(tg, tl, K, nullptr, nullptr, Sp, S_pre, per_wave, tbl, g, 1.f,
                         [&](const DescCtx& c, uint32_t uc, uint32_t u_stop) {

@@ -34,6 +34,7 @@ struct BlockLayer {
   unsigned flags;
   uint64_t per_wave;     // children per wave
   uint32_t xcd_chunk;    // work groups per XCD chunk (see k_layer_block); 1: plain launch order
+  uint32_t rows, row_wgs;  // rows of a 1-D launch (1: the grid's y) and work groups of a row (batch_item)
   // compensated sums only: element offsets of the low-order parts of the parent layer and of a
   // complex64 output layer from their high parts (0: none; a hi/lo layer is [2][B][S])
   int64_t par_lo, out_lo;
@@ -215,21 +216,28 @@ __device__ __forceinline__ void suffix_edges(const ChunkCtx<MAXD, SUF>& cx, Tupl
 // coefficients. The next tuple raises one position e (the first in which the two words differ) and
 // refills the later ones with the same mode, so that every suffix parent of b is the one after a's
 // (off[j] + 8 bytes) except the one that drops x_e: that is a's own parent for e = SUF - 1 (the
-// others unchanged) and lies at `offx` bytes for e < SUF - 1. a is not the block's last tuple, so
-// off[j] + 8 stays inside the parent block for every j. Per step and block this takes 5 loads of 16
-// bytes and a masked one in place of 10 of 8 bytes (whose lanes the cache serves at half its rate):
-// the last layer at n = 11, m = 32 25.9 -> 23.9 ms, of 170 instances (8, 20) 1.57 -> 1.46 ms.
+// others unchanged) and lies at b[e] for e < SUF - 1. off[j] + 8 bytes is inside the parent layer
+// for every j: it is past the parents of the block only where a = (x, m-1, .., m-1) drops x < m - 1,
+// and then another block follows. Per step and block this takes 5 loads of 16 bytes and a masked one
+// in place of 10 of 8 bytes (whose lanes the cache serves at half its rate): the last layer at n = 11,
+// m = 32 25.9 -> 23.9 ms, of 170 instances (8, 20) 1.57 -> 1.46 ms. Compensated sums, which are bound
+// by their arithmetic, keep the 10 loads: the selects cost 2 % there (n = 9, m = 22, 339 -> 346 us).
+template <int SUF>
+struct PairOffsets {
+  uint32_t a[SUF], b[SUF];  // suffix parents of the two children (bytes)
+  uint32_t x;               // b[e]
+  int e;
+};
 template <int MAXD, int SUF>
 __device__ __forceinline__ void pair_edges(const ChunkCtx<MAXD, SUF>& cx, TupleWordT<SUF> wa, TupleWordT<SUF> wb,
-                                           float2 (&c)[2][SUF], uint32_t (&off)[SUF], uint32_t& offx, int& e) {
-  uint32_t offb[SUF];
-  suffix_edges(cx, wa, c[0], off);
-  suffix_edges(cx, wb, c[1], offb);
+                                           float2 (&c)[2][SUF], PairOffsets<SUF>& o) {
+  suffix_edges(cx, wa, c[0], o.a);
+  suffix_edges(cx, wb, c[1], o.b);
   const uint32_t diff = ((uint32_t)wa ^ (uint32_t)wb) & 0x3f3f3f3fu;
-  e = (SUF == 5 && diff == 0u) ? 4 : (int)((uint32_t)__builtin_ctz(diff) >> 3);
-  offx = offb[0];
+  o.e = (SUF == 5 && diff == 0u) ? 4 : (int)((uint32_t)__builtin_ctz(diff) >> 3);
+  o.x = o.b[0];
 #pragma unroll
-  for (int j = 1; j < SUF - 1; ++j) offx = e == j ? offb[j] : offx;
+  for (int j = 1; j < SUF - 1; ++j) o.x = o.e == j ? o.b[j] : o.x;
 }
 
 // prod t_j! of a child from its tuple word and the block's prefix runs
@@ -399,13 +407,35 @@ __host__ __device__ inline size_t block_dyn_lds(int K, int me, int maxd) {
 // Work group `bid` of a 1-D grid in XCD chunks of C: the dispatcher deals work groups
 // round-robin to the 8 XCDs, and work group i = 8 t + x (XCD x) takes range 8 C (t / C) + C x + t % C,
 // so each XCD sweeps runs of C consecutive ranges while the eight XCDs stay in one region. The work
-// groups past the last whole multiple of 8 C keep their own index (a bijection of [0, gridDim.x)).
-__device__ __forceinline__ uint32_t xcd_chunk_index(uint32_t bid, uint32_t C) {
+// groups past the last whole multiple of 8 C keep their own index (a bijection of [0, n)).
+__device__ __forceinline__ uint32_t xcd_chunk_index(uint32_t bid, uint32_t C, uint32_t n) {
   if (C <= 1) return bid;
-  const uint32_t full = (gridDim.x / (8u * C)) * (8u * C);
+  const uint32_t full = (n / (8u * C)) * (8u * C);
   if (bid >= full) return bid;
   const uint32_t x = bid & 7u, t = bid >> 3;
   return (t / C) * 8u * C + x * C + (t % C);
+}
+
+// Row b of the batch and work group of the row. rows = 1: the row is blockIdx.y. Else the launch is
+// 1-D, rows x row_wgs work groups: whole eights of rows go to one XCD each (row 8 i + x to XCD x, its
+// work groups in order), so that a row's parent layer is read into one 4 MB L2 instead of eight, and
+// the rows left over are spread over all XCDs. Of 170 instances (8, 20) (5.3 MB of parents a row) the
+// last layer reads 1.7 GB beyond L2 instead of 6.9 GB; its time went 1.455 -> 1.434 ms (L1 and VALU
+// bind it), layer 7's 0.540 -> 0.504 ms.
+__device__ __forceinline__ uint32_t batch_item(uint32_t rows, uint32_t row_wgs, uint32_t xcd_chunk, int64_t* b) {
+  if (rows == 1u) {
+    *b = (int64_t)blockIdx.y;
+    return xcd_chunk_index(blockIdx.x, xcd_chunk, row_wgs);
+  }
+  const uint32_t full = (rows & ~7u) * row_wgs;
+  if (blockIdx.x < full) {
+    const uint32_t l = blockIdx.x >> 3, r = l / row_wgs;
+    *b = (int64_t)(8u * r + (blockIdx.x & 7u));
+    return l - r * row_wgs;
+  }
+  const uint32_t l = blockIdx.x - full, r = l / row_wgs;
+  *b = (int64_t)((rows & ~7u) + r);
+  return xcd_chunk_index(l - r * row_wgs, xcd_chunk, row_wgs);
 }
 
 __device__ __forceinline__ void wave_sync() {
@@ -614,7 +644,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(C
   const int ncg = (K + 1) * stride;
   uint64_t* cg_l = reinterpret_cast<uint64_t*>(smem);
   int* lo_l = reinterpret_cast<int*>(cg_l + ncg);
-  const int64_t b = blockIdx.y;
+  int64_t b;
+  const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
   fill_suffix_rows<SUF>(rows, a.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
@@ -628,7 +659,6 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(C
   // the far prefix streams one XCD reads are found by the others in the shared last-level cache.
   // At n = 11, m = 32 this measured 28.7 ms for the last layer against 30.3 ms in plain launch
   // order (C = 1) and 30.4 ms with C = 4096; contiguous eighths of the layer were slower still.
-  const uint32_t bid = xcd_chunk_index(blockIdx.x, a.xcd_chunk);
   const int wv = (int)rfl(threadIdx.x >> 6);
   const uint64_t g = uniform_u64(((uint64_t)bid * kWaves + wv) * a.per_wave);
   char* out_b = reinterpret_cast<char*>(out_all) + (size_t)b * a.S * (KIND == 1 ? 4 : 8);
@@ -655,20 +685,28 @@ __host__ __device__ inline size_t group_dyn_lds(int K, int me) {
 }
 
 // the suffix parents of two adjacent children (pair_edges): one 16-byte load for each dropped
-// position, and one 8-byte load in the lanes whose second child has a parent elsewhere
-template <int SUF>
-__device__ __forceinline__ void load_pair_parents(const float2* lp, const uint32_t (&off)[SUF], uint32_t offx, int e,
-                                                  float2 (&lv)[2][SUF]) {
-  float4 pv[SUF];
+// position, and one 8-byte load in the lanes whose second child has a parent elsewhere (SEP: a load
+// for each child and position)
+template <bool SEP, int SUF>
+__device__ __forceinline__ void load_pair_parents(const float2* lp, const PairOffsets<SUF>& o, float2 (&lv)[2][SUF]) {
+  if constexpr (SEP) {
 #pragma unroll
-  for (int j = 0; j < SUF; ++j) pv[j] = load_pair(lp, off[j]);
-  float2 xv = make_float2(0.f, 0.f);
-  if (e < SUF - 1) xv = at_bytes(lp, offx);
+    for (int j = 0; j < SUF; ++j) {
+      lv[0][j] = at_bytes(lp, o.a[j]);
+      lv[1][j] = at_bytes(lp, o.b[j]);
+    }
+  } else {
+    float4 pv[SUF];
 #pragma unroll
-  for (int j = 0; j < SUF; ++j) {
-    lv[0][j] = make_float2(pv[j].x, pv[j].y);
-    const float2 other = j == SUF - 1 ? lv[0][j] : xv;
-    lv[1][j] = make_float2(e == j ? other.x : pv[j].z, e == j ? other.y : pv[j].w);
+    for (int j = 0; j < SUF; ++j) pv[j] = load_pair(lp, o.a[j]);
+    float2 xv = make_float2(0.f, 0.f);
+    if (o.e < SUF - 1) xv = at_bytes(lp, o.x);
+#pragma unroll
+    for (int j = 0; j < SUF; ++j) {
+      lv[0][j] = make_float2(pv[j].x, pv[j].y);
+      const float2 other = j == SUF - 1 ? lv[0][j] : xv;
+      lv[1][j] = make_float2(o.e == j ? other.x : pv[j].z, o.e == j ? other.y : pv[j].w);
+    }
   }
 }
 
@@ -679,7 +717,7 @@ __device__ __forceinline__ void load_pair_parents(const float2* lp, const uint32
 // error at element offset olo of a complex64 output).
 template <int NS, int KIND, bool COMP = false>
 __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const float2* par, const float4& v0,
-                                                  const float2 (&lc)[2][5], const uint32_t (&off)[5], uint32_t offx, int e,
+                                                  const float2 (&lc)[2][5], const PairOffsets<5>& off,
                                                   uint32_t u, const uint32_t (&code)[2], const bool (&lead)[2], const float* rn,
                                                   float scale, void* out, const float4& v0lo = float4{},
                                                   int64_t plo = 0, int64_t olo = 0) {
@@ -700,7 +738,7 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
   }
   const float2* lp = par + LBp;
   float2 lv[2][5];
-  load_pair_parents(lp, off, offx, e, lv);
+  load_pair_parents<COMP>(lp, off, lv);
   const uint32_t lastrow = ((w6 >> 16) & 0xffu) + 1u;
   float res[2][2];
   BlockAcc accs[2];
@@ -724,7 +762,7 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
         sl[s] = load_pair(par + plo + base, u * 8u);
       }
       float2 ll[2][5];
-      load_pair_parents(lp + plo, off, offx, e, ll);
+      load_pair_parents<COMP>(lp + plo, off, ll);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
@@ -846,7 +884,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
   const int ncg = (K + 1) * stride;
   uint64_t* cg_l = reinterpret_cast<uint64_t*>(smem);
   int* lo_l = reinterpret_cast<int*>(cg_l + ncg);
-  const int64_t b = blockIdx.y;
+  int64_t b;
+  const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
   fill_suffix_rows<5>(rows, a.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
@@ -854,7 +893,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
   __syncthreads();
   const int wv = (int)rfl(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const uint32_t item = xcd_chunk_index(blockIdx.x, a.xcd_chunk) * kWaves + (uint32_t)wv;
+  const uint32_t item = bid * kWaves + (uint32_t)wv;
   if (item >= n_items) return;
   const uint4 it = items[item];
   const uint32_t r = rfl(it.x), u_b = rfl(it.y), u_e = rfl(it.z);
@@ -937,9 +976,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
       v0n = load_pair(sp0, (u + 128u) * 8u);
     }
     float2 lc[2][5];
-    uint32_t off[5], offx;
-    int e;
-    pair_edges(cx, tp.a, tp.b, lc, off, offx, e);
+    PairOffsets<5> off;
+    pair_edges(cx, tp.a, tp.b, lc, off);
     const uint32_t code[2] = {tuple_code<5>(tp.a), tuple_code<5>(tp.b)};
     const bool lead[2] = {skip0 && (int)((uint32_t)tp.a & 0xffu) == lo, skip0 && (int)((uint32_t)tp.b & 0xffu) == lo};
     float4 v0lo{};
@@ -948,7 +986,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
       uint4 bw[8];
       group_words(tbl, g, bw);
       group_dispatch<MAXD>(bw[1].x >> 24, [&](auto ns) {
-        group_block_pairs<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, offx, e, u, code, lead, rn, a.scale, out,
+        group_block_pairs<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, u, code, lead, rn, a.scale, out,
                                                             v0lo, COMP ? a.par_lo : 0, COMP ? a.out_lo : 0);
       });
     }

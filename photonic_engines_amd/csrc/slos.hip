@@ -641,6 +641,15 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
   return (dt.tuples5 && K - 5 >= 1 && K - 5 <= 8 && block_lds_fit(K, p->me, 5)) ? 5 : slos::kSuf;
 }
 
+// The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
+// there is one for every XCD and the grid's thread count stays below 2^32, else a row per grid y.
+dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
+  L->row_wgs = (uint32_t)wgs;
+  const bool flat = B >= 8 && wgs * (uint64_t)B < (1ull << 32) / slos::kBlockThreads;
+  L->rows = flat ? (uint32_t)B : 1u;
+  return flat ? dim3((unsigned)(wgs * (uint64_t)B)) : dim3((unsigned)wgs, (unsigned)B);
+}
+
 int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, int kind, bool comp, hipStream_t st) {
   slos::BlockLayer L;
   L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.S_par = a.S_par; L.S = a.S;
@@ -669,7 +678,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, in
     const uint64_t gwgs = ((uint64_t)gn + slos::kWaves - 1) / slos::kWaves;
     if (shg + slos::kBlockStaticLds <= lds_limit() && gwgs <= 0x7fffffffull) {
       L.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
-      const slos::BlockGrid bg{dim3((unsigned)gwgs, (unsigned)a.B), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
+      const slos::BlockGrid bg{batch_grid(gwgs, a.B, &L), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
       slos::launch_layer_group(a.K - suf, grp_last ? 1 : 0, comp, bg, a.par, a.out, L, gitems, gn);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
@@ -677,7 +686,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, in
   }
   const size_t sh = block_lds_fit(a.K, p->me, suf);
   if (!sh) return fail(SLOS_ERANGE, "block kernel LDS exceeds the GPU's LDS");
-  const slos::BlockGrid bg{dim3((unsigned)wgs, (unsigned)a.B), sh, st, dt.cg, dt.lo,
+  const slos::BlockGrid bg{batch_grid(wgs, a.B, &L), sh, st, dt.cg, dt.lo,
                            suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
   if (kind == 0) slos::launch_layer_block<0>(comp, a.K - suf, suf, bg, a.par, a.out, L);
   else if (kind == 1) slos::launch_layer_block<1>(comp, a.K - suf, suf, bg, a.par, a.out, L);
