@@ -13,22 +13,6 @@
 
 namespace slos {
 
-// prod_j t_j! of a sorted K-tuple (K <= KM) in FP64 (exact up to 18! per mode, far beyond the
-// float form)
-template <int KM>
-SLOS_HD double run_factorial_f64(const int (&p)[KM], int K, int multiset) {
-  double f = 1.0, run = 1.0;
-  if (multiset) {
-#pragma unroll
-    for (int i = 1; i < KM; ++i)
-      if (i < K) {
-        run = (p[i] == p[i - 1]) ? run + 1.0 : 1.0;
-        f *= run;
-      }
-  }
-  return f;
-}
-
 struct LayerArgsF64 {
   const uint64_t* cg;
   const int* lo;

@@ -105,16 +105,20 @@ SLOS_HD float run_factorial(const int* p, int K, int multiset) {
 template <int N>
 SLOS_HD constexpr int in_range(int i) { return i < 0 ? 0 : i >= N ? N - 1 : i; }
 
+// the index type of a space view (64-bit, or 32-bit for SpaceView32)
+template <class SV>
+using RankT = decltype(SV{}.C(0, 0));
+
 // sorted positions of lex index g of layer K (K <= KM) into p[0..K)
-template <int KM>
-SLOS_HD void unrank_fixed(const SpaceView& sv, uint64_t g, int K, int (&p)[KM]) {
+template <int KM, class SV>
+SLOS_HD void unrank_fixed(const SV& sv, RankT<SV> g, int K, int (&p)[KM]) {
   int l = 0;
 #pragma unroll
   for (int i = 0; i < KM; ++i) {
     p[i] = 0;
     if (i < K) {
       const int rem = K - i;
-      const uint64_t base = sv.C(rem, l);
+      const RankT<SV> base = sv.C(rem, l);
       int x = l;
       while (base - sv.C(rem, x + 1) <= g) ++x;
       g -= base - sv.C(rem, x);
@@ -125,10 +129,11 @@ SLOS_HD void unrank_fixed(const SpaceView& sv, uint64_t g, int K, int (&p)[KM]) 
 }
 
 // the parents of the K-tuple p (K <= KM), as for_each_parent
-template <int KM, class F>
-SLOS_HD void parents_fixed(const SpaceView& sv, int multiset, int K, const int (&p)[KM], F&& f) {
+template <int KM, class SV, class F>
+SLOS_HD void parents_fixed(const SV& sv, int multiset, int K, const int (&p)[KM], F&& f) {
+  typedef RankT<SV> R;
   int lop[KM + 1];
-  uint64_t suf[KM + 2];
+  R suf[KM + 2];
   int run[KM];
   lop[0] = 0;
 #pragma unroll
@@ -137,18 +142,18 @@ SLOS_HD void parents_fixed(const SpaceView& sv, int multiset, int K, const int (
   suf[KM + 1] = 0;
 #pragma unroll
   for (int i = KM - 1; i >= 0; --i) {
-    suf[i] = i < K ? suf[i + 1] + (sv.C(K - i, lop[i]) - sv.C(K - i, p[i])) : 0;
+    suf[i] = i < K ? suf[i + 1] + (sv.C(K - i, lop[i]) - sv.C(K - i, p[i])) : R(0);
     // copies of p[i] from i on (the count of a mode's first copy)
     const bool same = i + 1 < K && p[in_range<KM>(i + 1)] == p[i];
     run[i] = same ? run[in_range<KM>(i + 1)] + 1 : 1;
   }
-  uint64_t pre = 0;
+  R pre = 0;
 #pragma unroll
   for (int l = 0; l < KM; ++l) {
     if (l < K) {
       if (!multiset || l == 0 || p[l] != p[in_range<KM>(l - 1)]) {
         const int cnt = multiset ? run[l] : 1;
-        const uint64_t pr =
+        const R pr =
             (l == K - 1) ? pre
                          : pre + (sv.C(K - l - 1, lop[l]) - sv.C(K - l - 1, p[in_range<KM>(l + 1)])) + suf[l + 2];
         f(pr, p[l], cnt);
@@ -203,6 +208,22 @@ SLOS_HD float run_factorial_fixed(const int (&p)[KM], int K, int multiset) {
     for (int i = 1; i < KM; ++i)
       if (i < K) {
         run = (p[i] == p[i - 1]) ? run + 1.f : 1.f;
+        f *= run;
+      }
+  }
+  return f;
+}
+
+// prod_j t_j! of a sorted K-tuple (K <= KM) in FP64 (exact up to 18! per mode, far beyond the
+// float form)
+template <int KM>
+SLOS_HD double run_factorial_f64(const int (&p)[KM], int K, int multiset) {
+  double f = 1.0, run = 1.0;
+  if (multiset) {
+#pragma unroll
+    for (int i = 1; i < KM; ++i)
+      if (i < K) {
+        run = (p[i] == p[i - 1]) ? run + 1.0 : 1.0;
         f *= run;
       }
   }

@@ -25,6 +25,7 @@
 #include "layer_f64.hpp"
 #include "pull_index.hpp"
 #include "block_launch.hpp"
+#include "front.hpp"
 
 namespace {
 
@@ -761,6 +762,48 @@ int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   return SLOS_OK;
 }
 
+// The layers 1..kf that one launch of k_front takes (0: none): the largest kf <= layer for which the
+// layers below kf fit LDS with at most kFrontStates states, and which computes at most 2^21 states
+// again (all work groups together; with more the chip is full and a launch a layer costs less).
+int front_layers(const slos_plan* p, int64_t B, int layer, size_t elem, bool comp, size_t* lds, uint32_t* buf) {
+  int kf = 0;
+  if (B > 65535) return 0;
+  uint64_t below = 1, most = 1;  // states of the layers 0..k-1, the largest of them
+  for (int k = 1; k <= std::min(layer, slos::kFrontMax); ++k) {
+    const uint64_t S = p->size(k);
+    if (S >= (1ull << 31) || most > slos::kFrontStates) break;
+    const uint64_t wgs = (S + slos::kFrontThreads - 1) / slos::kFrontThreads;
+    if (wgs * below * (uint64_t)B > (1ull << 21)) break;
+    const size_t need = slos::front_lds(k, p->me, p->m, elem, most, comp);
+    if (need > lds_limit()) break;
+    kf = k;
+    *lds = need;
+    *buf = (uint32_t)most;
+    below += S;
+    most = std::max(most, S);
+  }
+  return kf;
+}
+
+// layers 1..kf (front_layers) in one launch; kind: of layer kf
+int run_front(const slos_plan* p, const DevTables& dt, int kf, const int* cols, const void* U, int64_t B, void* out,
+              int kind, double scale, unsigned flags, size_t lds, uint32_t buf, bool hilo_out, hipStream_t st) {
+  slos::FrontArgs a{};
+  a.cg = dt.cg; a.lo = dt.lo; a.tuples = dt.tuples; a.tuples5 = dt.tuples5;
+  a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.kf = kf; a.kind = kind; a.U = U;
+  for (int k = 0; k < kf; ++k) a.cols[k] = cols[k];
+  for (int k = 0; k <= kf; ++k) a.S[k] = (uint32_t)p->size(k);
+  a.buf = buf; a.out = out; a.scale = scale;
+  a.immediate = (flags & SLOS_FLAG_IMMEDIATE) ? 1u : 0u;
+  a.out_lo = hilo_out ? B * (int64_t)p->size(kf) : 0;
+  const uint64_t wgs = (p->size(kf) + slos::kFrontThreads - 1) / slos::kFrontThreads;
+  const RoctxRange range("slos first layers");
+  slos::launch_front((flags & SLOS_FLAG_F64) != 0, (flags & SLOS_FLAG_COMPENSATED) != 0,
+                     dim3((unsigned)wgs, (unsigned)B), lds, st, a);
+  HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
 bool mul_overflow(uint64_t a, uint64_t b, uint64_t* r) { return __builtin_mul_overflow(a, b, r); }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1465,12 +1508,24 @@ int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, int6
     HIP_TRY(hipGetLastError());
     return SLOS_OK;
   }
-  hipLaunchKernelGGL(slos::k_fill_ones_f64, g1, dim3(256), 0, st, ones, batch);
-  HIP_TRY(hipGetLastError());
+  const RoctxRange whole("slos_forward");
   const void* par = ones;
   uint64_t S_par = 1;
-  const RoctxRange whole("slos_forward");
-  for (int k = 1; k <= layer; ++k) {
+  size_t lds = 0;
+  uint32_t buf = 0;
+  const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 16, false, &lds, &buf);
+  if (kf) {
+    void* dst = kf == layer ? out : bufs[kf & 1];
+    const int rc = run_front(p, dt, kf, cols, U, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale,
+                             flags, lds, buf, false, st);
+    if (rc) return rc;
+    par = dst;
+    S_par = p->size(kf);
+  } else {
+    hipLaunchKernelGGL(slos::k_fill_ones_f64, g1, dim3(256), 0, st, ones, batch);
+    HIP_TRY(hipGetLastError());
+  }
+  for (int k = kf + 1; k <= layer; ++k) {
     const uint64_t S = p->size(k);
     const bool last = (k == layer);
     void* dst = last ? out : bufs[k & 1];
@@ -1494,9 +1549,6 @@ int forward_run(const slos_plan* p, const DevTables& dt, const void* U, int64_t 
   auto* base = static_cast<unsigned char*>(ws);
   float2* ones = reinterpret_cast<float2*>(base + w.ones);
   float2* bufs[2] = {reinterpret_cast<float2*>(base + w.even), reinterpret_cast<float2*>(base + w.odd)};
-  hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>((batch + 255) / 256, 4096)), dim3(256), 0, st,
-                     ones, batch);
-  HIP_TRY(hipGetLastError());
   if (layer == 0) {  // no photon: the vacuum
     hipLaunchKernelGGL(k_vacuum_out, dim3((unsigned)std::min<int64_t>((batch + 255) / 256, 4096)), dim3(256), 0, st, out,
                        batch, out_kind == SLOS_OUT_PROBS ? 1 : 0, (float)scale);
@@ -1509,7 +1561,22 @@ int forward_run(const slos_plan* p, const DevTables& dt, const void* U, int64_t 
   // compensated sums: every intermediate layer is a hi/lo pair [2][B][S] (the buffers are sized for it)
   const bool hilo = (flags & SLOS_FLAG_COMPENSATED) != 0;
   const RoctxRange whole("slos_forward");
-  for (int k = 1; k <= layer; ++k) {
+  size_t lds = 0;
+  uint32_t buf = 0;
+  const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 8, hilo, &lds, &buf);
+  if (kf) {
+    void* dst = kf == layer ? out : bufs[kf & 1];
+    rc = run_front(p, dt, kf, cols, U, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale, flags, lds,
+                   buf, hilo && kf < layer, st);
+    if (rc) return rc;
+    par = static_cast<const float2*>(dst);
+    S_par = p->size(kf);
+  } else {
+    hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>((batch + 255) / 256, 4096)), dim3(256), 0, st,
+                       ones, batch);
+    HIP_TRY(hipGetLastError());
+  }
+  for (int k = kf + 1; k <= layer; ++k) {
     const uint64_t S = p->size(k);
     const bool last = (k == layer);
     void* dst = last ? out : bufs[k & 1];

@@ -63,4 +63,13 @@ struct SpaceView {
   }
 };
 
+// the same tables with 32-bit counts (layers of fewer than 2^32 states)
+struct SpaceView32 {
+  const uint32_t* cg;
+  const int* lo;
+  int me;
+  int stride;
+  SLOS_HD uint32_t C(int r, int x) const { return cg[r * stride + x]; }
+};
+
 }  // namespace slos
