@@ -23,6 +23,7 @@
 #pragma once
 #include <stdint.h>
 
+#include "pull_index.hpp"
 #include "space.hpp"
 
 namespace slos {
@@ -300,29 +301,64 @@ inline TupleWordT<SUF> make_tuple_word(const SpaceView& sv, int multiset, uint64
   return w;
 }
 
+// sorted positions of lex index g of layer K (K <= KM), the last five from the 5-position suffix
+// words where they exist (words may be null): the search then ends with the prefix, a third of its
+// steps or fewer for K <= 8
+template <int KM, class SV>
+SLOS_HD void unrank_words(const SV& sv, const uint64_t* words, RankT<SV> g, int K, int (&p)[KM]) {
+  if (KM < 5 || K < 5 || !words) {
+    unrank_fixed<KM>(sv, g, K, p);
+    return;
+  }
+  int l = 0;
+#pragma unroll
+  for (int i = 0; i < KM; ++i) {
+    p[i] = 0;
+    if (i < K - 5) {
+      const int rem = K - i;
+      const RankT<SV> base = sv.C(rem, l);
+      int x = l;
+      while (base - sv.C(rem, x + 1) <= g) ++x;
+      g -= base - sv.C(rem, x);
+      p[i] = x;
+      l = sv.lo[x];
+    }
+  }
+  uint64_t w = words[(sv.C(5, 0) - sv.C(5, l)) + g];
+#pragma unroll
+  for (int i = 0; i < KM; ++i)
+    if (i >= K - 5 && i < K) {
+      p[i] = (int)((uint32_t)w & 63u);
+      w >>= 8;
+    }
+}
+
 // ---- the last layer in group order (5-position suffixes, multiset spaces) ----------------------
 // A block Q = (a, R) of the last layer drops its first photon into the parent block R of layer
 // K-1 (same tuple offsets u, since lo[last(Q)] = lo[last(R)]). The blocks (a, R), a = 0..R_0,
 // form the group of R: they share that parent block, their tuple words and their local-parent
 // ranks. A work item is (rank of R among the (d-1)-prefixes, u_begin, u_end): a range of suffix
 // positions of every block of the group, at most about 2048 children in all (measured best at
-// n = 11, m = 32: 27.5 ms for the last layer against 28.2 ms with 4096, 28.9 ms with 1024).
-constexpr uint32_t kGroupItemChildren = 2048;
-SLOS_HD uint32_t group_item_width(int G) {
-  const uint32_t w = (kGroupItemChildren / (uint32_t)G) & ~127u;
-  return w < 128u ? 128u : w;
-}
+// n = 11, m = 32: 27.5 ms for the last layer against 28.2 ms with 4096, 28.9 ms with 1024). A layer
+// of a few million children has too few such items to fill the chip and takes finer ones: 1024
+// children, ranges of at least 64 (us, layer 7 and 8 at n = 8, m = 24: 36.8 / 65.6 with 2048, 28.0 /
+// 55.8 so; at 14M children 88 / 92, at 37M 479 / 543).
+constexpr uint32_t kGroupItemChildren = 2048, kGroupItemWidth = 128;
+constexpr uint32_t kGroupFineChildren = 1024, kGroupFineWidth = 64;
 
-// the work items of layer K (prefix length d = K - 5 >= 2), 4 words each (r, u_b, u_e, 0)
+// the work items of layer K (prefix length d = K - 5 >= 2), 4 words each (r, u_b, u_e, 0): ranges of
+// about `children` children of the group, a multiple of `least` suffix positions
 template <class Vec>
-inline void group_items(const SpaceView& sv, int K, Vec& out) {
+inline void group_items(const SpaceView& sv, int K, Vec& out, uint32_t children = kGroupItemChildren,
+                        uint32_t least = kGroupItemWidth) {
   const int d = K - 5;
   const uint64_t nR = sv.C(d - 1, 0);
   int R[64];
   for (uint64_t r = 0; r < nR; ++r) {
     sv.unrank(r, d - 1, R);
     const uint32_t L = (uint32_t)sv.C(5, sv.lo[R[d - 2]]);
-    const uint32_t w = group_item_width(R[0] + 1);
+    uint32_t w = (children / (uint32_t)(R[0] + 1)) & ~(least - 1u);
+    if (w < least) w = least;
     for (uint32_t ub = 0; ub < L; ub += w) {
       out.push_back((uint32_t)r);
       out.push_back(ub);

@@ -3,8 +3,16 @@
 #pragma once
 #include "descend_block.hpp"
 #include "layer_block.hpp"
+#include "layer_block_f64.hpp"
 
 namespace slos {
+
+struct LayerArgs;
+struct LayerArgsF64;
+
+// k_layer_simple and its complex128 form (simple_kernels.hip)
+void launch_layer_simple(int kind, bool comp, dim3 grid, size_t lds, hipStream_t st, const LayerArgs& a);
+void launch_layer_f64_simple(int kind, dim3 grid, size_t lds, hipStream_t st, const LayerArgsF64& a);
 
 // grid, LDS, stream and the plan's device tables of one launch
 struct BlockGrid {
@@ -19,6 +27,8 @@ struct BlockGrid {
 
 // the stream-slot count instantiated for prefix width d (exact where the big layers live)
 inline int block_maxd(int d) { return d <= 4 ? 4 : d <= 8 ? d : 16; }
+// the same for the complex128 block kernel (d <= 8)
+inline int block_maxd_f64(int d) { return d <= 4 ? 4 : d <= 6 ? 6 : 8; }
 
 // k_layer_block for prefix width d = K - suf (block_kernels.hip, one object per KIND)
 template <int KIND>
@@ -27,6 +37,12 @@ void launch_layer_block(bool comp, int d, int suf, const BlockGrid& g, const flo
 // k_layer_group for prefix width d = K - 5 in 2..6 (group_kernels.hip)
 void launch_layer_group(int d, int kind, bool comp, const BlockGrid& g, const float2* par, void* out, const BlockLayer& L,
                         const uint4* items, uint32_t n_items);
+
+// the complex128 forms (f64_kernels.hip); the block kernel for prefixes of at most 8 positions
+void launch_layer_block_f64(int kind, int d, int suf, const BlockGrid& g, const double2* par, void* out,
+                            const BlockLayerF64& L);
+void launch_layer_group_f64(int d, int kind, const BlockGrid& g, const double2* par, void* out, const BlockLayerF64& L,
+                            const uint4* items, uint32_t n_items);
 
 // k_layer_block_group for prefix width d = K - 4 (uneven_kernels.hip)
 void launch_layer_block_group(bool comp, int d, uint32_t grid, size_t lds, hipStream_t st, const GroupLaunch& gl);

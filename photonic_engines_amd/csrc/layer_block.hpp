@@ -116,13 +116,13 @@ struct SufRow {
 };
 
 // rows for U[b, :, col] (Ucol = &U[b][0][col], stride m), positions < me; cg: the global table
-template <int SUF>
-__device__ __forceinline__ void fill_suffix_rows(SufRow* rows, const float2* Ucol, int m, const uint64_t* cg, int stride,
-                                                 int me) {
+// (Row: SufRow or its FP64 form, V: U's complex type)
+template <int SUF, class Row, class V>
+__device__ __forceinline__ void fill_suffix_rows(Row* rows, const V* Ucol, int m, const uint64_t* cg, int stride, int me) {
   for (int i = threadIdx.x; i < kSufRows; i += blockDim.x) {
     const int x = i & (kBlockModes - 1);
-    const float2 u = (i < kBlockModes && x < m) ? Ucol[(size_t)x * m] : make_float2(0.f, 0.f);
-    SufRow r;
+    const V u = (i < kBlockModes && x < m) ? Ucol[(size_t)x * m] : V{0, 0};
+    Row r;
     r.re = u.x;
     r.im = u.y;
     r.t0 = r.t1 = 0u;
@@ -178,38 +178,45 @@ struct ChunkCtx {
 
 // the suffix edges of one child from its tuple word: coefficients c[j] (edge 0 of a tau that
 // continues the prefix's last run is no edge: zero) and local-parent byte offsets off[j]
-template <int MAXD, int SUF>
-__device__ __forceinline__ void suffix_edges(const ChunkCtx<MAXD, SUF>& cx, TupleWordT<SUF> w, float2 (&c)[SUF],
-                                             uint32_t (&off)[SUF]) {
+// (Row: SufRow or its FP64 form, V: the complex type of the layers)
+template <int SUF, class Row, class V>
+__device__ __forceinline__ void suffix_edges_of(const Row* rows, uint32_t C0, int skip0, int lo, TupleWordT<SUF> w,
+                                                V (&c)[SUF], uint32_t (&off)[SUF]) {
   uint32_t lr[SUF];
   if constexpr (SUF == 4) {
     uint32_t a3[4], b2[4], b1[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const SufRow r = cx.rows[tw_byte(w, j)];
-      c[j] = make_float2(r.re, r.im);
+      const Row r = rows[tw_byte(w, j)];
+      c[j] = V{r.re, r.im};
       a3[j] = r.t0;
       b2[j] = r.t1 & 0xffffu;
       b1[j] = r.t1 >> 16;
     }
-    suffix_parent_ranks(cx.C0, a3, b2, b1, lr);
+    suffix_parent_ranks(C0, a3, b2, b1, lr);
   } else {
     const uint32_t lo32 = (uint32_t)w, hi32 = (uint32_t)(w >> 32);
     uint32_t t4[5], t3[5], t2[5], t1[5];
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
-      const SufRow r = cx.rows[j < 4 ? (lo32 >> (8 * j)) & 0xffu : hi32 & 0xffu];
-      c[j] = make_float2(r.re, r.im);
+      const Row r = rows[j < 4 ? (lo32 >> (8 * j)) & 0xffu : hi32 & 0xffu];
+      c[j] = V{r.re, r.im};
       t4[j] = r.t0 & 0xffffffu;
       t1[j] = r.t0 >> 24;
       t3[j] = r.t1 & 0xffffu;
       t2[j] = r.t1 >> 16;
     }
-    suffix_parent_ranks5(cx.C0, t4, t3, t2, t1, lr);
+    suffix_parent_ranks5(C0, t4, t3, t2, t1, lr);
   }
-  if (cx.skip0 && (int)((uint32_t)w & 0xffu) == cx.lo) c[0] = make_float2(0.f, 0.f);
+  if (skip0 && (int)((uint32_t)w & 0xffu) == lo) c[0] = V{0, 0};
 #pragma unroll
-  for (int j = 0; j < SUF; ++j) off[j] = lr[j] * 8u;
+  for (int j = 0; j < SUF; ++j) off[j] = lr[j] * (uint32_t)sizeof(V);
+}
+
+template <int MAXD, int SUF>
+__device__ __forceinline__ void suffix_edges(const ChunkCtx<MAXD, SUF>& cx, TupleWordT<SUF> w, float2 (&c)[SUF],
+                                             uint32_t (&off)[SUF]) {
+  suffix_edges_of<SUF>(cx.rows, cx.C0, cx.skip0, cx.lo, w, c, off);
 }
 
 // The suffix edges of two adjacent children a, b = a + 1 of a multiset space: c[0], c[1] their
@@ -496,6 +503,67 @@ __device__ __forceinline__ void block_children(const uint32_t* bj, const float2*
   }
 }
 
+// The block table of the blocks r .. r + 63: lane i computes the block of prefix r + i (one past the
+// last prefix is empty) and writes column i. Active slots are compacted to the front in ascending
+// prefix position (the summation order of the thread-per-state kernel); slots past the active count
+// carry slot 0's base and no edge.
+template <int MAXD, int SUF>
+__device__ __forceinline__ void fill_block_table(const BlockTables& tl, int K, int d, uint64_t r, uint64_t S_pre,
+                                                 uint32_t* tbl, int lane) {
+  constexpr int kModeW = (MAXD + 3) / 4;
+  constexpr int kBaseW = 8 + kModeW;
+  BlockInfo bi;
+  Streams<MAXD> st;
+  int q[MAXD];
+  const uint64_t ri = r + (uint64_t)lane;
+  const SpaceView sv{tl.cg, tl.lo, tl.me, tl.stride};
+  if (ri < S_pre) {
+    sv.unrank(ri, d, q);
+    block_info<MAXD, SUF>(tl, K, d, q, bi, st);
+  } else {
+    bi.L = 0;
+    bi.CB = bi.LBp = 0;
+    bi.toff = 0;
+    bi.lo = 0;
+    bi.skip0 = 0;
+    bi.lastrun = 0;
+    bi.fQ = 1.f;
+#pragma unroll
+    for (int s = 0; s < MAXD; ++s) {
+      st.base[s] = 0;
+      st.mode[s] = kNoEdgeRow;
+      st.active[s] = false;
+    }
+  }
+  wave_sync();  // every lane is done reading the previous batch
+  uint32_t* col = tbl + lane;
+  col[0 * kBlockBatch] = (uint32_t)bi.CB;
+  col[1 * kBlockBatch] = (uint32_t)(bi.CB >> 32);
+  col[2 * kBlockBatch] = (uint32_t)bi.LBp;
+  col[3 * kBlockBatch] = (uint32_t)(bi.LBp >> 32);
+  col[4 * kBlockBatch] = bi.L;
+  col[5 * kBlockBatch] = bi.toff;
+#pragma unroll
+  for (int w = 0; w < kModeW; ++w) col[(8 + w) * kBlockBatch] = kNoEdgeRow * 0x01010101u;
+#pragma unroll
+  for (int t = 0; t < MAXD; ++t) {
+    col[(kBaseW + 2 * t) * kBlockBatch] = (uint32_t)st.base[0];
+    col[(kBaseW + 2 * t + 1) * kBlockBatch] = (uint32_t)(st.base[0] >> 32);
+  }
+  uint32_t nact = 0;
+#pragma unroll
+  for (int s = 0; s < MAXD; ++s)
+    if (st.active[s]) {
+      reinterpret_cast<uint8_t*>(col + (8 + (nact >> 2)) * kBlockBatch)[nact & 3u] = (uint8_t)st.mode[s];
+      col[(kBaseW + 2 * nact) * kBlockBatch] = (uint32_t)st.base[s];
+      col[(kBaseW + 2 * nact + 1) * kBlockBatch] = (uint32_t)(st.base[s] >> 32);
+      ++nact;
+    }
+  col[6 * kBlockBatch] = (uint32_t)bi.lo | ((uint32_t)bi.skip0 << 8) | ((uint32_t)bi.lastrun << 16) | (nact << 24);
+  col[7 * kBlockBatch] = __builtin_bit_cast(uint32_t, bi.fQ);
+  wave_sync();
+}
+
 // One wave's share of a layer slice: the children [g, g + a.per_wave) of one instance, whose parent
 // layer is `par` and whose output layer starts at `out`. `rows` is the suffix table and `rn` the
 // readout norms (LDS), `tl` the counting tables in LDS, `tg` the same tables in global memory (for
@@ -506,13 +574,9 @@ template <int KIND, bool COMP, int MAXD, int SUF>
 __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTables& tl, const float2* __restrict__ par,
                                            void* __restrict__ out, const SufRow* rows, const float* rn,
                                            uint32_t* tbl, const BlockLayer& a, uint64_t g, int kind = 0) {
-  constexpr int kModeW = (MAXD + 3) / 4;
-  constexpr int kBaseW = 8 + kModeW;
   const int lane = threadIdx.x & 63;
   const int K = a.K;
-  const int me = tg.me, stride = tg.stride, multiset = tg.multiset;
-  const uint64_t* cg_l = tl.cg;
-  const int* lo_l = tl.lo;
+  const int stride = tg.stride, multiset = tg.multiset;
   const TupleWordT<SUF>* tuples = static_cast<const TupleWordT<SUF>*>(tg.tuples);
   const uint32_t C0 = (uint32_t)tg.cg[(SUF - 1) * stride];
   if (g >= a.S) return;
@@ -528,61 +592,7 @@ __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTab
   }
   while (g < g_end) {
     if (r >= a.S_pre) break;  // cannot happen while g < S; keeps the loop bounded regardless
-    // ---- lane i: data of the block of prefix r + i, into column i of the table ----
-    {
-      BlockInfo bi;
-      Streams<MAXD> st;
-      int q[MAXD];
-      const uint64_t ri = r + (uint64_t)lane;
-      const SpaceView sv{cg_l, lo_l, me, stride};
-      if (ri < a.S_pre) {
-        sv.unrank(ri, d, q);
-        block_info<MAXD, SUF>(tl, K, d, q, bi, st);
-      } else {
-        bi.L = 0;
-        bi.CB = bi.LBp = 0;
-        bi.toff = 0;
-        bi.lo = 0;
-        bi.skip0 = 0;
-        bi.lastrun = 0;
-        bi.fQ = 1.f;
-#pragma unroll
-        for (int s = 0; s < MAXD; ++s) {
-          st.base[s] = 0;
-          st.mode[s] = kNoEdgeRow;
-          st.active[s] = false;
-        }
-      }
-      wave_sync();  // every lane is done reading the previous batch
-      uint32_t* col = tbl + lane;
-      col[0 * kBlockBatch] = (uint32_t)bi.CB;
-      col[1 * kBlockBatch] = (uint32_t)(bi.CB >> 32);
-      col[2 * kBlockBatch] = (uint32_t)bi.LBp;
-      col[3 * kBlockBatch] = (uint32_t)(bi.LBp >> 32);
-      col[4 * kBlockBatch] = bi.L;
-      col[5 * kBlockBatch] = bi.toff;
-      // active slots compacted to the front in ascending prefix position (the summation order of
-      // the thread-per-state kernel); slots past the active count carry slot 0's base and no edge
-#pragma unroll
-      for (int w = 0; w < kModeW; ++w) col[(8 + w) * kBlockBatch] = kNoEdgeRow * 0x01010101u;
-#pragma unroll
-      for (int t = 0; t < MAXD; ++t) {
-        col[(kBaseW + 2 * t) * kBlockBatch] = (uint32_t)st.base[0];
-        col[(kBaseW + 2 * t + 1) * kBlockBatch] = (uint32_t)(st.base[0] >> 32);
-      }
-      uint32_t nact = 0;
-#pragma unroll
-      for (int s = 0; s < MAXD; ++s)
-        if (st.active[s]) {
-          reinterpret_cast<uint8_t*>(col + (8 + (nact >> 2)) * kBlockBatch)[nact & 3u] = (uint8_t)st.mode[s];
-          col[(kBaseW + 2 * nact) * kBlockBatch] = (uint32_t)st.base[s];
-          col[(kBaseW + 2 * nact + 1) * kBlockBatch] = (uint32_t)(st.base[s] >> 32);
-          ++nact;
-        }
-      col[6 * kBlockBatch] = (uint32_t)bi.lo | ((uint32_t)bi.skip0 << 8) | ((uint32_t)bi.lastrun << 16) | (nact << 24);
-      col[7 * kBlockBatch] = __builtin_bit_cast(uint32_t, bi.fQ);
-      wave_sync();
-    }
+    fill_block_table<MAXD, SUF>(tl, K, d, r, a.S_pre, tbl, lane);
     const int nb = (int)((a.S_pre - r < kBlockBatch) ? a.S_pre - r : kBlockBatch);
     for (int j = 0; j < nb && g < g_end; ++j) {
       const uint32_t* bj = tbl + j;

@@ -128,37 +128,35 @@ SLOS_HD void unrank_fixed(const SV& sv, RankT<SV> g, int K, int (&p)[KM]) {
   }
 }
 
-// the parents of the K-tuple p (K <= KM), as for_each_parent
+// The parents of the K-tuple p (K <= KM), as for_each_parent. With the counting recurrence
+// cg[r][x] = cg[r][x+1] + cg[r-1][lo[x]] the rank of an N-tuple telescopes, for every mask, to
+//   cg[N][0] - sum_{i <= N-2} cg[N-i][p_i + 1] - cg[1][p_(N-1)],
+// so a child needs two table entries a position: its own terms X (the positions after a dropped one
+// keep theirs) and the terms Y of the positions before a dropped one, which have one photon fewer.
 template <int KM, class SV, class F>
 SLOS_HD void parents_fixed(const SV& sv, int multiset, int K, const int (&p)[KM], F&& f) {
   typedef RankT<SV> R;
-  int lop[KM + 1];
-  R suf[KM + 2];
+  R Y[KM], SX[KM + 1];  // SX[i]: X_i + ... + X_(K-1)
   int run[KM];
-  lop[0] = 0;
-#pragma unroll
-  for (int i = 0; i < KM; ++i) lop[i + 1] = i < K ? sv.lo[p[i]] : 0;
-  suf[KM] = 0;
-  suf[KM + 1] = 0;
+  SX[KM] = 0;
 #pragma unroll
   for (int i = KM - 1; i >= 0; --i) {
-    suf[i] = i < K ? suf[i + 1] + (sv.C(K - i, lop[i]) - sv.C(K - i, p[i])) : R(0);
+    SX[i] = 0;
+    Y[i] = 0;
+    if (i < K) {
+      SX[i] = SX[i + 1] + (i == K - 1 ? sv.C(1, p[i]) : sv.C(K - i, p[i] + 1));
+      if (i < K - 1) Y[i] = i == K - 2 ? sv.C(1, p[i]) : sv.C(K - 1 - i, p[i] + 1);
+    }
     // copies of p[i] from i on (the count of a mode's first copy)
     const bool same = i + 1 < K && p[in_range<KM>(i + 1)] == p[i];
     run[i] = same ? run[in_range<KM>(i + 1)] + 1 : 1;
   }
-  R pre = 0;
+  R rest = K == 1 ? SX[1] : sv.C(K - 1, 0);  // cg[K-1][0] less the Y before l
 #pragma unroll
   for (int l = 0; l < KM; ++l) {
     if (l < K) {
-      if (!multiset || l == 0 || p[l] != p[in_range<KM>(l - 1)]) {
-        const int cnt = multiset ? run[l] : 1;
-        const R pr =
-            (l == K - 1) ? pre
-                         : pre + (sv.C(K - l - 1, lop[l]) - sv.C(K - l - 1, p[in_range<KM>(l + 1)])) + suf[l + 2];
-        f(pr, p[l], cnt);
-      }
-      if (l < K - 1) pre += sv.C(K - l - 1, lop[l]) - sv.C(K - l - 1, p[l]);
+      if (!multiset || l == 0 || p[l] != p[in_range<KM>(l - 1)]) f(rest - SX[l + 1], p[l], multiset ? run[l] : 1);
+      rest -= Y[l];
     }
   }
 }

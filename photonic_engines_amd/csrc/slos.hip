@@ -23,6 +23,7 @@
 #include "layer_block.hpp"
 #include "descend_block.hpp"
 #include "layer_f64.hpp"
+#include "layer_simple.hpp"
 #include "pull_index.hpp"
 #include "block_launch.hpp"
 #include "front.hpp"
@@ -56,6 +57,14 @@ struct DevTables {
   uint64_t* tuples5 = nullptr;             // the same for 5-position suffixes (may be absent)
   uint4* items[33] = {};                   // group-order work items of layer K (may be absent)
   uint32_t n_items[33] = {};
+  uint4* fine[33] = {};                    // the same in small items (may be absent)
+  uint32_t n_fine[33] = {};
+  // the items for a launch of `states` states in all
+  std::pair<const uint4*, uint32_t> group_items(int K, uint64_t states) const {
+    return fine[K] && states < kFineItems ? std::make_pair((const uint4*)fine[K], n_fine[K])
+                                          : std::make_pair((const uint4*)items[K], n_items[K]);
+  }
+  static constexpr uint64_t kFineItems = 1ull << 23;
 };
 
 struct slos_plan {
@@ -67,6 +76,7 @@ struct slos_plan {
   std::vector<slos::TupleWord> tuples;   // suffix-tuple words of the block kernel (empty: unused)
   std::vector<uint64_t> tuples5;         // 5-position suffix-tuple words (empty: unused)
   std::vector<uint32_t> items[33];       // group-order work items of layer K, 4 words each (empty: unused)
+  std::vector<uint32_t> fine[33];        // the same in small items, for layers of fewer than kFineItems states
   std::vector<DevTables> dev;
   std::mutex mu;
   slos::SpaceView host_view() const { return slos::SpaceView{cg.data(), lo.data(), me, me + 1}; }
@@ -135,121 +145,15 @@ int device_tables(const slos_plan* cp, DevTables* out) {
       HIP_TRY(hipMalloc(&t.items[K], p->items[K].size() * sizeof(uint32_t)));
       HIP_TRY(hipMemcpy(t.items[K], p->items[K].data(), p->items[K].size() * sizeof(uint32_t), hipMemcpyHostToDevice));
       t.n_items[K] = (uint32_t)(p->items[K].size() / 4);
+      if (!p->fine[K].empty()) {
+        HIP_TRY(hipMalloc(&t.fine[K], p->fine[K].size() * sizeof(uint32_t)));
+        HIP_TRY(hipMemcpy(t.fine[K], p->fine[K].data(), p->fine[K].size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        t.n_fine[K] = (uint32_t)(p->fine[K].size() / 4);
+      }
     }
   p->dev.push_back(t);
   *out = t;
   return SLOS_OK;
-}
-
-// ------------------------------------------------------------------------------------------
-// thread-per-state layer kernel: unrank, parent ranks by prefix/suffix sums, gather-MAC
-// ------------------------------------------------------------------------------------------
-
-struct Acc {
-  float re = 0.f, im = 0.f, cre = 0.f, cim = 0.f;
-};
-
-// (compensated arithmetic: no contraction, see bk_two_sum)
-__device__ __forceinline__ void two_sum(float& s, float& c, float x) {
-#pragma clang fp contract(off)
-  const float t = s + x;
-  const float bp = t - s;
-  c += (s - (t - bp)) + (x - bp);
-  s = t;
-}
-
-// acc += u * v, plain or compensated (product errors by fma, sums by two-sum)
-template <bool COMP>
-__device__ __forceinline__ void cmac(Acc& a, float2 u, float2 v) {
-  if constexpr (!COMP) {
-    a.re = fmaf(u.x, v.x, a.re);
-    a.re = fmaf(-u.y, v.y, a.re);
-    a.im = fmaf(u.x, v.y, a.im);
-    a.im = fmaf(u.y, v.x, a.im);
-  } else {
-#pragma clang fp contract(off)
-    float p, e;
-    p = u.x * v.x; e = fmaf(u.x, v.x, -p); two_sum(a.re, a.cre, p); a.cre += e;
-    p = -u.y * v.y; e = fmaf(-u.y, v.y, -p); two_sum(a.re, a.cre, p); a.cre += e;
-    p = u.x * v.y; e = fmaf(u.x, v.y, -p); two_sum(a.im, a.cim, p); a.cim += e;
-    p = u.y * v.x; e = fmaf(u.y, v.x, -p); two_sum(a.im, a.cim, p); a.cim += e;
-  }
-}
-
-struct LayerArgs {
-  const uint64_t* cg;
-  const int* lo;
-  int me, multiset, K, m, col;
-  const float2* U;        // [B][m][m]
-  const int32_t* cols;    // unused by the simple kernel
-  const float2* par;      // [B][S_par]
-  uint64_t S_par;
-  void* out;              // [B][S]
-  uint64_t S;
-  int64_t B;
-  float scale;
-  unsigned flags;
-  int64_t par_lo, out_lo;  // compensated sums: element offsets of the low-order parts (0: none)
-};
-
-// KIND 0: intermediate layer (complex64), 1: probabilities (float32), 2: scaled amplitudes
-// (K <= KM: the per-state position arrays stay in registers)
-template <int KIND, bool COMP, int KM>
-__global__ __launch_bounds__(256) void k_layer_simple(LayerArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int stride = a.me + 1;
-  const int ncg = (a.K + 1) * stride;
-  uint64_t* cg = reinterpret_cast<uint64_t*>(smem);
-  int* lo = reinterpret_cast<int*>(cg + ncg);
-  float2* ucol = reinterpret_cast<float2*>(smem + ((ncg * 8 + a.me * 4 + 15) & ~15));
-  for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = a.cg[i];
-  for (int i = threadIdx.x; i < a.me; i += blockDim.x) lo[i] = a.lo[i];
-  const slos::SpaceView sv{cg, lo, a.me, stride};
-  const int K = a.K;
-  for (int64_t b = blockIdx.y; b < a.B; b += gridDim.y) {
-    __syncthreads();
-    for (int j = threadIdx.x; j < a.m; j += blockDim.x)
-      ucol[j] = a.U[(size_t)b * a.m * a.m + (size_t)j * a.m + a.col];
-    __syncthreads();
-    const float2* pb = a.par + (size_t)b * a.S_par;
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < a.S;
-         g += (uint64_t)gridDim.x * blockDim.x) {
-      int p[KM];
-      slos::unrank_fixed<KM>(sv, g, K, p);
-      Acc acc;
-      slos::parents_fixed<KM>(sv, a.multiset, K, p,
-                              [&](uint64_t pr, int mode, int) { cmac<COMP>(acc, ucol[mode], pb[pr]); });
-      if constexpr (COMP) {
-        if (a.par_lo)  // the parents' low-order parts, into the correction terms
-          slos::parents_fixed<KM>(sv, a.multiset, K, p, [&](uint64_t pr, int mode, int) {
-            const float2 u = ucol[mode], w = pb[a.par_lo + pr];
-            acc.cre = fmaf(u.x, w.x, acc.cre);
-            acc.cre = fmaf(-u.y, w.y, acc.cre);
-            acc.cim = fmaf(u.x, w.y, acc.cim);
-            acc.cim = fmaf(u.y, w.x, acc.cim);
-          });
-      }
-      float re = COMP ? acc.re + acc.cre : acc.re, im = COMP ? acc.im + acc.cim : acc.im;
-      if constexpr (KIND == 0) {
-        reinterpret_cast<float2*>(a.out)[(size_t)b * a.S + g] = make_float2(re, im);
-        if constexpr (COMP) {
-          if (a.out_lo)  // the rounding error of the stored value (fast two-sum)
-            reinterpret_cast<float2*>(a.out)[a.out_lo + (size_t)b * a.S + g] =
-                make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
-        }
-      } else {
-        const float f = slos::run_factorial_fixed<KM>(p, K, a.multiset);
-        re *= a.scale;
-        im *= a.scale;
-        if constexpr (KIND == 1) {
-          reinterpret_cast<float*>(a.out)[(size_t)b * a.S + g] = slos::prob_readout(re, im, f);
-        } else {
-          const float s = (a.flags & SLOS_FLAG_IMMEDIATE) ? sqrtf(f) : 1.f;
-          reinterpret_cast<float2*>(a.out)[(size_t)b * a.S + g] = make_float2(re * s, im * s);
-        }
-      }
-    }
-  }
 }
 
 __global__ void k_fill_ones(float2* p, int64_t n) {
@@ -541,9 +445,9 @@ __global__ __launch_bounds__(256) void k_readout_adjoint_pull(const uint64_t* cg
         }
         const float2* ub = U + (size_t)b * m * m;
         const float2* pb = par + (size_t)b * S_par;
-        Acc acc;
+        slos::Acc acc;
         slos::parents_fixed<KM>(sv, multiset, K, p,
-                                [&](uint64_t pr, int mode, int) { cmac<false>(acc, ub[(size_t)mode * m + col], pb[pr]); });
+                                [&](uint64_t pr, int mode, int) { slos::cmac<false>(acc, ub[(size_t)mode * m + col], pb[pr]); });
         const float w = 2.f * s2 * f * gv;
         r = make_float2(w * acc.re, w * acc.im);
       }
@@ -642,6 +546,23 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
   return (dt.tuples5 && K - 5 >= 1 && K - 5 <= 8 && block_lds_fit(K, p->me, 5)) ? 5 : slos::kSuf;
 }
 
+// Whether layer K (S states, B rows) runs on the block or group-order kernel rather than one thread a
+// state, where both can. The block kernels share index work between states but wait on their own
+// set-up, and a block must be long enough to fill waves; the two give the same bits. Measured (us, block
+// or group order against thread):
+//   group order: 347k states 21 / 14, 2.0M 28 / 29, 7.9M 56 / 94; compensated 490k 44 / 17;
+//   blocks, multiset: 98k states 18.4 / 13.8, 475k 18.9 / 14.9, 2.3M (72,000 a block) 33 / 30, 9.3M (3,400 a
+//   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
+//   blocks, collision-free: 126k 41 / 15, 3.1M (209 a block) 101 / 55, 2.0M (4,680 a block) 39 / 32, 54.6M
+//   (92 a block) 1266 / 898, 7.6M (119,000 a block) 57 / 118.
+// The thread kernel's exact forms are those of at most 12 photons and 2^32 states.
+bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B) {
+  if (K > 12 || S >= (1ull << 32)) return true;
+  if (S * (uint64_t)B < (1ull << 21)) return false;
+  if (suf == 5 && !p->items[K].empty()) return true;
+  return S >= (p->multiset ? 256 : 8192) * p->size(K - suf);
+}
+
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
 // there is one for every XCD and the grid's thread count stays below 2^32, else a row per grid y.
 dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
@@ -651,7 +572,7 @@ dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
   return flat ? dim3((unsigned)(wgs * (uint64_t)B)) : dim3((unsigned)wgs, (unsigned)B);
 }
 
-int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, int kind, bool comp, hipStream_t st) {
+int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs& a, int kind, bool comp, hipStream_t st) {
   slos::BlockLayer L;
   L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.S_par = a.S_par; L.S = a.S;
   L.par_lo = a.par_lo; L.out_lo = a.out_lo;
@@ -673,8 +594,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const LayerArgs& a, in
   // complex64)
   const bool grp_last = kind == 1;
   if (suf == 5 && kind <= 1 && dt.items[a.K]) {
-    const uint4* gitems = dt.items[a.K];
-    const uint32_t gn = dt.n_items[a.K];
+    const auto [gitems, gn] = dt.group_items(a.K, a.S * (uint64_t)a.B);
     const size_t shg = slos::group_dyn_lds(a.K, p->me);
     const uint64_t gwgs = ((uint64_t)gn + slos::kWaves - 1) / slos::kWaves;
     if (shg + slos::kBlockStaticLds <= lds_limit() && gwgs <= 0x7fffffffull) {
@@ -710,29 +630,61 @@ void with_km(int photons, F&& f) {
 int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const float2* U, int64_t B,
                  const float2* par, uint64_t S_par, void* out, uint64_t S, int kind, float scale,
                  unsigned flags, hipStream_t st, bool par_hilo = false, bool out_hilo = false) {
-  LayerArgs a;
+  slos::LayerArgs a;
   a.cg = dt.cg; a.lo = dt.lo; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
-  a.U = U; a.cols = nullptr; a.par = par; a.S_par = S_par; a.out = out; a.S = S; a.B = B;
+  a.U = U; a.words = dt.tuples5; a.par = par; a.S_par = S_par; a.out = out; a.S = S; a.B = B;
   a.scale = scale; a.flags = flags;
   const bool comp = flags & SLOS_FLAG_COMPENSATED;
   a.par_lo = (comp && par_hilo) ? B * (int64_t)S_par : 0;
   a.out_lo = (comp && out_hilo && kind == 0) ? B * (int64_t)S : 0;
   if (!(flags & SLOS_FLAG_SIMPLE) && dt.tuples && K > slos::kSuf && K - slos::kSuf <= 16 &&
-      block_lds_fit(K, p->me, slos::kSuf))
+      block_lds_fit(K, p->me, slos::kSuf) && use_blocks(p, K, block_suffix(p, dt, K), S, B))
     return launch_block(p, dt, a, kind, comp, st);
   const size_t sh = (((size_t)(K + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8;
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
   const uint64_t blocks = std::min<uint64_t>((S + 255) / 256, 1u << 20);
   dim3 grid((unsigned)std::max<uint64_t>(blocks, 1), (unsigned)std::min<int64_t>(B, 65535));
-  with_km(K, [&](auto km) {
-    constexpr int KM = decltype(km)::value;
-    if (kind == 0 && !comp) hipLaunchKernelGGL((k_layer_simple<0, false, KM>), grid, dim3(256), sh, st, a);
-    else if (kind == 0) hipLaunchKernelGGL((k_layer_simple<0, true, KM>), grid, dim3(256), sh, st, a);
-    else if (kind == 1 && !comp) hipLaunchKernelGGL((k_layer_simple<1, false, KM>), grid, dim3(256), sh, st, a);
-    else if (kind == 1) hipLaunchKernelGGL((k_layer_simple<1, true, KM>), grid, dim3(256), sh, st, a);
-    else if (!comp) hipLaunchKernelGGL((k_layer_simple<2, false, KM>), grid, dim3(256), sh, st, a);
-    else hipLaunchKernelGGL((k_layer_simple<2, true, KM>), grid, dim3(256), sh, st, a);
-  });
+  slos::launch_layer_simple(kind, comp, grid, sh, st, a);
+  HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+// one complex128 layer on the block or group-order kernel; -1 where they do not apply (layers of
+// fewer than 5 photons, prefixes of more than 8 positions, spaces without tuple words)
+int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, int64_t B, const void* par,
+                     uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
+  if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
+  const int suf = dt.tuples5 && K > 5 ? 5 : slos::kSuf;
+  const int d = K - suf;
+  if (d > 8 || !use_blocks(p, K, suf, S, B)) return -1;
+  slos::BlockLayerF64 L{};
+  L.l.K = K; L.l.m = p->m; L.l.col = col; L.l.S_par = S_par; L.l.S = S; L.l.S_pre = p->size(d);
+  L.l.flags = flags;
+  L.U = static_cast<const double2*>(U);
+  L.scale = scale;
+  if (suf == 5 && kind <= 1 && dt.items[K]) {
+    const size_t sh = slos::group_dyn_lds64(K, p->me);
+    const auto [items, n_items] = dt.group_items(K, S * (uint64_t)B);
+    const uint64_t wgs = ((uint64_t)n_items + slos::kWaves - 1) / slos::kWaves;
+    if (sh + slos::kBlockStaticLds64 <= lds_limit() && wgs <= 0x7fffffffull) {
+      L.l.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
+      const slos::BlockGrid bg{batch_grid(wgs, B, &L.l), sh, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
+      slos::launch_layer_group_f64(d, kind, bg, static_cast<const double2*>(par), out, L, items, n_items);
+      HIP_TRY(hipGetLastError());
+      return SLOS_OK;
+    }
+  }
+  const size_t sh = slos::block_dyn_lds(K, p->me, slos::block_maxd_f64(d));
+  if (sh + slos::kBlockStaticLds64 > lds_limit()) return -1;
+  // children per wave as the complex64 block kernel
+  const uint64_t pw = (S / 16384 + 63) & ~63ull;
+  L.l.per_wave = std::min<uint64_t>(std::max<uint64_t>(pw, 256), kind == 0 ? 2048 : 4096);
+  L.l.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * L.l.per_wave));
+  const uint64_t wgs = ((S + L.l.per_wave - 1) / L.l.per_wave + slos::kWaves - 1) / slos::kWaves;
+  if (wgs > 0x7fffffffull) return -1;
+  const slos::BlockGrid bg{batch_grid(wgs, B, &L.l), sh, st, dt.cg, dt.lo,
+                           suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
+  slos::launch_layer_block_f64(kind, d, suf, bg, static_cast<const double2*>(par), out, L);
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
 }
@@ -741,8 +693,12 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
 // 2 scaled complex128 amplitudes (SLOS_FLAG_IMMEDIATE: times sqrt(prod t!))
 int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, int64_t B, const void* par,
                      uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
+  if (!(flags & SLOS_FLAG_SIMPLE)) {
+    const int rc = launch_block_f64(p, dt, K, col, U, B, par, S_par, out, S, kind, scale, flags, st);
+    if (rc >= 0) return rc;
+  }
   slos::LayerArgsF64 a;
-  a.cg = dt.cg; a.lo = dt.lo; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
+  a.cg = dt.cg; a.lo = dt.lo; a.words = dt.tuples5; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
   a.U = static_cast<const double2*>(U); a.par = static_cast<const double2*>(par); a.S_par = S_par;
   a.out = out; a.S = S; a.B = B; a.scale = scale;
   a.immediate = (flags & SLOS_FLAG_IMMEDIATE) ? 1u : 0u;
@@ -750,14 +706,7 @@ int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
   const uint64_t blocks = std::min<uint64_t>((S + 255) / 256, 1u << 20);
   dim3 grid((unsigned)std::max<uint64_t>(blocks, 1), (unsigned)std::min<int64_t>(B, 65535));
-#define SLOS_F64L(KM)                                                                         \
-  if (kind == 0) hipLaunchKernelGGL((slos::k_layer_f64<0, KM>), grid, dim3(256), sh, st, a);  \
-  else if (kind == 1) hipLaunchKernelGGL((slos::k_layer_f64<1, KM>), grid, dim3(256), sh, st, a); \
-  else hipLaunchKernelGGL((slos::k_layer_f64<2, KM>), grid, dim3(256), sh, st, a)
-  if (K <= 8) { SLOS_F64L(8); }
-  else if (K <= 16) { SLOS_F64L(16); }
-  else { SLOS_F64L(32); }
-#undef SLOS_F64L
+  slos::launch_layer_f64_simple(kind, grid, sh, st, a);
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
 }
@@ -1024,9 +973,9 @@ __global__ __launch_bounds__(256) void k_layer_simple_group(slos::GroupLaunch gl
       if (g >= it.S) break;
       int pos[KM];
       slos::unrank_fixed<KM>(sv, g, K, pos);
-      Acc acc;
+      slos::Acc acc;
       slos::parents_fixed<KM>(sv, it.multiset, K, pos,
-                              [&](uint64_t pr, int mode, int) { cmac<COMP>(acc, ucol[mode], pb[pr]); });
+                              [&](uint64_t pr, int mode, int) { slos::cmac<COMP>(acc, ucol[mode], pb[pr]); });
       if constexpr (COMP) {
         if (it.par_lo)  // the parents' low-order parts, into the correction terms
           slos::parents_fixed<KM>(sv, it.multiset, K, pos, [&](uint64_t pr, int mode, int) {
@@ -1297,7 +1246,11 @@ void build_tuples(slos_plan* p) {
     for (int K = 7; K <= p->n && K <= 11; ++K)
       if (p->multiset && p->size(K - 6) <= 0xffffffffull &&
           p->size(K) / slos::kGroupItemChildren + p->size(K - 6) <= (32u << 20))
+      {
         slos::group_items(sv, K, p->items[K]);
+        if (p->size(K) < DevTables::kFineItems)
+          slos::group_items(sv, K, p->fine[K], slos::kGroupFineChildren, slos::kGroupFineWidth);
+      }
   }
 }
 
@@ -1397,6 +1350,8 @@ int slos_plan_destroy(slos_plan* p) {
     if (t.tuples) (void)hipFree(t.tuples);
     if (t.tuples5) (void)hipFree(t.tuples5);
     for (auto* it : t.items)
+      if (it) (void)hipFree(it);
+    for (auto* it : t.fine)
       if (it) (void)hipFree(it);
   }
   (void)hipSetDevice(cur);
