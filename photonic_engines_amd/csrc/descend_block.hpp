@@ -1,6 +1,6 @@
 // Block-structured pull over children for one step of the uniform-loss recurrence
 // (photonic_engines/imperfections.py:254-276): q_{K-1}(t) = sum_a q_K(t + e_a) (t_a + 1) / K, for
-// multiset spaces (lo[x] = x). The index arithmetic (segment bases, tail offsets) is in
+// multiset spaces (lo[x] = x) without an insert table (child_walk.hpp). The index arithmetic (segment bases, tail offsets) is in
 // block_index.hpp.
 //
 // Work split, as in the forward block kernel: a wave owns a contiguous range of parents of layer

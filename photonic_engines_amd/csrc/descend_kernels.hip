@@ -1,9 +1,29 @@
 // k_descend_block and k_adjoint_block (descend_block.hpp).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "block_launch.hpp"
 
 namespace slos {
+
+namespace {
+
+template <class F>
+void with_prefix(int dp, F&& f) {
+  switch (dp) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 3: f(std::integral_constant<int, 3>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    case 5: f(std::integral_constant<int, 5>()); break;
+    case 6: f(std::integral_constant<int, 6>()); break;
+    case 7: f(std::integral_constant<int, 7>()); break;
+    default: f(std::integral_constant<int, 8>()); break;
+  }
+}
+
+}  // namespace
 
 void launch_descend_block(int maxd, const BlockGrid& g, int K, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
                           uint64_t S_pre, uint64_t per_wave, float scale, uint32_t xcd_chunk) {
@@ -22,6 +42,14 @@ void launch_descend_block(int maxd, const BlockGrid& g, int K, const float* qk, 
   else SLOS_DESC_E(8);
 #undef SLOS_DESC_E
 #undef SLOS_DESC
+}
+
+void launch_descend_insert(int dp, const BlockGrid& g, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
+                           uint64_t per_wave, float scale, uint32_t xcd_chunk, const uint32_t* ins) {
+  with_prefix(dp, [&](auto d) {
+    hipLaunchKernelGGL((k_descend_insert<decltype(d)::value>), g.grid, dim3(kBlockThreads), 0, g.st, g.cg, ins, g.me,
+                       qk, Sk, qout, Sp, per_wave, scale, xcd_chunk);
+  });
 }
 
 void launch_adjoint_block(int maxd, const BlockGrid& g, int K, int m, int col, const float2* U, const float2* psi,

@@ -55,6 +55,7 @@ struct DevTables {
   int* modes = nullptr;                    // the plan's input modes (spot permanents)
   slos::TupleWord* tuples = nullptr;       // block-kernel suffix-tuple words (may be absent)
   uint64_t* tuples5 = nullptr;             // the same for 5-position suffixes (may be absent)
+  uint32_t* insert = nullptr;              // insert table of the pulls over children (see insert_table)
   uint4* items[33] = {};                   // group-order work items of layer K (may be absent)
   uint32_t n_items[33] = {};
   uint4* fine[33] = {};                    // the same in small items (may be absent)
@@ -113,6 +114,11 @@ size_t lds_limit() {
   return lim;
 }
 
+__global__ void k_insert_table(const uint64_t* cg, const slos::TupleWord* tuples, int me, uint32_t n4, uint32_t* ins) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n4 * (uint32_t)me; i += gridDim.x * blockDim.x)
+    ins[i] = slos::insert_word(cg, me + 1, tuples[i % n4], (int)(i / n4));
+}
+
 int device_tables(const slos_plan* cp, DevTables* out) {
   slos_plan* p = const_cast<slos_plan*>(cp);
   int d = 0;
@@ -153,6 +159,40 @@ int device_tables(const slos_plan* cp, DevTables* out) {
     }
   p->dev.push_back(t);
   *out = t;
+  return SLOS_OK;
+}
+
+// The plan's insert table on the current GPU, built by the first pull over children that asks for it
+// (1.7 MB and about 50 us at 24 modes); null where the space has none, or while `st` is captured and
+// it is not there yet (nothing is allocated inside a capture).
+int insert_table(const slos_plan* cp, hipStream_t st, const uint32_t** out) {
+  slos_plan* p = const_cast<slos_plan*>(cp);
+  *out = nullptr;
+  const uint64_t n4 = p->tuples.size(), words = n4 * (uint64_t)p->me;
+  if (!p->multiset || !n4 || p->n <= 5 || p->size(5) > slos::kInsertTuples || words > slos::kInsertWords) return SLOS_OK;
+  int d = 0;
+  HIP_TRY(hipGetDevice(&d));
+  std::lock_guard<std::mutex> g(p->mu);
+  for (auto& t : p->dev)
+    if (t.device == d) {
+      if (!t.insert) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cap));
+        if (cap != hipStreamCaptureStatusNone) return SLOS_OK;
+        uint32_t* ins = nullptr;
+        HIP_TRY(hipMalloc(&ins, words * sizeof(uint32_t)));
+        hipLaunchKernelGGL(k_insert_table, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, t.cg, t.tuples, p->me,
+                           (uint32_t)n4, ins);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(st);  // other streams may read it from here on
+        if (e != hipSuccess) {
+          (void)hipFree(ins);
+          HIP_TRY(e);
+        }
+        t.insert = ins;
+      }
+      *out = t.insert;
+    }
   return SLOS_OK;
 }
 
@@ -1349,6 +1389,7 @@ int slos_plan_destroy(slos_plan* p) {
     (void)hipFree(t.modes);
     if (t.tuples) (void)hipFree(t.tuples);
     if (t.tuples5) (void)hipFree(t.tuples5);
+    if (t.insert) (void)hipFree(t.insert);
     for (auto* it : t.items)
       if (it) (void)hipFree(it);
     for (auto* it : t.fine)
@@ -1805,6 +1846,26 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   return SLOS_OK;
 }
 
+namespace {
+
+// Whether a pull over children takes the insert-table kernel, for a parent layer of Sp states in
+// S_pre blocks. Below, the thread-per-state kernel is the faster one: a wave of the walk spends a
+// fixed part of its time on each block, and on a small layer its few blocks run one after another.
+// Descents, us, walk / thread per state: 1.3M parents in blocks of 84 on average 69 / 84, 7.7M of 45
+// 286 / 388, 705k of 22 74 / 45, 490k of 126 39 / 36, 203k of 85 34 / 26, 658k of 427 37 / 47, 98k of
+// 4095 18 / 27, 200 rows of 12k in blocks of 159 49 / 105.
+bool insert_walk(uint64_t Sp, uint64_t S_pre, int64_t batch) {
+  const uint64_t block = Sp / S_pre;
+  return block >= 256 || (block >= 32 && Sp >= (1ull << 20) / (uint64_t)batch);
+}
+
+// Parents per wave of the insert-table kernels: few, so that the waves in flight read near one
+// another (descents, us, with 64 / 128 / 256 / 512: 2.0M parents 57 / 65 / 73 / 93, 7.9M 157 / 147 /
+// 157 / 202, 28M 588 / 467 / 460 / 555, 1.1G - / 20500 / 19100 / 19800).
+uint64_t insert_per_wave(uint64_t Sp) { return Sp < (1ull << 22) ? 64 : Sp < (1ull << 24) ? 128 : 256; }
+
+}  // namespace
+
 int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1, int64_t batch, unsigned flags,
                       double scale, slos_stream_t stream) {
   if (!p || !q_k || !q_km1) return fail(SLOS_EINVAL, "NULL argument");
@@ -1818,25 +1879,39 @@ int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1,
   char name[32];
   std::snprintf(name, sizeof name, "slos descent %d", k);
   const RoctxRange range(name);
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!(flags & SLOS_FLAG_SIMPLE) && p->multiset && dt.tuples && dp >= 1 && dp <= 8) {
-    const int maxd = dp <= 4 ? 4 : dp <= 6 ? 6 : 8;
-    const size_t shb = slos::desc_dyn_lds(k, p->me, maxd);
-    if (shb <= lds_limit()) {
-      // parents per wave: 1024 on layers of 2^27 parents or more, 512 below, fewer on small layers;
-      // XCD chunks of 2^16 parents (measured at n = 11, m = 32: the k = 11, 10, 9 steps 34.4, 9.0,
-      // 2.5 ms with 4096 per wave and chunks of 2^18, 32.6, 8.1, 2.0 ms so)
-      uint64_t pw = (Sp / 16384 + 63) & ~63ull;
-      pw = std::min<uint64_t>(std::max<uint64_t>(pw, 256), Sp >= (1ull << 27) ? 1024 : 512);
-      const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
-      if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
-      const dim3 grid((unsigned)wgs, (unsigned)batch);
-      const uint32_t xc = (uint32_t)std::max<uint64_t>(1, (1ull << 16) / ((uint64_t)slos::kWaves * pw));
-      const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-      const uint64_t S_pre = p->size(dp);
-      const slos::BlockGrid bg{grid, shb, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
-      slos::launch_descend_block(maxd, bg, k, q_k, Sk, q_km1, Sp, S_pre, pw, (float)scale, xc);
-      HIP_TRY(hipGetLastError());
-      return SLOS_OK;
+    const uint64_t S_pre = p->size(dp);
+    const uint32_t* ins = nullptr;
+    rc = insert_table(p, st, &ins);
+    if (rc) return rc;
+    if (ins) {
+      if (insert_walk(Sp, S_pre, batch)) {
+        const uint64_t pw = insert_per_wave(Sp);
+        const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
+        if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
+        const slos::BlockGrid bg{dim3((unsigned)wgs, (unsigned)batch), 0, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+        const uint32_t xc = (uint32_t)((1ull << 16) / ((uint64_t)slos::kWaves * pw));
+        slos::launch_descend_insert(dp, bg, q_k, Sk, q_km1, Sp, pw, (float)scale, xc, ins);
+        HIP_TRY(hipGetLastError());
+        return SLOS_OK;
+      }
+    } else {
+      const int maxd = dp <= 4 ? 4 : dp <= 6 ? 6 : 8;
+      const size_t shb = slos::desc_dyn_lds(k, p->me, maxd);
+      if (shb <= lds_limit()) {
+        // more than 41 modes, or no table yet. Parents per wave: 1024 on layers of 2^27 parents or more, 512 below,
+        // fewer on small layers; XCD chunks of 2^16 parents
+        uint64_t pw = (Sp / 16384 + 63) & ~63ull;
+        pw = std::min<uint64_t>(std::max<uint64_t>(pw, 256), Sp >= (1ull << 27) ? 1024 : 512);
+        const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
+        if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
+        const uint32_t xc = (uint32_t)std::max<uint64_t>(1, (1ull << 16) / ((uint64_t)slos::kWaves * pw));
+        const slos::BlockGrid bg{dim3((unsigned)wgs, (unsigned)batch), shb, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+        slos::launch_descend_block(maxd, bg, k, q_k, Sk, q_km1, Sp, S_pre, pw, (float)scale, xc);
+        HIP_TRY(hipGetLastError());
+        return SLOS_OK;
+      }
     }
   }
   const size_t sh = (size_t)(k + 1) * (p->me + 1) * 8 + (size_t)p->me * 4;

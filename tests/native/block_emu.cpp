@@ -499,6 +499,37 @@ int64_t emu_check_descend_block(int n, int m, int mask, int k, uint64_t first, u
   return bad;
 }
 
+// The children at and above last(P) of the same parents through the insert table's words, as the
+// device kernels use them, against slos::for_each_child (the modes below last(P) come first there).
+int64_t emu_check_insert(int n, int m, int mask, int k, uint64_t first, uint64_t count) {
+  constexpr int MAXD = 16;
+  Space s;
+  if (!build(n, m, mask, s) || !s.multiset || k - 1 < slos::kSuf + 1 || k > n || k - 1 - slos::kSuf > MAXD) return -1;
+  const int W = s.me + 1, D = k - 1, dp = D - slos::kSuf;
+  slos::SpaceView sv{s.cg.data(), s.lo.data(), s.me, W};
+  slos::BlockTables t{s.cg.data(), s.lo.data(), s.tuples.data(), s.me, W, s.multiset};
+  const uint64_t Sp = s.cg[(size_t)D * W], n5 = s.cg[(size_t)5 * W];
+  int64_t bad = 0;
+  for (uint64_t g = first; g < first + count && g < Sp; ++g) {
+    int q[MAXD];
+    const uint64_t u = slos::unrank_prefix<MAXD>(t, D, dp, g, q);
+    slos::DescBlock<MAXD> db;
+    slos::descend_block_info<MAXD>(t, k, dp, q, db);
+    const uint64_t tail = db.CB0 - (n5 - s.cg[(size_t)5 * W + db.lastP]);
+    std::vector<std::pair<uint64_t, int>> mine, ref;
+    for (int a = db.lastP; a < s.me; ++a) {
+      const uint32_t w = slos::insert_word(s.cg.data(), W, s.tuples[db.toff + u], a);
+      mine.push_back({tail + (w & slos::kInsertMask) / 4,
+                      (int)(w >> slos::kInsertShift) + (a == db.lastP ? db.lastrun : 0)});
+    }
+    slos::for_each_child(sv, s.multiset, k, g, [&](uint64_t r, int, int cnt) { ref.push_back({r, cnt}); });
+    if (ref.size() < mine.size()) { ++bad; continue; }
+    ref.erase(ref.begin(), ref.end() - (long)mine.size());
+    if (mine != ref) ++bad;
+  }
+  return bad;
+}
+
 // The block descent on a whole layer, in the device kernel's order of operations (float32 sums of
 // q * copies in ascending mode order, then times 1/k): out[t] for every parent t of layer k-1.
 int emu_descend_block(int n, int m, int mask, int k, const float* qk, float* out) {
