@@ -488,34 +488,40 @@ SLOS_HD int desc_tail_copies(const int (&s)[kSuf], int a, int lastP, int lastrun
   return 1 + (a == lastP ? lastrun : 0) + (s[0] == a) + (s[1] == a) + (s[2] == a) + (s[3] == a);
 }
 
-// The insert table of a multiset space: word a N4 + u for mode a and 4-tuple u (N4 of them) holds 4
-// times the index of the sorted 5-tuple (tuple u with a) in its low bits, and the copies of a in that
-// tuple in its top byte. A child of parent (P, u) with a mode a >= last(P) then lies at
+// The insert tables of a multiset space. First table: word a N4 + u for mode a and 4-tuple u (N4 of
+// them) holds 4 times the index of the sorted 5-tuple (tuple u with a) in its low bits, and the copies
+// of a in that tuple in its top byte. A child of parent (P, u) with a mode a >= last(P) then lies at
 //   CB0 - (N5 - cg[5][last(P)]) + index   (CB0: the first child with prefix P)
-// and holds the word's copies of a, and for a = last(P) those in P besides.
+// and holds the word's copies of a, and for a = last(P) those in P besides. Second table, behind it:
+// the same for the last kInsertModes modes alone (from X on): word (a - X) cg[5][X] + u, u a 5-tuple
+// of these modes, the index that of its 6-tuple among theirs.
 constexpr int kInsertShift = 24;
 constexpr uint32_t kInsertMask = (1u << kInsertShift) - 1u;
 constexpr uint64_t kInsertTuples = 4u << 20;  // 5-tuples the index field holds
-constexpr uint64_t kInsertWords = 4u << 20;   // largest table: 16 MB (41 modes)
-SLOS_HD uint32_t insert_word(const uint64_t* cg, int W, TupleWord w, int a) {
-  int t[5];
+constexpr uint64_t kInsertWords = 4u << 20;   // largest first table: 16 MB (41 modes)
+constexpr int kInsertModes = 8;
+SLOS_HD int insert_from(int me) { return me > kInsertModes ? me - kInsertModes : 0; }
+
+// the word of mode a and the sorted N-tuple t of modes >= from
+template <int N>
+SLOS_HD uint32_t insert_word(const uint64_t* cg, int W, const int (&t)[N], int a, int from) {
+  int c[N + 1];
   int n = 0, copies = 1;
   bool placed = false;
 #pragma unroll
-  for (int i = 0; i < kSuf; ++i) {
-    const int x = (int)(tw_byte(w, i) & 63u);
-    copies += x == a;
-    if (!placed && a < x) {
-      t[n++] = a;
+  for (int i = 0; i < N; ++i) {
+    copies += t[i] == a;
+    if (!placed && a < t[i]) {
+      c[n++] = a;
       placed = true;
     }
-    t[n++] = x;
+    c[n++] = t[i];
   }
-  if (!placed) t[n++] = a;
-  uint64_t r = cg[5 * W];
+  if (!placed) c[n++] = a;
+  uint64_t r = cg[(N + 1) * W + from];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) r -= cg[(5 - i) * W + t[i] + 1];
-  r -= cg[W + t[4]];
+  for (int i = 0; i < N; ++i) r -= cg[(N + 1 - i) * W + c[i] + 1];
+  r -= cg[W + c[N]];
   return ((uint32_t)r << 2) | ((uint32_t)copies << kInsertShift);
 }
 

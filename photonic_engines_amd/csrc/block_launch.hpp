@@ -48,14 +48,15 @@ void launch_layer_group_f64(int d, int kind, const BlockGrid& g, const double2* 
 // k_layer_block_group for prefix width d = K - 4 (uneven_kernels.hip)
 void launch_layer_block_group(bool comp, int d, uint32_t grid, size_t lds, hipStream_t st, const GroupLaunch& gl);
 
-// k_descend_block and k_adjoint_block with maxd (4, 6 or 8) prefix slots (descend_kernels.hip)
+// k_descend_block with maxd (4, 6 or 8) prefix slots (descend_kernels.hip)
 void launch_descend_block(int maxd, const BlockGrid& g, int K, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
                           uint64_t S_pre, uint64_t per_wave, float scale, uint32_t xcd_chunk);
 // the insert-table form for a prefix of dp (1 to 8) positions
 void launch_descend_insert(int dp, const BlockGrid& g, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
                            uint64_t per_wave, float scale, uint32_t xcd_chunk, const uint32_t* ins);
-void launch_adjoint_block(int maxd, const BlockGrid& g, int K, int m, int col, const float2* U, const float2* psi,
-                          const float2* gk, uint64_t Sk, float2* gout, uint64_t Sp, uint64_t S_pre, uint64_t per_wave,
-                          uint32_t xcd_chunk, double2* partial);
+// the adjoint of one layer, at most 32 modes
+void launch_adjoint_insert(int dp, const BlockGrid& g, int m, int col, const float2* U, const float2* psi,
+                           const float2* gk, uint64_t Sk, float2* gout, uint64_t Sp, uint64_t per_wave,
+                           uint32_t xcd_chunk, double2* partial, const uint32_t* ins);
 
 }  // namespace slos

@@ -1,4 +1,5 @@
-// k_descend_block and k_adjoint_block (descend_block.hpp).
+// The pulls over children: k_descend_insert and k_adjoint_insert (child_walk.hpp), k_descend_block
+// (descend_block.hpp).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -52,22 +53,16 @@ void launch_descend_insert(int dp, const BlockGrid& g, const float* qk, uint64_t
   });
 }
 
-void launch_adjoint_block(int maxd, const BlockGrid& g, int K, int m, int col, const float2* U, const float2* psi,
-                          const float2* gk, uint64_t Sk, float2* gout, uint64_t Sp, uint64_t S_pre, uint64_t per_wave,
-                          uint32_t xcd_chunk, double2* partial) {
-  const auto* tuples = static_cast<const TupleWord*>(g.tuples);
-#define SLOS_ADJ(D, E)                                                                                             \
-  hipLaunchKernelGGL((k_adjoint_block<D, E>), g.grid, dim3(kBlockThreads), g.lds, g.st, g.cg, g.lo, tuples, g.me, \
-                     g.me + 1, K, m, col, U, psi, gk, Sk, gout, Sp, S_pre, per_wave, xcd_chunk, partial)
-#define SLOS_ADJ_E(D)                \
-  do {                               \
-    if (g.me <= 16) SLOS_ADJ(D, 16); \
-    else SLOS_ADJ(D, 32);            \
-  } while (0)
-  if (maxd == 4) SLOS_ADJ_E(4);
-  else if (maxd == 6) SLOS_ADJ_E(6);
-  else SLOS_ADJ_E(8);
-#undef SLOS_ADJ_E
+void launch_adjoint_insert(int dp, const BlockGrid& g, int m, int col, const float2* U, const float2* psi,
+                           const float2* gk, uint64_t Sk, float2* gout, uint64_t Sp, uint64_t per_wave,
+                           uint32_t xcd_chunk, double2* partial, const uint32_t* ins) {
+#define SLOS_ADJ(E)                                                                                                     \
+  hipLaunchKernelGGL((k_adjoint_insert<decltype(d)::value, E>), g.grid, dim3(kBlockThreads), 0, g.st, g.cg, ins, g.me, \
+                     m, col, U, psi, gk, Sk, gout, Sp, per_wave, xcd_chunk, partial)
+  with_prefix(dp, [&](auto d) {
+    if (g.me <= 16) SLOS_ADJ(16);
+    else SLOS_ADJ(32);
+  });
 #undef SLOS_ADJ
 }
 

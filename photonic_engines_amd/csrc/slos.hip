@@ -114,9 +114,28 @@ size_t lds_limit() {
   return lim;
 }
 
-__global__ void k_insert_table(const uint64_t* cg, const slos::TupleWord* tuples, int me, uint32_t n4, uint32_t* ins) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n4 * (uint32_t)me; i += gridDim.x * blockDim.x)
-    ins[i] = slos::insert_word(cg, me + 1, tuples[i % n4], (int)(i / n4));
+__global__ void k_insert_table(const uint64_t* cg, const slos::TupleWord* tuples, int me, uint32_t n4, uint32_t words,
+                               uint32_t* ins) {
+  const int W = me + 1, X = slos::insert_from(me);
+  const uint32_t first = n4 * (uint32_t)me, n5 = (uint32_t)cg[5 * W + X];
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) {
+    if (i < first) {
+      const slos::TupleWord w = tuples[i % n4];
+      const int t[4] = {(int)(w & 63u), (int)((w >> 8) & 63u), (int)((w >> 16) & 63u), (int)((w >> 24) & 63u)};
+      ins[i] = slos::insert_word<4>(cg, W, t, (int)(i / n4), 0);
+    } else {
+      uint64_t r = (i - first) % n5;
+      int t[5], x = X;
+      for (int l = 0; l < 5; ++l) {  // 5-tuple r of the modes from X on
+        const uint64_t* c = cg + (5 - l) * W;
+        const uint64_t top = c[x];
+        while (x < me - 1 && top - c[x + 1] <= r) ++x;
+        r -= top - c[x];
+        t[l] = x;
+      }
+      ins[i] = slos::insert_word<5>(cg, W, t, X + (int)((i - first) / n5), X);
+    }
+  }
 }
 
 int device_tables(const slos_plan* cp, DevTables* out) {
@@ -162,14 +181,21 @@ int device_tables(const slos_plan* cp, DevTables* out) {
   return SLOS_OK;
 }
 
+bool has_insert_table(const slos_plan* p) {
+  return p->multiset && !p->tuples.empty() && p->n > 5 && p->size(5) <= slos::kInsertTuples &&
+         p->tuples.size() * (uint64_t)p->me <= slos::kInsertWords;
+}
+
 // The plan's insert table on the current GPU, built by the first pull over children that asks for it
 // (1.7 MB and about 50 us at 24 modes); null where the space has none, or while `st` is captured and
 // it is not there yet (nothing is allocated inside a capture).
 int insert_table(const slos_plan* cp, hipStream_t st, const uint32_t** out) {
   slos_plan* p = const_cast<slos_plan*>(cp);
   *out = nullptr;
-  const uint64_t n4 = p->tuples.size(), words = n4 * (uint64_t)p->me;
-  if (!p->multiset || !n4 || p->n <= 5 || p->size(5) > slos::kInsertTuples || words > slos::kInsertWords) return SLOS_OK;
+  if (!has_insert_table(p)) return SLOS_OK;
+  const uint64_t n4 = p->tuples.size(), first = n4 * (uint64_t)p->me;
+  const int X = slos::insert_from(p->me);
+  const uint64_t words = first + (uint64_t)(p->me - X) * p->cg[(size_t)5 * (p->me + 1) + X];
   int d = 0;
   HIP_TRY(hipGetDevice(&d));
   std::lock_guard<std::mutex> g(p->mu);
@@ -182,7 +208,7 @@ int insert_table(const slos_plan* cp, hipStream_t st, const uint32_t** out) {
         uint32_t* ins = nullptr;
         HIP_TRY(hipMalloc(&ins, words * sizeof(uint32_t)));
         hipLaunchKernelGGL(k_insert_table, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, t.cg, t.tuples, p->me,
-                           (uint32_t)n4, ins);
+                           (uint32_t)n4, (uint32_t)words, ins);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(st);  // other streams may read it from here on
         if (e != hipSuccess) {
@@ -551,7 +577,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adjoint_layer(const uint64_t* c
 }
 
 // gU[b][j][col] += sum over blocks of partial[b][block][j]
-__global__ __launch_bounds__(64) void k_reduce_gu(const double2* __restrict__ partial, int nblk, int me, int m, int col,
+constexpr int kReduceThreads = 256;
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_gu(const double2* __restrict__ partial, int nblk, int me, int m, int col,
                                                   float2* __restrict__ gU, int accumulate) {
   const int64_t b = blockIdx.y;
   const int j = blockIdx.x;
@@ -565,7 +592,14 @@ __global__ __launch_bounds__(64) void k_reduce_gu(const double2* __restrict__ pa
     sr += __shfl_down(sr, o, 64);
     si += __shfl_down(si, o, 64);
   }
+  __shared__ double2 wave[kReduceThreads / 64];
+  if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = make_double2(sr, si);
+  __syncthreads();
   if (threadIdx.x == 0) {
+    for (int w = 1; w < kReduceThreads / 64; ++w) {
+      sr += wave[w].x;
+      si += wave[w].y;
+    }
     float2* dst = gU + (size_t)b * m * m + (size_t)j * m + col;
     if (accumulate) *dst = make_float2(dst->x + (float)sr, dst->y + (float)si);
     else *dst = make_float2((float)sr, (float)si);
@@ -1748,48 +1782,40 @@ static int adjoint_blocks(uint64_t Sp) { return (int)std::max<uint64_t>(1, std::
 
 namespace {
 
-// parents per XCD chunk of the block adjoint (see slos::xcd_chunk_index)
-constexpr uint64_t kDescChunkParents = 1ull << 18;
+// parents per XCD chunk of the insert-table adjoint (see slos::xcd_chunk_index)
+constexpr uint64_t kAdjChunkParents = 1ull << 18;
 
-// How one adjoint layer runs: the block kernel (multiset spaces whose parent layer has a 1..8
+// How one adjoint layer runs: the insert-table kernel (multiset spaces whose parent layer has a 1..8
 // position prefix before its 4-position suffix, up to 32 modes) or the thread-per-state kernel;
 // `nblk` work groups, each writing one FP64 partial per mode.
 struct AdjLaunch {
-  bool block = false;
-  int maxd = 0;
+  bool walk = false;
   uint64_t per_wave = 0;
   uint32_t xcd_chunk = 1;
-  size_t lds = 0;
+  size_t lds = 0;   // of the thread-per-state kernel
   uint64_t nblk = 0;
 };
 
 int adjoint_launch(const slos_plan* p, int k, AdjLaunch* L) {
   const uint64_t Sp = p->size(k - 1);
   const int dp = k - 1 - slos::kSuf;
-  if (p->multiset && !p->tuples.empty() && dp >= 1 && dp <= 8 && p->me <= 32) {
-    const int maxd = dp <= 4 ? 4 : dp <= 6 ? 6 : 8;
-    const size_t shb = slos::desc_dyn_lds(k, p->me, maxd);
-    if (shb + sizeof(double) * 2 * slos::kWaves * 32 <= lds_limit()) {
-      // parents per wave: at most about 2^16 work groups (FP64 partials per mode), at least 256
-      // (at n = 8, m = 24 the top layer took 0.46 ms with at least 2048 a wave, 0.25 ms so)
-      uint64_t pw = (Sp / ((uint64_t)slos::kWaves << 16) + 63) & ~63ull;
-      pw = std::max<uint64_t>(pw, 256);
-      const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
-      if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
-      L->block = true;
-      L->maxd = maxd;
-      L->per_wave = pw;
-      L->xcd_chunk = (uint32_t)std::max<uint64_t>(1, kDescChunkParents / ((uint64_t)slos::kWaves * pw));
-      L->lds = shb;
-      L->nblk = wgs;
-      return SLOS_OK;
-    }
+  L->lds = (((size_t)(k + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8 +
+           (size_t)kAdjThreads * p->me * 8;
+  L->walk = has_insert_table(p) && dp >= 1 && dp <= 8 && p->me <= 32;
+  if (L->walk) {
+    // parents per wave: at most about 2^16 work groups (FP64 partials per mode), and else as few as
+    // pay for a wave's sum over its lanes (us with 128 / 256 / 512: 2.0M parents 137 / 119 / 112,
+    // 475k 55 / 60 / 73, 2.2M 147 / 130 / 153, 76k 57 / 80 / 92)
+    uint64_t pw = (Sp / ((uint64_t)slos::kWaves << 16) + slos::kAdjChunk - 1) & ~(uint64_t)(slos::kAdjChunk - 1);
+    pw = std::max<uint64_t>(pw, Sp < (1ull << 20) ? 128 : 256);
+    const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
+    if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
+    L->per_wave = pw;
+    L->xcd_chunk = (uint32_t)std::max<uint64_t>(1, kAdjChunkParents / ((uint64_t)slos::kWaves * pw));
+    L->nblk = wgs;
+    return SLOS_OK;
   }
-  const size_t sh = (((size_t)(k + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8 +
-                    (size_t)kAdjThreads * p->me * 8;
-  if (sh > lds_limit()) return fail(SLOS_ERANGE, "adjoint LDS exceeds the GPU's LDS (too many modes)");
-  L->block = false;
-  L->lds = sh;
+  if (L->lds > lds_limit()) return fail(SLOS_ERANGE, "adjoint LDS exceeds the GPU's LDS (too many modes)");
   L->nblk = adjoint_blocks(Sp);
   return SLOS_OK;
 }
@@ -1827,12 +1853,17 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   const auto* gk = static_cast<const float2*>(grad_k);
   auto* gout = static_cast<float2*>(grad_prev);
   auto* part = static_cast<double2*>(ws);
-  if (L.block && dt.tuples) {
-    const dim3 grid((unsigned)L.nblk, (unsigned)batch);
-    const uint64_t S_pre = p->size(k - 1 - slos::kSuf);
-    const slos::BlockGrid bg{grid, L.lds, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
-    slos::launch_adjoint_block(L.maxd, bg, k, p->m, col, Uf, psi, gk, Sk, gout, Sp, S_pre, L.per_wave, L.xcd_chunk, part);
-  } else {
+  const uint32_t* ins = nullptr;
+  if (L.walk) {
+    rc = insert_table(p, st, &ins);
+    if (rc) return rc;
+  }
+  if (ins) {
+    const slos::BlockGrid bg{dim3((unsigned)L.nblk, (unsigned)batch), 0, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+    slos::launch_adjoint_insert(k - 1 - slos::kSuf, bg, p->m, col, Uf, psi, gk, Sk, gout, Sp, L.per_wave, L.xcd_chunk,
+                                part, ins);
+  } else {  // (also inside a capture that comes before the first use of the table)
+    if (L.lds > lds_limit()) return fail(SLOS_ERANGE, "adjoint LDS exceeds the GPU's LDS (too many modes)");
     with_km(k - 1, [&](auto km) {
       hipLaunchKernelGGL((k_adjoint_layer<decltype(km)::value>), dim3((unsigned)L.nblk, (unsigned)batch),
                          dim3(kAdjThreads), L.lds, st, dt.cg, dt.lo, p->me, p->multiset, k, p->m, col, Uf, psi, gk, Sk,
@@ -1840,7 +1871,7 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
     });
   }
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_gu, dim3((unsigned)p->me, (unsigned)batch), dim3(64), 0, st,
+  hipLaunchKernelGGL(k_reduce_gu, dim3((unsigned)p->me, (unsigned)batch), dim3(kReduceThreads), 0, st,
                      static_cast<const double2*>(ws), (int)L.nblk, p->me, p->m, col, static_cast<float2*>(grad_U), accumulate);
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
@@ -1848,20 +1879,21 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
 
 namespace {
 
-// Whether a pull over children takes the insert-table kernel, for a parent layer of Sp states in
-// S_pre blocks. Below, the thread-per-state kernel is the faster one: a wave of the walk spends a
-// fixed part of its time on each block, and on a small layer its few blocks run one after another.
-// Descents, us, walk / thread per state: 1.3M parents in blocks of 84 on average 69 / 84, 7.7M of 45
-// 286 / 388, 705k of 22 74 / 45, 490k of 126 39 / 36, 203k of 85 34 / 26, 658k of 427 37 / 47, 98k of
-// 4095 18 / 27, 200 rows of 12k in blocks of 159 49 / 105.
-bool insert_walk(uint64_t Sp, uint64_t S_pre, int64_t batch) {
-  const uint64_t block = Sp / S_pre;
-  return block >= 256 || (block >= 32 && Sp >= (1ull << 20) / (uint64_t)batch);
+// Whether a descent of `batch` rows with prefixes of dp positions takes the insert-table kernel. Its
+// waves spend a fixed part of their time on each block, and on a small layer their blocks run one
+// after another: with few parents a block the thread-per-state kernel is the faster one. Descents, us,
+// walk / thread per state: blocks of 296 parents on average, 203k in all, 25 / 25; of 324, 32k in all,
+// 18 / 23; of 189, 76k in all, 29 / 24; of 133, 7.7M in all, 179 / 387; of 34, 4.6M in all, 134 / 186;
+// of 24, 7.8M in all, 300 / 312; of 56, 705k in all, 53 / 44; of 10, 1.1M in all, 110 / 58.
+bool insert_walk(const slos_plan* p, int dp, uint64_t Sp, int64_t batch) {
+  const int X = slos::insert_from(p->me);
+  const uint64_t blocks = (X ? p->cg[(size_t)dp * (p->me + 1) + (p->me - X)] : 0) + p->size(dp - 1);
+  return Sp / blocks >= 256 || (Sp / blocks >= 32 && Sp >= (1ull << 20) / (uint64_t)batch);
 }
 
 // Parents per wave of the insert-table kernels: few, so that the waves in flight read near one
-// another (descents, us, with 64 / 128 / 256 / 512: 2.0M parents 57 / 65 / 73 / 93, 7.9M 157 / 147 /
-// 157 / 202, 28M 588 / 467 / 460 / 555, 1.1G - / 20500 / 19100 / 19800).
+// another (descents, us, with 64 / 128 / 256 / 512, measured without the merged blocks: 2.0M parents 57
+// / 65 / 73 / 93, 7.9M 157 / 147 / 157 / 202, 28M 588 / 467 / 460 / 555, 1.1G - / 20500 / 19100 / 19800).
 uint64_t insert_per_wave(uint64_t Sp) { return Sp < (1ull << 22) ? 64 : Sp < (1ull << 24) ? 128 : 256; }
 
 }  // namespace
@@ -1886,7 +1918,7 @@ int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1,
     rc = insert_table(p, st, &ins);
     if (rc) return rc;
     if (ins) {
-      if (insert_walk(Sp, S_pre, batch)) {
+      if (insert_walk(p, dp, Sp, batch)) {
         const uint64_t pw = insert_per_wave(Sp);
         const uint64_t wgs = ((Sp + pw - 1) / pw + slos::kWaves - 1) / slos::kWaves;
         if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");

@@ -515,17 +515,37 @@ int64_t emu_check_insert(int n, int m, int mask, int k, uint64_t first, uint64_t
     const uint64_t u = slos::unrank_prefix<MAXD>(t, D, dp, g, q);
     slos::DescBlock<MAXD> db;
     slos::descend_block_info<MAXD>(t, k, dp, q, db);
+    const slos::TupleWord tw = s.tuples[db.toff + u];
+    int sx[slos::kSuf];
+    for (int j = 0; j < slos::kSuf; ++j) sx[j] = (int)((tw >> (8 * j)) & 63u);
     const uint64_t tail = db.CB0 - (n5 - s.cg[(size_t)5 * W + db.lastP]);
     std::vector<std::pair<uint64_t, int>> mine, ref;
     for (int a = db.lastP; a < s.me; ++a) {
-      const uint32_t w = slos::insert_word(s.cg.data(), W, s.tuples[db.toff + u], a);
+      const uint32_t w = slos::insert_word<4>(s.cg.data(), W, sx, a, 0);
       mine.push_back({tail + (w & slos::kInsertMask) / 4,
                       (int)(w >> slos::kInsertShift) + (a == db.lastP ? db.lastrun : 0)});
     }
     slos::for_each_child(sv, s.multiset, k, g, [&](uint64_t r, int, int cnt) { ref.push_back({r, cnt}); });
     if (ref.size() < mine.size()) { ++bad; continue; }
+    std::vector<std::pair<uint64_t, int>> all(ref);
     ref.erase(ref.begin(), ref.end() - (long)mine.size());
     if (mine != ref) ++bad;
+    // the second table: suffixes of 5 positions, all of them among the last modes
+    const int X = slos::insert_from(s.me);
+    if (sx[0] < X || db.lastP < X) continue;
+    const int s5[5] = {db.lastP, sx[0], sx[1], sx[2], sx[3]};
+    uint64_t base = s.cg[(size_t)k * W];
+    for (int l = 0; l < dp - 1; ++l) base -= s.cg[(size_t)(k - l) * W + db.p[l] + 1];
+    const int x0 = std::max(X, dp > 1 ? db.p[dp - 2] : 0);
+    mine.clear();
+    for (int a = x0; a < s.me; ++a) {
+      const uint32_t w = slos::insert_word<5>(s.cg.data(), W, s5, a, X);
+      int more = 0;
+      for (int l = 0; l < dp - 1; ++l) more += db.p[l] == a;
+      mine.push_back({base - s.cg[(size_t)6 * W + X] + (w & slos::kInsertMask) / 4, (int)(w >> slos::kInsertShift) + more});
+    }
+    all.erase(all.begin(), all.end() - (long)mine.size());
+    if (mine != all) ++bad;
   }
   return bad;
 }

@@ -41,3 +41,34 @@ def test_descents_equal_the_thread_kernel(n, m, mask, rows):
         out = plan.loss_descend(k, q, scale=0.75)
         assert torch.equal(out, plan.loss_descend(k, q, flags=nat.FLAG_SIMPLE, scale=0.75)), k
         q = out
+
+
+# parent prefixes of 1 to 8 positions on both sides of 16 modes; every parent in the last eight modes;
+# a last step of the walk of one parent
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,mask,rows", [(6, 32, "fock", 1), (7, 16, "fock", 3), (8, 17, "tail_empty", 1),
+                                           (8, 24, "fock", 1), (9, 9, "fock", 2), (10, 12, "fock", 1),
+                                           (13, 4, "fock", 5), (13, 9, "fock", 1)])
+def test_adjoint_against_complex128(n, m, mask, rows):
+    """One adjoint layer against the complex128 kernel on random layers. A term of grad_prev is one of
+    2 me fused products a component, one of dL/dU a product in float32 sums of at most 2 x 8 parents a
+    lane (FP64 beyond): errors within these counts, and two roundings, times the sums of magnitudes."""
+    plan = _plan(n, m, mask)
+    me = m if mask == "fock" else m - 2
+    g = torch.Generator("cuda").manual_seed(17 * n + m)
+
+    def rand(*shape):
+        return torch.randn(shape, dtype=torch.complex64, device="cuda", generator=g)
+
+    U = rand(rows, m, m)
+    for k in range(n, 5, -1):
+        psi, gk, col = rand(rows, plan.sizes[k - 1]), rand(rows, plan.sizes[k]), k % m
+        gU, ref_U, mag_U = torch.zeros_like(U), *(torch.zeros_like(U, dtype=torch.complex128) for _ in range(2))
+        out = plan.adjoint_layer(U, k, col, psi, gk, gU)
+        wide = [x.to(torch.complex128) for x in (U, psi, gk)]
+        ref = plan.adjoint_layer(wide[0], k, col, wide[1], wide[2], ref_U)
+        size = [x.abs().to(torch.complex128) for x in wide]
+        mag = plan.adjoint_layer(size[0], k, col, size[1], size[2], mag_U)
+        eps = 2.0 ** -24 * 2 ** 0.5
+        assert ((out - ref).abs() <= (2 * me + 2) * eps * mag.real).all(), k
+        assert ((gU - ref_U).abs() <= (2 * 8 + 2) * eps * mag_U.real).all(), k
