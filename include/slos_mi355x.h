@@ -170,6 +170,22 @@ int slos_adjoint_layer(const slos_plan* plan, const void* U, int64_t batch, int 
                        const void* grad_k, void* grad_prev, void* grad_U, int accumulate, void* workspace,
                        size_t workspace_bytes, slos_stream_t stream);
 
+/* A forward and its whole backward in one call each (complex64, plain sums; the autograd pair of
+ * kernel.py:216-257 where every layer is kept). slos_forward_saved runs layers 1..layer (1 <= layer <= n)
+ * over the columns modes[0..layer-1] (NULL: the plan's own), keeps layers 0..layer-1 in `saved`
+ * (slos_saved_bytes bytes, opaque) and writes to `out` the probabilities |amp * scale|^2 prod t_j!
+ * (probs != 0) or the raw amplitudes of the last one. slos_backward takes the gradient of that output
+ * (grad_kind 0: complex64 amplitudes; 1: float32 probabilities, layer = n; 2: the same for a gradient
+ * that is zero almost everywhere) and writes grad_U, complex64 [batch][m][m], all of it. Workspace >=
+ * slos_backward_workspace bytes. batch <= 65535; nothing but a plan's first use allocates. */
+int slos_saved_bytes(const slos_plan* plan, int64_t batch, int layer, size_t* bytes);
+int slos_forward_saved(const slos_plan* plan, const void* U, int64_t batch, const int32_t* modes, int layer, int probs,
+                       void* out, double scale, void* saved, size_t saved_bytes, slos_stream_t stream);
+int slos_backward_workspace(const slos_plan* plan, int64_t batch, int layer, int grad_kind, size_t* bytes);
+int slos_backward(const slos_plan* plan, const void* U, int64_t batch, const int32_t* modes, int layer,
+                  const void* saved, size_t saved_bytes, const void* grad, int grad_kind, double scale, void* grad_U,
+                  void* workspace, size_t workspace_bytes, slos_stream_t stream);
+
 /* One step of the uniform photon-removal recurrence of output loss (imperfections.py:254-276):
  * q_{k-1}(t) = scale * (sum_j q_k(t + e_j) (t_j + 1)) / k, for 1 <= k <= n. Pull form (each
  * (k-1)-photon state gathers its children), no atomics; children in ascending mode order. q_k:

@@ -1,4 +1,4 @@
-// k_layer_block for one KIND (SLOS_BLOCK_KIND, given by the Makefile): 0 raw, 1 probabilities, 2 amplitudes.
+// k_layer_block for one KIND (SLOS_BLOCK_KIND, given by the Makefile): 0 raw, 1 probabilities, 2 amplitudes, 4 readout's adjoint.
 #include <hip/hip_runtime.h>
 
 #include "block_launch.hpp"
@@ -10,8 +10,8 @@ void launch_layer_block(bool comp, int d, int suf, const BlockGrid& g, const flo
   // one stream slot per prefix position: exact widths where the big layers live (d = K - suf)
 #define SLOS_BLK(D, S)                                                                                                \
   do {                                                                                                                \
-    if (comp)                                                                                                         \
-      hipLaunchKernelGGL((k_layer_block<KIND, true, D, S>), g.grid, dim3(kBlockThreads), g.lds, g.st, g.cg, g.lo,     \
+    if (comp && KIND != 4)                                                                                            \
+      hipLaunchKernelGGL((k_layer_block<KIND == 4 ? 0 : KIND, true, D, S>), g.grid, dim3(kBlockThreads), g.lds, g.st, g.cg, g.lo,     \
                          g.tuples, g.me, g.me + 1, g.multiset, par, out, L);                                          \
     else                                                                                                              \
       hipLaunchKernelGGL((k_layer_block<KIND, false, D, S>), g.grid, dim3(kBlockThreads), g.lds, g.st, g.cg, g.lo,    \

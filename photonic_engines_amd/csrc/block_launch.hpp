@@ -35,7 +35,7 @@ inline int block_maxd_f64(int d) { return d <= 4 ? 4 : d <= 6 ? 6 : 8; }
 template <int KIND>
 void launch_layer_block(bool comp, int d, int suf, const BlockGrid& g, const float2* par, void* out, const BlockLayer& L);
 
-// k_layer_group for prefix width d = K - 5 in 2..6 (group_kernels.hip)
+// k_layer_group for prefix width d = K - 5 in 2..6, kind 0, 1 or 4 (group_kernels.hip)
 void launch_layer_group(int d, int kind, bool comp, const BlockGrid& g, const float2* par, void* out, const BlockLayer& L,
                         const uint4* items, uint32_t n_items);
 

@@ -38,6 +38,7 @@ struct FrontArgs {
   double scale;
   unsigned immediate;
   int64_t out_lo;            // compensated sums: offset of layer kf's low-order parts (0: none)
+  void* below[kFrontMax];    // layers 0..kf-1 in memory [B][S_k] too, for a backward pass (null: not)
 };
 
 // LDS: cg rows 0..kf (32-bit), lo, the input columns, two layers (twice with low-order parts)

@@ -61,6 +61,8 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
     bufs[0][0] = T2{1, 0};
     if constexpr (COMP) bufs[0][a.buf] = T2{0, 0};
   }
+  const bool keep = a.below[0] && blockIdx.x == 0;  // one work group a row writes the layers below kf
+  if (keep && threadIdx.x == 0) static_cast<T2*>(a.below[0])[b] = T2{1, 0};
   const SpaceView32 sv{cg, lo, a.me, stride};
   auto layer = [&](auto km, int K, bool last) {
     constexpr int KM = decltype(km)::value;
@@ -102,6 +104,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
       }
       if (!last) {
         dst[g] = T2{re, im};
+        if (keep) (static_cast<T2*>(a.below[K]) + (size_t)b * S)[g] = T2{re, im};
         if constexpr (COMP) dst[a.buf + g] = T2{s.c.cre - (re - s.c.re), s.c.cim - (im - s.c.im)};
       } else if (a.kind == 0) {
         T2* out = static_cast<T2*>(a.out) + (size_t)b * S;

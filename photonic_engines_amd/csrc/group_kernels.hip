@@ -13,7 +13,9 @@ void launch_layer_group(int d, int kind, bool comp, const BlockGrid& g, const fl
                      g.me + 1, par, out, L, items, n_items)
 #define SLOS_GRP_D(D)                                                   \
   do {                                                                  \
-    if (kind == 1) {                                                    \
+    if (kind == 4) {                                                    \
+      SLOS_GRP(D, 4, false);                                            \
+    } else if (kind == 1) {                                             \
       if (comp) SLOS_GRP(D, 1, true);                                   \
       else SLOS_GRP(D, 1, false);                                       \
     } else {                                                            \

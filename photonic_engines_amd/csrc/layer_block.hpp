@@ -38,6 +38,7 @@ struct BlockLayer {
   // compensated sums only: element offsets of the low-order parts of the parent layer and of a
   // complex64 output layer from their high parts (0: none; a hi/lo layer is [2][B][S])
   int64_t par_lo, out_lo;
+  const float* gp = nullptr;  // KIND 4: dL/dp [B][S]
 };
 
 __device__ __forceinline__ uint32_t rfl(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -52,6 +53,13 @@ __device__ __forceinline__ float2 uniform_f2(float2 v) {
   return make_float2(__builtin_bit_cast(float, rfl(__builtin_bit_cast(uint32_t, v.x))),
                      __builtin_bit_cast(float, rfl(__builtin_bit_cast(uint32_t, v.y))));
 }
+// dL/d(raw amplitude) of one state from dL/dp = gv: 2 s^2 f gv amp (zero where gv is, whatever the amplitude)
+__device__ __forceinline__ float2 readout_gradient(float re, float im, float s2, float f, float gv) {
+  if (gv == 0.f) return make_float2(0.f, 0.f);
+  const float w = 2.f * s2 * f * gv;
+  return make_float2(w * re, w * im);
+}
+
 // element `off` bytes past a scalar base: lets the compiler use base-in-SGPR addressing
 template <class T>
 __device__ __forceinline__ const T& at_bytes(const T* base, uint32_t off) {
@@ -174,6 +182,7 @@ struct ChunkCtx {
   unsigned flags;
   int kind;  // KIND 3 only: 1 probabilities, 0 raw amplitudes
   int64_t plo = 0, olo = 0;  // compensated sums: low-order parts of the parents / the output (elements)
+  const float* gb = nullptr;  // KIND 4: dL/dp of the block's first child
 };
 
 // the suffix edges of one child from its tuple word: coefficients c[j] (edge 0 of a tau that
@@ -309,6 +318,10 @@ __device__ __forceinline__ void sweep(const ChunkCtx<MAXD, SUF>& cx, uint32_t uc
           *reinterpret_cast<float2*>(cx.ob + u[c] * 8u + cx.olo * 8) =
               make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
       }
+    } else if constexpr (KIND == 4) {
+      if (in[c])
+        *reinterpret_cast<float2*>(cx.ob + u[c] * 8u) =
+            readout_gradient(re, im, cx.scale, child_norm_w(cx, tw[c]), at_bytes(cx.gb, u[c] * 4u));
     } else {
       const float f = child_norm_w(cx, tw[c]);
       re *= cx.scale;
@@ -380,6 +393,13 @@ __device__ __forceinline__ void sweep_pairs(const ChunkCtx<MAXD, SUF>& cx, uint3
   }
   if (KIND == 0 || (KIND == 3 && cx.kind == 0)) {
     const float4 v = make_float4(res[0][0], res[0][1], res[1][0], res[1][1]);
+    __builtin_memcpy(reinterpret_cast<float2*>(cx.ob) + u, &v, 16);
+  } else if constexpr (KIND == 4) {
+    float2 gv;
+    __builtin_memcpy(&gv, cx.gb + u, 8);
+    const float2 a = readout_gradient(res[0][0], res[0][1], cx.scale, f[0], gv.x);
+    const float2 b = readout_gradient(res[1][0], res[1][1], cx.scale, f[1], gv.y);
+    const float4 v = make_float4(a.x, a.y, b.x, b.y);
     __builtin_memcpy(reinterpret_cast<float2*>(cx.ob) + u, &v, 16);
   } else {
     float re0 = res[0][0] * cx.scale, im0 = res[0][1] * cx.scale;
@@ -466,6 +486,7 @@ struct BlockSweep {
   unsigned flags;
   int kind;
   int64_t plo, olo;
+  const float* gb;
 };
 
 // Children [u0, u_stop) of one block with its first NS stream slots of the block table column `bj`
@@ -485,7 +506,7 @@ __device__ __forceinline__ void block_children(const uint32_t* bj, const float2*
   }
   ChunkCtx<NS, SUF> cx{sp,       coef,    bs.lp,       static_cast<const TupleWordT<SUF>*>(bs.tb),
                        bs.ob,    bs.rows, bs.rn,       bs.C0,    bs.u_stop, bs.lane, bs.fQ, bs.lastrun,
-                       bs.skip0, bs.lo,   bs.multiset, bs.scale, bs.flags,  bs.kind, bs.plo, bs.olo};
+                       bs.skip0, bs.lo,   bs.multiset, bs.scale, bs.flags,  bs.kind, bs.plo, bs.olo, bs.gb};
   const uint32_t u_stop = bs.u_stop;
   uint32_t uc = bs.u0;
   if constexpr (!COMP) {
@@ -573,7 +594,8 @@ __device__ __forceinline__ void fill_block_table(const BlockTables& tl, int K, i
 template <int KIND, bool COMP, int MAXD, int SUF>
 __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTables& tl, const float2* __restrict__ par,
                                            void* __restrict__ out, const SufRow* rows, const float* rn,
-                                           uint32_t* tbl, const BlockLayer& a, uint64_t g, int kind = 0) {
+                                           uint32_t* tbl, const BlockLayer& a, uint64_t g, int kind = 0,
+                                           const float* __restrict__ gp = nullptr) {
   const int lane = threadIdx.x & 63;
   const int K = a.K;
   const int stride = tg.stride, multiset = tg.multiset;
@@ -617,7 +639,7 @@ __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTab
       const uint32_t u_stop = (uint32_t)(((uint64_t)L - u0 < avail) ? (uint64_t)L : u0 + avail);
       const BlockSweep bs{par + LBp, tuples + toff, reinterpret_cast<char*>(out) + CB * (probs ? 4 : 8), rows, rn, C0,
                           (uint32_t)u0, u_stop, lane, fQ, lastrun, skip0, blo, multiset, a.scale, a.flags, kind,
-                          COMP ? a.par_lo : 0, COMP ? a.out_lo : 0};
+                          COMP ? a.par_lo : 0, COMP ? a.out_lo : 0, KIND == 4 ? gp + CB : nullptr};
       // one sweep per count of active prefix streams, so inactive slots cost no loads or FMAs
       if constexpr (MAXD > 8) {
         block_children<KIND, COMP, MAXD, MAXD, SUF>(bj, par, bs);
@@ -636,7 +658,8 @@ __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTab
 }
 
 
-// KIND 0: intermediate layer (complex64), 1: probabilities (float32), 2: scaled amplitudes;
+// KIND 0: intermediate layer (complex64), 1: probabilities (float32), 2: scaled amplitudes,
+// 4: the readout's adjoint (complex64, readout_gradient; scale is its square);
 // SUF: suffix length (4, or 5 with the 8-byte tuple words). Occupancy: 5 waves per SIMD for the
 // plain 4-suffix sweep; 4 for the 5-suffix sweep (its widest prefixes would spill at 96 registers,
 // and 4 measured slightly faster at n = 11, m = 32 as well); 3 for compensated sums and wide prefixes.
@@ -674,7 +697,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(C
   char* out_b = reinterpret_cast<char*>(out_all) + (size_t)b * a.S * (KIND == 1 ? 4 : 8);
   uint32_t* tbl = reinterpret_cast<uint32_t*>(smem + block_table_offset(K, me)) +
                   (size_t)wv * kBlockBatch * block_words(MAXD);
-  block_wave<KIND, COMP, MAXD, SUF>(tg, tl, par_all + (size_t)b * a.S_par, out_b, rows, rn, tbl, a, g);
+  block_wave<KIND, COMP, MAXD, SUF>(tg, tl, par_all + (size_t)b * a.S_par, out_b, rows, rn, tbl, a, g, 0,
+                                    KIND == 4 ? a.gp + (size_t)b * a.S : nullptr);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -721,7 +745,8 @@ __device__ __forceinline__ void load_pair_parents(const float2* lp, const PairOf
 }
 
 // one block of the group for the pair step: NS stream slots (slot 0 shared), both children;
-// KIND 1 writes probabilities (float32), KIND 0 the raw complex64 amplitudes of a middle layer
+// KIND 1 writes probabilities (float32), KIND 0 the raw complex64 amplitudes of a middle layer, KIND 4
+// (gp: dL/dp of the row) their gradients by the readout
 // COMP: compensated sums as the block kernel's sweep (two-sum accumulation; with plo the parents'
 // low-order parts at element offset plo, slot 0's in v0lo; with olo the stored value's rounding
 // error at element offset olo of a complex64 output).
@@ -729,7 +754,7 @@ template <int NS, int KIND, bool COMP = false>
 __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const float2* par, const float4& v0,
                                                   const float2 (&lc)[2][5], const PairOffsets<5>& off,
                                                   uint32_t u, const uint32_t (&code)[2], const bool (&lead)[2], const float* rn,
-                                                  float scale, void* out, const float4& v0lo = float4{},
+                                                  float scale, void* out, const float* gp, const float4& v0lo = float4{},
                                                   int64_t plo = 0, int64_t olo = 0) {
   const uint64_t CB = (uint64_t)bw[0].x | ((uint64_t)bw[0].y << 32);
   const uint64_t LBp = (uint64_t)bw[0].z | ((uint64_t)bw[0].w << 32);
@@ -799,6 +824,15 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
         __builtin_memcpy(static_cast<float2*>(out) + olo + CB + u, &e, 16);
       }
     }
+  } else if constexpr (KIND == 4) {
+    float2 gv, g[2];
+    __builtin_memcpy(&gv, gp + CB + u, 8);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const float f = fQ * rn[(lead[c] ? lastrow : 0u) * 16u + code[c]];
+      g[c] = readout_gradient(res[c][0], res[c][1], scale, f, c == 0 ? gv.x : gv.y);
+    }
+    __builtin_memcpy(static_cast<float2*>(out) + CB + u, g, 16);
   } else {
     float pr[2];
 #pragma unroll
@@ -816,7 +850,7 @@ template <int NS, int KIND, bool COMP = false>
 __device__ __forceinline__ void group_block_one(const uint4 (&bw)[8], const float2* par, const float2& v0,
                                                 const float2 (&lc)[5], const uint32_t (&off)[5], uint32_t u, bool in,
                                                 uint32_t code, bool lead, const float* rn, float scale, void* out,
-                                                const float2& v0lo = float2{}, int64_t plo = 0, int64_t olo = 0) {
+                                                const float* gp, const float2& v0lo = float2{}, int64_t plo = 0, int64_t olo = 0) {
   const uint64_t CB = (uint64_t)bw[0].x | ((uint64_t)bw[0].y << 32);
   const uint64_t LBp = (uint64_t)bw[0].z | ((uint64_t)bw[0].w << 32);
   const uint32_t w6 = bw[1].x;
@@ -860,7 +894,9 @@ __device__ __forceinline__ void group_block_one(const uint4 (&bw)[8], const floa
     }
   } else {
     const float f = fQ * rn[(lead ? ((w6 >> 16) & 0xffu) + 1u : 0u) * 16u + code];
-    if (in) static_cast<float*>(out)[CB + u] = prob_readout(re * scale, im * scale, f);
+    if constexpr (KIND == 4) {
+      if (in) static_cast<float2*>(out)[CB + u] = readout_gradient(re, im, scale, f, gp[CB + u]);
+    } else if (in) static_cast<float*>(out)[CB + u] = prob_readout(re * scale, im * scale, f);
   }
 }
 
@@ -914,7 +950,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
   const int G = (int)rfl((uint32_t)R[0]) + 1;  // blocks (a, R), a = 0..R_0 (lo[x] = x)
   uint32_t* tbl = reinterpret_cast<uint32_t*>(smem + group_table_offset(K, me)) + (size_t)wv * me * kGroupWords;
   const float2* par = par_all + (size_t)b * a.S_par;
-  void* out = static_cast<char*>(out_all) + (size_t)b * a.S * (KIND == 0 ? 8 : 4);
+  void* out = static_cast<char*>(out_all) + (size_t)b * a.S * (KIND == 1 ? 4 : 8);
+  const float* gp = KIND == 4 ? a.gp + (size_t)b * a.S : nullptr;
   if (lane < G) {
     int q[MAXD];
     q[0] = lane;
@@ -996,7 +1033,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
       uint4 bw[8];
       group_words(tbl, g, bw);
       group_dispatch<MAXD>(bw[1].x >> 24, [&](auto ns) {
-        group_block_pairs<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, u, code, lead, rn, a.scale, out,
+        group_block_pairs<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, u, code, lead, rn, a.scale, out, gp,
                                                             v0lo, COMP ? a.par_lo : 0, COMP ? a.out_lo : 0);
       });
     }
@@ -1018,8 +1055,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
       uint4 bw[8];
       group_words(tbl, g, bw);
       group_dispatch<MAXD>(bw[1].x >> 24, [&](auto ns) {
-        group_block_one<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, u, in, code, lead, rn, a.scale, out, v0lo,
-                                                          COMP ? a.par_lo : 0, COMP ? a.out_lo : 0);
+        group_block_one<decltype(ns)::value, KIND, COMP>(bw, par, v0, lc, off, u, in, code, lead, rn, a.scale, out, gp,
+                                                          v0lo,                                                          COMP ? a.par_lo : 0, COMP ? a.out_lo : 0);
       });
     }
   }

@@ -55,9 +55,11 @@ struct LayerArgs {
   float scale;
   unsigned flags;
   int64_t par_lo, out_lo;  // compensated sums: element offsets of the low-order parts (0: none)
+  const float* gp = nullptr;  // KIND 4: dL/dp [B][S]
 };
 
-// KIND 0: intermediate layer (complex64), 1: probabilities (float32), 2: scaled amplitudes
+// KIND 0: intermediate layer (complex64), 1: probabilities (float32), 2: scaled amplitudes, 4: the
+// readout's adjoint (readout_gradient)
 // (K <= KM: the per-state position arrays stay in registers; SV: 32-bit counts where the layer has
 // fewer than 2^32 states; EXACT: K = KM). Bound by VALU instructions, most of them index arithmetic: with
 // K known the compiler drops the guards and selects of the unrolled loops, the ranks take two table
@@ -107,6 +109,10 @@ __global__ __launch_bounds__(256) void k_layer_simple(LayerArgs a) {
             reinterpret_cast<float2*>(a.out)[a.out_lo + (size_t)b * a.S + g] =
                 make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
         }
+      } else if constexpr (KIND == 4) {
+        const uint64_t c = (uint64_t)b * a.S + g;
+        reinterpret_cast<float2*>(a.out)[c] =
+            readout_gradient(re, im, a.scale, run_factorial_fixed<KM>(p, K, a.multiset), a.gp[c]);
       } else {
         const float f = run_factorial_fixed<KM>(p, K, a.multiset);
         re *= a.scale;

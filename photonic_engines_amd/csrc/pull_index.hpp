@@ -162,23 +162,24 @@ SLOS_HD void parents_fixed(const SV& sv, int multiset, int K, const int (&p)[KM]
 }
 
 // the children in layer k of the (k-1)-tuple p (k - 1 <= KM), as for_each_child
-template <int KM, class F>
-SLOS_HD void children_fixed(const SpaceView& sv, int multiset, int k, const int (&p)[KM], F&& f) {
+template <int KM, class SV, class F>
+SLOS_HD void children_fixed(const SV& sv, int multiset, int k, const int (&p)[KM], F&& f) {
+  typedef RankT<SV> R;
   const int P = k - 1;
-  uint64_t SP[KM + 1];
+  R SP[KM + 1];
   SP[KM] = 0;
 #pragma unroll
   for (int i = KM - 1; i >= 0; --i) {
     const int lov = i == 0 ? 0 : sv.lo[p[in_range<KM>(i - 1)]];
     SP[i] = i < P ? SP[i + 1] + (sv.C(P - i, lov) - sv.C(P - i, p[i])) : 0;
   }
-  uint64_t PB = 0;
+  R PB = 0;
   int lo_i = 0, run = 0;
 #pragma unroll
   for (int i = 0; i <= KM; ++i) {
     const int pi = p[in_range<KM>(i)], pprev = p[in_range<KM>(i - 1)];
     if (i < P) {
-      const uint64_t base = PB + sv.C(k - i, lo_i) - sv.C(k - i - 1, pi) + SP[in_range<KM + 1>(i + 1)];
+      const R base = PB + sv.C(k - i, lo_i) - sv.C(k - i - 1, pi) + SP[in_range<KM + 1>(i + 1)];
       for (int j = lo_i; j < pi; ++j) {
         if (sv.lo[j] > pi) break;
         const int cnt = (multiset && i > 0 && j == pprev) ? run + 1 : 1;
@@ -188,7 +189,7 @@ SLOS_HD void children_fixed(const SpaceView& sv, int multiset, int k, const int 
       run = (i > 0 && pi == pprev) ? run + 1 : 1;
       lo_i = sv.lo[pi];
     } else if (i == P) {
-      const uint64_t base = PB + sv.C(1, lo_i);
+      const R base = PB + sv.C(1, lo_i);
       for (int j = lo_i; j < sv.me; ++j) {
         const int cnt = (multiset && i > 0 && j == pprev) ? run + 1 : 1;
         f(base - sv.C(1, j), j, cnt);

@@ -49,6 +49,7 @@ void launch_layer_simple(int kind, bool comp, dim3 grid, size_t lds, hipStream_t
     if (!comp) {
       if (kind == 0) hipLaunchKernelGGL((k_layer_simple<0, false, KM, SV, EX>), grid, dim3(256), lds, st, a);
       else if (kind == 1) hipLaunchKernelGGL((k_layer_simple<1, false, KM, SV, EX>), grid, dim3(256), lds, st, a);
+      else if (kind == 4) hipLaunchKernelGGL((k_layer_simple<4, false, KM, SV, EX>), grid, dim3(256), lds, st, a);
       else hipLaunchKernelGGL((k_layer_simple<2, false, KM, SV, EX>), grid, dim3(256), lds, st, a);
     } else {
       if (kind == 0) hipLaunchKernelGGL((k_layer_simple<0, true, KM, SV, EX>), grid, dim3(256), lds, st, a);

@@ -527,35 +527,37 @@ __global__ __launch_bounds__(256) void k_readout_adjoint_pull(const uint64_t* cg
 // each block then reduces its rows to partial[b][block][j] (FP64 stage in k_reduce_gu)
 // (k - 1 <= KM)
 constexpr int kAdjThreads = 64;
-template <int KM>
+template <int KM, class SV = slos::SpaceView, bool EXACT = false>
 __global__ __launch_bounds__(kAdjThreads) void k_adjoint_layer(const uint64_t* cg_g, const int* lo_g, int me, int multiset,
-                                                             int k, int m, int col, const float2* __restrict__ U,
+                                                             int kk, int m, int col, const float2* __restrict__ U,
                                                              const float2* __restrict__ psi, const float2* __restrict__ gk,
                                                              uint64_t Sk, float2* __restrict__ gout, uint64_t Sp,
                                                              double2* __restrict__ partial, int want_psi_grad) {
   extern __shared__ __align__(16) unsigned char smem[];
+  typedef slos::RankT<SV> R;
+  const int k = EXACT ? KM + 1 : kk;
   const int stride = me + 1;
   const int ncg = (k + 1) * stride;
-  uint64_t* cg = reinterpret_cast<uint64_t*>(smem);
+  R* cg = reinterpret_cast<R*>(smem);
   int* lo = reinterpret_cast<int*>(cg + ncg);
   float2* ucol = reinterpret_cast<float2*>(smem + ((ncg * 8 + me * 4 + 15) & ~15));
   float2* slots = ucol + m;  // [kAdjThreads][me]
   const int64_t b = blockIdx.y;
-  for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = cg_g[i];
+  for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = (R)cg_g[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo[i] = lo_g[i];
   for (int j = threadIdx.x; j < m; j += blockDim.x) ucol[j] = U[(size_t)b * m * m + (size_t)j * m + col];
   float2* my = slots + (size_t)threadIdx.x * me;
   for (int j = 0; j < me; ++j) my[j] = make_float2(0.f, 0.f);
   __syncthreads();
-  const slos::SpaceView sv{cg, lo, me, stride};
+  const SV sv{cg, lo, me, stride};
   const float2* gb = gk + (size_t)b * Sk;
   const float2* pb = psi + (size_t)b * Sp;
   for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < Sp; t += (uint64_t)gridDim.x * blockDim.x) {
     const float2 ps = pb[t];
     int p[KM];
-    slos::unrank_fixed<KM>(sv, t, k - 1, p);
+    slos::unrank_fixed<KM>(sv, (R)t, k - 1, p);
     float gr = 0.f, gi = 0.f;
-    slos::children_fixed<KM>(sv, multiset, k, p, [&](uint64_t c, int j, int) {
+    slos::children_fixed<KM>(sv, multiset, k, p, [&](R c, int j, int) {
       const float2 gv = gb[c];
       const float2 u = ucol[j];
       gr += u.x * gv.x + u.y * gv.y;   // conj(u) * gv
@@ -606,6 +608,62 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_gu(const double2* __r
   }
 }
 
+// All of dL/dU in one launch: work group (j, b) sums the partials of mode j of every layer in FP64 and
+// writes row j of gU[b], the layers' sums added to their columns from the last layer down (columns that
+// are no input mode, and modes outside the space, are zero).
+struct ReduceArgs {
+  uint64_t part[kMaxPhotons];  // layer k's partials [B][nblk][me], at k - 1
+  uint32_t nblk[kMaxPhotons];
+  int col[kMaxPhotons];
+  int layers;
+};
+constexpr int kReduceAllThreads = 512;
+__global__ __launch_bounds__(kReduceAllThreads) void k_reduce_all(ReduceArgs a, const double2* __restrict__ partial, int me,
+                                                                  int m, float2* __restrict__ gU) {
+  constexpr int kW = kReduceAllThreads / 64;
+  __shared__ double2 wave[kMaxPhotons][kW];
+  __shared__ float2 sum[kMaxPhotons];
+  const int64_t b = blockIdx.y;
+  const int j = blockIdx.x;
+  const int w = threadIdx.x >> 6;
+  if (j < me) {
+    for (int l = 0; l < a.layers; ++l) {
+      const uint32_t nblk = a.nblk[l];
+      double sr = 0, si = 0;
+      if (nblk > (uint32_t)w * 64u) {
+        const double2* src = partial + a.part[l] + (size_t)b * nblk * me + j;
+        for (uint32_t r = threadIdx.x; r < nblk; r += kReduceAllThreads) {
+          const double2 v = src[(size_t)r * me];
+          sr += v.x;
+          si += v.y;
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+          sr += __shfl_down(sr, o, 64);
+          si += __shfl_down(si, o, 64);
+        }
+      }
+      if ((threadIdx.x & 63) == 0) wave[l][w] = make_double2(sr, si);
+    }
+    __syncthreads();
+    if (threadIdx.x < a.layers) {
+      double sr = 0, si = 0;
+      for (int i = 0; i < kW; ++i) {
+        sr += wave[threadIdx.x][i].x;
+        si += wave[threadIdx.x][i].y;
+      }
+      sum[threadIdx.x] = make_float2((float)sr, (float)si);
+    }
+    __syncthreads();
+  }
+  for (int c = threadIdx.x; c < m; c += blockDim.x) {
+    float2 v = make_float2(0.f, 0.f);
+    if (j < me)
+      for (int l = a.layers - 1; l >= 0; --l)
+        if (a.col[l] == c) v = make_float2(v.x + sum[l].x, v.y + sum[l].y);
+    gU[(size_t)b * m * m + (size_t)j * m + c] = v;
+  }
+}
+
 // dynamic LDS of the single-plan block kernel for layer K with suffix length suf, or 0 if it
 // does not fit the GPU's LDS
 size_t block_lds_fit(int K, int me, int suf) {
@@ -648,7 +706,7 @@ dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
 
 int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs& a, int kind, bool comp, hipStream_t st) {
   slos::BlockLayer L;
-  L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.S_par = a.S_par; L.S = a.S;
+  L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.S_par = a.S_par; L.S = a.S; L.gp = a.gp;
   L.par_lo = a.par_lo; L.out_lo = a.out_lo;
   const int suf = block_suffix(p, dt, a.K);
   L.S_pre = p->size(a.K - suf);
@@ -666,15 +724,14 @@ int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs&
   if (a.B > 65535) return fail(SLOS_ERANGE, "batch > 65535");
   // layers in group order where their work items exist (plain or compensated sums; probabilities or
   // complex64)
-  const bool grp_last = kind == 1;
-  if (suf == 5 && kind <= 1 && dt.items[a.K]) {
+  if (suf == 5 && kind != 2 && dt.items[a.K]) {
     const auto [gitems, gn] = dt.group_items(a.K, a.S * (uint64_t)a.B);
     const size_t shg = slos::group_dyn_lds(a.K, p->me);
     const uint64_t gwgs = ((uint64_t)gn + slos::kWaves - 1) / slos::kWaves;
     if (shg + slos::kBlockStaticLds <= lds_limit() && gwgs <= 0x7fffffffull) {
       L.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
       const slos::BlockGrid bg{batch_grid(gwgs, a.B, &L), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
-      slos::launch_layer_group(a.K - suf, grp_last ? 1 : 0, comp, bg, a.par, a.out, L, gitems, gn);
+      slos::launch_layer_group(a.K - suf, kind, comp, bg, a.par, a.out, L, gitems, gn);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
     }
@@ -685,6 +742,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs&
                            suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
   if (kind == 0) slos::launch_layer_block<0>(comp, a.K - suf, suf, bg, a.par, a.out, L);
   else if (kind == 1) slos::launch_layer_block<1>(comp, a.K - suf, suf, bg, a.par, a.out, L);
+  else if (kind == 4) slos::launch_layer_block<4>(false, a.K - suf, suf, bg, a.par, a.out, L);
   else slos::launch_layer_block<2>(comp, a.K - suf, suf, bg, a.par, a.out, L);
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
@@ -703,8 +761,10 @@ void with_km(int photons, F&& f) {
 // hi/lo pair [2][B][S], the low-order parts after the high ones
 int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const float2* U, int64_t B,
                  const float2* par, uint64_t S_par, void* out, uint64_t S, int kind, float scale,
-                 unsigned flags, hipStream_t st, bool par_hilo = false, bool out_hilo = false) {
+                 unsigned flags, hipStream_t st, bool par_hilo = false, bool out_hilo = false,
+                 const float* gp = nullptr) {
   slos::LayerArgs a;
+  a.gp = gp;
   a.cg = dt.cg; a.lo = dt.lo; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
   a.U = U; a.words = dt.tuples5; a.par = par; a.S_par = S_par; a.out = out; a.S = S; a.B = B;
   a.scale = scale; a.flags = flags;
@@ -810,8 +870,11 @@ int front_layers(const slos_plan* p, int64_t B, int layer, size_t elem, bool com
 
 // layers 1..kf (front_layers) in one launch; kind: of layer kf
 int run_front(const slos_plan* p, const DevTables& dt, int kf, const int* cols, const void* U, int64_t B, void* out,
-              int kind, double scale, unsigned flags, size_t lds, uint32_t buf, bool hilo_out, hipStream_t st) {
+              int kind, double scale, unsigned flags, size_t lds, uint32_t buf, bool hilo_out, hipStream_t st,
+              void* const* below = nullptr) {
   slos::FrontArgs a{};
+  if (below)
+    for (int k = 0; k < kf; ++k) a.below[k] = below[k];
   a.cg = dt.cg; a.lo = dt.lo; a.tuples = dt.tuples; a.tuples5 = dt.tuples5;
   a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.kf = kf; a.kind = kind; a.U = U;
   for (int k = 0; k < kf; ++k) a.cols[k] = cols[k];
@@ -1754,26 +1817,36 @@ int slos_readout_adjoint(const slos_plan* p, int64_t batch, const void* amps, co
   return SLOS_OK;
 }
 
+namespace {
+
+int run_readout_pull(const slos_plan* p, const DevTables& dt, const float2* U, int64_t batch, int col, const float2* psi_prev,
+                     const float* grad_p, double scale, float2* grad_amps, hipStream_t st) {
+  const int K = p->n;
+  const uint64_t S = p->size(K);
+  dim3 grid((unsigned)std::max<uint64_t>(1, std::min<uint64_t>((S + 255) / 256, 1u << 20)),
+            (unsigned)std::min<int64_t>(batch, 16));
+  with_km(K, [&](auto km) {
+    hipLaunchKernelGGL((k_readout_adjoint_pull<decltype(km)::value>), grid, dim3(256), 0, st, dt.cg, dt.lo, p->me,
+                       p->multiset, K, p->m, col, U, psi_prev, p->size(K - 1), grad_p, grad_amps, S, batch,
+                       (float)(scale * scale));
+  });
+  HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+}  // namespace
+
 int slos_readout_adjoint_pull(const slos_plan* p, const void* U, int64_t batch, const void* psi_prev,
                               const float* grad_p, double scale, void* grad_amps, slos_stream_t stream) {
   if (!p || !U || !psi_prev || !grad_p || !grad_amps) return fail(SLOS_EINVAL, "NULL argument");
   if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
   if (p->n < 1) return fail(SLOS_EINVAL, "no photon layer");
   DevTables dt;
-  int rc = device_tables(p, &dt);
+  const int rc = device_tables(p, &dt);
   if (rc) return rc;
-  const int K = p->n;
-  const uint64_t S = p->size(K);
-  dim3 grid((unsigned)std::max<uint64_t>(1, std::min<uint64_t>((S + 255) / 256, 1u << 20)),
-            (unsigned)std::min<int64_t>(batch, 16));
-  with_km(K, [&](auto km) {
-    hipLaunchKernelGGL((k_readout_adjoint_pull<decltype(km)::value>), grid, dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), dt.cg, dt.lo, p->me, p->multiset, K, p->m,
-                       p->modes[K - 1], static_cast<const float2*>(U), static_cast<const float2*>(psi_prev),
-                       p->size(K - 1), grad_p, static_cast<float2*>(grad_amps), S, batch, (float)(scale * scale));
-  });
-  HIP_TRY(hipGetLastError());
-  return SLOS_OK;
+  return run_readout_pull(p, dt, static_cast<const float2*>(U), batch, p->modes[p->n - 1],
+                          static_cast<const float2*>(psi_prev), grad_p, scale, static_cast<float2*>(grad_amps),
+                          reinterpret_cast<hipStream_t>(stream));
 }
 
 // work groups of the thread-per-state adjoint (grid-stride over the parents; one FP64 partial per
@@ -1832,6 +1905,40 @@ int slos_adjoint_workspace(const slos_plan* p, int64_t batch, int k, size_t* byt
   return SLOS_OK;
 }
 
+namespace {
+
+// the FP64 partials of layer k's dL/dU column and (unless null) grad_prev, as `L` (adjoint_launch)
+int run_adjoint(const slos_plan* p, const DevTables& dt, const AdjLaunch& L, const float2* U, int64_t batch, int k, int col,
+                const float2* psi, const float2* gk, float2* gout, double2* part, hipStream_t st) {
+  const uint64_t Sp = p->size(k - 1), Sk = p->size(k);
+  const uint32_t* ins = nullptr;
+  if (L.walk) {
+    const int rc = insert_table(p, st, &ins);
+    if (rc) return rc;
+  }
+  if (ins) {
+    const slos::BlockGrid bg{dim3((unsigned)L.nblk, (unsigned)batch), 0, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
+    slos::launch_adjoint_insert(k - 1 - slos::kSuf, bg, p->m, col, U, psi, gk, Sk, gout, Sp, L.per_wave, L.xcd_chunk, part,
+                                ins);
+  } else {  // (also inside a capture that comes before the first use of the table)
+    if (L.lds > lds_limit()) return fail(SLOS_ERANGE, "adjoint LDS exceeds the GPU's LDS (too many modes)");
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)L.nblk, (unsigned)batch), dim3(kAdjThreads), L.lds, st, dt.cg, dt.lo, p->me,
+                         p->multiset, k, p->m, col, U, psi, gk, Sk, gout, Sp, part, gout != nullptr);
+    };
+    const bool narrow = Sk < (1ull << 32);
+    if (narrow && k == 2) launch(k_adjoint_layer<1, slos::SpaceView32, true>);
+    else if (narrow && k == 3) launch(k_adjoint_layer<2, slos::SpaceView32, true>);
+    else if (narrow && k == 4) launch(k_adjoint_layer<3, slos::SpaceView32, true>);
+    else if (narrow && k == 5) launch(k_adjoint_layer<4, slos::SpaceView32, true>);
+    else with_km(k - 1, [&](auto km) { launch(k_adjoint_layer<decltype(km)::value>); });
+  }
+  HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+}  // namespace
+
 int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, int col, const void* psi_prev,
                        const void* grad_k, void* grad_prev, void* grad_U, int accumulate, void* ws, size_t ws_bytes,
                        slos_stream_t stream) {
@@ -1839,7 +1946,6 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   if (k < 1 || k > p->n) return fail(SLOS_EINVAL, "layer out of range");
   if (col < 0 || col >= p->m) return fail(SLOS_EINVAL, "input mode out of range");
   if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
-  const uint64_t Sp = p->size(k - 1), Sk = p->size(k);
   AdjLaunch L;
   int rc = adjoint_launch(p, k, &L);
   if (rc) return rc;
@@ -1848,31 +1954,174 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   rc = device_tables(p, &dt);
   if (rc) return rc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const auto* Uf = static_cast<const float2*>(U);
-  const auto* psi = static_cast<const float2*>(psi_prev);
-  const auto* gk = static_cast<const float2*>(grad_k);
-  auto* gout = static_cast<float2*>(grad_prev);
-  auto* part = static_cast<double2*>(ws);
-  const uint32_t* ins = nullptr;
-  if (L.walk) {
-    rc = insert_table(p, st, &ins);
-    if (rc) return rc;
-  }
-  if (ins) {
-    const slos::BlockGrid bg{dim3((unsigned)L.nblk, (unsigned)batch), 0, st, dt.cg, dt.lo, dt.tuples, p->me, p->multiset};
-    slos::launch_adjoint_insert(k - 1 - slos::kSuf, bg, p->m, col, Uf, psi, gk, Sk, gout, Sp, L.per_wave, L.xcd_chunk,
-                                part, ins);
-  } else {  // (also inside a capture that comes before the first use of the table)
-    if (L.lds > lds_limit()) return fail(SLOS_ERANGE, "adjoint LDS exceeds the GPU's LDS (too many modes)");
-    with_km(k - 1, [&](auto km) {
-      hipLaunchKernelGGL((k_adjoint_layer<decltype(km)::value>), dim3((unsigned)L.nblk, (unsigned)batch),
-                         dim3(kAdjThreads), L.lds, st, dt.cg, dt.lo, p->me, p->multiset, k, p->m, col, Uf, psi, gk, Sk,
-                         gout, Sp, part, grad_prev != nullptr);
-    });
-  }
-  HIP_TRY(hipGetLastError());
+  rc = run_adjoint(p, dt, L, static_cast<const float2*>(U), batch, k, col, static_cast<const float2*>(psi_prev),
+                   static_cast<const float2*>(grad_k), static_cast<float2*>(grad_prev), static_cast<double2*>(ws), st);
+  if (rc) return rc;
   hipLaunchKernelGGL(k_reduce_gu, dim3((unsigned)p->me, (unsigned)batch), dim3(kReduceThreads), 0, st,
                      static_cast<const double2*>(ws), (int)L.nblk, p->me, p->m, col, static_cast<float2*>(grad_U), accumulate);
+  HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+namespace {
+
+// the layers 0..layer-1 a backward pass reads, one after another [batch][S_k] at multiples of 256 bytes
+int saved_layout(const slos_plan* p, int64_t batch, int layer, std::vector<size_t>* at, size_t* total) {
+  uint64_t sum = 0;
+  for (int k = 0; k < layer; ++k) {
+    uint64_t bytes;
+    at->push_back((size_t)sum);
+    if (mul_overflow(p->size(k), (uint64_t)batch * sizeof(float2), &bytes) || bytes > (1ull << 62) ||
+        __builtin_add_overflow(sum, align256((size_t)bytes), &sum))
+      return fail(SLOS_ERANGE, "layer sizes overflow");
+  }
+  *total = (size_t)sum;
+  return SLOS_OK;
+}
+
+// workspace of a backward pass: the partials of every layer, and the gradients of two layers in turn
+struct BackLayout {
+  std::vector<AdjLaunch> L;       // of layer k at k - 1
+  std::vector<size_t> part;       // its partials (bytes from the workspace's begin)
+  size_t g[2] = {0, 0};           // gradients of the layers layer, layer - 2, ..; layer - 1, ..
+  size_t total = 0;
+};
+
+int back_layout(const slos_plan* p, int64_t batch, int layer, bool readout, BackLayout* b) {
+  size_t sum = 0;
+  for (int k = 1; k <= layer; ++k) {
+    AdjLaunch L;
+    const int rc = adjoint_launch(p, k, &L);
+    if (rc) return rc;
+    b->L.push_back(L);
+    b->part.push_back(sum);
+    sum += align256((size_t)batch * L.nblk * p->me * sizeof(double2));
+  }
+  for (int i = 0; i < 2; ++i) {
+    const int k = readout ? layer - i : layer - 1 - i;  // the largest layer of the two buffers
+    b->g[i] = sum;
+    if (k >= 1) sum += align256((size_t)batch * p->size(k) * sizeof(float2));
+  }
+  b->total = sum;
+  return SLOS_OK;
+}
+
+}  // namespace
+
+int slos_saved_bytes(const slos_plan* p, int64_t batch, int layer, size_t* bytes) {
+  if (!p || !bytes) return fail(SLOS_EINVAL, "NULL argument");
+  if (layer < 1 || layer > p->n || batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "bad argument");
+  std::vector<size_t> at;
+  return saved_layout(p, batch, layer, &at, bytes);
+}
+
+int slos_forward_saved(const slos_plan* p, const void* U, int64_t batch, const int32_t* modes, int layer, int probs,
+                       void* out, double scale, void* saved, size_t saved_bytes, slos_stream_t stream) {
+  int cols[kMaxPhotons] = {};
+  WsLayout w;
+  int rc = forward_check(p, U, batch, modes, layer, probs ? SLOS_OUT_PROBS : SLOS_OUT_AMPS, out, 0u, cols, &w);
+  if (rc) return rc;
+  if (layer < 1 || batch > 65535) return fail(SLOS_EINVAL, "bad argument");
+  std::vector<size_t> at;
+  size_t total = 0;
+  rc = saved_layout(p, batch, layer, &at, &total);
+  if (rc) return rc;
+  if (!saved || saved_bytes < total) return fail(SLOS_ENOMEM, "buffer of the layers too small");
+  DevTables dt;
+  rc = device_tables(p, &dt);
+  if (rc) return rc;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  void* layers[kMaxPhotons];
+  for (int k = 0; k < layer; ++k) layers[k] = static_cast<unsigned char*>(saved) + at[k];
+  const RoctxRange whole("slos_forward");
+  size_t lds = 0;
+  uint32_t buf = 0;
+  const int kf = front_layers(p, batch, layer - 1, 8, false, &lds, &buf);
+  if (kf) {
+    rc = run_front(p, dt, kf, cols, U, batch, layers[kf], 0, 1.0, 0u, lds, buf, false, st, layers);
+    if (rc) return rc;
+  } else {
+    hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>((batch + 255) / 256, 4096)), dim3(256), 0, st,
+                       static_cast<float2*>(layers[0]), batch);
+    HIP_TRY(hipGetLastError());
+  }
+  for (int k = kf + 1; k <= layer; ++k) {
+    const bool last = k == layer;
+    rc = launch_layer(p, dt, k, cols[k - 1], static_cast<const float2*>(U), batch,
+                      static_cast<const float2*>(layers[k - 1]), p->size(k - 1), last ? out : layers[k], p->size(k),
+                      last && probs ? 1 : 0, last ? (float)scale : 1.f, 0u, st);
+    if (rc) return rc;
+  }
+  return SLOS_OK;
+}
+
+int slos_backward_workspace(const slos_plan* p, int64_t batch, int layer, int grad_kind, size_t* bytes) {
+  if (!p || !bytes) return fail(SLOS_EINVAL, "NULL argument");
+  if (layer < 1 || layer > p->n || batch < 1 || batch > 65535 || grad_kind < 0 || grad_kind > 2)
+    return fail(SLOS_EINVAL, "bad argument");
+  BackLayout b;
+  const int rc = back_layout(p, batch, layer, grad_kind != 0, &b);
+  *bytes = b.total;
+  return rc;
+}
+
+int slos_backward(const slos_plan* p, const void* U, int64_t batch, const int32_t* modes, int layer, const void* saved,
+                  size_t saved_bytes, const void* grad, int grad_kind, double scale, void* grad_U, void* ws,
+                  size_t ws_bytes, slos_stream_t stream) {
+  if (!p || !U || !saved || !grad || !grad_U || !ws) return fail(SLOS_EINVAL, "NULL argument");
+  if (layer < 1 || layer > p->n || batch < 1 || batch > 65535 || grad_kind < 0 || grad_kind > 2)
+    return fail(SLOS_EINVAL, "bad argument");
+  if (grad_kind != 0 && layer != p->n) return fail(SLOS_EINVAL, "probabilities are those of the last layer");
+  ReduceArgs ra{};
+  std::vector<size_t> at;
+  size_t total = 0;
+  int rc = saved_layout(p, batch, layer, &at, &total);
+  if (rc) return rc;
+  if (saved_bytes < total) return fail(SLOS_ENOMEM, "buffer of the layers too small");
+  BackLayout b;
+  rc = back_layout(p, batch, layer, grad_kind != 0, &b);
+  if (rc) return rc;
+  if (ws_bytes < b.total) return fail(SLOS_ENOMEM, "workspace too small");
+  for (int k = 0; k < layer; ++k) {
+    ra.col[k] = modes ? modes[k] : p->modes[k];
+    if (ra.col[k] < 0 || ra.col[k] >= p->m) return fail(SLOS_EINVAL, "input mode out of range");
+    ra.part[k] = b.part[k] / sizeof(double2);
+    ra.nblk[k] = (uint32_t)b.L[k].nblk;
+  }
+  ra.layers = layer;
+  DevTables dt;
+  rc = device_tables(p, &dt);
+  if (rc) return rc;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const RoctxRange whole("slos_backward");
+  const auto* Uf = static_cast<const float2*>(U);
+  auto* base = static_cast<unsigned char*>(ws);
+  auto psi = [&](int k) { return reinterpret_cast<const float2*>(static_cast<const unsigned char*>(saved) + at[k]); };
+  const auto* gk = static_cast<const float2*>(grad);
+  int next = 0;
+  if (grad_kind != 0) {
+    auto* g = reinterpret_cast<float2*>(base + b.g[0]);
+    const auto* gp = static_cast<const float*>(grad);
+    if (grad_kind == 1) {  // the amplitudes again, with the readout's adjoint in the same pass
+      rc = launch_layer(p, dt, layer, ra.col[layer - 1], Uf, batch, psi(layer - 1), p->size(layer - 1), g, p->size(layer), 4,
+                        (float)(scale * scale), 0u, st, false, false, gp);
+    } else {
+      rc = run_readout_pull(p, dt, Uf, batch, ra.col[layer - 1], psi(layer - 1), gp, scale, g, st);
+    }
+    if (rc) return rc;
+    gk = g;
+    next = 1;
+  }
+  for (int k = layer; k >= 1; --k) {
+    auto* gout = k > 1 ? reinterpret_cast<float2*>(base + b.g[next]) : nullptr;
+    rc = run_adjoint(p, dt, b.L[k - 1], Uf, batch, k, ra.col[k - 1], psi(k - 1), gk, gout,
+                     reinterpret_cast<double2*>(base + b.part[k - 1]), st);
+    if (rc) return rc;
+    gk = gout;
+    next ^= 1;
+  }
+  hipLaunchKernelGGL(k_reduce_all, dim3((unsigned)p->m, (unsigned)batch), dim3(kReduceAllThreads), 0, st, ra,
+                     reinterpret_cast<const double2*>(base), p->me, p->m, static_cast<float2*>(grad_U));
   HIP_TRY(hipGetLastError());
   return SLOS_OK;
 }

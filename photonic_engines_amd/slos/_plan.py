@@ -243,6 +243,38 @@ class Plan:
                          nat.stream_handle(U.device)), "slos_adjoint_layer")
         return gprev
 
+    def saved_bytes(self, batch: int, layer: int) -> int:
+        """Device bytes forward_saved keeps: the layers 0..layer-1 of `batch` rows."""
+        out = ctypes.c_size_t()
+        nat.check(self._lib.slos_saved_bytes(self._h, batch, layer, ctypes.byref(out)), "slos_saved_bytes")
+        return int(out.value)
+
+    def forward_saved(self, U: torch.Tensor, modes, layer: int, probs: bool, scale: float, saved_bytes: int):
+        """(output, saved): the last layer's probabilities (scaled) or raw amplitudes of a contiguous
+        complex64 U [B, m, m], B <= MAX_ROWS, and the layers below it for `backward`."""
+        B, dev = U.shape[0], U.device
+        out = torch.empty((B, self.sizes[layer]), dtype=torch.float32 if probs else torch.complex64, device=dev)
+        saved = torch.empty(saved_bytes, dtype=torch.uint8, device=dev)
+        nat.check(self._lib.slos_forward_saved(self._h, nat.ptr(U), B, (ctypes.c_int32 * layer)(*modes), layer,
+                                               int(probs), nat.ptr(out), float(scale), nat.ptr(saved), saved_bytes,
+                                               nat.stream_handle(dev)), "slos_forward_saved")
+        return out, saved
+
+    def backward(self, U: torch.Tensor, modes, layer: int, saved: torch.Tensor, grad: torch.Tensor, grad_kind: int,
+                 scale: float) -> torch.Tensor:
+        """dL/dU from the gradient of forward_saved's output (grad_kind 0: of the raw amplitudes, 1: of
+        the probabilities, 2: of the probabilities, zero almost everywhere)."""
+        B, dev = U.shape[0], U.device
+        wsb = ctypes.c_size_t()
+        nat.check(self._lib.slos_backward_workspace(self._h, B, layer, grad_kind, ctypes.byref(wsb)),
+                  "slos_backward_workspace")
+        ws = torch.empty(max(int(wsb.value), 1), dtype=torch.uint8, device=dev)
+        gU = torch.empty_like(U)
+        nat.check(self._lib.slos_backward(self._h, nat.ptr(U), B, (ctypes.c_int32 * layer)(*modes), layer, nat.ptr(saved),
+                                          saved.numel(), nat.ptr(grad), grad_kind, float(scale), nat.ptr(gU), nat.ptr(ws),
+                                          ws.numel(), nat.stream_handle(dev)), "slos_backward")
+        return gU
+
     def loss_descend(self, k: int, q: torch.Tensor, flags: int = 0, scale: float = 1.0) -> torch.Tensor:
         """q_{k-1} = scale * descent of q_k ([B, S_k] float32, or float64 in FP64, contiguous on the GPU)."""
         out = torch.empty((q.shape[0], self.sizes[k - 1]), dtype=q.dtype, device=q.device)

@@ -1,9 +1,10 @@
 """Hand-written adjoint of the SLOS recurrence behind torch.autograd.Function.
 
 Replaces autograd through gather / mul / scatter_add_ (photonic_engines/slos/kernel.py:216-257)
-and the opt-in recomputing layer (_CheckpointedLayer, kernel.py:40-80). A forward keeps only every
-other layer (the even ones); the backward recomputes each odd layer once from the even layer below
-it, then runs the recurrence backwards with the adjoint kernels:
+and the opt-in recomputing layer (_CheckpointedLayer, kernel.py:40-80). A forward keeps the layers below
+the last where they are small (KEEP_BYTES), else every other layer (the even ones), and the backward
+then recomputes each odd layer once from the even layer below it; it runs the recurrence backwards with
+the adjoint kernels:
 
   readout   g_n = 2 s^2 prod(t!) dL/dp * psi_n            (p = |s psi_n|^2 prod t!)
   layer k   g_{k-1}[t] = sum_j conj(U[j, i_k]) g_k[t + e_j]
@@ -23,6 +24,7 @@ from __future__ import annotations
 import torch
 
 from .. import _native as nat
+from ._plan import MAX_ROWS
 
 
 def _layer_flags(kernel) -> int:
@@ -86,6 +88,22 @@ def _sparse(grad_p: torch.Tensor) -> bool:
     return int(torch.count_nonzero(sample)) * SPARSE_READOUT <= sample.numel()
 
 
+# A forward keeps every layer below the last while these take at most KEEP_BYTES (and the kernel was not
+# asked for checkpointing): forward and backward are then one native call each, and no layer is
+# recomputed but the last, in the pass that applies the readout's adjoint. Above it the even layers are
+# kept and the odd ones recomputed, layer by layer.
+KEEP_BYTES = 1 << 30
+
+
+def _kept_bytes(kernel, Ug: torch.Tensor, layer: int, cf: int) -> int | None:
+    """Bytes of the layers a forward keeps for the native backward, or None where it does not apply
+    (complex128 and compensated sums have the layer-by-layer backward only)."""
+    if cf or Ug.dtype != torch.complex64 or kernel.gradient_checkpointing or not 1 <= Ug.shape[0] <= MAX_ROWS:
+        return None
+    n = kernel._plan.saved_bytes(Ug.shape[0], layer)
+    return n if n <= KEEP_BYTES else None
+
+
 def _user_grad(gU: torch.Tensor, ctx) -> torch.Tensor:
     gU = gU.to(device=ctx.user_device, dtype=ctx.user_dtype)
     return gU.squeeze(0) if len(ctx.user_shape) == 2 else gU
@@ -96,11 +114,14 @@ class SLOSProbs(torch.autograd.Function):
     def forward(ctx, U_user: torch.Tensor, Ug: torch.Tensor, kernel) -> torch.Tensor:
         plan, modes, n = kernel._plan, kernel.input_modes, kernel.n
         cf = _layer_flags(kernel)                        # every layer as in the forward without grad
-        saved, psi = _checkpointed_forward(plan, Ug, modes, n, cf)
-        p = plan.layer_step(Ug, n, modes[n - 1], psi, nat.OUT_PROBS, scale=kernel._input_norm, flags=cf)
-        ctx.kernel, ctx.saved, ctx.Ug, ctx.cf = kernel, saved, Ug, cf
+        ctx.kernel, ctx.Ug, ctx.cf = kernel, Ug, cf
         ctx.user_shape, ctx.user_dtype, ctx.user_device = U_user.shape, U_user.dtype, U_user.device
-        return p
+        kept = _kept_bytes(kernel, Ug, n, cf)
+        if kept is not None:
+            p, ctx.saved = plan.forward_saved(Ug, modes, n, True, kernel._input_norm, kept)
+            return p
+        ctx.saved, psi = _checkpointed_forward(plan, Ug, modes, n, cf)
+        return plan.layer_step(Ug, n, modes[n - 1], psi, nat.OUT_PROBS, scale=kernel._input_norm, flags=cf)
 
     @staticmethod
     def backward(ctx, grad_p: torch.Tensor):
@@ -108,6 +129,10 @@ class SLOSProbs(torch.autograd.Function):
         plan, modes, n = kernel._plan, kernel.input_modes, kernel.n
         rdt = torch.float64 if Ug.dtype == torch.complex128 else torch.float32
         grad_p = grad_p.to(device=Ug.device, dtype=rdt).contiguous()
+        if isinstance(saved, torch.Tensor):
+            gU = plan.backward(Ug, modes, n, saved, grad_p, 2 if _sparse(grad_p) else 1, kernel._input_norm)
+            ctx.saved = None
+            return _user_grad(gU, ctx), None, None
         psi_prev = saved[n - 1] if (n - 1) in saved else plan.layer_step(Ug, n - 1, modes[n - 2], saved[n - 2],
                                                                           nat.OUT_RAW, flags=cf)
         if Ug.dtype == torch.complex64 and not cf and _sparse(grad_p):
@@ -130,17 +155,24 @@ class SLOSRaw(torch.autograd.Function):
         plan = kernel._plan
         modes = [int(c) for c in modes]
         cf = _layer_flags(kernel)
-        saved, psi = _checkpointed_forward(plan, Ug, modes, layer, cf)
-        out = _hi(plan.layer_step(Ug, layer, modes[layer - 1], psi, nat.OUT_RAW, flags=cf))
-        ctx.kernel, ctx.saved, ctx.Ug, ctx.cf, ctx.modes, ctx.layer = kernel, saved, Ug, cf, modes, layer
+        ctx.kernel, ctx.Ug, ctx.cf, ctx.modes, ctx.layer = kernel, Ug, cf, modes, layer
         ctx.user_shape, ctx.user_dtype, ctx.user_device = U_user.shape, U_user.dtype, U_user.device
-        return out
+        kept = _kept_bytes(kernel, Ug, layer, cf)
+        if kept is not None:
+            out, ctx.saved = plan.forward_saved(Ug, modes, layer, False, 1.0, kept)
+            return out
+        ctx.saved, psi = _checkpointed_forward(plan, Ug, modes, layer, cf)
+        return _hi(plan.layer_step(Ug, layer, modes[layer - 1], psi, nat.OUT_RAW, flags=cf))
 
     @staticmethod
     def backward(ctx, grad_out: torch.Tensor):
         kernel, saved, Ug, cf, modes, layer = ctx.kernel, ctx.saved, ctx.Ug, ctx.cf, ctx.modes, ctx.layer
         plan = kernel._plan
         g = grad_out.to(device=Ug.device, dtype=Ug.dtype).contiguous()
+        if isinstance(saved, torch.Tensor):
+            gU = plan.backward(Ug, modes, layer, saved, g, 0, 1.0)
+            ctx.saved = None
+            return _user_grad(gU, ctx), None, None, None, None
         psi_prev = saved[layer - 1] if (layer - 1) in saved else plan.layer_step(
             Ug, layer - 1, modes[layer - 2], saved[layer - 2], nat.OUT_RAW, flags=cf)
         gU = _adjoint_layers(plan, Ug, modes, layer, saved, cf, g, psi_prev)
