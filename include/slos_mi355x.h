@@ -197,6 +197,18 @@ int slos_loss_descend(const slos_plan* plan, int k, const float* q_k, float* q_k
                       double scale,
                       slos_stream_t stream);
 
+/* The x-model's distribution on the last layer (species.py:123-146) of 3 <= n <= 24 photons in one
+ * call: float32 out [batch][S_n] = the sum over the sets T of at most `order` (1 <= order <= n)
+ * distinguishable photons of weights[|T|] times the distribution of the others interfering and T raised
+ * (slos_raise), the terms sharing their raises. `weights`: n + 2 floats, on the host or (weights_on_device)
+ * the GPU: weights[L], L <= n - 2, of each set of L photons, and weights[n + 1] of all sets of n - 1
+ * and n photons together. flags: SLOS_FLAG_COMPENSATED or 0 (the forwards' sums). U: complex64
+ * [batch][m][m], W: float32 |U|^2, batch <= 65535; the sets of all sizes together at most 2^20. */
+int slos_xmodel_workspace(const slos_plan* plan, int64_t batch, int order, unsigned flags, size_t* bytes);
+int slos_xmodel(const slos_plan* plan, const void* U, const float* W, int64_t batch, int order,
+                const float* weights, int weights_on_device, float* out, unsigned flags, void* workspace, size_t workspace_bytes,
+                slos_stream_t stream);
+
 /* Probability-level raise of partial distinguishability (species.classical_raise,
  * slos/species.py:37-56): a photon that interferes with nothing enters column col, and
  * q_k(c) = sum_{j distinct in c} w[b][j] q_{k-1}(c - e_j) with w[b][j] = |U[b, j, col]|^2 (device

@@ -133,6 +133,35 @@ SLOS_HD void unrank_fixed(const SV& sv, RankT<SV> g, int K, int (&p)[KM]) {
 //   cg[N][0] - sum_{i <= N-2} cg[N-i][p_i + 1] - cg[1][p_(N-1)],
 // so a child needs two table entries a position: its own terms X (the positions after a dropped one
 // keep theirs) and the terms Y of the positions before a dropped one, which have one photon fewer.
+// parent_ranks: the rank without position l, for every l < K, and whether l is its mode's first copy (a
+// repeated position's rank is its first copy's).
+template <int KM, class SV>
+SLOS_HD void parent_ranks(const SV& sv, int multiset, int K, const int (&p)[KM], RankT<SV> (&rank)[KM], bool (&first)[KM]) {
+  typedef RankT<SV> R;
+  R Y[KM], SX[KM + 1];
+  SX[KM] = 0;
+#pragma unroll
+  for (int i = KM - 1; i >= 0; --i) {
+    SX[i] = 0;
+    Y[i] = 0;
+    if (i < K) {
+      SX[i] = SX[i + 1] + (i == K - 1 ? sv.C(1, p[i]) : sv.C(K - i, p[i] + 1));
+      if (i < K - 1) Y[i] = i == K - 2 ? sv.C(1, p[i]) : sv.C(K - 1 - i, p[i] + 1);
+    }
+  }
+  R rest = K == 1 ? SX[1] : sv.C(K - 1, 0);
+#pragma unroll
+  for (int l = 0; l < KM; ++l) {
+    first[l] = false;
+    rank[l] = 0;
+    if (l < K) {
+      rank[l] = rest - SX[l + 1];
+      first[l] = !multiset || l == 0 || p[l] != p[in_range<KM>(l - 1)];
+      rest -= Y[l];
+    }
+  }
+}
+
 template <int KM, class SV, class F>
 SLOS_HD void parents_fixed(const SV& sv, int multiset, int K, const int (&p)[KM], F&& f) {
   typedef RankT<SV> R;

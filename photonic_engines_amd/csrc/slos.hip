@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -27,6 +28,7 @@
 #include "pull_index.hpp"
 #include "block_launch.hpp"
 #include "front.hpp"
+#include "raise.hpp"
 
 namespace {
 
@@ -55,6 +57,7 @@ struct DevTables {
   int* modes = nullptr;                    // the plan's input modes (spot permanents)
   slos::TupleWord* tuples = nullptr;       // block-kernel suffix-tuple words (may be absent)
   uint64_t* tuples5 = nullptr;             // the same for 5-position suffixes (may be absent)
+  uint32_t* xm[33] = {};                   // x-model rows of the levels 0..L (see xmodel_tables)
   uint32_t* insert = nullptr;              // insert table of the pulls over children (see insert_table)
   uint4* items[33] = {};                   // group-order work items of layer K (may be absent)
   uint32_t n_items[33] = {};
@@ -68,6 +71,16 @@ struct DevTables {
   static constexpr uint64_t kFineItems = 1ull << 23;
 };
 
+// The rows of the x-model's levels 0..L (raise.hpp): masks of a level from at[level] on, and from
+// off[level] on, per row of the level, the index of its first source in the next level (one more entry:
+// their number); `zeros`: as many zero entries as the largest level has rows, and one.
+struct XRows {
+  std::vector<uint32_t> words;
+  std::vector<size_t> at, off, rows;
+  size_t zeros = 0;
+  uint64_t most = 0;
+};
+
 struct slos_plan {
   int n = 0, m = 0, mask = 0, me = 0, multiset = 1, shift = 0;
   std::vector<int> modes;
@@ -78,6 +91,7 @@ struct slos_plan {
   std::vector<uint64_t> tuples5;         // 5-position suffix-tuple words (empty: unused)
   std::vector<uint32_t> items[33];       // group-order work items of layer K, 4 words each (empty: unused)
   std::vector<uint32_t> fine[33];        // the same in small items, for layers of fewer than kFineItems states
+  std::unique_ptr<const XRows> xrows[33];  // x-model rows of the levels 0..L, built by the first call
   std::vector<DevTables> dev;
   std::mutex mu;
   slos::SpaceView host_view() const { return slos::SpaceView{cg.data(), lo.data(), me, me + 1}; }
@@ -1487,6 +1501,8 @@ int slos_plan_destroy(slos_plan* p) {
     if (t.tuples) (void)hipFree(t.tuples);
     if (t.tuples5) (void)hipFree(t.tuples5);
     if (t.insert) (void)hipFree(t.insert);
+    for (auto* x : t.xm)
+      if (x) (void)hipFree(x);
     for (auto* it : t.items)
       if (it) (void)hipFree(it);
     for (auto* it : t.fine)
@@ -2203,6 +2219,238 @@ int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1,
                        dt.cg, dt.lo, p->me, p->multiset, k, q_k, Sk, q_km1, Sp, batch, (float)scale);
   });
   HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+namespace {
+
+constexpr uint64_t kXRows = 1u << 20;  // rows of all levels together
+
+bool xmodel_rows(int n, int levels, XRows* x) {
+  std::vector<uint32_t> level{0u};
+  uint64_t total = 0;
+  for (int L = 0; L <= levels; ++L) {
+    total += level.size();
+    if (total > kXRows) return false;
+    x->rows.push_back(level.size());
+    x->most = std::max<uint64_t>(x->most, level.size());
+    x->at.push_back(x->words.size());
+    x->words.insert(x->words.end(), level.begin(), level.end());
+    x->off.push_back(x->words.size());
+    std::vector<uint32_t> next;
+    for (const uint32_t t : level) {
+      x->words.push_back((uint32_t)next.size());
+      const int first = t ? __builtin_ctz(t) : n;
+      for (int j = 0; j < first; ++j) next.push_back(t | (1u << j));
+      if (next.size() > kXRows) return false;
+    }
+    x->words.push_back((uint32_t)next.size());
+    level.swap(next);
+  }
+  x->zeros = x->words.size();
+  x->words.insert(x->words.end(), x->most + 1, 0u);
+  return true;
+}
+
+// the plan's rows of the levels 0..levels (null: more than kXRows)
+const XRows* xmodel_host_rows(const slos_plan* cp, int levels) {
+  slos_plan* p = const_cast<slos_plan*>(cp);
+  std::lock_guard<std::mutex> g(p->mu);
+  if (!p->xrows[levels]) {
+    auto x = std::make_unique<XRows>();
+    if (!xmodel_rows(p->n, levels, x.get())) return nullptr;
+    p->xrows[levels] = std::move(x);
+  }
+  return p->xrows[levels].get();
+}
+
+// the same on the current GPU
+int xmodel_tables(const slos_plan* cp, int levels, const XRows& x, const uint32_t** out) {
+  slos_plan* p = const_cast<slos_plan*>(cp);
+  int d = 0;
+  HIP_TRY(hipGetDevice(&d));
+  std::lock_guard<std::mutex> g(p->mu);
+  for (auto& t : p->dev)
+    if (t.device == d) {
+      if (!t.xm[levels]) {
+        uint32_t* dev = nullptr;
+        HIP_TRY(hipMalloc(&dev, x.words.size() * sizeof(uint32_t)));
+        const hipError_t e = hipMemcpy(dev, x.words.data(), x.words.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+          (void)hipFree(dev);
+          HIP_TRY(e);
+        }
+        t.xm[levels] = dev;
+      }
+      *out = t.xm[levels];
+      return SLOS_OK;
+    }
+  return fail(SLOS_EINVAL, "no device tables");
+}
+
+struct XLayout {
+  const XRows* rows = nullptr;
+  int levels = 0;                 // the most distinguishable photons beside at least two interfering ones
+  size_t A[2] = {0, 0}, chain[2] = {0, 0}, scale = 0, one = 0, up = 0, fwd = 0, total = 0;
+  std::vector<uint32_t> chunk;    // rows of one forward, per level
+};
+
+int xmodel_layout(const slos_plan* p, int64_t B, int order, unsigned flags, XLayout* x) {
+  const int n = p->n;
+  if (n < 3 || n > slos::kRaisePhotons || order < 1 || order > n || B < 1 || B > 65535)
+    return fail(SLOS_EINVAL, "bad argument");
+  x->levels = std::min(order, n - 2);
+  x->rows = xmodel_host_rows(p, x->levels);
+  if (!x->rows) return fail(SLOS_ERANGE, "too many subsets");
+  uint64_t A[2] = {0, 0}, up = 0, fwd = 0;
+  for (int L = 0; L <= x->levels; ++L) {
+    const uint64_t R = x->rows->rows[L];
+    uint64_t bytes;
+    if (mul_overflow(p->size(n - L), R * (uint64_t)B * sizeof(float), &bytes) || bytes > (1ull << 62))
+      return fail(SLOS_ERANGE, "layer sizes overflow");
+    if (L) A[L & 1] = std::max(A[L & 1], bytes);
+    WsLayout w;
+    const int rc = forward_layout(p, B, n - L, &w, (flags & SLOS_FLAG_COMPENSATED) != 0, false);
+    if (rc) return rc;
+    const uint64_t row = w.total + (uint64_t)B * p->m * p->m * sizeof(float2);
+    const uint64_t fit = std::min<uint64_t>({R, 65535u / (uint64_t)B, (1ull << 30) / row});
+    x->chunk.push_back((uint32_t)std::max<uint64_t>(1, fit));
+    WsLayout wc;
+    const int rc2 = forward_layout(p, B * (int64_t)x->chunk[L], n - L, &wc, (flags & SLOS_FLAG_COMPENSATED) != 0, false);
+    if (rc2) return rc2;
+    fwd = std::max<uint64_t>(fwd, wc.total);
+    up = std::max<uint64_t>(up, (uint64_t)x->chunk[L] * (uint64_t)B * p->m * p->m * sizeof(float2));
+  }
+  size_t sum = 0;
+  auto take = [&](size_t* at, uint64_t bytes) {
+    *at = sum;
+    sum += align256((size_t)bytes);
+  };
+  take(&x->A[0], A[0]);
+  take(&x->A[1], A[1]);
+  take(&x->chain[0], (uint64_t)B * sizeof(float));
+  take(&x->chain[1], (uint64_t)B * p->size(1) * sizeof(float));
+  take(&x->scale, x->rows->most * sizeof(float));
+  take(&x->one, sizeof(float));
+  take(&x->up, up);
+  take(&x->fwd, fwd);
+  x->total = sum;
+  return SLOS_OK;
+}
+
+}  // namespace
+
+int slos_xmodel_workspace(const slos_plan* p, int64_t batch, int order, unsigned flags, size_t* bytes) {
+  if (!p || !bytes) return fail(SLOS_EINVAL, "NULL argument");
+  XLayout x;
+  const int rc = xmodel_layout(p, batch, order, flags, &x);
+  *bytes = x.total;
+  return rc;
+}
+
+int slos_xmodel(const slos_plan* p, const void* U, const float* W, int64_t batch, int order, const float* weights,
+                int weights_on_device, float* out, unsigned flags, void* ws, size_t ws_bytes, slos_stream_t stream) {
+  if (!p || !U || !W || !weights || !out || !ws) return fail(SLOS_EINVAL, "NULL argument");
+  if (flags & ~(unsigned)SLOS_FLAG_COMPENSATED) return fail(SLOS_EINVAL, "unsupported flag");
+  XLayout x;
+  int rc = xmodel_layout(p, batch, order, flags, &x);
+  if (rc) return rc;
+  if (ws_bytes < x.total) return fail(SLOS_ENOMEM, "workspace too small");
+  DevTables dt;
+  rc = device_tables(p, &dt);
+  if (rc) return rc;
+  const uint32_t* tab = nullptr;
+  rc = xmodel_tables(p, x.levels, *x.rows, &tab);
+  if (rc) return rc;
+  const int n = p->n;
+  const int B = (int)batch;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const RoctxRange whole("slos_xmodel");
+  auto* base = static_cast<unsigned char*>(ws);
+  auto* scale = reinterpret_cast<float*>(base + x.scale);
+  auto* one = reinterpret_cast<float*>(base + x.one);
+  auto level = [&](int L) { return L ? reinterpret_cast<float*>(base + x.A[L & 1]) : out; };
+  // the terms of L distinguishable photons: every subset's forward, and the rows' weights
+  auto start = [&](int L) {
+    const uint32_t R = (uint32_t)x.rows->rows[L];
+    const int g = n - L;
+    int cols[kMaxPhotons];
+    for (int i = 0; i < g; ++i) cols[i] = i;
+    for (uint32_t r0 = 0; r0 < R; r0 += x.chunk[L]) {
+      slos::SubsetArgs a{};
+      a.U = static_cast<const float2*>(U);
+      a.Up = reinterpret_cast<float2*>(base + x.up);
+      a.masks = tab + x.rows->at[L];
+      a.r0 = r0;
+      a.rows = std::min(x.chunk[L], R - r0);
+      a.B = B; a.m = p->m; a.n = n; a.g = g;
+      a.row_scale = scale;
+      for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
+      slos::launch_subsets(st, a);
+      HIP_TRY(hipGetLastError());
+      const int64_t rows = (int64_t)a.rows * B;
+      WsLayout w;
+      int rc = forward_layout(p, rows, g, &w, (flags & SLOS_FLAG_COMPENSATED) != 0, false);
+      if (rc) return rc;
+      rc = forward_run(p, dt, a.Up, rows, cols, g, SLOS_OUT_PROBS, level(L) + (size_t)r0 * B * p->size(g), 1.0, flags, w,
+                       base + x.fwd, st);
+      if (rc) return rc;
+    }
+    return (int)SLOS_OK;
+  };
+  // targets += their sources, raised (off: see RaiseArgs), the targets scaled
+  auto raise = [&](int K, const float* q, float* to, uint32_t targets, const uint32_t* off, int photon, const float* row_scale,
+                   int weight) {
+    slos::RaiseArgs a{};
+    a.cg = dt.cg; a.lo = dt.lo; a.words = dt.tuples5; a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.K = K; a.B = B;
+    a.S_par = p->size(K - 1); a.S = p->size(K);
+    a.q = q; a.out = to; a.targets = targets; a.off = off; a.photon = photon; a.photons = off ? n : 1;
+    a.row_scale = row_scale;
+    if (weight < 0) a.weight_value = 1.f;
+    else if (weights_on_device) a.weight = weights + weight;
+    else a.weight_value = weights[weight];
+    a.W = W;
+    for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
+    const size_t lds = slos::raise_lds(K, p->me, a.photons);
+    if (lds > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
+    const uint64_t wgs = (a.S + 255) / 256;
+    if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
+    // a work group takes all targets of its states where there are enough states: 2048 work groups fill
+    // the chip
+    const uint64_t parts = std::min<uint64_t>({targets, 65535u, (2048 + wgs * B - 1) / (wgs * B)});
+    a.rows_per = (uint32_t)((targets + parts - 1) / parts);
+    const unsigned z = (targets + a.rows_per - 1) / a.rows_per;
+    slos::launch_raise(dim3((unsigned)wgs, (unsigned)B, z), lds, st, a);
+    HIP_TRY(hipGetLastError());
+    return (int)SLOS_OK;
+  };
+  const int top = x.levels;
+  rc = start(top);
+  if (rc) return rc;
+  rc = raise(n - top, level(top), level(top), (uint32_t)x.rows->rows[top], tab + x.rows->zeros, 0, scale, top);
+  if (rc) return rc;
+  if (order >= n - 1) {
+    // the terms with fewer than two interfering photons: photons 0 and 1 raised from the vacuum into
+    // the set of the others
+    auto* c0 = reinterpret_cast<float*>(base + x.chain[0]);
+    auto* c1 = reinterpret_cast<float*>(base + x.chain[1]);
+    slos::launch_chain_start(st, c0, B, one, weights_on_device ? weights + n + 1 : nullptr,
+                             weights_on_device ? 0.f : weights[n + 1]);
+    HIP_TRY(hipGetLastError());
+    rc = raise(1, c0, c1, 1, nullptr, 0, nullptr, -1);
+    if (rc) return rc;
+    const uint32_t others = ((1u << n) - 1u) & ~3u;
+    const uint32_t* masks = x.rows->words.data() + x.rows->at[top];
+    const size_t row = std::find(masks, masks + x.rows->rows[top], others) - masks;
+    rc = raise(2, c1, level(top) + row * B * p->size(2), 1, nullptr, 1, one, -1);
+    if (rc) return rc;
+  }
+  for (int L = top; L >= 1; --L) {
+    rc = start(L - 1);
+    if (rc) return rc;
+    rc = raise(n - L + 1, level(L), level(L - 1), (uint32_t)x.rows->rows[L - 1], tab + x.rows->off[L - 1], 0, scale, L - 1);
+    if (rc) return rc;
+  }
   return SLOS_OK;
 }
 

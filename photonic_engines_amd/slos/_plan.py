@@ -243,6 +243,23 @@ class Plan:
                          nat.stream_handle(U.device)), "slos_adjoint_layer")
         return gprev
 
+    def xmodel(self, U: torch.Tensor, W: torch.Tensor, order: int, weights, flags: int = 0) -> torch.Tensor:
+        """The x-model's distribution [B, S_n] of a contiguous complex64 U [B, m, m] (slos_xmodel);
+        W its float32 squared magnitudes, `weights` a float32 GPU tensor or a list of n + 2 floats."""
+        B, dev = U.shape[0], U.device
+        wsb = ctypes.c_size_t()
+        nat.check(self._lib.slos_xmodel_workspace(self._h, B, order, int(flags), ctypes.byref(wsb)), "slos_xmodel_workspace")
+        need, out_bytes = int(wsb.value), 4 * B * self.sizes[self.n]
+        self.preflight(out_bytes + need, dev, f"SLOS x-model (n={self.n}, m={self.m}, batch {B}: output {out_bytes:,} B, "
+                       f"workspace {need:,} B)")
+        out = torch.empty((B, self.sizes[self.n]), dtype=torch.float32, device=dev)
+        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+        on_device = isinstance(weights, torch.Tensor)
+        wp = nat.ptr(weights) if on_device else (ctypes.c_float * len(weights))(*weights)
+        nat.check(self._lib.slos_xmodel(self._h, nat.ptr(U), nat.ptr(W), B, order, wp, int(on_device), nat.ptr(out), int(flags),
+                                        nat.ptr(ws), need, nat.stream_handle(dev)), "slos_xmodel")
+        return out
+
     def saved_bytes(self, batch: int, layer: int) -> int:
         """Device bytes forward_saved keeps: the layers 0..layer-1 of `batch` rows."""
         out = ctypes.c_size_t()

@@ -35,6 +35,7 @@ import torch
 
 from .. import _native as nat
 from ..imperfections import spec
+from ._plan import MAX_ROWS
 
 
 def _needs_grad(U: torch.Tensor) -> bool:
@@ -191,6 +192,33 @@ def _raise_rows(kernel, q: torch.Tensor, k: int, W: torch.Tensor) -> torch.Tenso
     return kernel._plan.layer_step(Uw, k + 1, 0, qc, nat.OUT_RAW).real
 
 
+# sets of distinguishable photons the one-call x-model takes, and its photons
+_NATIVE_SETS, _NATIVE_PHOTONS = 1 << 20, 24
+
+
+def _weights(x: torch.Tensor, n: int, b_max: int) -> torch.Tensor:
+    """float64 [n + 2] (and x's own shape): x^(n-L) (1-x)^L, the weight of each set of L distinguishable photons, for L = 0..n,
+    then the weight of all sets of n - 1 and n photons that b_max admits together. Differentiable in x."""
+    L = torch.arange(n + 1, dtype=torch.float64, device=x.device).reshape(-1, *([1] * x.dim()))
+    xd = x.double()
+    w = xd ** (n - L) * (1 - xd) ** L
+    top = sum(math.comb(n, k) * w[k] for k in (n, n - 1) if 0 <= k <= b_max)
+    return torch.cat([w, torch.as_tensor(top, dtype=w.dtype, device=x.device).expand(1, *x.shape)])
+
+
+def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, b_max: int) -> torch.Tensor | None:
+    """The mixture [B, S_n] in one native call (slos_xmodel), or None where that does not apply: with a
+    gradient, in FP64, without a distinguishable photon or with fewer than three photons."""
+    n = len(kernel.input_modes)
+    if (Ub.dtype != torch.complex64 or _needs_grad(Ub) or _needs_grad(x) or x.dim() != 0 or b_max < 1
+            or not 3 <= n <= _NATIVE_PHOTONS or not 1 <= Ub.shape[0] <= MAX_ROWS
+            or sum(math.comb(n, L) for L in range(min(b_max, n - 2) + 2)) > _NATIVE_SETS):
+        return None
+    w = _weights(x.detach(), n, b_max)
+    return kernel._plan.xmodel(Ub, Ub.abs() ** 2, b_max, w.tolist() if w.device.type == "cpu" else w.float(),
+                               nat.FLAG_COMPENSATED if kernel.compensated else 0)
+
+
 def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torch.Tensor:
     """The x-model distribution on the final layer ([S] or [B, S], rdtype): the sum over the
     interfering subsets G of the input photons of x^|G| (1 - x)^(n - |G|) species_probs(G, rest).
@@ -205,19 +233,23 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
     one batched layer step, and the contributions are added in ascending order of T. A[()] is the
     result. The final layer then takes n raises instead of one per subset. An interfering set of
     fewer than two photons is itself classical: its photons join T (a single photon's
-    distribution is its column |U[:, c]|^2)."""
+    distribution is its column |U[:, c]|^2). Without a gradient, in complex64, all of it is one native
+    call (_native_x) with the same bits."""
     d = spec(indist)
     if d.x is None:
         raise NotImplementedError("strong simulation: the x-model only (random species need a partition sum)")
     Ub, batched = _batched_u(kernel, U)
     rdt = kernel.rdtype
-    x = indist if isinstance(indist, torch.Tensor) else torch.tensor(d.x, dtype=rdt)
-    x = x.to(dtype=rdt, device=Ub.device)
+    x = indist.to(dtype=rdt) if isinstance(indist, torch.Tensor) else torch.tensor(d.x, dtype=rdt)
     cols = kernel.input_modes
     n = len(cols)
+    b_max = n if order is None else max(0, min(int(order), n))
+    native = _native_x(kernel, Ub, x, b_max)
+    if native is not None:
+        return kernel._out(native, batched)
+    weights = _weights(x, n, b_max).to(dtype=rdt, device=Ub.device)
     B, m = Ub.shape[0], Ub.shape[-1]
     dev = Ub.device
-    b_max = n if order is None else max(0, min(int(order), n))
     per = max(1, (2 << 30) // (rdt.itemsize * kernel.layers.size(n) * max(B, 1)))
     A: dict = {}
 
@@ -227,7 +259,7 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
     def start(L):
         # the terms whose distinguishable set has L photons (at least two interfering): weight
         # x^(n-L) (1-x)^L
-        w = x ** (n - L) * (1 - x) ** L
+        w = weights[L]
         bads = list(combinations(range(n), L))
         for i0 in range(0, len(bads), per):
             chunk = bads[i0:i0 + per]
@@ -238,13 +270,8 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
 
     # fewer than two interfering photons: the whole input is classical, every photon raised from the
     # vacuum (C(n, L) such terms for L = n and n - 1)
-    wc = None
-    for L in (n, n - 1):
-        if 0 <= L <= b_max and n - L <= 1:
-            t = math.comb(n, L) * (x ** (n - L) * (1 - x) ** L)
-            wc = t if wc is None else wc + t
-    if wc is not None and n >= 1:
-        add(tuple(range(n)), wc * torch.ones((B, 1), dtype=rdt, device=dev))
+    if b_max >= n - 1 and n >= 1:
+        add(tuple(range(n)), weights[n + 1] * torch.ones((B, 1), dtype=rdt, device=dev))
     for L in range(n, 0, -1):
         if L <= b_max and n - L >= 2:
             start(L)
@@ -278,7 +305,7 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
         for ti, t in enumerate(order):
             add(t, acc[ti])
     if n >= 2:
-        add((), _subset_forwards(kernel, Ub, cols, [list(cols)])[0] * (x ** n))
+        add((), _subset_forwards(kernel, Ub, cols, [list(cols)])[0] * weights[0])
     if () not in A:  # no photon
         add((), torch.ones((B, 1), dtype=rdt, device=dev))
     out = A[()]

@@ -5,7 +5,7 @@ tests/test_imperfections.py:432-460). Tolerance: complex64 engine, max|dp| <= 1e
 import numpy as np
 import pytest
 import torch
-from helpers import haar_unitary
+from helpers import haar_unitary, occupation_list
 
 from oracle import slos_oracle as so
 from photonic_engines_amd.imperfections import Distinguishability, truncation_bound
@@ -129,3 +129,24 @@ def test_x_model_n10_m20_against_fp64(order):
         assert abs(mass - 1) < 1e-9
     else:
         assert abs(mass - (1 - truncation_bound(n, x, order))) < 1e-9
+
+
+@pytest.mark.parametrize("n,m,occ,mask,rows,order", [
+    (3, 5, [1, 1, 1, 0, 0], "fock", 0, None), (4, 6, [2, 0, 1, 1, 0, 0], "fock", 3, None),
+    (5, 9, None, "fock", 2, 2), (5, 9, None, "fock", 0, 4), (6, 12, None, "dual_rail", 0, None),
+    (5, 8, None, "unbunched", 2, 3), (6, 9, [2, 2, 2, 0, 0, 0, 0, 0, 0], "tail_empty", 0, 1), (7, 10, None, "fock", 0, 6),
+    (8, 12, None, "fock", 0, None), (9, 10, None, "fock", 0, 3)])
+def test_one_call_mixture_against_fp64(n, m, occ, mask, rows, order):
+    """The x-model in one native call against the layer-by-layer FP64 x-model: every order on either side
+    of the classical terms, rows, masks, repeated columns."""
+    occ = occ or occupation_list(n, m, mask)
+    U = torch.stack([haar_unitary(m, n * m + i) for i in range(max(1, rows))])
+    U = (U if rows else U[0]).to(torch.complex64)
+    ref = FockSLOSKernel(n, m, occ, mask=mask, device="cuda", dtype=torch.complex128).probs(
+        U.to(torch.complex128).cuda(), indist=0.85, order=order)
+    k = FockSLOSKernel(n, m, occ, mask=mask, device="cuda")
+    for x in (0.85, torch.tensor(0.85, device="cuda")):
+        p = k.probs(U.cuda(), indist=x, order=order)
+        assert p.shape == ref.shape and p.dtype == torch.float32
+        assert float((p - ref).abs().max()) <= TOL
+        assert abs(float(p.sum()) - float(ref.sum())) <= 1e-5 * max(1, rows)
