@@ -126,6 +126,12 @@ int slos_forward(const slos_plan* plan, const void* U, int64_t batch, const int3
                  int layer, int out_kind, void* out, double scale, unsigned flags,
                  void* workspace, size_t workspace_bytes, slos_stream_t stream);
 
+/* slos_forward on matrices with strides: element (b, row, col) of U at strides[0] b + strides[1] row +
+ * strides[2] col elements from `U` (any values, zero and negative ones included). */
+int slos_forward_strided(const slos_plan* plan, const void* U, const int64_t* strides, int64_t batch,
+                         const int32_t* modes, int layer, int out_kind, void* out, double scale, unsigned flags,
+                         void* workspace, size_t workspace_bytes, slos_stream_t stream);
+
 /* slos_forward without a workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. It calls no hipMalloc / hipFree: the intermediate layers live in a

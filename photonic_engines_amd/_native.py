@@ -35,6 +35,8 @@ SIGNATURES = {
     "slos_forward_workspace": (_c.c_int, [_vp, _c.c_int64, _c.c_int, _c.c_uint, _c.POINTER(_c.c_size_t)]),
     "slos_forward": (_c.c_int, [_vp, _vp, _c.c_int64, _i32p, _c.c_int, _c.c_int, _vp, _c.c_double, _c.c_uint,
                                 _vp, _c.c_size_t, _vp]),
+    "slos_forward_strided": (_c.c_int, [_vp, _vp, _c.POINTER(_c.c_int64), _c.c_int64, _i32p, _c.c_int, _c.c_int, _vp,
+                                        _c.c_double, _c.c_uint, _vp, _c.c_size_t, _vp]),
     "slos_forward_noalloc": (_c.c_int, [_vp, _vp, _c.c_int64, _i32p, _c.c_int, _c.c_int, _vp, _c.c_double,
                                         _c.c_uint, _vp]),
     "slos_layer_step": (_c.c_int, [_vp, _vp, _c.c_int64, _c.c_int, _c.c_int, _vp, _c.c_int, _vp, _c.c_double,
@@ -118,6 +120,11 @@ def check(rc: int, what: str) -> None:
     if rc == SLOS_ERANGE:
         raise OverflowError(msg)
     raise NativeError(msg)
+
+
+def raw_stream(device: torch.device) -> int:
+    """The current stream of `device` as an integer handle."""
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def stream_handle(device: torch.device) -> ctypes.c_void_p:

@@ -31,6 +31,7 @@ struct FrontArgs {
   int me, multiset, m, kf;
   int kind;                  // of layer kf: 0 raw, 1 probabilities, 2 scaled amplitudes
   const void* U;             // [B][m][m]
+  MatrixStride us;           // U's strides
   int cols[kFrontMax];       // input column of layer k at cols[k - 1]
   uint32_t S[kFrontMax + 1];
   uint32_t buf;              // LDS elements of one ping-pong buffer

@@ -50,12 +50,12 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
   T2* ucols = reinterpret_cast<T2*>(smem + (((ncg + a.me) * 4 + 15) & ~15));
   T2* bufs[2] = {ucols + a.kf * a.m, ucols + a.kf * a.m + (COMP ? 2 : 1) * a.buf};
   const int64_t b = blockIdx.y;
-  const T2* U = static_cast<const T2*>(a.U) + (size_t)b * a.m * a.m;
+  const T2* U = static_cast<const T2*>(a.U) + b * a.us.B;
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = (uint32_t)a.cg[i];
   for (int i = threadIdx.x; i < a.me; i += blockDim.x) lo[i] = a.lo[i];
   for (int i = threadIdx.x; i < a.kf * a.m; i += blockDim.x) {
     const int k = i / a.m, j = i - k * a.m;
-    ucols[i] = U[(size_t)j * a.m + a.cols[k]];
+    ucols[i] = U[j * a.us.R + a.cols[k] * a.us.C];
   }
   if (threadIdx.x == 0) {
     bufs[0][0] = T2{1, 0};

@@ -27,6 +27,7 @@ constexpr int kWaves = kBlockThreads / 64;
 struct BlockLayer {
   int K, m, col;
   const float2* U;       // [B][m][m]
+  MatrixStride us;       // U's strides
   uint64_t S_par;        // parent layer size
   uint64_t S;            // child layer size
   uint64_t S_pre;        // number of d-prefixes (layer d of the space)
@@ -123,13 +124,14 @@ struct SufRow {
   uint32_t t0, t1;
 };
 
-// rows for U[b, :, col] (Ucol = &U[b][0][col], stride m), positions < me; cg: the global table
+// rows for U[b, :, col] (Ucol = &U[b][0][col], rows `down` apart), positions < me; cg: the global table
 // (Row: SufRow or its FP64 form, V: U's complex type)
 template <int SUF, class Row, class V>
-__device__ __forceinline__ void fill_suffix_rows(Row* rows, const V* Ucol, int m, const uint64_t* cg, int stride, int me) {
+__device__ __forceinline__ void fill_suffix_rows(Row* rows, const V* Ucol, int64_t down, int m, const uint64_t* cg, int stride,
+                                                 int me) {
   for (int i = threadIdx.x; i < kSufRows; i += blockDim.x) {
     const int x = i & (kBlockModes - 1);
-    const V u = (i < kBlockModes && x < m) ? Ucol[(size_t)x * m] : V{0, 0};
+    const V u = (i < kBlockModes && x < m) ? Ucol[x * down] : V{0, 0};
     Row r;
     r.re = u.x;
     r.im = u.y;
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(C
   const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
-  fill_suffix_rows<SUF>(rows, a.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
+  fill_suffix_rows<SUF>(rows, a.U + b * a.us.B + a.col * a.us.C, a.us.R, a.m, cg_t, stride, me);
   fill_norm_rows<SUF>(rn);
   __syncthreads();
   const BlockTables tg{cg_t, lo_t, tuples, me, stride, multiset};  // global: scalar loads
@@ -934,7 +936,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
   const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
-  fill_suffix_rows<5>(rows, a.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
+  fill_suffix_rows<5>(rows, a.U + b * a.us.B + a.col * a.us.C, a.us.R, a.m, cg_t, stride, me);
   fill_norm_rows<5>(rn);
   __syncthreads();
   const int wv = (int)rfl(threadIdx.x >> 6);
@@ -1141,12 +1143,12 @@ k_layer_block_group(GroupLaunch gl) {
       for (int i = threadIdx.x; i < it.me; i += blockDim.x) lo_l[i] = it.lo[i];
       cur = it.cg;
     }
-    fill_suffix_rows<kSuf>(rows, it.U + (size_t)b * it.m * it.m + it.col, it.m, it.cg, stride, it.me);
+    fill_suffix_rows<kSuf>(rows, it.U + (size_t)b * it.m * it.m + it.col, it.m, it.m, it.cg, stride, it.me);
     __syncthreads();
     const BlockTables tg{it.cg, it.lo, it.tuples, it.me, stride, it.multiset};
     const BlockTables tl{cg_l, lo_l, it.tuples, it.me, stride, it.multiset};
     BlockLayer a;
-    a.K = K; a.m = it.m; a.col = it.col; a.U = it.U; a.S_par = it.S_par; a.S = it.S; a.S_pre = it.S_pre;
+    a.K = K; a.m = it.m; a.col = it.col; a.U = it.U; a.us = packed_stride(it.m); a.S_par = it.S_par; a.S = it.S; a.S_pre = it.S_pre;
     a.scale = it.scale; a.flags = it.flags; a.per_wave = it.per_wave; a.xcd_chunk = 1;
     a.par_lo = it.par_lo; a.out_lo = it.out_lo;
     const uint64_t g = uniform_u64(((uint64_t)w * kWaves + wv) * it.per_wave);

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
   const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
-  fill_suffix_rows<SUF>(rows, p.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
+  fill_suffix_rows<SUF>(rows, p.U + b * a.us.B + a.col * a.us.C, a.us.R, a.m, cg_t, stride, me);
   fill_norm_rows<SUF>(rn);
   __syncthreads();
   const BlockTables tg{cg_t, lo_t, tuples, me, stride, multiset};  // global: scalar loads
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
   const uint32_t bid = batch_item(a.rows, a.row_wgs, a.xcd_chunk, &b);
   for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg_l[i] = cg_t[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo_l[i] = lo_t[i];
-  fill_suffix_rows<5>(rows, p.U + (size_t)b * a.m * a.m + a.col, a.m, cg_t, stride, me);
+  fill_suffix_rows<5>(rows, p.U + b * a.us.B + a.col * a.us.C, a.us.R, a.m, cg_t, stride, me);
   fill_norm_rows<5>(rn);
   __syncthreads();
   const int wv = (int)rfl(threadIdx.x >> 6);

@@ -46,6 +46,7 @@ struct LayerArgs {
   const int* lo;
   int me, multiset, K, m, col;
   const float2* U;        // [B][m][m]
+  MatrixStride us;        // U's strides
   const uint64_t* words;  // 5-position suffix words (or null)
   const float2* par;      // [B][S_par]
   uint64_t S_par;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(256) void k_layer_simple(LayerArgs a) {
   for (int64_t b = blockIdx.y; b < a.B; b += gridDim.y) {
     __syncthreads();
     for (int j = threadIdx.x; j < a.m; j += blockDim.x)
-      ucol[j] = a.U[(size_t)b * a.m * a.m + (size_t)j * a.m + a.col];
+      ucol[j] = a.U[b * a.us.B + j * a.us.R + a.col * a.us.C];
     __syncthreads();
     const float2* pb = a.par + (size_t)b * a.S_par;
     for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < a.S;

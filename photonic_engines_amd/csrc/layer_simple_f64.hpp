@@ -15,6 +15,7 @@ struct LayerArgsF64 {
   const uint64_t* words;  // 5-position suffix words (or null)
   int me, multiset, K, m, col;
   const double2* U;    // [B][m][m]
+  MatrixStride us;        // U's strides
   const double2* par;  // [B][S_par]
   uint64_t S_par;
   void* out;           // [B][S]: complex128 (kinds 0, 2) or float64 (kind 1)
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(256) void k_layer_f64(LayerArgsF64 a) {
   double2* ucol = reinterpret_cast<double2*>(smem + space_lds_f64(K, a.me));
   for (int64_t b = blockIdx.y; b < a.B; b += gridDim.y) {
     __syncthreads();
-    for (int j = threadIdx.x; j < a.m; j += blockDim.x) ucol[j] = a.U[(size_t)b * a.m * a.m + (size_t)j * a.m + a.col];
+    for (int j = threadIdx.x; j < a.m; j += blockDim.x) ucol[j] = a.U[b * a.us.B + j * a.us.R + a.col * a.us.C];
     __syncthreads();
     const double2* pb = a.par + (size_t)b * a.S_par;
     for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < a.S; g += (uint64_t)gridDim.x * blockDim.x) {

@@ -720,7 +720,7 @@ dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
 
 int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs& a, int kind, bool comp, hipStream_t st) {
   slos::BlockLayer L;
-  L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.S_par = a.S_par; L.S = a.S; L.gp = a.gp;
+  L.K = a.K; L.m = a.m; L.col = a.col; L.U = a.U; L.us = a.us; L.S_par = a.S_par; L.S = a.S; L.gp = a.gp;
   L.par_lo = a.par_lo; L.out_lo = a.out_lo;
   const int suf = block_suffix(p, dt, a.K);
   L.S_pre = p->size(a.K - suf);
@@ -773,14 +773,14 @@ void with_km(int photons, F&& f) {
 
 // par_hilo / out_hilo (compensated sums only): the parent layer / the complex64 output layer is a
 // hi/lo pair [2][B][S], the low-order parts after the high ones
-int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const float2* U, int64_t B,
+int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const float2* U, slos::MatrixStride us, int64_t B,
                  const float2* par, uint64_t S_par, void* out, uint64_t S, int kind, float scale,
                  unsigned flags, hipStream_t st, bool par_hilo = false, bool out_hilo = false,
                  const float* gp = nullptr) {
   slos::LayerArgs a;
   a.gp = gp;
   a.cg = dt.cg; a.lo = dt.lo; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
-  a.U = U; a.words = dt.tuples5; a.par = par; a.S_par = S_par; a.out = out; a.S = S; a.B = B;
+  a.U = U; a.us = us; a.words = dt.tuples5; a.par = par; a.S_par = S_par; a.out = out; a.S = S; a.B = B;
   a.scale = scale; a.flags = flags;
   const bool comp = flags & SLOS_FLAG_COMPENSATED;
   a.par_lo = (comp && par_hilo) ? B * (int64_t)S_par : 0;
@@ -799,7 +799,7 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
 
 // one complex128 layer on the block or group-order kernel; -1 where they do not apply (layers of
 // fewer than 5 photons, prefixes of more than 8 positions, spaces without tuple words)
-int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, int64_t B, const void* par,
+int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, slos::MatrixStride us, int64_t B, const void* par,
                      uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
   if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
   const int suf = dt.tuples5 && K > 5 ? 5 : slos::kSuf;
@@ -809,6 +809,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   L.l.K = K; L.l.m = p->m; L.l.col = col; L.l.S_par = S_par; L.l.S = S; L.l.S_pre = p->size(d);
   L.l.flags = flags;
   L.U = static_cast<const double2*>(U);
+  L.l.us = us;
   L.scale = scale;
   if (suf == 5 && kind <= 1 && dt.items[K]) {
     const size_t sh = slos::group_dyn_lds64(K, p->me);
@@ -839,15 +840,15 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
 
 // one complex128 layer (thread-per-state, FP64): kind 0 raw complex128, 1 float64 probabilities,
 // 2 scaled complex128 amplitudes (SLOS_FLAG_IMMEDIATE: times sqrt(prod t!))
-int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, int64_t B, const void* par,
+int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, slos::MatrixStride us, int64_t B, const void* par,
                      uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
   if (!(flags & SLOS_FLAG_SIMPLE)) {
-    const int rc = launch_block_f64(p, dt, K, col, U, B, par, S_par, out, S, kind, scale, flags, st);
+    const int rc = launch_block_f64(p, dt, K, col, U, us, B, par, S_par, out, S, kind, scale, flags, st);
     if (rc >= 0) return rc;
   }
   slos::LayerArgsF64 a;
   a.cg = dt.cg; a.lo = dt.lo; a.words = dt.tuples5; a.me = p->me; a.multiset = p->multiset; a.K = K; a.m = p->m; a.col = col;
-  a.U = static_cast<const double2*>(U); a.par = static_cast<const double2*>(par); a.S_par = S_par;
+  a.U = static_cast<const double2*>(U); a.us = us; a.par = static_cast<const double2*>(par); a.S_par = S_par;
   a.out = out; a.S = S; a.B = B; a.scale = scale;
   a.immediate = (flags & SLOS_FLAG_IMMEDIATE) ? 1u : 0u;
   const size_t sh = slos::space_lds_f64(K, p->me) + (size_t)p->m * 16;
@@ -883,14 +884,14 @@ int front_layers(const slos_plan* p, int64_t B, int layer, size_t elem, bool com
 }
 
 // layers 1..kf (front_layers) in one launch; kind: of layer kf
-int run_front(const slos_plan* p, const DevTables& dt, int kf, const int* cols, const void* U, int64_t B, void* out,
+int run_front(const slos_plan* p, const DevTables& dt, int kf, const int* cols, const void* U, slos::MatrixStride us, int64_t B, void* out,
               int kind, double scale, unsigned flags, size_t lds, uint32_t buf, bool hilo_out, hipStream_t st,
               void* const* below = nullptr) {
   slos::FrontArgs a{};
   if (below)
     for (int k = 0; k < kf; ++k) a.below[k] = below[k];
   a.cg = dt.cg; a.lo = dt.lo; a.tuples = dt.tuples; a.tuples5 = dt.tuples5;
-  a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.kf = kf; a.kind = kind; a.U = U;
+  a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.kf = kf; a.kind = kind; a.U = U; a.us = us;
   for (int k = 0; k < kf; ++k) a.cols[k] = cols[k];
   for (int k = 0; k <= kf; ++k) a.S[k] = (uint32_t)p->size(k);
   a.buf = buf; a.out = out; a.scale = scale;
@@ -1259,7 +1260,7 @@ int group_layer_per_plan(const slos_group* G, int K, const GroupArgs& a, const G
     const float2* par = K == 1 ? reinterpret_cast<const float2*>(a.ws + w.ones[g]) : bufs[(K - 1) & 1];
     const bool last = K == p->n;
     void* out = last ? static_cast<void*>(a.out[g]) : static_cast<void*>(bufs[K & 1]);
-    const int rc = launch_layer(p, dts[g], K, p->modes[K - 1], a.U[g], a.B[g], par, p->size(K - 1), out, p->size(K),
+    const int rc = launch_layer(p, dts[g], K, p->modes[K - 1], a.U[g], slos::packed_stride(p->m), a.B[g], par, p->size(K - 1), out, p->size(K),
                                 last ? 1 : 0, last ? a.scale[g] : 1.f, a.flags & ~SLOS_FLAG_HILO, st, hilo && K >= 2,
                                 hilo && !last);
     if (rc) return rc;
@@ -1604,7 +1605,7 @@ int forward_check(const slos_plan* p, const void* U, int64_t batch, const int32_
 }
 
 // the complex128 forward (SLOS_FLAG_F64): the same layer walk as forward_run, FP64 kernels
-int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, int64_t batch, const int* cols, int layer,
+int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, slos::MatrixStride us, int64_t batch, const int* cols, int layer,
                     int out_kind, void* out, double scale, unsigned flags, const WsLayout& w, void* ws,
                     hipStream_t st) {
   auto* base = static_cast<unsigned char*>(ws);
@@ -1625,7 +1626,7 @@ int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, int6
   const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 16, false, &lds, &buf);
   if (kf) {
     void* dst = kf == layer ? out : bufs[kf & 1];
-    const int rc = run_front(p, dt, kf, cols, U, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale,
+    const int rc = run_front(p, dt, kf, cols, U, us, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale,
                              flags, lds, buf, false, st);
     if (rc) return rc;
     par = dst;
@@ -1642,7 +1643,7 @@ int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, int6
     char name[32];
     std::snprintf(name, sizeof name, "slos layer %d", k);
     const RoctxRange range(name);
-    const int rc = launch_layer_f64(p, dt, k, cols[k - 1], U, batch, par, S_par, dst, S, kind, scale, flags, st);
+    const int rc = launch_layer_f64(p, dt, k, cols[k - 1], U, us, batch, par, S_par, dst, S, kind, scale, flags, st);
     if (rc) return rc;
     par = dst;
     S_par = S;
@@ -1651,9 +1652,9 @@ int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, int6
 }
 
 // the layer launches of a forward whose workspace `ws` follows layout `w` (no allocation)
-int forward_run(const slos_plan* p, const DevTables& dt, const void* U, int64_t batch, const int* cols, int layer,
+int forward_run(const slos_plan* p, const DevTables& dt, const void* U, slos::MatrixStride us, int64_t batch, const int* cols, int layer,
                 int out_kind, void* out, double scale, unsigned flags, const WsLayout& w, void* ws, hipStream_t st) {
-  if (flags & SLOS_FLAG_F64) return forward_run_f64(p, dt, U, batch, cols, layer, out_kind, out, scale, flags, w, ws, st);
+  if (flags & SLOS_FLAG_F64) return forward_run_f64(p, dt, U, us, batch, cols, layer, out_kind, out, scale, flags, w, ws, st);
   int rc = SLOS_OK;
   auto* base = static_cast<unsigned char*>(ws);
   float2* ones = reinterpret_cast<float2*>(base + w.ones);
@@ -1675,7 +1676,7 @@ int forward_run(const slos_plan* p, const DevTables& dt, const void* U, int64_t 
   const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 8, hilo, &lds, &buf);
   if (kf) {
     void* dst = kf == layer ? out : bufs[kf & 1];
-    rc = run_front(p, dt, kf, cols, U, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale, flags, lds,
+    rc = run_front(p, dt, kf, cols, U, us, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale, flags, lds,
                    buf, hilo && kf < layer, st);
     if (rc) return rc;
     par = static_cast<const float2*>(dst);
@@ -1693,7 +1694,7 @@ int forward_run(const slos_plan* p, const DevTables& dt, const void* U, int64_t 
     char name[32];
     std::snprintf(name, sizeof name, "slos layer %d", k);
     const RoctxRange range(name);
-    rc = launch_layer(p, dt, k, cols[k - 1], Uf, batch, par, S_par, dst, S, kind, (float)scale, flags & ~SLOS_FLAG_HILO,
+    rc = launch_layer(p, dt, k, cols[k - 1], Uf, us, batch, par, S_par, dst, S, kind, (float)scale, flags & ~SLOS_FLAG_HILO,
                       st, hilo && k >= 2, hilo && !last);
     if (rc) return rc;
     par = static_cast<const float2*>(dst);
@@ -1754,19 +1755,27 @@ int resident_tables(const slos_plan* cp, DevTables* out) {
 
 }  // namespace
 
-int slos_forward(const slos_plan* p, const void* U, int64_t batch, const int32_t* modes, int layer, int out_kind,
+int slos_forward_strided(const slos_plan* p, const void* U, const int64_t* strides, int64_t batch, const int32_t* modes, int layer, int out_kind,
                  void* out, double scale, unsigned flags, void* ws, size_t ws_bytes, slos_stream_t stream) {
   int cols[kMaxPhotons] = {};  // layer <= n <= 32 (checked before cols is written)
   WsLayout w;
   int rc = forward_check(p, U, batch, modes, layer, out_kind, out, flags, cols, &w);
   if (rc) return rc;
+  if (!strides) return fail(SLOS_EINVAL, "NULL argument");
   if (!ws || ws_bytes < w.total)
     return fail(SLOS_ENOMEM, "workspace too small: need " + std::to_string(w.total) + " bytes");
   DevTables dt;
   rc = device_tables(p, &dt);
   if (rc) return rc;
-  return forward_run(p, dt, U, batch, cols, layer, out_kind, out, scale, flags, w, ws,
+  return forward_run(p, dt, U, slos::MatrixStride{strides[0], strides[1], strides[2]}, batch, cols, layer, out_kind, out, scale, flags, w, ws,
                      reinterpret_cast<hipStream_t>(stream));
+}
+
+int slos_forward(const slos_plan* p, const void* U, int64_t batch, const int32_t* modes, int layer, int out_kind,
+                 void* out, double scale, unsigned flags, void* ws, size_t ws_bytes, slos_stream_t stream) {
+  if (!p) return fail(SLOS_EINVAL, "NULL argument");
+  const int64_t m = p->m, packed[3] = {m * m, m, 1};
+  return slos_forward_strided(p, U, packed, batch, modes, layer, out_kind, out, scale, flags, ws, ws_bytes, stream);
 }
 
 int slos_forward_noalloc(const slos_plan* p, const void* U, int64_t batch, const int32_t* modes, int layer,
@@ -1785,7 +1794,7 @@ int slos_forward_noalloc(const slos_plan* p, const void* U, int64_t batch, const
   void* ws = nullptr;
   rc = scratch_address(&ws);
   if (rc) return rc;
-  return forward_run(p, dt, U, batch, cols, layer, out_kind, out, scale, flags, w, ws,
+  return forward_run(p, dt, U, slos::packed_stride(p->m), batch, cols, layer, out_kind, out, scale, flags, w, ws,
                      reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -1803,13 +1812,13 @@ int slos_layer_step(const slos_plan* p, const void* U, int64_t batch, int k, int
   if (flags & SLOS_FLAG_F64) {
     if (flags & (SLOS_FLAG_COMPENSATED | SLOS_FLAG_HILO))
       return fail(SLOS_EINVAL, "SLOS_FLAG_F64 computes in FP64: no compensated sums");
-    return launch_layer_f64(p, dt, k, col, U, batch, psi_prev, p->size(k - 1), out, p->size(k), kind, scale, flags,
+    return launch_layer_f64(p, dt, k, col, U, slos::packed_stride(p->m), batch, psi_prev, p->size(k - 1), out, p->size(k), kind, scale, flags,
                             reinterpret_cast<hipStream_t>(stream));
   }
   const bool hilo = (flags & SLOS_FLAG_HILO) && (flags & SLOS_FLAG_COMPENSATED);
   if ((flags & SLOS_FLAG_HILO) && !(flags & SLOS_FLAG_COMPENSATED))
     return fail(SLOS_EINVAL, "SLOS_FLAG_HILO needs SLOS_FLAG_COMPENSATED");
-  return launch_layer(p, dt, k, col, static_cast<const float2*>(U), batch, static_cast<const float2*>(psi_prev),
+  return launch_layer(p, dt, k, col, static_cast<const float2*>(U), slos::packed_stride(p->m), batch, static_cast<const float2*>(psi_prev),
                       p->size(k - 1), out, p->size(k), kind, (float)scale, flags & ~SLOS_FLAG_HILO,
                       reinterpret_cast<hipStream_t>(stream), hilo, hilo && kind == 0);
 }
@@ -2054,7 +2063,7 @@ int slos_forward_saved(const slos_plan* p, const void* U, int64_t batch, const i
   uint32_t buf = 0;
   const int kf = front_layers(p, batch, layer - 1, 8, false, &lds, &buf);
   if (kf) {
-    rc = run_front(p, dt, kf, cols, U, batch, layers[kf], 0, 1.0, 0u, lds, buf, false, st, layers);
+    rc = run_front(p, dt, kf, cols, U, slos::packed_stride(p->m), batch, layers[kf], 0, 1.0, 0u, lds, buf, false, st, layers);
     if (rc) return rc;
   } else {
     hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>((batch + 255) / 256, 4096)), dim3(256), 0, st,
@@ -2063,7 +2072,7 @@ int slos_forward_saved(const slos_plan* p, const void* U, int64_t batch, const i
   }
   for (int k = kf + 1; k <= layer; ++k) {
     const bool last = k == layer;
-    rc = launch_layer(p, dt, k, cols[k - 1], static_cast<const float2*>(U), batch,
+    rc = launch_layer(p, dt, k, cols[k - 1], static_cast<const float2*>(U), slos::packed_stride(p->m), batch,
                       static_cast<const float2*>(layers[k - 1]), p->size(k - 1), last ? out : layers[k], p->size(k),
                       last && probs ? 1 : 0, last ? (float)scale : 1.f, 0u, st);
     if (rc) return rc;
@@ -2119,7 +2128,7 @@ int slos_backward(const slos_plan* p, const void* U, int64_t batch, const int32_
     auto* g = reinterpret_cast<float2*>(base + b.g[0]);
     const auto* gp = static_cast<const float*>(grad);
     if (grad_kind == 1) {  // the amplitudes again, with the readout's adjoint in the same pass
-      rc = launch_layer(p, dt, layer, ra.col[layer - 1], Uf, batch, psi(layer - 1), p->size(layer - 1), g, p->size(layer), 4,
+      rc = launch_layer(p, dt, layer, ra.col[layer - 1], Uf, slos::packed_stride(p->m), batch, psi(layer - 1), p->size(layer - 1), g, p->size(layer), 4,
                         (float)(scale * scale), 0u, st, false, false, gp);
     } else {
       rc = run_readout_pull(p, dt, Uf, batch, ra.col[layer - 1], psi(layer - 1), gp, scale, g, st);
@@ -2392,7 +2401,7 @@ int slos_xmodel(const slos_plan* p, const void* U, const float* W, int64_t batch
       WsLayout w;
       int rc = forward_layout(p, rows, g, &w, (flags & SLOS_FLAG_COMPENSATED) != 0, false);
       if (rc) return rc;
-      rc = forward_run(p, dt, a.Up, rows, cols, g, SLOS_OUT_PROBS, level(L) + (size_t)r0 * B * p->size(g), 1.0, flags, w,
+      rc = forward_run(p, dt, a.Up, slos::packed_stride(p->m), rows, cols, g, SLOS_OUT_PROBS, level(L) + (size_t)r0 * B * p->size(g), 1.0, flags, w,
                        base + x.fwd, st);
       if (rc) return rc;
     }

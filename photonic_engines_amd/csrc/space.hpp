@@ -30,6 +30,12 @@
 
 namespace slos {
 
+// a batch of matrices in memory: element (b, row, col) at b * B + row * R + col * C
+struct MatrixStride {
+  int64_t B, R, C;
+};
+SLOS_HD MatrixStride packed_stride(int m) { return MatrixStride{(int64_t)m * m, m, 1}; }
+
 struct SpaceView {
   const uint64_t* cg;  // (rows) x (me + 1), row-major
   const int* lo;       // me

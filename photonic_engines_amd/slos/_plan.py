@@ -30,6 +30,9 @@ def _dtype_flags(cdtype: torch.dtype, flags: int) -> int:
 MAX_ROWS = 65535
 
 
+_Strides = ctypes.c_int64 * 3
+
+
 def _row_ranges(B: int) -> list[tuple[int, int]]:
     return [(i, min(B, i + MAX_ROWS)) for i in range(0, B, MAX_ROWS)]
 
@@ -45,6 +48,7 @@ class Plan:
             raise ValueError(f"unknown mask {mask!r}")
         self.n, self.m, self.mask = int(n), int(m), mask
         self.modes = [int(i) for i in input_modes]
+        self._forward_sizes: dict = {}  # (batch, flags, dtype) -> sizes of a forward, by formula
         if len(self.modes) != self.n:
             raise ValueError(f"input has {len(self.modes)} photons, expected n={n}")
         arr = (ctypes.c_int32 * self.n)(*self.modes)
@@ -242,6 +246,37 @@ class Plan:
                          nat.ptr(gprev[i:j]) if want_prev else None, nat.ptr(grad_U[i:j]), 1, nat.ptr(ws), ws.numel(),
                          nat.stream_handle(U.device)), "slos_adjoint_layer")
         return gprev
+
+    def probs(self, U: torch.Tensor, scale: float, flags: int) -> torch.Tensor:
+        """The probabilities [S_n] of a matrix [m, m] or [B, S_n] of a batch (B <= MAX_ROWS) on the GPU, in
+        whatever strides it has: forward without a copy of U, in as few host operations as it takes
+        (a small forward's launches take less time than these)."""
+        batched = U.dim() == 3
+        B = U.shape[0] if batched else 1
+        dev = U.device
+        key = (B, flags, U.dtype)
+        known = self._forward_sizes.get(key)
+        if known is None:
+            f = _dtype_flags(U.dtype, flags)
+            odt = _out_dtypes(U.dtype)[0]
+            ws_bytes = max(1, self.workspace_bytes(B, self.n, f))
+            if len(self._forward_sizes) >= 64:
+                self._forward_sizes.clear()
+            known = self._forward_sizes[key] = (f, odt, ws_bytes, ws_bytes + B * self.sizes[self.n] * odt.itemsize)
+        f, odt, ws_bytes, need = known
+        if need >= self.PREFLIGHT_MIN:
+            self.preflight(need, dev, f"SLOS forward (n={self.n}, m={self.m}, batch {B}: "
+                           f"output {need - ws_bytes:,} B, workspace {ws_bytes:,} B)")
+        S = self.sizes[self.n]
+        out = torch.empty((B, S) if batched else (S,), dtype=odt, device=dev)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        strides = U.stride()
+        rc = self._lib.slos_forward_strided(
+            self._h, U.data_ptr(), _Strides(*(strides if batched else (0, *strides))), B, None, self.n, nat.OUT_PROBS,
+            out.data_ptr(), scale, f, ws.data_ptr(), ws_bytes, nat.raw_stream(dev))
+        if rc:
+            nat.check(rc, "slos_forward")
+        return out
 
     def xmodel(self, U: torch.Tensor, W: torch.Tensor, order: int, weights, flags: int = 0) -> torch.Tensor:
         """The x-model's distribution [B, S_n] of a contiguous complex64 U [B, m, m] (slos_xmodel);

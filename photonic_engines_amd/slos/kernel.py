@@ -140,6 +140,15 @@ class FockSLOSKernel:
         dev = nat.require_gpu(U.device if U.device.type == "cuda" else self.device)
         return U.to(device=dev, dtype=self.cdtype).contiguous(), batched
 
+    def _direct(self, U: torch.Tensor) -> bool:
+        """Whether a forward can read U where it is: on a GPU, as its result, in the kernel's dtype, any
+        strides (a lazily conjugated or negated view has other values than its memory)."""
+        shape = U.shape
+        d = len(shape)
+        return (U.is_cuda and U.dtype == self.cdtype and self.device.type == "cuda" and (d == 2 or d == 3)
+                and shape[d - 1] == self.m and shape[d - 2] == self.m and not U.is_conj() and not U.is_neg()
+                and (d == 2 or 1 <= shape[0] <= MAX_ROWS))
+
     def _out(self, t: torch.Tensor, batched: bool) -> torch.Tensor:
         t = t if batched else t.squeeze(0)
         return t.to(self.device) if self.device.type != "cuda" else t
@@ -213,6 +222,8 @@ class FockSLOSKernel:
                 p = SLOSProbs.apply(U, Ug, self)
                 p = p if batched else p.squeeze(0)
                 p = p.to(self.device) if self.device.type != "cuda" else p
+            elif loss is None and self._direct(U):
+                return self._plan.probs(U, self._input_norm, self._flags())
             else:
                 Ug, batched = self._prepare(U)
                 # a loss without gradient: the readout applies the weight of layer n (|amp s|^2 w_n)
