@@ -2008,7 +2008,7 @@ int saved_layout(const slos_plan* p, int64_t batch, int layer, std::vector<size_
 struct BackLayout {
   std::vector<AdjLaunch> L;       // of layer k at k - 1
   std::vector<size_t> part;       // its partials (bytes from the workspace's begin)
-  size_t g[2] = {0, 0};           // gradients of the layers layer, layer - 2, ..; layer - 1, ..
+  size_t g[2] = {0, 0};           // gradients of the layers top, top - 2, ..; top - 1, .. (top: `layer`, or the one below)
   size_t total = 0;
 };
 
@@ -2022,10 +2022,12 @@ int back_layout(const slos_plan* p, int64_t batch, int layer, bool readout, Back
     b->part.push_back(sum);
     sum += align256((size_t)batch * L.nblk * p->me * sizeof(double2));
   }
+  // (a mask's layers need not shrink with the photons: the largest of those a buffer holds in turn)
   for (int i = 0; i < 2; ++i) {
-    const int k = readout ? layer - i : layer - 1 - i;  // the largest layer of the two buffers
+    uint64_t most = 0;
+    for (int k = readout ? layer - i : layer - 1 - i; k >= 1; k -= 2) most = std::max(most, p->size(k));
     b->g[i] = sum;
-    if (k >= 1) sum += align256((size_t)batch * p->size(k) * sizeof(float2));
+    sum += align256((size_t)batch * most * sizeof(float2));
   }
   b->total = sum;
   return SLOS_OK;

@@ -179,3 +179,27 @@ def test_memory_plan_and_preflight():
         UnevenBatch([k128])
     big = Plan(12, 64, "fock", list(range(12)))
     assert big.memory_plan(1)["output"] == 4 * math.comb(75, 12)              # ~105 TB of probabilities
+
+
+def test_backward_workspace_holds_the_largest_layer_of_each_buffer():
+    """The gradients of every other layer share a buffer; a mask's layers need not shrink with the photons
+    (dual rail, 5 photons: 1, 10, 40, 80, 80, 32 states)."""
+    L = nat.lib()
+    for mask, n, m in (("dual_rail", 5, 10), ("sparse_1in4", 4, 16), ("unbunched", 6, 8), ("fock", 5, 9)):
+        step = {"dual_rail": 2, "sparse_1in4": 4}.get(mask, 1)
+        modes = (ctypes.c_int32 * n)(*[step * i for i in range(n)])
+        h = ctypes.c_void_p()
+        assert L.slos_plan_create(n, m, nat.MASK_IDS[mask], modes, ctypes.byref(h)) == 0
+        sizes = []
+        for k in range(n + 1):
+            s = ctypes.c_uint64()
+            assert L.slos_layer_size(h, k, ctypes.byref(s)) == 0
+            sizes.append(s.value)
+        for batch in (1, 3):
+            for kind in (0, 1):
+                b = ctypes.c_size_t()
+                assert L.slos_backward_workspace(h, batch, n, kind, ctypes.byref(b)) == 0
+                top = n if kind else n - 1
+                partials = n * -(-16 * batch * (m - 2 if mask == "tail_empty" else m) // 256) * 256  # at least
+                assert b.value >= partials + 8 * batch * (max(sizes[top:0:-2]) + max(sizes[top - 1:0:-2], default=0))
+        L.slos_plan_destroy(h)
