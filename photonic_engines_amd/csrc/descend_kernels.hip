@@ -1,9 +1,10 @@
 // The pulls over children: k_descend_insert and k_adjoint_insert (child_walk.hpp), k_descend_block
-// (descend_block.hpp).
+// (descend_block.hpp), k_adjoint_modes (adjoint_modes.hpp).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
+#include "adjoint_modes.hpp"
 #include "block_launch.hpp"
 
 namespace slos {
@@ -64,6 +65,28 @@ void launch_adjoint_insert(int dp, const BlockGrid& g, int m, int col, const flo
     else SLOS_ADJ(32);
   });
 #undef SLOS_ADJ
+}
+
+void launch_adjoint_modes(int P, dim3 grid, hipStream_t st, const AdjointModesArgs& a) {
+#define SLOS_MODES(N)                                                                                                   \
+  do {                                                                                                                  \
+    if (a.me <= 32) {                                                                                                   \
+      if (a.multiset) hipLaunchKernelGGL((k_adjoint_modes<N, 32, true>), grid, dim3(kModesThreads), 0, st, a);          \
+      else hipLaunchKernelGGL((k_adjoint_modes<N, 32, false>), grid, dim3(kModesThreads), 0, st, a);                    \
+    } else {                                                                                                            \
+      if (a.multiset) hipLaunchKernelGGL((k_adjoint_modes<N, 64, true>), grid, dim3(kModesThreads), 0, st, a);          \
+      else hipLaunchKernelGGL((k_adjoint_modes<N, 64, false>), grid, dim3(kModesThreads), 0, st, a);                    \
+    }                                                                                                                   \
+  } while (0)
+  switch (P) {
+    case 0: SLOS_MODES(0); break;
+    case 1: SLOS_MODES(1); break;
+    case 2: SLOS_MODES(2); break;
+    case 3: SLOS_MODES(3); break;
+    case 4: SLOS_MODES(4); break;
+    default: SLOS_MODES(5); break;
+  }
+#undef SLOS_MODES
 }
 
 }  // namespace slos

@@ -29,6 +29,7 @@
 #include "block_launch.hpp"
 #include "front.hpp"
 #include "raise.hpp"
+#include "adjoint_modes.hpp"
 
 namespace {
 
@@ -631,7 +632,8 @@ struct ReduceArgs {
   int col[kMaxPhotons];
   int layers;
 };
-constexpr int kReduceAllThreads = 512;
+constexpr int kReduceAllThreads = 1024;
+constexpr uint32_t kFew = 512;  // partials of a layer that one wave sums
 __global__ __launch_bounds__(kReduceAllThreads) void k_reduce_all(ReduceArgs a, const double2* __restrict__ partial, int me,
                                                                   int m, float2* __restrict__ gU) {
   constexpr int kW = kReduceAllThreads / 64;
@@ -641,12 +643,14 @@ __global__ __launch_bounds__(kReduceAllThreads) void k_reduce_all(ReduceArgs a, 
   const int j = blockIdx.x;
   const int w = threadIdx.x >> 6;
   if (j < me) {
+    // a layer of few partials is one wave's, the layers in turn; the others take all waves
     for (int l = 0; l < a.layers; ++l) {
       const uint32_t nblk = a.nblk[l];
+      const bool few = nblk <= kFew;
       double sr = 0, si = 0;
-      if (nblk > (uint32_t)w * 64u) {
+      if (!few || l % kW == w) {
         const double2* src = partial + a.part[l] + (size_t)b * nblk * me + j;
-        for (uint32_t r = threadIdx.x; r < nblk; r += kReduceAllThreads) {
+        for (uint32_t r = few ? threadIdx.x & 63u : threadIdx.x; r < nblk; r += few ? 64u : (uint32_t)kReduceAllThreads) {
           const double2 v = src[(size_t)r * me];
           sr += v.x;
           si += v.y;
@@ -1883,23 +1887,45 @@ namespace {
 // parents per XCD chunk of the insert-table adjoint (see slos::xcd_chunk_index)
 constexpr uint64_t kAdjChunkParents = 1ull << 18;
 
-// How one adjoint layer runs: the insert-table kernel (multiset spaces whose parent layer has a 1..8
-// position prefix before its 4-position suffix, up to 32 modes) or the thread-per-state kernel;
-// `nblk` work groups, each writing one FP64 partial per mode.
+// How one adjoint layer runs: the kernel with a lane a mode, the insert-table kernel or the
+// thread-per-state kernel; `nblk` work groups, each writing one FP64 partial per mode.
 struct AdjLaunch {
   bool walk = false;
+  uint32_t turns = 0;  // parents a group, of the kernel with a lane a mode (0: another kernel)
   uint64_t per_wave = 0;
   uint32_t xcd_chunk = 1;
   size_t lds = 0;   // of the thread-per-state kernel
   uint64_t nblk = 0;
 };
 
-int adjoint_launch(const slos_plan* p, int k, AdjLaunch* L) {
-  const uint64_t Sp = p->size(k - 1);
+// the insert-table kernel: parent prefixes of 1..8 positions, up to 32 modes (its sums' registers)
+bool adjoint_walk(const slos_plan* p, int k) {
   const int dp = k - 1 - slos::kSuf;
+  return has_insert_table(p) && dp >= 1 && dp <= 8 && p->me <= 32;
+}
+
+// Whether an adjoint layer takes the kernel with a lane a mode. It is quick to start and computes each
+// child's index anew: the one for few parents, and for many modes, where the thread-per-state kernel has
+// few waves (its sums' LDS). Adjoint layers with their sums, us, lane a mode / walk: 98k parents in all (24
+// modes) 31 / 35, 171k (14) 35 / 29, 377k (32) 68 / 57; lane a mode / thread per state: 17k (24) 26 / 38, 119k (14)
+// 30 / 34, 273k (12) 54 / 42, 886k (20) 100 / 116, 209k (32) 44 / 92, 766k (64) 234 / 592, 1.1M (40) 268 / 417.
+bool adjoint_modes(const slos_plan* p, int k, int64_t batch) {
+  if (k - 1 > slos::kModesPhotons || p->me > 64 || p->size(k) >= (1ull << 31)) return false;
+  return p->size(k - 1) <= (1ull << 17) / (uint64_t)batch || (!adjoint_walk(p, k) && p->me >= 20);
+}
+
+// modes: the kernel with a lane a mode, else the walk or the thread-per-state kernel
+int adjoint_launch(const slos_plan* p, int k, bool modes, AdjLaunch* L) {
+  const uint64_t Sp = p->size(k - 1);
   L->lds = (((size_t)(k + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8 +
            (size_t)kAdjThreads * p->me * 8;
-  L->walk = has_insert_table(p) && dp >= 1 && dp <= 8 && p->me <= 32;
+  if (modes) {
+    const uint32_t groups = slos::modes_groups(p->me);
+    L->turns = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, Sp / (groups * 64u)));
+    L->nblk = (Sp + groups * L->turns - 1) / (groups * L->turns);
+    return SLOS_OK;
+  }
+  L->walk = adjoint_walk(p, k);
   if (L->walk) {
     // parents per wave: at most about 2^16 work groups (FP64 partials per mode), and else as few as
     // pay for a wave's sum over its lanes (us with 128 / 256 / 512: 2.0M parents 137 / 119 / 112,
@@ -1923,10 +1949,16 @@ int adjoint_launch(const slos_plan* p, int k, AdjLaunch* L) {
 int slos_adjoint_workspace(const slos_plan* p, int64_t batch, int k, size_t* bytes) {
   if (!p || !bytes) return fail(SLOS_EINVAL, "NULL argument");
   if (k < 1 || k > p->n || batch < 1) return fail(SLOS_EINVAL, "bad argument");
-  AdjLaunch L;
-  int rc = adjoint_launch(p, k, &L);
-  if (rc) return rc;
-  *bytes = (size_t)batch * L.nblk * p->me * sizeof(double2);
+  // (enough for every smaller batch too, whichever kernel that takes)
+  uint64_t nblk = 0;
+  for (const bool modes : {false, true}) {
+    if (modes && !adjoint_modes(p, k, 1)) break;
+    AdjLaunch L;
+    const int rc = adjoint_launch(p, k, modes, &L);
+    if (rc && !(rc == SLOS_ERANGE && adjoint_modes(p, k, batch))) return rc;
+    nblk = std::max(nblk, L.nblk);
+  }
+  *bytes = (size_t)batch * nblk * p->me * sizeof(double2);
   return SLOS_OK;
 }
 
@@ -1936,6 +1968,16 @@ namespace {
 int run_adjoint(const slos_plan* p, const DevTables& dt, const AdjLaunch& L, const float2* U, int64_t batch, int k, int col,
                 const float2* psi, const float2* gk, float2* gout, double2* part, hipStream_t st) {
   const uint64_t Sp = p->size(k - 1), Sk = p->size(k);
+  if (L.turns) {
+    slos::AdjointModesArgs a{};
+    a.cg = dt.cg; a.lo = dt.lo; a.tuples = dt.tuples; a.tuples5 = dt.tuples5;
+    a.me = p->me; a.multiset = p->multiset; a.m = p->m; a.col = col;
+    a.U = U; a.psi = psi; a.gk = gk; a.gout = gout; a.Sp = (uint32_t)Sp; a.Sk = (uint32_t)Sk; a.turns = L.turns;
+    a.partial = part;
+    slos::launch_adjoint_modes(k - 1, dim3((unsigned)L.nblk, (unsigned)batch), st, a);
+    HIP_TRY(hipGetLastError());
+    return SLOS_OK;
+  }
   const uint32_t* ins = nullptr;
   if (L.walk) {
     const int rc = insert_table(p, st, &ins);
@@ -1972,7 +2014,7 @@ int slos_adjoint_layer(const slos_plan* p, const void* U, int64_t batch, int k, 
   if (col < 0 || col >= p->m) return fail(SLOS_EINVAL, "input mode out of range");
   if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
   AdjLaunch L;
-  int rc = adjoint_launch(p, k, &L);
+  int rc = adjoint_launch(p, k, adjoint_modes(p, k, batch), &L);
   if (rc) return rc;
   if (!ws || ws_bytes < (size_t)batch * L.nblk * p->me * sizeof(double2)) return fail(SLOS_ENOMEM, "workspace too small");
   DevTables dt;
@@ -2016,7 +2058,7 @@ int back_layout(const slos_plan* p, int64_t batch, int layer, bool readout, Back
   size_t sum = 0;
   for (int k = 1; k <= layer; ++k) {
     AdjLaunch L;
-    const int rc = adjoint_launch(p, k, &L);
+    const int rc = adjoint_launch(p, k, adjoint_modes(p, k, batch), &L);
     if (rc) return rc;
     b->L.push_back(L);
     b->part.push_back(sum);

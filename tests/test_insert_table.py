@@ -21,10 +21,11 @@ def test_insert_table_children(emu, n, m, mask, k, first):  # noqa: F811
 
 
 def _plan(n, m, mask):
-    modes = m if mask == "fock" else m - 2
+    modes = m - 2 if mask == "tail_empty" else m
+    step = {"dual_rail": 2, "sparse_1in4": 4}.get(mask, 1)
     occ = [0] * m
     for i in range(n):
-        occ[i % modes] += 1
+        occ[step * i % modes] += 1
     return FockSLOSKernel(n, m, occ, mask=mask, device="cuda")._plan
 
 
@@ -44,24 +45,27 @@ def test_descents_equal_the_thread_kernel(n, m, mask, rows):
 
 
 # parent prefixes of 1 to 8 positions on both sides of 16 modes; every parent in the last eight modes;
-# a last step of the walk of one parent
+# a last step of the walk of one parent; the layers of at most five parent photons by a lane a mode, in
+# groups of 32 and 64 lanes, and thread per state with many rows; masks with inadmissible children
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,m,mask,rows", [(6, 32, "fock", 1), (7, 16, "fock", 3), (8, 17, "tail_empty", 1),
+@pytest.mark.parametrize("n,m,mask,rows", [(5, 33, "fock", 1), (4, 64, "fock", 2), (6, 8, "fock", 200), (5, 7, "fock", 1200),
+                                           (6, 14, "unbunched", 2), (5, 40, "dual_rail", 1), (4, 24, "sparse_1in4", 3),
+                                           (1, 1, "fock", 1), (2, 6, "tail_empty", 4), (6, 32, "fock", 1), (7, 16, "fock", 3), (8, 17, "tail_empty", 1),
                                            (8, 24, "fock", 1), (9, 9, "fock", 2), (10, 12, "fock", 1),
                                            (13, 4, "fock", 5), (13, 9, "fock", 1)])
 def test_adjoint_against_complex128(n, m, mask, rows):
     """One adjoint layer against the complex128 kernel on random layers. A term of grad_prev is one of
     2 me fused products a component, one of dL/dU a product in float32 sums of at most 2 x 8 parents a
-    lane (FP64 beyond): errors within these counts, and two roundings, times the sums of magnitudes."""
+    lane or thread (FP64 beyond): errors within these counts, and two roundings, times the sums of magnitudes."""
     plan = _plan(n, m, mask)
-    me = m if mask == "fock" else m - 2
+    me = m - 2 if mask == "tail_empty" else m
     g = torch.Generator("cuda").manual_seed(17 * n + m)
 
     def rand(*shape):
         return torch.randn(shape, dtype=torch.complex64, device="cuda", generator=g)
 
     U = rand(rows, m, m)
-    for k in range(n, 5, -1):
+    for k in range(n, 0, -1):
         psi, gk, col = rand(rows, plan.sizes[k - 1]), rand(rows, plan.sizes[k]), k % m
         gU, ref_U, mag_U = torch.zeros_like(U), *(torch.zeros_like(U, dtype=torch.complex128) for _ in range(2))
         out = plan.adjoint_layer(U, k, col, psi, gk, gU)
