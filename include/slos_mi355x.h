@@ -203,6 +203,12 @@ int slos_loss_descend(const slos_plan* plan, int k, const float* q_k, float* q_k
                       double scale,
                       slos_stream_t stream);
 
+/* Every step of that recurrence, from layer n to the vacuum: out[k] (k < n) = scale[k] times the descent
+ * of out[k + 1] (of q for k = n - 1), float32 [batch][S_k] on the GPU; `out` and `scale` on the host. The
+ * same values as slos_loss_descend's, the last small layers in one launch. */
+int slos_loss_thin(const slos_plan* plan, const float* q, float* const* out, const double* scale, int64_t batch,
+                   slos_stream_t stream);
+
 /* The x-model's distribution on the last layer (species.py:123-146) of 3 <= n <= 24 photons in one
  * call: float32 out [batch][S_n] = the sum over the sets T of at most `order` (1 <= order <= n)
  * distinguishable photons of weights[|T|] times the distribution of the others interfering and T raised

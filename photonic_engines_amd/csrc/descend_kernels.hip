@@ -1,11 +1,14 @@
 // The pulls over children: k_descend_insert and k_adjoint_insert (child_walk.hpp), k_descend_block
-// (descend_block.hpp), k_adjoint_modes (adjoint_modes.hpp).
+// (descend_block.hpp), k_adjoint_modes (adjoint_modes.hpp), k_descend_tail
+// (descend_tail.hpp).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "adjoint_modes.hpp"
 #include "block_launch.hpp"
+#include "descend_tail.hpp"
+#include "pull_index.hpp"
 
 namespace slos {
 
@@ -87,6 +90,61 @@ void launch_adjoint_modes(int P, dim3 grid, hipStream_t st, const AdjointModesAr
     default: SLOS_MODES(5); break;
   }
 #undef SLOS_MODES
+}
+
+__global__ __launch_bounds__(kTailThreads) void k_descend_tail(TailArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int stride = a.me + 1;
+  const int ncg = (a.top + 1) * stride;
+  float* bufs = reinterpret_cast<float*>(smem);  // the even layers, then the odd ones
+  uint32_t* cg = reinterpret_cast<uint32_t*>(bufs + 2 * kTailStates);
+  int* lo = reinterpret_cast<int*>(cg + ncg);
+  const size_t b = blockIdx.y;
+  for (int i = threadIdx.x; i < ncg; i += kTailThreads) cg[i] = (uint32_t)a.cg[i];
+  for (int i = threadIdx.x; i < a.me; i += kTailThreads) lo[i] = a.lo[i];
+  const SpaceView32 sv{cg, lo, a.me, stride};
+  auto layer = [&](auto km, int k) {
+    constexpr int KM = decltype(km)::value;
+    const int P = k - 1;
+    const float* q = k == a.top ? a.q + b * a.S[a.top] : bufs + (k & 1) * kTailStates;
+    float* keep = bufs + (P & 1) * kTailStates;
+    float* out = a.out[P] + b * a.S[P];
+    const float invk = 1.f / (float)k, scale = a.scale[P];
+    for (uint32_t t = threadIdx.x; t < a.S[P]; t += kTailThreads) {
+      int p[KM];
+      if (KM <= 4 && a.tuples && P == KM && (a.multiset || KM == 4)) {
+        const TupleWord w = a.tuples[t];
+#pragma unroll
+        for (int i = 0; i < KM; ++i) p[i] = (int)(tw_byte(w, (4 - KM + i) & 3) & 63u);
+      } else {
+        unrank_fixed<KM>(sv, t, P, p);
+      }
+      float acc = 0.f;
+      children_fixed<KM>(sv, a.multiset, k, p, [&](uint32_t c, int, int cnt) { acc = fmaf(q[c], (float)cnt, acc); });
+      const float v = (acc * invk) * scale;
+      keep[t] = v;
+      out[t] = v;
+    }
+  };
+  for (int k = a.top; k >= 1; --k) {
+    __syncthreads();
+    switch (k - 1) {
+      case 0:
+      case 1: layer(std::integral_constant<int, 1>{}, k); break;
+      case 2: layer(std::integral_constant<int, 2>{}, k); break;
+      case 3: layer(std::integral_constant<int, 3>{}, k); break;
+      case 4: layer(std::integral_constant<int, 4>{}, k); break;
+      case 5:
+      case 6:
+      case 7:
+      case 8: layer(std::integral_constant<int, 8>{}, k); break;
+      default: layer(std::integral_constant<int, kTailTop>{}, k); break;
+    }
+  }
+}
+
+void launch_descend_tail(dim3 grid, size_t lds, hipStream_t st, const TailArgs& a) {
+  hipLaunchKernelGGL(k_descend_tail, grid, dim3(kTailThreads), lds, st, a);
 }
 
 }  // namespace slos

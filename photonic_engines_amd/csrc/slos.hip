@@ -30,6 +30,7 @@
 #include "front.hpp"
 #include "raise.hpp"
 #include "adjoint_modes.hpp"
+#include "descend_tail.hpp"
 
 namespace {
 
@@ -369,27 +370,29 @@ __global__ __launch_bounds__(64) void k_spot_ryser(const uint64_t* cg_g, const i
 // uniform loss: q_{k-1}(t) = sum_j q_k(t + e_j) (t_j + 1) / k  (pull over children, no atomics)
 // ------------------------------------------------------------------------------------------
 // (child ranks: slos::children_fixed in pull_index.hpp; k - 1 <= KM)
-template <int KM>
-__global__ __launch_bounds__(256) void k_descend(const uint64_t* cg_g, const int* lo_g, int me, int multiset, int k,
+template <int KM, class SV = slos::SpaceView, bool EXACT = false>
+__global__ __launch_bounds__(256) void k_descend(const uint64_t* cg_g, const int* lo_g, int me, int multiset, int kk,
                                                  const float* __restrict__ qk, uint64_t Sk,
                                                  float* __restrict__ qout, uint64_t Sp, int64_t B, float scale) {
   extern __shared__ __align__(16) unsigned char smem[];
+  typedef slos::RankT<SV> R;
+  const int k = EXACT ? KM + 1 : kk;
   const int stride = me + 1;
   const int ncg = (k + 1) * stride;
-  uint64_t* cg = reinterpret_cast<uint64_t*>(smem);
+  R* cg = reinterpret_cast<R*>(smem);
   int* lo = reinterpret_cast<int*>(cg + ncg);
-  for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = cg_g[i];
+  for (int i = threadIdx.x; i < ncg; i += blockDim.x) cg[i] = (R)cg_g[i];
   for (int i = threadIdx.x; i < me; i += blockDim.x) lo[i] = lo_g[i];
   __syncthreads();
-  const slos::SpaceView sv{cg, lo, me, stride};
+  const SV sv{cg, lo, me, stride};
   const float invk = 1.f / (float)k;
   for (int64_t b = blockIdx.y; b < B; b += gridDim.y) {
     const float* qb = qk + (size_t)b * Sk;
     for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < Sp; t += (uint64_t)gridDim.x * blockDim.x) {
       int p[KM];
-      slos::unrank_fixed<KM>(sv, t, k - 1, p);
+      slos::unrank_fixed<KM>(sv, (R)t, k - 1, p);
       float acc = 0.f;
-      slos::children_fixed<KM>(sv, multiset, k, p, [&](uint64_t c, int, int cnt) { acc = fmaf(qb[c], (float)cnt, acc); });
+      slos::children_fixed<KM>(sv, multiset, k, p, [&](R c, int, int cnt) { acc = fmaf(qb[c], (float)cnt, acc); });
       qout[(size_t)b * Sp + t] = (acc * invk) * scale;
     }
   }
@@ -2216,24 +2219,20 @@ uint64_t insert_per_wave(uint64_t Sp) { return Sp < (1ull << 22) ? 64 : Sp < (1u
 
 }  // namespace
 
-int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1, int64_t batch, unsigned flags,
-                      double scale, slos_stream_t stream) {
-  if (!p || !q_k || !q_km1) return fail(SLOS_EINVAL, "NULL argument");
-  if (k < 1 || k > p->n) return fail(SLOS_EINVAL, "layer out of range");
-  if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
-  DevTables dt;
-  int rc = device_tables(p, &dt);
-  if (rc) return rc;
+namespace {
+
+// one step of the loss recurrence
+int run_descend(const slos_plan* p, const DevTables& dt, int k, const float* q_k, float* q_km1, int64_t batch,
+                unsigned flags, double scale, hipStream_t st) {
   const uint64_t Sp = p->size(k - 1), Sk = p->size(k);
   const int dp = k - 1 - slos::kSuf;
   char name[32];
   std::snprintf(name, sizeof name, "slos descent %d", k);
   const RoctxRange range(name);
-  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!(flags & SLOS_FLAG_SIMPLE) && p->multiset && dt.tuples && dp >= 1 && dp <= 8) {
     const uint64_t S_pre = p->size(dp);
     const uint32_t* ins = nullptr;
-    rc = insert_table(p, st, &ins);
+    const int rc = insert_table(p, st, &ins);
     if (rc) return rc;
     if (ins) {
       if (insert_walk(p, dp, Sp, batch)) {
@@ -2267,11 +2266,78 @@ int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1,
   const size_t sh = (size_t)(k + 1) * (p->me + 1) * 8 + (size_t)p->me * 4;
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
   dim3 grid((unsigned)std::max<uint64_t>(1, std::min<uint64_t>((Sp + 255) / 256, 1u << 20)), (unsigned)batch);
-  with_km(k - 1, [&](auto km) {
-    hipLaunchKernelGGL((k_descend<decltype(km)::value>), grid, dim3(256), sh, reinterpret_cast<hipStream_t>(stream),
-                       dt.cg, dt.lo, p->me, p->multiset, k, q_k, Sk, q_km1, Sp, batch, (float)scale);
-  });
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), sh, st, dt.cg, dt.lo, p->me, p->multiset, k, q_k, Sk, q_km1, Sp, batch,
+                       (float)scale);
+  };
+  // (known photons and 32-bit ranks, as the forward's thread kernel: the step 5 -> 4 at 24 modes 14 -> 6 us)
+  switch (Sk < (1ull << 32) ? k - 1 : 0) {
+    case 1: launch(k_descend<1, slos::SpaceView32, true>); break;
+    case 2: launch(k_descend<2, slos::SpaceView32, true>); break;
+    case 3: launch(k_descend<3, slos::SpaceView32, true>); break;
+    case 4: launch(k_descend<4, slos::SpaceView32, true>); break;
+    case 5: launch(k_descend<5, slos::SpaceView32, true>); break;
+    case 6: launch(k_descend<6, slos::SpaceView32, true>); break;
+    case 7: launch(k_descend<7, slos::SpaceView32, true>); break;
+    case 8: launch(k_descend<8, slos::SpaceView32, true>); break;
+    default: with_km(k - 1, [&](auto km) { launch(k_descend<decltype(km)::value>); }); break;
+  }
   HIP_TRY(hipGetLastError());
+  return SLOS_OK;
+}
+
+// the layer k from which one launch takes every step down (descend_tail.hpp), or 0
+int tail_top(const slos_plan* p) {
+  int top = 0;
+  for (int k = 1; k <= std::min(p->n, slos::kTailTop); ++k) {
+    const uint64_t Sp = p->size(k - 1);
+    if (Sp > slos::kTailStates || Sp * (uint64_t)p->me > slos::kTailEdges || p->size(k) >= (1ull << 31)) break;
+    top = k;
+  }
+  return slos::tail_lds(top, p->me) <= lds_limit() ? top : 0;
+}
+
+}  // namespace
+
+int slos_loss_descend(const slos_plan* p, int k, const float* q_k, float* q_km1, int64_t batch, unsigned flags,
+                      double scale, slos_stream_t stream) {
+  if (!p || !q_k || !q_km1) return fail(SLOS_EINVAL, "NULL argument");
+  if (k < 1 || k > p->n) return fail(SLOS_EINVAL, "layer out of range");
+  if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
+  DevTables dt;
+  const int rc = device_tables(p, &dt);
+  if (rc) return rc;
+  return run_descend(p, dt, k, q_k, q_km1, batch, flags, scale, reinterpret_cast<hipStream_t>(stream));
+}
+
+int slos_loss_thin(const slos_plan* p, const float* q, float* const* out, const double* scale, int64_t batch,
+                   slos_stream_t stream) {
+  if (!p || !q || !scale || (p->n > 0 && !out)) return fail(SLOS_EINVAL, "NULL argument");
+  if (batch < 1 || batch > 65535) return fail(SLOS_EINVAL, "batch must be in [1, 65535]");
+  for (int k = 0; k < p->n; ++k)
+    if (!out[k]) return fail(SLOS_EINVAL, "NULL argument");
+  DevTables dt;
+  int rc = device_tables(p, &dt);
+  if (rc) return rc;
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int top = tail_top(p);
+  for (int k = p->n; k > top; --k) {
+    rc = run_descend(p, dt, k, k == p->n ? q : out[k], out[k - 1], batch, 0u, scale[k - 1], st);
+    if (rc) return rc;
+  }
+  if (top) {
+    const RoctxRange range("slos last descents");
+    slos::TailArgs a{};
+    a.cg = dt.cg; a.lo = dt.lo; a.tuples = dt.tuples; a.me = p->me; a.multiset = p->multiset; a.top = top;
+    a.q = top == p->n ? q : out[top];
+    for (int k = 0; k <= top; ++k) a.S[k] = (uint32_t)p->size(k);
+    for (int k = 0; k < top; ++k) {
+      a.out[k] = out[k];
+      a.scale[k] = (float)scale[k];
+    }
+    slos::launch_descend_tail(dim3(1, (unsigned)batch), slos::tail_lds(top, p->me), st, a);
+    HIP_TRY(hipGetLastError());
+  }
   return SLOS_OK;
 }
 

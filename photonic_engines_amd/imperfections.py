@@ -210,23 +210,25 @@ class _Descend(torch.autograd.Function):
 
 
 def carried_weights(n: int, eta: Eta, device, dtype=torch.float32) -> torch.Tensor | None:
-    """The binomial weights of layers 0..n in the probabilities' dtype (float32, or float64) when
-    the weighted blocks can be carried down the layers (a loss without gradient whose weights are
-    all positive), else None."""
+    """The binomial weights of layers 0..n in the probabilities' dtype (float32, or float64), on the host
+    (they go to the kernels as arguments), when the weighted blocks can be carried down the layers (a
+    loss without gradient whose weights are all positive), else None."""
     e = _eta(eta)
     if e is None or (isinstance(e, torch.Tensor) and e.requires_grad):
         return None
-    w = binomial_pmf(n, e, dtype=torch.float64, device=device).to(dtype)
+    # (on the host from the start, unless eta is on the GPU: no launches, nothing to wait for)
+    w = binomial_pmf(n, e, dtype=torch.float64, device=device if isinstance(e, torch.Tensor) and e.is_cuda else "cpu")
+    w = w.cpu().to(dtype)
     return w if bool((w > 0).all()) else None
 
 
 def thin_distribution(layers, probs: torch.Tensor, eta: Eta, chunk: int | None = None,
-                      _top_weighted: bool = False) -> LossyDistribution:
+                      _top_weighted: torch.Tensor | None = None) -> LossyDistribution:
     """Uniform output loss on the n-photon distribution `probs` ([S] or [B, S] over
     layers.final_states), returned as a LossyDistribution over 0..n photons
     (imperfections.py:309-337). Differentiable in probs and eta. `chunk` is accepted for
-    signature compatibility (the pull kernels need no edge chunks). `_top_weighted`: `probs` already
-    carries the weight of layer n (the forward's readout applied it)."""
+    signature compatibility (the pull kernels need no edge chunks). `_top_weighted`: the carried
+    weights, when `probs` already has that of layer n (the forward's readout applied it)."""
     n = layers.n
     e = _eta(eta)
     user_dev = probs.device
@@ -236,17 +238,13 @@ def thin_distribution(layers, probs: torch.Tensor, eta: Eta, chunk: int | None =
     q_top = (probs if batched else probs.unsqueeze(0)).to(device=dev, dtype=rdt).contiguous()
     plan = layers._plan
     grad = torch.is_grad_enabled() and (q_top.requires_grad or (isinstance(e, torch.Tensor) and e.requires_grad))
-    w32 = None if grad else carried_weights(n, e, dev, dtype=rdt)
-    if _top_weighted and w32 is None:
-        raise ValueError("_top_weighted needs a loss whose weights can be carried down the layers")
+    w32 = _top_weighted if _top_weighted is not None else None if grad else carried_weights(n, e, dev, dtype=rdt)
     if w32 is not None:
         # carry the weights down the layers: block[k-1] = descent(block[k]) * w[k-1] / w[k], one pass
         # per layer and no unweighted copies
-        ratio = (w32[:-1].double() / w32[1:].double()).cpu().tolist()
-        blocks = [None] * (n + 1)
-        blocks[n] = q_top if _top_weighted else q_top * w32[n]
-        for k in range(n, 0, -1):
-            blocks[k - 1] = plan.loss_descend(k, blocks[k], scale=ratio[k - 1])
+        ratio = (w32[:-1].double() / w32[1:].double()).tolist()
+        top = q_top if _top_weighted is not None else q_top * float(w32[n])
+        blocks = [*plan.loss_thin(top, ratio), top]
         out = []
         for b in blocks:
             b = b if batched else b.squeeze(0)

@@ -342,6 +342,20 @@ class Plan:
             nat.check(rc, "slos_loss_descend")
         return out
 
+    def loss_thin(self, q: torch.Tensor, scale) -> list:
+        """[q_0, .., q_{n-1}], q_k = scale[k] * descent of q_{k+1}, from q = q_n ([B, S_n] float32 or float64,
+        contiguous on the GPU)."""
+        B, n = q.shape[0], self.n
+        if q.dtype != torch.float32 or not 1 <= B <= MAX_ROWS:
+            res = [q]
+            for k in range(n, 0, -1):
+                res.append(self.loss_descend(k, res[-1], scale=scale[k - 1]))
+            return res[:0:-1]
+        out = [torch.empty((B, self.sizes[k]), dtype=q.dtype, device=q.device) for k in range(n)]
+        nat.check(self._lib.slos_loss_thin(self._h, nat.ptr(q), (ctypes.c_void_p * n)(*[t.data_ptr() for t in out]),
+                                           (ctypes.c_double * n)(*scale), B, nat.stream_handle(q.device)), "slos_loss_thin")
+        return out
+
     def loss_ascend(self, k: int, g: torch.Tensor) -> torch.Tensor:
         """Adjoint of loss_descend: [B, S_{k-1}] -> [B, S_k] (float32 or float64)."""
         out = torch.empty((g.shape[0], self.sizes[k]), dtype=g.dtype, device=g.device)

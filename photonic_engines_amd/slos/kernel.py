@@ -236,7 +236,7 @@ class FockSLOSKernel:
                               batched)
                 if w32 is not None:
                     from ..imperfections import thin_distribution
-                    return thin_distribution(self.layers, p, loss, _top_weighted=True)
+                    return thin_distribution(self.layers, p, loss, _top_weighted=w32)
         except torch.cuda.OutOfMemoryError as e:
             self._add_oom_hint(e)
             raise

@@ -76,3 +76,20 @@ def test_adjoint_against_complex128(n, m, mask, rows):
         eps = 2.0 ** -24 * 2 ** 0.5
         assert ((out - ref).abs() <= (2 * me + 2) * eps * mag.real).all(), k
         assert ((gU - ref_U).abs() <= (2 * 8 + 2) * eps * mag_U.real).all(), k
+
+
+# every step in one call: steps of the walk and thread per state, then the last layers in one launch: from
+# layer n on; from a layer of few states below larger ones; masks; nothing below the table's layers
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,mask,rows", [(1, 1, "fock", 1), (3, 12, "fock", 5), (6, 24, "fock", 2), (9, 5, "fock", 1),
+                                           (5, 64, "fock", 1), (12, 3, "fock", 3), (6, 20, "unbunched", 2),
+                                           (8, 16, "dual_rail", 1), (7, 14, "tail_empty", 4), (5, 24, "sparse_1in4", 1)])
+def test_all_descents_in_one_call(n, m, mask, rows):
+    plan = _plan(n, m, mask)
+    q = torch.rand((rows, plan.sizes[n]), device="cuda", generator=torch.Generator("cuda").manual_seed(n + m))
+    scale = [0.5 + 0.05 * k for k in range(n)]
+    out = plan.loss_thin(q, scale)
+    assert len(out) == n
+    for k in range(n, 0, -1):
+        q = plan.loss_descend(k, q, flags=nat.FLAG_SIMPLE, scale=scale[k - 1])
+        assert torch.equal(out[k - 1], q), k
