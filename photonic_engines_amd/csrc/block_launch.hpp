@@ -51,7 +51,7 @@ void launch_layer_block_group(bool comp, int d, uint32_t grid, size_t lds, hipSt
 // k_descend_block with maxd (4, 6 or 8) prefix slots (descend_kernels.hip)
 void launch_descend_block(int maxd, const BlockGrid& g, int K, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
                           uint64_t S_pre, uint64_t per_wave, float scale, uint32_t xcd_chunk);
-// the insert-table form for a prefix of dp (1 to 8) positions
+// the insert-table form for a prefix of dp (0 to 8) positions
 void launch_descend_insert(int dp, const BlockGrid& g, const float* qk, uint64_t Sk, float* qout, uint64_t Sp,
                            uint64_t per_wave, float scale, uint32_t xcd_chunk, const uint32_t* ins);
 // the adjoint of one layer, at most 32 modes

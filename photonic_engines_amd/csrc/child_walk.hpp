@@ -1,5 +1,5 @@
 // Pulls over children through the insert table (block_index.hpp: insert_word), for multiset spaces of
-// at most 41 modes and parent layers D = K - 1 = DP + 4, DP = 1..8: one step of the uniform-loss
+// at most 41 modes and parent layers D = K - 1 = DP + 4, DP = 0..8: one step of the uniform-loss
 // recurrence (photonic_engines/imperfections.py:254-276), q_{K-1}(t) = sum_a q_K(t + e_a) (t_a + 1) / K.
 //
 // A wave owns a contiguous range of parents and takes it block by block (a block: the parents (P, u)
@@ -45,6 +45,11 @@ __device__ __forceinline__ void child_walk(const uint64_t* __restrict__ cg, int 
   const int lane = threadIdx.x & 63;
   if (g >= Sp) return;
   const uint64_t g_end = g + per_wave < Sp ? g + per_wave : Sp;
+  if constexpr (DP == 0) {  // no prefix: one block, every mode through the table
+    sweep(ChildBlock{0, 0, 0, 1u, 0u, (uint32_t)Sp, 0}, (uint32_t)g, (uint32_t)g_end);
+    return;
+  }
+  constexpr int D1 = DP > 0 ? DP : 1;
   uint64_t row[DP + 1];  // lane x: cg[K - l][x + 1]
 #pragma unroll
   for (int l = 0; l <= DP; ++l) row[l] = lane < me ? cg[(K - l) * W + lane + 1] : 0u;
@@ -55,7 +60,7 @@ __device__ __forceinline__ void child_walk(const uint64_t* __restrict__ cg, int 
   const uint32_t n4 = (uint32_t)cg[4 * W], n5X = rl(c5, X);
   // the prefix of parent g: position l is the number of modes x >= its predecessor that g's rank
   // among the tuples from there on has passed
-  int p[DP];
+  int p[D1];
   uint64_t u0 = g;
   {
     uint64_t top = Sp;
@@ -77,9 +82,9 @@ __device__ __forceinline__ void child_walk(const uint64_t* __restrict__ cg, int 
   }
   while (g < g_end) {
     ChildBlock b;
-    // suffixes of 5 positions from X on, else of 4 (p[DP - 1] >= X: the first of the run it begins)
-    const bool merged = p[DP - 1] >= X;
-    b.x0 = p[DP - 1];
+    // suffixes of 5 positions from X on, else of 4 (p[D1 - 1] >= X: the first of the run it begins)
+    const bool merged = p[D1 - 1] >= X;
+    b.x0 = p[D1 - 1];
     const uint32_t L = rl(merged ? c5 : c4, b.x0);
     b.CBp = g - u0;
     uint64_t lower = cK, own = row[0];  // lane a: lower - own = its stream's base

@@ -17,6 +17,7 @@ namespace {
 template <class F>
 void with_prefix(int dp, F&& f) {
   switch (dp) {
+    case 0: f(std::integral_constant<int, 0>()); break;
     case 1: f(std::integral_constant<int, 1>()); break;
     case 2: f(std::integral_constant<int, 2>()); break;
     case 3: f(std::integral_constant<int, 3>()); break;
@@ -119,8 +120,7 @@ __global__ __launch_bounds__(kTailThreads) void k_descend_tail(TailArgs a) {
       } else {
         unrank_fixed<KM>(sv, t, P, p);
       }
-      float acc = 0.f;
-      children_fixed<KM>(sv, a.multiset, k, p, [&](uint32_t c, int, int cnt) { acc = fmaf(q[c], (float)cnt, acc); });
+      const float acc = children_sum<KM>(sv, a.multiset, k, p, q);
       const float v = (acc * invk) * scale;
       keep[t] = v;
       out[t] = v;

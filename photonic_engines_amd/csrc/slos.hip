@@ -198,7 +198,7 @@ int device_tables(const slos_plan* cp, DevTables* out) {
 }
 
 bool has_insert_table(const slos_plan* p) {
-  return p->multiset && !p->tuples.empty() && p->n > 5 && p->size(5) <= slos::kInsertTuples &&
+  return p->multiset && !p->tuples.empty() && p->n >= 5 && p->size(5) <= slos::kInsertTuples &&
          p->tuples.size() * (uint64_t)p->me <= slos::kInsertWords;
 }
 
@@ -392,7 +392,8 @@ __global__ __launch_bounds__(256) void k_descend(const uint64_t* cg_g, const int
       int p[KM];
       slos::unrank_fixed<KM>(sv, (R)t, k - 1, p);
       float acc = 0.f;
-      slos::children_fixed<KM>(sv, multiset, k, p, [&](R c, int, int cnt) { acc = fmaf(qb[c], (float)cnt, acc); });
+      if constexpr (EXACT) acc = slos::children_sum<KM>(sv, multiset, k, p, qb);
+      else slos::children_fixed<KM>(sv, multiset, k, p, [&](R c, int, int cnt) { acc = fmaf(qb[c], (float)cnt, acc); });
       qout[(size_t)b * Sp + t] = (acc * invk) * scale;
     }
   }
@@ -1901,10 +1902,10 @@ struct AdjLaunch {
   uint64_t nblk = 0;
 };
 
-// the insert-table kernel: parent prefixes of 1..8 positions, up to 32 modes (its sums' registers)
+// the insert-table kernel: parent prefixes of 0..8 positions, up to 32 modes (its sums' registers)
 bool adjoint_walk(const slos_plan* p, int k) {
   const int dp = k - 1 - slos::kSuf;
-  return has_insert_table(p) && dp >= 1 && dp <= 8 && p->me <= 32;
+  return has_insert_table(p) && dp >= 0 && dp <= 8 && p->me <= 32;
 }
 
 // Whether an adjoint layer takes the kernel with a lane a mode. It is quick to start and computes each
@@ -2208,7 +2209,7 @@ namespace {
 // of 24, 7.8M in all, 300 / 312; of 56, 705k in all, 53 / 44; of 10, 1.1M in all, 110 / 58.
 bool insert_walk(const slos_plan* p, int dp, uint64_t Sp, int64_t batch) {
   const int X = slos::insert_from(p->me);
-  const uint64_t blocks = (X ? p->cg[(size_t)dp * (p->me + 1) + (p->me - X)] : 0) + p->size(dp - 1);
+  const uint64_t blocks = dp == 0 ? 1 : (X ? p->cg[(size_t)dp * (p->me + 1) + (p->me - X)] : 0) + p->size(dp - 1);
   return Sp / blocks >= 256 || (Sp / blocks >= 32 && Sp >= (1ull << 20) / (uint64_t)batch);
 }
 
@@ -2229,7 +2230,7 @@ int run_descend(const slos_plan* p, const DevTables& dt, int k, const float* q_k
   char name[32];
   std::snprintf(name, sizeof name, "slos descent %d", k);
   const RoctxRange range(name);
-  if (!(flags & SLOS_FLAG_SIMPLE) && p->multiset && dt.tuples && dp >= 1 && dp <= 8) {
+  if (!(flags & SLOS_FLAG_SIMPLE) && p->multiset && dt.tuples && dp >= 0 && dp <= 8) {
     const uint64_t S_pre = p->size(dp);
     const uint32_t* ins = nullptr;
     const int rc = insert_table(p, st, &ins);
@@ -2245,7 +2246,7 @@ int run_descend(const slos_plan* p, const DevTables& dt, int k, const float* q_k
         HIP_TRY(hipGetLastError());
         return SLOS_OK;
       }
-    } else {
+    } else if (dp >= 1) {
       const int maxd = dp <= 4 ? 4 : dp <= 6 ? 6 : 8;
       const size_t shb = slos::desc_dyn_lds(k, p->me, maxd);
       if (shb <= lds_limit()) {

@@ -29,16 +29,16 @@ def _plan(n, m, mask):
     return FockSLOSKernel(n, m, occ, mask=mask, device="cuda")._plan
 
 
-# (n, m, mask, rows): parent prefixes of 1 to 8 positions, blocks of one parent up to the longest, the
+# (n, m, mask, rows): parent prefixes of 0 to 8 positions, blocks of one parent up to the longest, the
 # largest mode count of the table, several rows, and the thread-per-state side of the rule
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,m,mask,rows", [(6, 41, "fock", 1), (7, 12, "fock", 200), (8, 24, "fock", 1),
+@pytest.mark.parametrize("n,m,mask,rows", [(5, 41, "fock", 1), (5, 9, "fock", 3), (6, 41, "fock", 1), (7, 12, "fock", 200), (8, 24, "fock", 1),
                                            (9, 18, "tail_empty", 3), (10, 21, "fock", 1), (11, 17, "fock", 1),
                                            (12, 16, "fock", 1), (13, 16, "fock", 1), (9, 9, "fock", 2)])
 def test_descents_equal_the_thread_kernel(n, m, mask, rows):
     plan = _plan(n, m, mask)
     q = torch.rand((rows, plan.sizes[n]), device="cuda", generator=torch.Generator("cuda").manual_seed(n * m))
-    for k in range(n, 5, -1):
+    for k in range(n, 4, -1):
         out = plan.loss_descend(k, q, scale=0.75)
         assert torch.equal(out, plan.loss_descend(k, q, flags=nat.FLAG_SIMPLE, scale=0.75)), k
         q = out
@@ -48,7 +48,7 @@ def test_descents_equal_the_thread_kernel(n, m, mask, rows):
 # a last step of the walk of one parent; the layers of at most five parent photons by a lane a mode, in
 # groups of 32 and 64 lanes, and thread per state with many rows; masks with inadmissible children
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,m,mask,rows", [(5, 33, "fock", 1), (4, 64, "fock", 2), (6, 8, "fock", 200), (5, 7, "fock", 1200),
+@pytest.mark.parametrize("n,m,mask,rows", [(5, 33, "fock", 1), (5, 32, "fock", 4), (4, 64, "fock", 2), (6, 8, "fock", 200), (5, 7, "fock", 1200),
                                            (6, 14, "unbunched", 2), (5, 40, "dual_rail", 1), (4, 24, "sparse_1in4", 3),
                                            (1, 1, "fock", 1), (2, 6, "tail_empty", 4), (6, 32, "fock", 1), (7, 16, "fock", 3), (8, 17, "tail_empty", 1),
                                            (8, 24, "fock", 1), (9, 9, "fock", 2), (10, 12, "fock", 1),
