@@ -60,7 +60,7 @@ enum {
 };
 
 /* flags of slos_forward */
-#define SLOS_FLAG_COMPENSATED 1u /* two-sum (compensated) FP32 accumulation of every child sum */
+#define SLOS_FLAG_COMPENSATED 1u /* child sums in FP64, layers as hi/lo pairs of floats */
 #define SLOS_FLAG_IMMEDIATE 2u   /* amplitudes in the per-edge sqrt normalisation (kernel.py:239-244):
                                     raw amplitude * sqrt(prod_j t_j!) */
 #define SLOS_FLAG_SIMPLE 4u      /* force the thread-per-state kernel (ablation / debugging) */
@@ -315,7 +315,7 @@ int slos_group_replay(slos_group* group, slos_stream_t stream);
 
 /* complex128 / float64 twins (FockSLOSKernel(dtype=torch.complex128), kernel.py:92,117-118) of
  * the entry points with typed float pointers or no flags argument; same arguments and results
- * as their complex64 forms, in FP64, thread-per-state:
+ * as their complex64 forms, in FP64, thread-per-state kernels:
  *   slos_loss_descend_f64   slos_loss_descend (imperfections.py:254-276) on float64 q
  *   slos_loss_ascend_f64    slos_loss_ascend on float64 gradients
  *   slos_readout_adjoint_f64  slos_readout_adjoint: complex128 amps / grad_amps, float64 grad_p

@@ -24,10 +24,10 @@ struct Pair<double> {
 template <class T, bool COMP>
 struct Sum {
   T re = 0, im = 0;
-  BlockAcc c{0.f, 0.f, 0.f, 0.f};
+  BlockAcc<COMP> c;
   __device__ __forceinline__ void add(typename Pair<T>::type u, typename Pair<T>::type v) {
     if constexpr (std::is_same<T, float>::value) {
-      bk_cmac<COMP>(c, u, v);
+      bk_cmac(c, u, v);
     } else {
       re = fma(u.x, v.x, re);
       re = fma(-u.y, v.y, re);
@@ -90,14 +90,15 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
       Sum<T, COMP> s;
       parents_fixed<KM>(sv, a.multiset, K, p, [&](uint32_t pr, int mode, int) { s.add(ucol[mode], par[pr]); });
       if constexpr (COMP) {
-        if (K > 1)  // the parents' low-order parts, into the correction terms
+        if (K > 1)  // the parents' low-order parts
           parents_fixed<KM>(sv, a.multiset, K, p,
                             [&](uint32_t pr, int mode, int) { bk_lo_mac(s.c, ucol[mode], par[a.buf + pr]); });
       }
       T re, im;
       if constexpr (std::is_same<T, float>::value) {
-        re = COMP ? s.c.re + s.c.cre : s.c.re;
-        im = COMP ? s.c.im + s.c.cim : s.c.im;
+        const float2 sum = s.c.value();
+        re = sum.x;
+        im = sum.y;
       } else {
         re = s.re;
         im = s.im;
@@ -105,12 +106,12 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
       if (!last) {
         dst[g] = T2{re, im};
         if (keep) (static_cast<T2*>(a.below[K]) + (size_t)b * S)[g] = T2{re, im};
-        if constexpr (COMP) dst[a.buf + g] = T2{s.c.cre - (re - s.c.re), s.c.cim - (im - s.c.im)};
+        if constexpr (COMP) dst[a.buf + g] = s.c.rest(T2{re, im});
       } else if (a.kind == 0) {
         T2* out = static_cast<T2*>(a.out) + (size_t)b * S;
         out[g] = T2{re, im};
         if constexpr (COMP)
-          if (a.out_lo) out[a.out_lo + g] = T2{s.c.cre - (re - s.c.re), s.c.cim - (im - s.c.im)};
+          if (a.out_lo) out[a.out_lo + g] = s.c.rest(T2{re, im});
       } else {
         T f;
         if constexpr (std::is_same<T, float>::value) f = run_factorial_fixed<KM>(p, K, a.multiset);

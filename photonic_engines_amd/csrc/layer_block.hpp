@@ -74,44 +74,48 @@ __device__ __forceinline__ float prob_readout(float re, float im, float f) {
   return (re * re + im * im) * f;
 }
 
+// One complex sum of products. Plain: fused multiply-adds in FP32. Compensated: the products, exact in
+// FP64, and their sum in FP64, whose fused multiply-add has the rate of FP32's here; the products with
+// the parents' low-order parts in FP32. (Products split by fma and summed by FP32 two-sums took 36
+// operations a product of complex numbers, and bound these layers: at n = 9, m = 22 layers 7, 8 and 9 took 56, 79
+// and 190 us so, 33, 60 and 152 us as here; at n = 10 layer 10 740 -> 474 us. The group-order kernel's
+// registers then allow three waves a SIMD: with four, spilling, 210 us, with two 180 us.) A layer stores a value's nearest float and, as its low-order part, the rest.
+template <bool COMP>
 struct BlockAcc {
-  float re, im, cre, cim;
+  float re = 0.f, im = 0.f;
+  __device__ __forceinline__ float2 value() const { return make_float2(re, im); }
+};
+template <>
+struct BlockAcc<true> {
+  double re = 0.0, im = 0.0;
+  float lre = 0.f, lim = 0.f;
+  __device__ __forceinline__ float2 value() const { return make_float2((float)(re + (double)lre), (float)(im + (double)lim)); }
+  // what the stored value leaves
+  __device__ __forceinline__ float2 rest(float2 v) const {
+    return make_float2((float)((re + (double)lre) - (double)v.x), (float)((im + (double)lim) - (double)v.y));
+  }
 };
 
-// Compensated arithmetic must not be contracted: a product fused into the next addition would make
-// the two-sum's error terms wrong, so these bodies turn contraction off.
-__device__ __forceinline__ void bk_two_sum(float& s, float& c, float x) {
-#pragma clang fp contract(off)
-  const float t = s + x;
-  const float bp = t - s;
-  c += (s - (t - bp)) + (x - bp);
-  s = t;
+// acc += u * v
+__device__ __forceinline__ void bk_cmac(BlockAcc<false>& a, float2 u, float2 v) {
+  a.re = fmaf(u.x, v.x, a.re);
+  a.re = fmaf(-u.y, v.y, a.re);
+  a.im = fmaf(u.x, v.y, a.im);
+  a.im = fmaf(u.y, v.x, a.im);
+}
+__device__ __forceinline__ void bk_cmac(BlockAcc<true>& a, float2 u, float2 v) {
+  a.re = fma((double)u.x, (double)v.x, a.re);
+  a.re = fma(-(double)u.y, (double)v.y, a.re);
+  a.im = fma((double)u.x, (double)v.y, a.im);
+  a.im = fma((double)u.y, (double)v.x, a.im);
 }
 
-// acc += u * v; COMP: products split exactly by fma, sums by two-sum, errors kept in cre / cim
-template <bool COMP>
-__device__ __forceinline__ void bk_cmac(BlockAcc& a, float2 u, float2 v) {
-  if constexpr (!COMP) {
-    a.re = fmaf(u.x, v.x, a.re);
-    a.re = fmaf(-u.y, v.y, a.re);
-    a.im = fmaf(u.x, v.y, a.im);
-    a.im = fmaf(u.y, v.x, a.im);
-  } else {
-#pragma clang fp contract(off)
-    float p, e;
-    p = u.x * v.x; e = fmaf(u.x, v.x, -p); bk_two_sum(a.re, a.cre, p); a.cre += e;
-    p = -u.y * v.y; e = fmaf(-u.y, v.y, -p); bk_two_sum(a.re, a.cre, p); a.cre += e;
-    p = u.x * v.y; e = fmaf(u.x, v.y, -p); bk_two_sum(a.im, a.cim, p); a.cim += e;
-    p = u.y * v.x; e = fmaf(u.y, v.x, -p); bk_two_sum(a.im, a.cim, p); a.cim += e;
-  }
-}
-
-// the low-order part w of a hi/lo parent value: acc.c += u * w (plain products into the correction)
-__device__ __forceinline__ void bk_lo_mac(BlockAcc& a, float2 u, float2 w) {
-  a.cre = fmaf(u.x, w.x, a.cre);
-  a.cre = fmaf(-u.y, w.y, a.cre);
-  a.cim = fmaf(u.x, w.y, a.cim);
-  a.cim = fmaf(u.y, w.x, a.cim);
+// the low-order part w of a hi/lo parent value: acc += u * w
+__device__ __forceinline__ void bk_lo_mac(BlockAcc<true>& a, float2 u, float2 w) {
+  a.lre = fmaf(u.x, w.x, a.lre);
+  a.lre = fmaf(-u.y, w.y, a.lre);
+  a.lim = fmaf(u.x, w.y, a.lim);
+  a.lim = fmaf(u.y, w.x, a.lim);
 }
 
 // One row of the per-launch suffix table (LDS, kSufRows rows, row = tuple-word byte): the U
@@ -296,29 +300,26 @@ __device__ __forceinline__ void sweep(const ChunkCtx<MAXD, SUF>& cx, uint32_t uc
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    BlockAcc acc{0.f, 0.f, 0.f, 0.f};
+    BlockAcc<COMP> acc;
 #pragma unroll
-    for (int s = 0; s < MAXD; ++s) bk_cmac<COMP>(acc, cx.coef[s], sv[c][s]);
+    for (int s = 0; s < MAXD; ++s) bk_cmac(acc, cx.coef[s], sv[c][s]);
 #pragma unroll
-    for (int jj = 0; jj < SUF; ++jj) bk_cmac<COMP>(acc, lc[c][jj], lv[c][jj]);
+    for (int jj = 0; jj < SUF; ++jj) bk_cmac(acc, lc[c][jj], lv[c][jj]);
     if constexpr (COMP) {
-      if (cx.plo) {  // the parents' low-order parts, into the correction terms (plain products)
+      if (cx.plo) {  // the parents' low-order parts
 #pragma unroll
         for (int s = 0; s < MAXD; ++s) bk_lo_mac(acc, cx.coef[s], at_bytes(cx.sp[s] + cx.plo, u[c] * 8u));
 #pragma unroll
         for (int jj = 0; jj < SUF; ++jj) bk_lo_mac(acc, lc[c][jj], at_bytes(cx.lp + cx.plo, loff[c][jj]));
       }
     }
-    // (plain sums: the correction terms are zero and are not added)
-    float re = COMP ? acc.re + acc.cre : acc.re, im = COMP ? acc.im + acc.cim : acc.im;
+    const float2 sum = acc.value();
+    float re = sum.x, im = sum.y;
     if (KIND == 0 || (KIND == 3 && cx.kind == 0)) {
       if (in[c]) *reinterpret_cast<float2*>(cx.ob + u[c] * 8u) = make_float2(re, im);
       if constexpr (COMP) {
-        // the rounding error of the stored value (fast two-sum: |acc.re| >= |acc.cre| as the
-        // correction is the accumulated rounding error of the sum)
         if (cx.olo && in[c])
-          *reinterpret_cast<float2*>(cx.ob + u[c] * 8u + cx.olo * 8) =
-              make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
+          *reinterpret_cast<float2*>(cx.ob + u[c] * 8u + cx.olo * 8) = acc.rest(sum);
       }
     } else if constexpr (KIND == 4) {
       if (in[c])
@@ -383,14 +384,15 @@ __device__ __forceinline__ void sweep_pairs(const ChunkCtx<MAXD, SUF>& cx, uint3
   float f[2] = {1.f, 1.f};
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    BlockAcc acc{0.f, 0.f, 0.f, 0.f};
+    BlockAcc<COMP> acc;
 #pragma unroll
     for (int s = 0; s < MAXD; ++s)
-      bk_cmac<COMP>(acc, cx.coef[s], c == 0 ? make_float2(sv[s].x, sv[s].y) : make_float2(sv[s].z, sv[s].w));
+      bk_cmac(acc, cx.coef[s], c == 0 ? make_float2(sv[s].x, sv[s].y) : make_float2(sv[s].z, sv[s].w));
 #pragma unroll
-    for (int jj = 0; jj < SUF; ++jj) bk_cmac<COMP>(acc, lc[c][jj], lv[c][jj]);
-    res[c][0] = COMP ? acc.re + acc.cre : acc.re;
-    res[c][1] = COMP ? acc.im + acc.cim : acc.im;
+    for (int jj = 0; jj < SUF; ++jj) bk_cmac(acc, lc[c][jj], lv[c][jj]);
+    const float2 sum = acc.value();
+    res[c][0] = sum.x;
+    res[c][1] = sum.y;
     if (!(KIND == 0 || (KIND == 3 && cx.kind == 0))) f[c] = child_norm_w(cx, tw[c]);
   }
   if (KIND == 0 || (KIND == 3 && cx.kind == 0)) {
@@ -721,37 +723,28 @@ __host__ __device__ inline size_t group_dyn_lds(int K, int me) {
 }
 
 // the suffix parents of two adjacent children (pair_edges): one 16-byte load for each dropped
-// position, and one 8-byte load in the lanes whose second child has a parent elsewhere (SEP: a load
-// for each child and position)
-template <bool SEP, int SUF>
+// position, and one 8-byte load in the lanes whose second child has a parent elsewhere
+template <int SUF>
 __device__ __forceinline__ void load_pair_parents(const float2* lp, const PairOffsets<SUF>& o, float2 (&lv)[2][SUF]) {
-  if constexpr (SEP) {
+  float4 pv[SUF];
 #pragma unroll
-    for (int j = 0; j < SUF; ++j) {
-      lv[0][j] = at_bytes(lp, o.a[j]);
-      lv[1][j] = at_bytes(lp, o.b[j]);
-    }
-  } else {
-    float4 pv[SUF];
+  for (int j = 0; j < SUF; ++j) pv[j] = load_pair(lp, o.a[j]);
+  float2 xv = make_float2(0.f, 0.f);
+  if (o.e < SUF - 1) xv = at_bytes(lp, o.x);
 #pragma unroll
-    for (int j = 0; j < SUF; ++j) pv[j] = load_pair(lp, o.a[j]);
-    float2 xv = make_float2(0.f, 0.f);
-    if (o.e < SUF - 1) xv = at_bytes(lp, o.x);
-#pragma unroll
-    for (int j = 0; j < SUF; ++j) {
-      lv[0][j] = make_float2(pv[j].x, pv[j].y);
-      const float2 other = j == SUF - 1 ? lv[0][j] : xv;
-      lv[1][j] = make_float2(o.e == j ? other.x : pv[j].z, o.e == j ? other.y : pv[j].w);
-    }
+  for (int j = 0; j < SUF; ++j) {
+    lv[0][j] = make_float2(pv[j].x, pv[j].y);
+    const float2 other = j == SUF - 1 ? lv[0][j] : xv;
+    lv[1][j] = make_float2(o.e == j ? other.x : pv[j].z, o.e == j ? other.y : pv[j].w);
   }
 }
 
 // one block of the group for the pair step: NS stream slots (slot 0 shared), both children;
 // KIND 1 writes probabilities (float32), KIND 0 the raw complex64 amplitudes of a middle layer, KIND 4
 // (gp: dL/dp of the row) their gradients by the readout
-// COMP: compensated sums as the block kernel's sweep (two-sum accumulation; with plo the parents'
-// low-order parts at element offset plo, slot 0's in v0lo; with olo the stored value's rounding
-// error at element offset olo of a complex64 output).
+// COMP: compensated sums as the block kernel's sweep (with plo the parents' low-order parts at element
+// offset plo, slot 0's in v0lo; with olo the stored value's low-order part at element offset olo of a
+// complex64 output).
 template <int NS, int KIND, bool COMP = false>
 __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const float2* par, const float4& v0,
                                                   const float2 (&lc)[2][5], const PairOffsets<5>& off,
@@ -775,22 +768,22 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
   }
   const float2* lp = par + LBp;
   float2 lv[2][5];
-  load_pair_parents<COMP>(lp, off, lv);
+  load_pair_parents(lp, off, lv);
   const uint32_t lastrow = ((w6 >> 16) & 0xffu) + 1u;
   float res[2][2];
-  BlockAcc accs[2];
+  BlockAcc<COMP> accs[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    BlockAcc acc{0.f, 0.f, 0.f, 0.f};
+    BlockAcc<COMP> acc;
 #pragma unroll
     for (int s = 0; s < NS; ++s)
-      bk_cmac<COMP>(acc, coef[s], c == 0 ? make_float2(sv[s].x, sv[s].y) : make_float2(sv[s].z, sv[s].w));
+      bk_cmac(acc, coef[s], c == 0 ? make_float2(sv[s].x, sv[s].y) : make_float2(sv[s].z, sv[s].w));
 #pragma unroll
-    for (int j = 0; j < 5; ++j) bk_cmac<COMP>(acc, lc[c][j], lv[c][j]);
+    for (int j = 0; j < 5; ++j) bk_cmac(acc, lc[c][j], lv[c][j]);
     accs[c] = acc;
   }
   if constexpr (COMP) {
-    if (plo) {  // the parents' low-order parts, into the correction terms (plain products)
+    if (plo) {  // the parents' low-order parts
       float4 sl[NS];
       sl[0] = v0lo;
 #pragma unroll
@@ -799,7 +792,7 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
         sl[s] = load_pair(par + plo + base, u * 8u);
       }
       float2 ll[2][5];
-      load_pair_parents<COMP>(lp + plo, off, ll);
+      load_pair_parents(lp + plo, off, ll);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
@@ -812,17 +805,17 @@ __device__ __forceinline__ void group_block_pairs(const uint4 (&bw)[8], const fl
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    res[c][0] = COMP ? accs[c].re + accs[c].cre : accs[c].re;
-    res[c][1] = COMP ? accs[c].im + accs[c].cim : accs[c].im;
+    const float2 sum = accs[c].value();
+    res[c][0] = sum.x;
+    res[c][1] = sum.y;
   }
   if constexpr (KIND == 0) {
     const float4 v = make_float4(res[0][0], res[0][1], res[1][0], res[1][1]);
     __builtin_memcpy(static_cast<float2*>(out) + CB + u, &v, 16);
     if constexpr (COMP) {
-      // the rounding error of the stored value (fast two-sum, as the block kernel)
       if (olo) {
-        const float4 e = make_float4(accs[0].cre - (res[0][0] - accs[0].re), accs[0].cim - (res[0][1] - accs[0].im),
-                                     accs[1].cre - (res[1][0] - accs[1].re), accs[1].cim - (res[1][1] - accs[1].im));
+        const float2 e0 = accs[0].rest(make_float2(res[0][0], res[0][1])), e1 = accs[1].rest(make_float2(res[1][0], res[1][1]));
+        const float4 e = make_float4(e0.x, e0.y, e1.x, e1.y);
         __builtin_memcpy(static_cast<float2*>(out) + olo + CB + u, &e, 16);
       }
     }
@@ -871,11 +864,11 @@ __device__ __forceinline__ void group_block_one(const uint4 (&bw)[8], const floa
   float2 lv[5];
 #pragma unroll
   for (int j = 0; j < 5; ++j) lv[j] = at_bytes(lp, off[j]);
-  BlockAcc acc{0.f, 0.f, 0.f, 0.f};
+  BlockAcc<COMP> acc;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) bk_cmac<COMP>(acc, coef[s], sv[s]);
+  for (int s = 0; s < NS; ++s) bk_cmac(acc, coef[s], sv[s]);
 #pragma unroll
-  for (int j = 0; j < 5; ++j) bk_cmac<COMP>(acc, lc[j], lv[j]);
+  for (int j = 0; j < 5; ++j) bk_cmac(acc, lc[j], lv[j]);
   if constexpr (COMP) {
     if (plo) {
       bk_lo_mac(acc, coef[0], v0lo);
@@ -888,11 +881,12 @@ __device__ __forceinline__ void group_block_one(const uint4 (&bw)[8], const floa
       for (int j = 0; j < 5; ++j) bk_lo_mac(acc, lc[j], at_bytes(lp + plo, off[j]));
     }
   }
-  const float re = COMP ? acc.re + acc.cre : acc.re, im = COMP ? acc.im + acc.cim : acc.im;
+  const float2 sum = acc.value();
+  const float re = sum.x, im = sum.y;
   if constexpr (KIND == 0) {
     if (in) static_cast<float2*>(out)[CB + u] = make_float2(re, im);
     if constexpr (COMP) {
-      if (olo && in) static_cast<float2*>(out)[olo + CB + u] = make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
+      if (olo && in) static_cast<float2*>(out)[olo + CB + u] = acc.rest(sum);
     }
   } else {
     const float f = fQ * rn[(lead ? ((w6 >> 16) & 0xffu) + 1u : 0u) * 16u + code];
@@ -919,7 +913,7 @@ __device__ __forceinline__ void group_dispatch(uint32_t nact, F&& f) {
 }
 
 template <int MAXD, int KIND, bool COMP = false>
-__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_layer_group(
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(COMP ? 3 : 4))) void k_layer_group(
     const uint64_t* __restrict__ cg_t, const int* __restrict__ lo_t, const uint64_t* __restrict__ tuples5, int me,
     int stride, const float2* __restrict__ par_all, void* __restrict__ out_all, BlockLayer a,
     const uint4* __restrict__ items, uint32_t n_items) {
@@ -1032,6 +1026,13 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4
     float4 v0lo{};
     if (COMP && a.par_lo) v0lo = load_pair(sp0 + a.par_lo, u * 8u);
     for (int g = 0; g < G; ++g) {
+      if constexpr (COMP) {
+        // (opaque in every turn: else the coefficients are kept widened to FP64 for all of them, and spill)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int j = 0; j < 5; ++j) asm volatile("" : "+v"(lc[c][j].x), "+v"(lc[c][j].y));
+      }
       uint4 bw[8];
       group_words(tbl, g, bw);
       group_dispatch<MAXD>(bw[1].x >> 24, [&](auto ns) {

@@ -10,37 +10,6 @@
 
 namespace slos {
 
-struct Acc {
-  float re = 0.f, im = 0.f, cre = 0.f, cim = 0.f;
-};
-
-// (compensated arithmetic: no contraction, see bk_two_sum)
-__device__ __forceinline__ void two_sum(float& s, float& c, float x) {
-#pragma clang fp contract(off)
-  const float t = s + x;
-  const float bp = t - s;
-  c += (s - (t - bp)) + (x - bp);
-  s = t;
-}
-
-// acc += u * v, plain or compensated (product errors by fma, sums by two-sum)
-template <bool COMP>
-__device__ __forceinline__ void cmac(Acc& a, float2 u, float2 v) {
-  if constexpr (!COMP) {
-    a.re = fmaf(u.x, v.x, a.re);
-    a.re = fmaf(-u.y, v.y, a.re);
-    a.im = fmaf(u.x, v.y, a.im);
-    a.im = fmaf(u.y, v.x, a.im);
-  } else {
-#pragma clang fp contract(off)
-    float p, e;
-    p = u.x * v.x; e = fmaf(u.x, v.x, -p); two_sum(a.re, a.cre, p); a.cre += e;
-    p = -u.y * v.y; e = fmaf(-u.y, v.y, -p); two_sum(a.re, a.cre, p); a.cre += e;
-    p = u.x * v.y; e = fmaf(u.x, v.y, -p); two_sum(a.im, a.cim, p); a.cim += e;
-    p = u.y * v.x; e = fmaf(u.y, v.x, -p); two_sum(a.im, a.cim, p); a.cim += e;
-  }
-}
-
 struct LayerArgs {
   const uint64_t* cg;
   const int* lo;
@@ -90,25 +59,18 @@ __global__ __launch_bounds__(256) void k_layer_simple(LayerArgs a) {
          g += (uint64_t)gridDim.x * blockDim.x) {
       int p[KM];
       unrank_words<KM>(sv, a.words, (R)g, K, p);
-      Acc acc;
-      parents_fixed<KM>(sv, a.multiset, K, p, [&](R pr, int mode, int) { cmac<COMP>(acc, ucol[mode], pb[pr]); });
+      BlockAcc<COMP> acc;
+      parents_fixed<KM>(sv, a.multiset, K, p, [&](R pr, int mode, int) { bk_cmac(acc, ucol[mode], pb[pr]); });
       if constexpr (COMP) {
-        if (a.par_lo)  // the parents' low-order parts, into the correction terms
-          parents_fixed<KM>(sv, a.multiset, K, p, [&](R pr, int mode, int) {
-            const float2 u = ucol[mode], w = pb[a.par_lo + pr];
-            acc.cre = fmaf(u.x, w.x, acc.cre);
-            acc.cre = fmaf(-u.y, w.y, acc.cre);
-            acc.cim = fmaf(u.x, w.y, acc.cim);
-            acc.cim = fmaf(u.y, w.x, acc.cim);
-          });
+        if (a.par_lo)  // the parents' low-order parts
+          parents_fixed<KM>(sv, a.multiset, K, p, [&](R pr, int mode, int) { bk_lo_mac(acc, ucol[mode], pb[a.par_lo + pr]); });
       }
-      float re = COMP ? acc.re + acc.cre : acc.re, im = COMP ? acc.im + acc.cim : acc.im;
+      const float2 sum = acc.value();
+      float re = sum.x, im = sum.y;
       if constexpr (KIND == 0) {
         reinterpret_cast<float2*>(a.out)[(size_t)b * a.S + g] = make_float2(re, im);
         if constexpr (COMP) {
-          if (a.out_lo)  // the rounding error of the stored value (fast two-sum)
-            reinterpret_cast<float2*>(a.out)[a.out_lo + (size_t)b * a.S + g] =
-                make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
+          if (a.out_lo) reinterpret_cast<float2*>(a.out)[a.out_lo + (size_t)b * a.S + g] = acc.rest(sum);
         }
       } else if constexpr (KIND == 4) {
         const uint64_t c = (uint64_t)b * a.S + g;

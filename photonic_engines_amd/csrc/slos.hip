@@ -530,9 +530,9 @@ __global__ __launch_bounds__(256) void k_readout_adjoint_pull(const uint64_t* cg
         }
         const float2* ub = U + (size_t)b * m * m;
         const float2* pb = par + (size_t)b * S_par;
-        slos::Acc acc;
+        slos::BlockAcc<false> acc;
         slos::parents_fixed<KM>(sv, multiset, K, p,
-                                [&](uint64_t pr, int mode, int) { slos::cmac<false>(acc, ub[(size_t)mode * m + col], pb[pr]); });
+                                [&](uint64_t pr, int mode, int) { slos::bk_cmac(acc, ub[(size_t)mode * m + col], pb[pr]); });
         const float w = 2.f * s2 * f * gv;
         r = make_float2(w * acc.re, w * acc.im);
       }
@@ -1133,20 +1133,16 @@ __global__ __launch_bounds__(256) void k_layer_simple_group(slos::GroupLaunch gl
       if (g >= it.S) break;
       int pos[KM];
       slos::unrank_fixed<KM>(sv, g, K, pos);
-      slos::Acc acc;
+      slos::BlockAcc<COMP> acc;
       slos::parents_fixed<KM>(sv, it.multiset, K, pos,
-                              [&](uint64_t pr, int mode, int) { slos::cmac<COMP>(acc, ucol[mode], pb[pr]); });
+                              [&](uint64_t pr, int mode, int) { slos::bk_cmac(acc, ucol[mode], pb[pr]); });
       if constexpr (COMP) {
-        if (it.par_lo)  // the parents' low-order parts, into the correction terms
-          slos::parents_fixed<KM>(sv, it.multiset, K, pos, [&](uint64_t pr, int mode, int) {
-            const float2 u = ucol[mode], v = pb[it.par_lo + pr];
-            acc.cre = fmaf(u.x, v.x, acc.cre);
-            acc.cre = fmaf(-u.y, v.y, acc.cre);
-            acc.cim = fmaf(u.x, v.y, acc.cim);
-            acc.cim = fmaf(u.y, v.x, acc.cim);
-          });
+        if (it.par_lo)  // the parents' low-order parts
+          slos::parents_fixed<KM>(sv, it.multiset, K, pos,
+                                  [&](uint64_t pr, int mode, int) { slos::bk_lo_mac(acc, ucol[mode], pb[it.par_lo + pr]); });
       }
-      float re = COMP ? acc.re + acc.cre : acc.re, im = COMP ? acc.im + acc.cim : acc.im;
+      const float2 sum = acc.value();
+      float re = sum.x, im = sum.y;
       if (it.kind == 1) {
         const float f = slos::run_factorial_fixed<KM>(pos, K, it.multiset);
         re *= it.scale;
@@ -1155,9 +1151,7 @@ __global__ __launch_bounds__(256) void k_layer_simple_group(slos::GroupLaunch gl
       } else {
         reinterpret_cast<float2*>(it.out)[(size_t)b * it.S + g] = make_float2(re, im);
         if constexpr (COMP) {
-          if (it.out_lo)
-            reinterpret_cast<float2*>(it.out)[it.out_lo + (size_t)b * it.S + g] =
-                make_float2(acc.cre - (re - acc.re), acc.cim - (im - acc.im));
+          if (it.out_lo) reinterpret_cast<float2*>(it.out)[it.out_lo + (size_t)b * it.S + g] = acc.rest(sum);
         }
       }
     }

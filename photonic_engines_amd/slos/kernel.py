@@ -13,10 +13,10 @@ Device model: the engine always computes on an AMD GPU. `device` is where U is t
 where results are returned; a CPU `device` (the reference's default) therefore means host-resident
 inputs and outputs around the same GPU computation. Without a visible GPU the engine raises.
 
-Precision: complex64 end to end (float32 probabilities); `compensated=True` (keyword) accumulates
-every child sum with fma-split products and two-sum (a compensated dot product), as an accuracy
-option. `dtype=torch.complex128` computes every layer in complex128 and the probabilities in
-float64 (kernel.py:117-118), on the thread-per-state FP64 kernels.
+Precision: complex64 end to end (float32 probabilities); `compensated=True` (keyword) sums every
+child's products, exact, in FP64 and carries each layer with its rounding errors (a compensated dot
+product), as an accuracy option. `dtype=torch.complex128` computes every layer in complex128 and the probabilities in
+float64 (kernel.py:117-118).
 """
 from __future__ import annotations
 
