@@ -73,7 +73,7 @@ enum {
                                     slos_layer_step in complex128: U, the layers and the amplitudes
                                     complex128, the probabilities float64, every sum in FP64 (the
                                     reference's dtype=torch.complex128, kernel.py:92,117-118).
-                                    Thread-per-state kernels; not with SLOS_FLAG_COMPENSATED */
+                                    Not with SLOS_FLAG_COMPENSATED */
 
 /* Version string of the library. */
 const char* slos_version(void);
@@ -215,10 +215,10 @@ int slos_loss_thin(const slos_plan* plan, const float* q, float* const* out, con
  * (slos_raise), the terms sharing their raises. `weights`: n + 2 floats, on the host or (weights_on_device)
  * the GPU: weights[L], L <= n - 2, of each set of L photons, and weights[n + 1] of all sets of n - 1
  * and n photons together. flags: SLOS_FLAG_COMPENSATED or 0 (the forwards' sums). U: complex64
- * [batch][m][m], W: float32 |U|^2, batch <= 65535; the sets of all sizes together at most 2^20. */
+ * [batch][m][m], batch <= 65535; the sets of all sizes together at most 2^20. */
 int slos_xmodel_workspace(const slos_plan* plan, int64_t batch, int order, unsigned flags, size_t* bytes);
-int slos_xmodel(const slos_plan* plan, const void* U, const float* W, int64_t batch, int order,
-                const float* weights, int weights_on_device, float* out, unsigned flags, void* workspace, size_t workspace_bytes,
+int slos_xmodel(const slos_plan* plan, const void* U, int64_t batch, int order, const float* weights,
+                int weights_on_device, float* out, unsigned flags, void* workspace, size_t workspace_bytes,
                 slos_stream_t stream);
 
 /* Probability-level raise of partial distinguishability (species.classical_raise,

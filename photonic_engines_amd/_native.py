@@ -56,7 +56,7 @@ SIGNATURES = {
     "slos_loss_thin": (_c.c_int, [_vp, _vp, _c.POINTER(_vp), _f64p, _c.c_int64, _vp]),
     "slos_loss_ascend": (_c.c_int, [_vp, _c.c_int, _vp, _vp, _c.c_int64, _vp]),
     "slos_xmodel_workspace": (_c.c_int, [_vp, _c.c_int64, _c.c_int, _c.c_uint, _c.POINTER(_c.c_size_t)]),
-    "slos_xmodel": (_c.c_int, [_vp, _vp, _vp, _c.c_int64, _c.c_int, _vp, _c.c_int, _vp, _c.c_uint, _vp, _c.c_size_t, _vp]),
+    "slos_xmodel": (_c.c_int, [_vp, _vp, _c.c_int64, _c.c_int, _vp, _c.c_int, _vp, _c.c_uint, _vp, _c.c_size_t, _vp]),
     "slos_raise": (_c.c_int, [_vp, _c.c_int, _vp, _vp, _vp, _c.c_int64, _vp]),
     "slos_loss_descend_f64": (_c.c_int, [_vp, _c.c_int, _vp, _vp, _c.c_int64, _c.c_double, _vp]),
     "slos_loss_ascend_f64": (_c.c_int, [_vp, _c.c_int, _vp, _vp, _c.c_int64, _vp]),

@@ -32,7 +32,7 @@ struct RaiseArgs {
   const float* row_scale;  // out holds the targets' own terms, to be scaled by these (null: nothing) ..
   const float* weight;     // .. and by this (device, or null: weight_value)
   float weight_value;
-  const float* W;          // |U|^2 [B][m][m]
+  const float2* U;         // [B][m][m]
   int cols[kRaisePhotons]; // input column of each photon
 };
 

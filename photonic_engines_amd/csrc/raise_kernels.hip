@@ -13,6 +13,12 @@ __device__ __forceinline__ float add_rounded(float a, float b) {
   return a + b;
 }
 
+// |u|^2, every operation rounded
+__device__ __forceinline__ float square_rounded(float2 u) {
+#pragma clang fp contract(off)
+  return u.x * u.x + u.y * u.y;
+}
+
 // One child a thread: its positions and its parents' ranks once, for all rows of the work group. A row
 // costs a gather, an LDS weight and a multiply-add per parent and source; the gathers are 4 bytes a
 // lane from one row, near one another. Bound by the cache's rate for them. A source's parents are summed
@@ -35,7 +41,8 @@ __global__ __launch_bounds__(256) void k_raise_rows(RaiseArgs a) {
   for (int i = threadIdx.x; i < a.me; i += blockDim.x) lo[i] = a.lo[i];
   for (int i = threadIdx.x; i < a.photons * a.me; i += blockDim.x) {
     const int j = i / a.me, x = i - j * a.me;
-    wl[i] = a.W[(size_t)b * a.m * a.m + (size_t)x * a.m + a.cols[a.off ? j : a.photon]];
+    const float2 u = a.U[(size_t)b * a.m * a.m + (size_t)x * a.m + a.cols[a.off ? j : a.photon]];
+    wl[i] = square_rounded(u);
   }
   __syncthreads();
   const SV sv{cg, lo, a.me, stride};

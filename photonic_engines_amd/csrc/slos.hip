@@ -2462,9 +2462,9 @@ int slos_xmodel_workspace(const slos_plan* p, int64_t batch, int order, unsigned
   return rc;
 }
 
-int slos_xmodel(const slos_plan* p, const void* U, const float* W, int64_t batch, int order, const float* weights,
-                int weights_on_device, float* out, unsigned flags, void* ws, size_t ws_bytes, slos_stream_t stream) {
-  if (!p || !U || !W || !weights || !out || !ws) return fail(SLOS_EINVAL, "NULL argument");
+int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, const float* weights, int weights_on_device,
+                float* out, unsigned flags, void* ws, size_t ws_bytes, slos_stream_t stream) {
+  if (!p || !U || !weights || !out || !ws) return fail(SLOS_EINVAL, "NULL argument");
   if (flags & ~(unsigned)SLOS_FLAG_COMPENSATED) return fail(SLOS_EINVAL, "unsupported flag");
   XLayout x;
   int rc = xmodel_layout(p, batch, order, flags, &x);
@@ -2523,7 +2523,7 @@ int slos_xmodel(const slos_plan* p, const void* U, const float* W, int64_t batch
     if (weight < 0) a.weight_value = 1.f;
     else if (weights_on_device) a.weight = weights + weight;
     else a.weight_value = weights[weight];
-    a.W = W;
+    a.U = static_cast<const float2*>(U);
     for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
     const size_t lds = slos::raise_lds(K, p->me, a.photons);
     if (lds > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");

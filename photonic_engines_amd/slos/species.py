@@ -42,6 +42,11 @@ def _needs_grad(U: torch.Tensor) -> bool:
     return U.requires_grad and torch.is_grad_enabled()
 
 
+def _squares(u: torch.Tensor) -> torch.Tensor:
+    """|u|^2 without the root (and its rounding) of abs."""
+    return u.real.square() + u.imag.square()
+
+
 def _complex_of(q: torch.Tensor) -> torch.dtype:
     """The complex dtype of the layer steps over real probabilities q (float64: complex128)."""
     return torch.complex128 if q.dtype == torch.float64 else torch.complex64
@@ -104,7 +109,7 @@ def layer_probs(kernel, Ub: torch.Tensor, cols: Sequence[int]) -> torch.Tensor:
 def classical_raise(kernel, q: torch.Tensor, k: int, col: int, Ub: torch.Tensor) -> torch.Tensor:
     """One photon that interferes with nothing enters column `col`: the layer-k distribution
     q [B, S_k] becomes the layer-(k+1) one, q'(t + e_j) = sum q(t) |U[j, col]|^2."""
-    w = (Ub[:, :, int(col)].abs() ** 2).to(q.dtype).contiguous()
+    w = _squares(Ub[:, :, int(col)]).to(q.dtype).contiguous()
     if _needs_grad(Ub) or q.requires_grad:
         return _raise_steps(kernel, q.contiguous(), k, [w])
     if q.dtype == torch.float64:  # FP64: the raise as a complex128 layer step
@@ -215,7 +220,7 @@ def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, b_max: int) -> torch.Te
             or sum(math.comb(n, L) for L in range(min(b_max, n - 2) + 2)) > _NATIVE_SETS):
         return None
     w = _weights(x.detach(), n, b_max)
-    return kernel._plan.xmodel(Ub, Ub.abs() ** 2, b_max, w.tolist() if w.device.type == "cpu" else w.float(),
+    return kernel._plan.xmodel(Ub, b_max, w.tolist() if w.device.type == "cpu" else w.float(),
                                nat.FLAG_COMPENSATED if kernel.compensated else 0)
 
 
@@ -292,7 +297,7 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
         rows = [srcs[t][j] for j in range(len(cnt)) for t in order[:cnt[j]]]
         q = torch.cat([A[T] for T in rows], 0)                                        # [len(Ts) * B, S_k]
         ct = torch.as_tensor([cols[T[0]] for T in rows], dtype=torch.int64, device=dev)
-        W = (Ub[:, :, ct].abs() ** 2).permute(2, 0, 1).reshape(len(rows) * B, m).to(rdt)
+        W = _squares(Ub[:, :, ct]).permute(2, 0, 1).reshape(len(rows) * B, m).to(rdt)
         r = _raise_rows(kernel, q, k, W)
         r = r.reshape(len(rows), B, r.shape[-1])
         for T in Ts:
