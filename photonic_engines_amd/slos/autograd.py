@@ -98,7 +98,9 @@ KEEP_BYTES = 1 << 30
 def _kept_bytes(kernel, Ug: torch.Tensor, layer: int, cf: int) -> int | None:
     """Bytes of the layers a forward keeps for the native backward, or None where it does not apply
     (complex128 and compensated sums have the layer-by-layer backward only)."""
-    if cf or Ug.dtype != torch.complex64 or kernel.gradient_checkpointing or not 1 <= Ug.shape[0] <= MAX_ROWS:
+    if cf or Ug.dtype != torch.complex64 or not 1 <= Ug.shape[0] <= MAX_ROWS:
+        return None
+    if getattr(kernel, "gradient_checkpointing", False):  # (superposition kernels have no such option)
         return None
     n = kernel._plan.saved_bytes(Ug.shape[0], layer)
     return n if n <= KEEP_BYTES else None
