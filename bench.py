@@ -166,7 +166,7 @@ def bench_lossy(kern, U: torch.Tensor, eta: float = 0.9, steps: int = 3) -> dict
     d_bytes = 4 * S[n] + 4 * S[n - 1]
     outputs = int(sum(S[: n + 1]))
     return {"eta": eta, "ms_per_step": dt * 1e3, "outputs": outputs, "probs_per_s": outputs / dt,
-            "descent_top": {"kernel": f"k_descend_block (layer {n} -> {n - 1})", "kernel_ms": d_ms,
+            "descent_top": {"kernel": f"k_descend_insert (layer {n} -> {n - 1})", "kernel_ms": d_ms,
                             "alg_bytes": d_bytes, "achieved_GBps": d_bytes / (d_ms * 1e-3) / 1e9,
                             "frac": d_bytes / (d_ms * 1e-3) / 1e9 / PEAK_HBM_GBS},
             "max_abs_block_mass_minus_binomial": max(abs(a - b) for a, b in zip(masses, pmf))}
@@ -251,7 +251,7 @@ def bench_adjoint(steps: int = 5) -> dict:
     a_bytes = 8 * S[n] + 16 * S[n - 1]
     return {"workload": "n=8 m=24, first 8 modes, L = -mean log p over 1,024 sampled outputs", "states": int(S[n]),
             "ms_per_step": dt * 1e3, "grad_nonzero_columns": int((g.abs().sum(0) > 0).sum()),
-            "adjoint_top": {"kernel": "k_adjoint_block (layer 8 -> 7, with dL/dU partials and their FP64 sum)",
+            "adjoint_top": {"kernel": "k_adjoint_insert (layer 8 -> 7, with dL/dU partials and their FP64 sum)",
                             "kernel_ms": a_ms, "alg_bytes": a_bytes,
                             "achieved_GBps": a_bytes / (a_ms * 1e-3) / 1e9,
                             "frac": a_bytes / (a_ms * 1e-3) / 1e9 / PEAK_HBM_GBS}}
