@@ -5,8 +5,8 @@
 // layers 1 .. kf-1 for itself, in LDS, and then its own 1,024 states of layer kf: the same parent sums
 // in the same order (bit-identical), computed again by every work group, which costs less than the
 // launches as long as layer kf-1 has at most kFrontStates states and the work groups of all rows
-// together do not fill the chip (see front_layers in slos.hip). A launch takes 10 us where the tuple
-// words give the positions and 15-17 us where they are unranked; it replaces the fill and 3 to 6
+// together do not fill the chip (see front_layers in slos.hip). A launch takes about 10 us (where the
+// tuple words do not give the positions they are searched for, see k_front); it replaces the fill and 3 to 6
 // launches of 5 us or more: probs(U) at n = 4, m = 12 34.8 -> 21.5 us, n = 6, m = 18 42.6 -> 24.3 us
 // (both now a matter of host time), n = 8, m = 24 126 -> 107 us.
 #pragma once

@@ -84,6 +84,12 @@ __global__ __launch_bounds__(kFrontThreads) void k_front(FrontArgs a) {
         const uint64_t w = a.tuples5[g];
 #pragma unroll
         for (int i = 0; i < KM; ++i) p[i] = (int)(tw_byte(w, i) & 63u);
+      } else if (a.me >= 3 * KM) {
+        // one search of log2(me) reads a position where a walk over the modes is long: us a forward against the
+        // walk, n = 3, m = 64 11.5 / 27.3, n = 4, m = 32 20.5 / 30.3, n = 4, m = 24 14.6 / 19.4, n = 4, m = 12
+        // 10.8 / 11.9, n = 6, m = 18 17.1 / 17.2. Below 3 modes a position the walk takes few more reads than
+        // the searches do.
+        unrank_search<KM>(sv, g, K, p);
       } else {
         unrank_fixed<KM>(sv, g, K, p);
       }

@@ -128,6 +128,29 @@ SLOS_HD void unrank_fixed(const SV& sv, RankT<SV> g, int K, int (&p)[KM]) {
   }
 }
 
+// unrank_fixed with a binary search a position: K log2(me) dependent table reads in place of up to me + K
+template <int KM, class SV>
+SLOS_HD void unrank_search(const SV& sv, RankT<SV> g, int K, int (&p)[KM]) {
+  int l = 0;
+#pragma unroll
+  for (int i = 0; i < KM; ++i) {
+    p[i] = 0;
+    if (i < K) {
+      const int rem = K - i;
+      const RankT<SV> base = sv.C(rem, l);
+      int x = l, top = sv.me - 1;  // the largest x with base - C(rem, x) <= g is in [x, top]
+      while (x < top) {
+        const int mid = (x + top + 1) / 2;
+        if (base - sv.C(rem, mid) <= g) x = mid;
+        else top = mid - 1;
+      }
+      g -= base - sv.C(rem, x);
+      p[i] = x;
+      l = sv.lo[x];
+    }
+  }
+}
+
 // The parents of the K-tuple p (K <= KM), as for_each_parent. With the counting recurrence
 // cg[r][x] = cg[r][x+1] + cg[r-1][lo[x]] the rank of an N-tuple telescopes, for every mask, to
 //   cg[N][0] - sum_{i <= N-2} cg[N-i][p_i + 1] - cg[1][p_(N-1)],

@@ -499,6 +499,27 @@ int64_t emu_check_descend_block(int n, int m, int mask, int k, uint64_t first, u
   return bad;
 }
 
+// unrank_search against unrank_fixed over the first `count` states of layer k and every `step`-th after
+int64_t emu_check_unrank_search(int n, int m, int mask, int k, uint64_t count, uint64_t step) {
+  constexpr int KM = 8;
+  Space s;
+  if (!build(n, m, mask, s) || k < 1 || k > n || k > KM || step < 1) return -1;
+  slos::SpaceView sv{s.cg.data(), s.lo.data(), s.me, s.me + 1};
+  const uint64_t S = s.cg[(size_t)k * (s.me + 1)];
+  int64_t bad = 0;
+  for (uint64_t g = 0; g < S; g += g < count ? 1 : step) {
+    int p[KM], q[KM];
+    slos::unrank_fixed<KM>(sv, g, k, p);
+    slos::unrank_search<KM>(sv, g, k, q);
+    for (int i = 0; i < KM; ++i)
+      if (p[i] != q[i]) {
+        ++bad;
+        break;
+      }
+  }
+  return bad;
+}
+
 // The children at and above last(P) of the same parents through the insert table's words, as the
 // device kernels use them, against slos::for_each_child (the modes below last(P) come first there).
 int64_t emu_check_insert(int n, int m, int mask, int k, uint64_t first, uint64_t count) {

@@ -20,6 +20,15 @@ def test_insert_table_children(emu, n, m, mask, k, first):  # noqa: F811
     assert emu.emu_check_insert(n, m, pull.MASK_IDS[mask], k, first, 200_000) == 0
 
 
+@pytest.mark.parametrize("n,m,mask", [(1, 1, "fock"), (2, 3, "fock"), (4, 64, "fock"), (5, 9, "tail_empty"), (4, 64, "unbunched"),
+                                      (3, 3, "unbunched"), (6, 24, "dual_rail"), (4, 40, "sparse_1in4"), (8, 12, "fock")])
+def test_binary_search_for_positions(emu, n, m, mask):  # noqa: F811
+    emu.emu_check_unrank_search.restype = ctypes.c_int64
+    emu.emu_check_unrank_search.argtypes = [ctypes.c_int] * 4 + [ctypes.c_uint64] * 2
+    for k in range(1, n + 1):
+        assert emu.emu_check_unrank_search(n, m, pull.MASK_IDS[mask], k, 100_000, 997) == 0
+
+
 def _plan(n, m, mask):
     modes = m - 2 if mask == "tail_empty" else m
     step = {"dual_rail": 2, "sparse_1in4": 4}.get(mask, 1)
