@@ -280,7 +280,7 @@ class Plan:
 
     def xmodel(self, U: torch.Tensor, order: int, weights, flags: int = 0) -> torch.Tensor:
         """The x-model's distribution [B, S_n] of a contiguous complex64 U [B, m, m] (slos_xmodel);
-        `weights` a float32 GPU tensor or a list of n + 2 floats."""
+        `weights` a list of n + 2 floats."""
         B, dev = U.shape[0], U.device
         wsb = ctypes.c_size_t()
         nat.check(self._lib.slos_xmodel_workspace(self._h, B, order, int(flags), ctypes.byref(wsb)), "slos_xmodel_workspace")
@@ -289,10 +289,8 @@ class Plan:
                        f"workspace {need:,} B)")
         out = torch.empty((B, self.sizes[self.n]), dtype=torch.float32, device=dev)
         ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
-        on_device = isinstance(weights, torch.Tensor)
-        wp = nat.ptr(weights) if on_device else (ctypes.c_float * len(weights))(*weights)
-        nat.check(self._lib.slos_xmodel(self._h, nat.ptr(U), B, order, wp, int(on_device), nat.ptr(out), int(flags),
-                                        nat.ptr(ws), need, nat.stream_handle(dev)), "slos_xmodel")
+        nat.check(self._lib.slos_xmodel(self._h, nat.ptr(U), B, order, (ctypes.c_float * len(weights))(*weights), 0,
+                                        nat.ptr(out), int(flags), nat.ptr(ws), need, nat.stream_handle(dev)), "slos_xmodel")
         return out
 
     def saved_bytes(self, batch: int, layer: int) -> int:

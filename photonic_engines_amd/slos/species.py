@@ -211,17 +211,17 @@ def _weights(x: torch.Tensor, n: int, b_max: int) -> torch.Tensor:
     return torch.cat([w, torch.as_tensor(top, dtype=w.dtype, device=x.device).expand(1, *x.shape)])
 
 
-def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, b_max: int) -> torch.Tensor | None:
+def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, value: float, b_max: int) -> torch.Tensor | None:
     """The mixture [B, S_n] in one native call (slos_xmodel), or None where that does not apply: with a
-    gradient, in FP64, without a distinguishable photon or with fewer than three photons."""
+    gradient, in FP64, without a distinguishable photon or with fewer than three photons. `value`: x on the
+    host, as its check read it; the weights go to the kernels from there (x may be on another GPU than U)."""
     n = len(kernel.input_modes)
     if (Ub.dtype != torch.complex64 or _needs_grad(Ub) or _needs_grad(x) or x.dim() != 0 or b_max < 1
             or not 3 <= n <= _NATIVE_PHOTONS or not 1 <= Ub.shape[0] <= MAX_ROWS
             or sum(math.comb(n, L) for L in range(min(b_max, n - 2) + 2)) > _NATIVE_SETS):
         return None
-    w = _weights(x.detach(), n, b_max)
-    return kernel._plan.xmodel(Ub, b_max, w.tolist() if w.device.type == "cpu" else w.float(),
-                               nat.FLAG_COMPENSATED if kernel.compensated else 0)
+    w = _weights(torch.tensor(value, dtype=x.dtype), n, b_max)
+    return kernel._plan.xmodel(Ub, b_max, w.tolist(), nat.FLAG_COMPENSATED if kernel.compensated else 0)
 
 
 def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torch.Tensor:
@@ -249,7 +249,7 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
     cols = kernel.input_modes
     n = len(cols)
     b_max = n if order is None else max(0, min(int(order), n))
-    native = _native_x(kernel, Ub, x, b_max)
+    native = _native_x(kernel, Ub, x, d.x, b_max)
     if native is not None:
         return kernel._out(native, batched)
     weights = _weights(x, n, b_max).to(dtype=rdt, device=Ub.device)
