@@ -209,7 +209,7 @@ int slos_loss_descend(const slos_plan* plan, int k, const float* q_k, float* q_k
 int slos_loss_thin(const slos_plan* plan, const float* q, float* const* out, const double* scale, int64_t batch,
                    slos_stream_t stream);
 
-/* The x-model's distribution on the last layer (species.py:123-146) of 3 <= n <= 24 photons in one
+/* The x-model's distribution on the last layer (species.py:123-146) of 3 <= n <= 24 photons, n <= m, in one
  * call: float32 out [batch][S_n] = the sum over the sets T of at most `order` (1 <= order <= n)
  * distinguishable photons of weights[|T|] times the distribution of the others interfering and T raised
  * (slos_raise), the terms sharing their raises. `weights`: n + 2 floats, on the host or (weights_on_device)

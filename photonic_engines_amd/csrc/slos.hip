@@ -2413,6 +2413,8 @@ int xmodel_layout(const slos_plan* p, int64_t B, int order, unsigned flags, XLay
   const int n = p->n;
   if (n < 3 || n > slos::kRaisePhotons || order < 1 || order > n || B < 1 || B > 65535)
     return fail(SLOS_EINVAL, "bad argument");
+  // (a subset's photons are laid out as the columns of an m x m matrix)
+  if (n > p->m) return fail(SLOS_EINVAL, "more photons than modes");
   x->levels = std::min(order, n - 2);
   x->rows = xmodel_host_rows(p, x->levels);
   if (!x->rows) return fail(SLOS_ERANGE, "too many subsets");

@@ -213,11 +213,11 @@ def _weights(x: torch.Tensor, n: int, b_max: int) -> torch.Tensor:
 
 def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, value: float, b_max: int) -> torch.Tensor | None:
     """The mixture [B, S_n] in one native call (slos_xmodel), or None where that does not apply: with a
-    gradient, in FP64, without a distinguishable photon or with fewer than three photons. `value`: x on the
+    gradient, in FP64, without a distinguishable photon, with fewer than three photons or more than modes. `value`: x on the
     host, as its check read it; the weights go to the kernels from there (x may be on another GPU than U)."""
     n = len(kernel.input_modes)
     if (Ub.dtype != torch.complex64 or _needs_grad(Ub) or _needs_grad(x) or x.dim() != 0 or b_max < 1
-            or not 3 <= n <= _NATIVE_PHOTONS or not 1 <= Ub.shape[0] <= MAX_ROWS
+            or not 3 <= n <= min(_NATIVE_PHOTONS, Ub.shape[-1]) or not 1 <= Ub.shape[0] <= MAX_ROWS
             or sum(math.comb(n, L) for L in range(min(b_max, n - 2) + 2)) > _NATIVE_SETS):
         return None
     w = _weights(torch.tensor(value, dtype=x.dtype), n, b_max)

@@ -1,9 +1,11 @@
 """The host side of the x-model (photonic_engines/slos/species.py:123-146), without a GPU."""
+import ctypes
 import math
 from types import SimpleNamespace
 
 import torch
 
+from photonic_engines_amd import _native as nat
 from photonic_engines_amd.imperfections import Distinguishability
 from photonic_engines_amd.slos import species
 
@@ -24,3 +26,19 @@ def test_weights_of_an_x_on_another_device(monkeypatch):
     ref.append(math.comb(n, n) * ref[n] + math.comb(n, n - 1) * ref[n - 1])
     # x in float32 (half an ulp, 2^-24): x^(n-L) (1-x)^L is off by at most (n - L + L x / (1 - x)) 2^-24 < 3 n 2^-24
     assert all(abs(a - b) <= 3 * n * 2.0 ** -24 * b for a, b in zip(w, ref, strict=True))
+
+
+def test_more_photons_than_modes_are_refused():
+    """A subset's photons are the columns of an m x m matrix: with n > m the one-call x-model would write
+    past it. The C entries refuse; the layer-by-layer form, which raises for it, gets the call."""
+    L = nat.lib()
+    for n, m, rc in ((3, 2, nat.SLOS_EINVAL), (13, 10, nat.SLOS_EINVAL), (3, 3, nat.SLOS_OK), (13, 13, nat.SLOS_OK)):
+        h = ctypes.c_void_p()
+        assert L.slos_plan_create(n, m, nat.MASK_IDS["fock"], (ctypes.c_int32 * n)(*[i % m for i in range(n)]), ctypes.byref(h)) == 0
+        b = ctypes.c_size_t()
+        assert L.slos_xmodel_workspace(h, 1, 1, 0, ctypes.byref(b)) == rc
+        L.slos_plan_destroy(h)
+    kernel = SimpleNamespace(_plan=SimpleNamespace(xmodel=lambda *a: torch.zeros(1, 4)), input_modes=[0, 0, 1], compensated=False)
+    for m in (2, 3):
+        native = species._native_x(kernel, torch.zeros(1, m, m, dtype=torch.complex64), torch.tensor(0.7), 0.7, 1)
+        assert (native is None) == (m == 2)
