@@ -74,6 +74,9 @@ enum {
                                     complex128, the probabilities float64, every sum in FP64 (the
                                     reference's dtype=torch.complex128, kernel.py:92,117-118).
                                     Not with SLOS_FLAG_COMPENSATED */
+#define SLOS_FLAG_BLOCK 32u      /* force the block and group-order kernels on every layer that they can take,
+                                    whatever its size, and a launch for every layer (debugging; without
+                                    effect beside SLOS_FLAG_SIMPLE) */
 
 /* Version string of the library. */
 const char* slos_version(void);

@@ -18,7 +18,7 @@ LIB_PATH = os.environ.get("SLOS_MI355X_LIB") or os.path.join(_HERE, "_build", "l
 SLOS_OK, SLOS_EINVAL, SLOS_ENOMEM, SLOS_EHIP, SLOS_ERANGE, SLOS_ENODEV = range(6)
 MASK_IDS = {"fock": 0, "unbunched": 1, "dual_rail": 2, "sparse_1in4": 3, "tail_empty": 4}
 OUT_PROBS, OUT_AMPS, OUT_RAW = 0, 1, 2
-FLAG_COMPENSATED, FLAG_IMMEDIATE, FLAG_SIMPLE, FLAG_HILO, FLAG_F64 = 1, 2, 4, 8, 16
+FLAG_COMPENSATED, FLAG_IMMEDIATE, FLAG_SIMPLE, FLAG_HILO, FLAG_F64, FLAG_BLOCK = 1, 2, 4, 8, 16, 32
 
 # every symbol include/slos_mi355x.h declares: (name, restype, argtypes)
 _c = ctypes

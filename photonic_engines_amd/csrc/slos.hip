@@ -794,7 +794,7 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
   a.par_lo = (comp && par_hilo) ? B * (int64_t)S_par : 0;
   a.out_lo = (comp && out_hilo && kind == 0) ? B * (int64_t)S : 0;
   if (!(flags & SLOS_FLAG_SIMPLE) && dt.tuples && K > slos::kSuf && K - slos::kSuf <= 16 &&
-      block_lds_fit(K, p->me, slos::kSuf) && use_blocks(p, K, block_suffix(p, dt, K), S, B))
+      block_lds_fit(K, p->me, slos::kSuf) && (flags & SLOS_FLAG_BLOCK || use_blocks(p, K, block_suffix(p, dt, K), S, B)))
     return launch_block(p, dt, a, kind, comp, st);
   const size_t sh = (((size_t)(K + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8;
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
@@ -812,7 +812,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
   const int suf = dt.tuples5 && K > 5 ? 5 : slos::kSuf;
   const int d = K - suf;
-  if (d > 8 || !use_blocks(p, K, suf, S, B)) return -1;
+  if (d > 8 || !(flags & SLOS_FLAG_BLOCK || use_blocks(p, K, suf, S, B))) return -1;
   slos::BlockLayerF64 L{};
   L.l.K = K; L.l.m = p->m; L.l.col = col; L.l.S_par = S_par; L.l.S = S; L.l.S_pre = p->size(d);
   L.l.flags = flags;
@@ -1625,7 +1625,7 @@ int forward_run_f64(const slos_plan* p, const DevTables& dt, const void* U, slos
   uint64_t S_par = 1;
   size_t lds = 0;
   uint32_t buf = 0;
-  const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 16, false, &lds, &buf);
+  const int kf = (flags & (SLOS_FLAG_SIMPLE | SLOS_FLAG_BLOCK)) ? 0 : front_layers(p, batch, layer, 16, false, &lds, &buf);
   if (kf) {
     void* dst = kf == layer ? out : bufs[kf & 1];
     const int rc = run_front(p, dt, kf, cols, U, us, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale,
@@ -1675,7 +1675,7 @@ int forward_run(const slos_plan* p, const DevTables& dt, const void* U, slos::Ma
   const RoctxRange whole("slos_forward");
   size_t lds = 0;
   uint32_t buf = 0;
-  const int kf = (flags & SLOS_FLAG_SIMPLE) ? 0 : front_layers(p, batch, layer, 8, hilo, &lds, &buf);
+  const int kf = (flags & (SLOS_FLAG_SIMPLE | SLOS_FLAG_BLOCK)) ? 0 : front_layers(p, batch, layer, 8, hilo, &lds, &buf);
   if (kf) {
     void* dst = kf == layer ? out : bufs[kf & 1];
     rc = run_front(p, dt, kf, cols, U, us, batch, dst, kf < layer ? 0 : out_kind == SLOS_OUT_PROBS ? 1 : 2, scale, flags, lds,
