@@ -872,12 +872,11 @@ int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
 // layers below kf fit LDS with at most kFrontStates states, which computes at most 2^21 states again (all
 // work groups together; with more the chip is full and a launch a layer costs less), and whose work
 // groups, of every row, are at most 512: two a CU, the chip once. Each takes 10 us or more however few
-// states its row has, so that with many rows a launch a layer is the shorter way, us, so / a launch a layer: n = 4,
-// m = 8, 512 work groups 17 / 27, 1024 31 / 29, 2048 59 / 42; n = 3, m = 6, 1024 22 / 24, 4096 80 / 35, 60000 1117 / 337;
-// n = 2, m = 4, 60000 818 / 218. With 5 photons or more they replace more launches and are worth twice as
-// many: n = 5, m = 10, 1024 34 / 39, 2048 66 / 59; n = 6, m = 6, 1024 32 / 36, 1536 46 / 43. From 100 modes on a thread's
-// search for its positions, which k_front shortens, outweighs both: n = 2, m = 100, 20480 419 / 466; n = 2,
-// m = 200, 10240 223 / 368; n = 1, m = 300, 2048 28 / 56; but n = 2, m = 64, 3072 62 / 54.
+// states its row has, so that with many rows a launch a layer is the shorter way, us, so / a launch a layer:
+// n = 4, m = 8, 512 work groups 17 / 27, 1024 31 / 27, 2048 59 / 29; n = 5, m = 10, 512 19 / 30, 1024 34 / 33,
+// 2048 66 / 49; n = 6, m = 6, 1024 32 / 30; n = 3, m = 6, 60000 1117 / 153; n = 2, m = 4, 60000 818 / 84. From
+// 128 modes on a thread's search for its positions, which k_front shortens, outweighs that: n = 2, m = 200,
+// 5120 113 / 145; n = 1, m = 300, 2048 28 / 45; n = 2, m = 1500, 1100 52 / 704; but n = 2, m = 100, 5120 107 / 89.
 int front_layers(const slos_plan* p, int64_t B, int layer, size_t elem, bool comp, size_t* lds, uint32_t* buf) {
   int kf = 0;
   if (B > 65535) return 0;
@@ -889,7 +888,7 @@ int front_layers(const slos_plan* p, int64_t B, int layer, size_t elem, bool com
     if (wgs * below * (uint64_t)B > (1ull << 21)) break;
     const size_t need = slos::front_lds(k, p->me, p->m, elem, most, comp);
     if (need > lds_limit()) break;
-    if (p->me >= 100 || wgs * (uint64_t)B <= (k > 4 ? 1024u : 512u)) {
+    if (p->me >= 128 || wgs * (uint64_t)B <= 512u) {
       kf = k;
       *lds = need;
       *buf = (uint32_t)most;
