@@ -709,8 +709,14 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
 //   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
 //   blocks, collision-free: 126k 41 / 15, 3.1M (209 a block) 101 / 55, 2.0M (4,680 a block) 39 / 32, 54.6M
 //   (92 a block) 1266 / 898, 7.6M (119,000 a block) 57 / 118.
-// The thread kernel's exact forms are those of at most 12 photons and 2^32 states.
-bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B) {
+// The thread kernel's exact forms are those of at most 12 photons and 2^32 states. The line holds for
+// compensated sums (8 photons, 1.1M states 27 / 24, 2.2M 33 / 45, 9 photons, 3.1M 46 / 63; collision-free 3.1M (209 a
+// block) 115 / 72, 10.7M 106 / 153) and for complex128 (f64: 1.1M 26 / 18, 2.2M 28 / 32, 3.1M 39 / 45; 3.1M (209 a
+// block) 101 / 54, 10.7M 80 / 117). At 13 photons, the most the complex128 block kernel takes, its blocks of tens of
+// states lose to the thread kernel's 16-photon form up to some ten million: 203k states 96 / 15, 5.2M 229 / 172,
+// 10.4M 350 / 336 (raw layers 424 / 296), 37M 959 / 1220 (1113 / 1096), 120M 2209 / 3978.
+bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool f64) {
+  if (f64 && K > 12 && S < (1ull << 32)) return S * (uint64_t)B >= (1ull << 25);
   if (K > 12 || S >= (1ull << 32)) return true;
   if (S * (uint64_t)B < (1ull << 21)) return false;
   if (suf == 5 && !p->items[K].empty()) return true;
@@ -794,7 +800,7 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
   a.par_lo = (comp && par_hilo) ? B * (int64_t)S_par : 0;
   a.out_lo = (comp && out_hilo && kind == 0) ? B * (int64_t)S : 0;
   if (!(flags & SLOS_FLAG_SIMPLE) && dt.tuples && K > slos::kSuf && K - slos::kSuf <= 16 &&
-      block_lds_fit(K, p->me, slos::kSuf) && (flags & SLOS_FLAG_BLOCK || use_blocks(p, K, block_suffix(p, dt, K), S, B)))
+      block_lds_fit(K, p->me, slos::kSuf) && (flags & SLOS_FLAG_BLOCK || use_blocks(p, K, block_suffix(p, dt, K), S, B, false)))
     return launch_block(p, dt, a, kind, comp, st);
   const size_t sh = (((size_t)(K + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8;
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
@@ -812,7 +818,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
   const int suf = dt.tuples5 && K > 5 ? 5 : slos::kSuf;
   const int d = K - suf;
-  if (d > 8 || !(flags & SLOS_FLAG_BLOCK || use_blocks(p, K, suf, S, B))) return -1;
+  if (d > 8 || !(flags & SLOS_FLAG_BLOCK || use_blocks(p, K, suf, S, B, true))) return -1;
   slos::BlockLayerF64 L{};
   L.l.K = K; L.l.m = p->m; L.l.col = col; L.l.S_par = S_par; L.l.S = S; L.l.S_pre = p->size(d);
   L.l.flags = flags;
