@@ -709,6 +709,16 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
 //   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
 //   blocks, collision-free: 126k 41 / 15, 3.1M (209 a block) 101 / 55, 2.0M (4,680 a block) 39 / 32, 54.6M
 //   (92 a block) 1266 / 898, 7.6M (119,000 a block) 57 / 118.
+// Shorter blocks pay where the layer is large: a state costs 6 us / 10^6 in blocks and 13 to 19 by threads, a
+// block some 2.6 us / 1000 besides, and the launch some 40 us of waves that wait on their first blocks. So
+// the line is one of states times states a block, 2^34 for set masks, on layers of less than 2^20 states
+// (rows of a batch, whose parents stay in the L2) 2^32:
+//   8.4e9 (5.9M states, 1,441 a block) 93 / 81, 2.2e10 (10.5M, 2,120) 119 / 141, 7.5e9 (14.3M, 522) 227 / 206, 2.2e10 (28M,
+//   780) 348 / 397, 6e9 (30M, 210) 586 / 464, 2.1e10 (64.5M, 320) 973 / 1027, 1.8e10 (129M, 142) 2158 / 2331, 8.2e11
+//   (273M, 2,992) 1996 / 4186; rows: 2.7e9 (10 of 735k, 363) 107 / 94, 6.3e9 (200 of 78k, 408) 131 / 152, 1.3e10 (50 of 735k,
+//   363) 351 / 439, 1.4e10 (20 of 143k, 4,750) 24 / 35.
+// and 2^33 for the multiset layers that have no group order: 12 photons, 1.8e9 (17.4M, 101) 364 / 268, 7.7e9 (52M, 149)
+//   768 / 790 (compensated 1607 / 1334, complex128 948 / 917), 3e10 (141M, 214) 1482 / 2317.
 // The thread kernel's exact forms are those of at most 12 photons and 2^32 states. The line holds for
 // compensated sums (8 photons, 1.1M states 27 / 24, 2.2M 33 / 45, 9 photons, 3.1M 46 / 63; collision-free 3.1M (209 a
 // block) 115 / 72, 10.7M 106 / 153) and for complex128 (f64: 1.1M 26 / 18, 2.2M 28 / 32, 3.1M 39 / 45; 3.1M (209 a
@@ -720,7 +730,9 @@ bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool 
   if (K > 12 || S >= (1ull << 32)) return true;
   if (S * (uint64_t)B < (1ull << 21)) return false;
   if (suf == 5 && !p->items[K].empty()) return true;
-  return S >= (p->multiset ? 256 : 8192) * p->size(K - suf);
+  const double per = (double)S / (double)p->size(K - suf), states = (double)S * (double)B;
+  if (per >= (p->multiset ? 256.0 : 8192.0)) return true;
+  return states * per >= (double)(p->multiset ? 1ull << 33 : S < (1ull << 20) ? 1ull << 32 : 1ull << 34);
 }
 
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
