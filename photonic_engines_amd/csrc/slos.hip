@@ -2291,8 +2291,13 @@ int run_descend(const slos_plan* p, const DevTables& dt, int k, const float* q_k
     hipLaunchKernelGGL(kernel, grid, dim3(256), sh, st, dt.cg, dt.lo, p->me, p->multiset, k, q_k, Sk, q_km1, Sp, batch,
                        (float)scale);
   };
-  // (known photons and 32-bit ranks, as the forward's thread kernel: the step 5 -> 4 at 24 modes 14 -> 6 us)
-  switch (Sk < (1ull << 32) ? k - 1 : 0) {
+  // Known photons and 32-bit ranks, as the forward's thread kernel, with the gathers of every mode in turn (children_sum): the
+  // step 5 -> 4 at 24 modes 14 -> 6 us. In a set mask most modes take no photon where many are taken, and the walk
+  // over the admissible ones is shorter from 6 parent photons on (sparse_1in4: 5): us, walk / every mode, 6 -> 5 at 26 modes
+  // 18 / 14, at 40 54 / 52, 7 -> 6 at 26 modes 19 / 23, 8 -> 7 35 / 51, 9 -> 8 75 / 116, at 40 5195 / 6388; sparse_1in4, 36
+  // modes, 5 -> 4 16.5 / 16.0, 6 -> 5 15.8 / 18.5, 9 -> 8 19 / 59.
+  const int every = p->multiset ? 8 : p->shift == 2 ? 4 : 5;
+  switch (Sk < (1ull << 32) && k - 1 <= every ? k - 1 : 0) {
     case 1: launch(k_descend<1, slos::SpaceView32, true>); break;
     case 2: launch(k_descend<2, slos::SpaceView32, true>); break;
     case 3: launch(k_descend<3, slos::SpaceView32, true>); break;
