@@ -127,11 +127,12 @@ __global__ __launch_bounds__(kModesThreads) void k_adjoint_modes(AdjointModesArg
     if (!MULTISET) child = child && (first || before <= jj) && lo_j <= after;
     const float2 ps = psi[tt];
     const float2 g = child ? gk[idx] : make_float2(0.f, 0.f);
-    acc.x += (double)fmaf(ps.y, g.y, ps.x * g.x);  // conj(psi) * g
-    acc.y += (double)fmaf(-ps.y, g.x, ps.x * g.y);
+    // (the products are selected, not g alone: where there is no child, an infinite or NaN psi or U adds nothing)
+    acc.x += child ? (double)fmaf(ps.y, g.y, ps.x * g.x) : 0.0;  // conj(psi) * g
+    acc.y += child ? (double)fmaf(-ps.y, g.x, ps.x * g.y) : 0.0;
     if (gout) {
-      const float gr = group_sum<G>(fmaf(u.y, g.y, u.x * g.x));   // conj(u) * g
-      const float gi = group_sum<G>(fmaf(-u.y, g.x, u.x * g.y));
+      const float gr = group_sum<G>(child ? fmaf(u.y, g.y, u.x * g.x) : 0.f);   // conj(u) * g
+      const float gi = group_sum<G>(child ? fmaf(-u.y, g.x, u.x * g.y) : 0.f);
       if (in && j == G - 1) gout[t] = make_float2(gr, gi);
     }
   }
