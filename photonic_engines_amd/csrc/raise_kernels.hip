@@ -46,34 +46,34 @@ __global__ __launch_bounds__(256) void k_raise_rows(RaiseArgs a) {
   }
   __syncthreads();
   const SV sv{cg, lo, a.me, stride};
-  const uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= a.S) return;
-  int p[KM];
-  unrank_words<KM>(sv, a.words, (R)c, K, p);
-  R par[KM];      // the parent without position l
-  bool real[KM];  // (a repeated position is no further parent)
-  parent_ranks<KM>(sv, a.multiset, K, p, par, real);
   const float wt = a.weight ? *a.weight : a.weight_value;
   const uint32_t r0 = blockIdx.z * a.rows_per;
   const uint32_t r1 = r0 + a.rows_per < a.targets ? r0 + a.rows_per : a.targets;
-  for (uint32_t r = r0; r < r1; ++r) {
-    const uint32_t s0 = a.off ? a.off[r] : 0u, s1 = a.off ? a.off[r + 1] : 1u;
-    float acc = 0.f;
+  for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.S; c += (uint64_t)gridDim.x * blockDim.x) {
+    int p[KM];
+    unrank_words<KM>(sv, a.words, (R)c, K, p);
+    R par[KM];      // the parent without position l
+    bool real[KM];  // (a repeated position is no further parent)
+    parent_ranks<KM>(sv, a.multiset, K, p, par, real);
+    for (uint32_t r = r0; r < r1; ++r) {
+      const uint32_t s0 = a.off ? a.off[r] : 0u, s1 = a.off ? a.off[r + 1] : 1u;
+      float acc = 0.f;
 #pragma unroll 2
-    for (uint32_t s = s0; s < s1; ++s) {
-      const float* q = a.q + ((size_t)s * a.B + b) * a.S_par;
-      const float* w = wl + (size_t)(s - s0) * a.me;
-      float v[KM];
+      for (uint32_t s = s0; s < s1; ++s) {
+        const float* q = a.q + ((size_t)s * a.B + b) * a.S_par;
+        const float* w = wl + (size_t)(s - s0) * a.me;
+        float v[KM];
 #pragma unroll
-      for (int l = 0; l < KM; ++l) v[l] = l < K ? q[par[l]] : 0.f;
-      float sum = 0.f;
+        for (int l = 0; l < KM; ++l) v[l] = l < K ? q[par[l]] : 0.f;
+        float sum = 0.f;
 #pragma unroll
-      for (int l = 0; l < KM; ++l)
-        if (l < K) sum = fmaf(w[p[l]], real[l] ? v[l] : 0.f, sum);
-      acc = add_rounded(acc, sum);
+        for (int l = 0; l < KM; ++l)
+          if (l < K) sum = fmaf(w[p[l]], real[l] ? v[l] : 0.f, sum);
+        acc = add_rounded(acc, sum);
+      }
+      float* o = a.out + ((size_t)r * a.B + b) * a.S + c;
+      *o = a.row_scale ? add_rounded((*o * a.row_scale[r]) * wt, acc) : acc;
     }
-    float* o = a.out + ((size_t)r * a.B + b) * a.S + c;
-    *o = a.row_scale ? add_rounded((*o * a.row_scale[r]) * wt, acc) : acc;
   }
 }
 

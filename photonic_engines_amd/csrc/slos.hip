@@ -2560,8 +2560,7 @@ int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, con
     for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
     const size_t lds = slos::raise_lds(K, p->me, a.photons);
     if (lds > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
-    const uint64_t wgs = (a.S + 255) / 256;
-    if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
+    const uint64_t wgs = std::min<uint64_t>((a.S + 255) / 256, 1u << 20);  // (a launch has at most 2^32 threads)
     // a work group takes all targets of its states where there are enough states: 2048 work groups fill
     // the chip
     const uint64_t parts = std::min<uint64_t>({targets, 65535u, (2048 + wgs * B - 1) / (wgs * B)});
