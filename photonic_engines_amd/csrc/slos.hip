@@ -2511,6 +2511,9 @@ int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, con
   if (rc) return rc;
   const int n = p->n;
   const int B = (int)batch;
+  int photons[kMaxPhotons];  // their columns, in order (k_subset_columns counts equal ones next to each other)
+  std::copy(p->modes.begin(), p->modes.end(), photons);
+  std::sort(photons, photons + n);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const RoctxRange whole("slos_xmodel");
   auto* base = static_cast<unsigned char*>(ws);
@@ -2532,7 +2535,7 @@ int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, con
       a.rows = std::min(x.chunk[L], R - r0);
       a.B = B; a.m = p->m; a.n = n; a.g = g;
       a.row_scale = scale;
-      for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
+      for (int j = 0; j < n; ++j) a.cols[j] = photons[j];
       slos::launch_subsets(st, a);
       HIP_TRY(hipGetLastError());
       const int64_t rows = (int64_t)a.rows * B;
@@ -2557,7 +2560,7 @@ int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, con
     else if (weights_on_device) a.weight = weights + weight;
     else a.weight_value = weights[weight];
     a.U = static_cast<const float2*>(U);
-    for (int j = 0; j < n; ++j) a.cols[j] = p->modes[j];
+    for (int j = 0; j < n; ++j) a.cols[j] = photons[j];
     const size_t lds = slos::raise_lds(K, p->me, a.photons);
     if (lds > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
     const uint64_t wgs = std::min<uint64_t>((a.S + 255) / 256, 1u << 20);  // (a launch has at most 2^32 threads)

@@ -1,4 +1,5 @@
 """The one-call x-model (slos_xmodel; photonic_engines/slos/species.py:123-146)."""
+import ctypes
 import itertools
 import math
 
@@ -7,7 +8,9 @@ import pytest
 import torch
 from helpers import haar_unitary
 
+from photonic_engines_amd import _native as nat
 from photonic_engines_amd.slos import FockSLOSKernel
+from photonic_engines_amd.slos._plan import Plan
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -46,3 +49,29 @@ def test_more_than_2_to_32_states():
         # (at most 12 factors and a sum of at most 24 permutations' products on 4 layers, each within 2^-24 of
         # the products' own size, which a Haar matrix's entries bound by 24 (4 / m)^4)
         assert abs(float(p[i]) - ref) <= 1e-4 * ref + 1e-6 * 24 * (4 / m) ** 4, (i, t)
+
+
+@pytest.mark.parametrize("modes", [[0, 1, 0, 3], [2, 0, 2, 2], [3, 1, 0, 2]])
+@pytest.mark.parametrize("weights_on_device", [0, 1])
+def test_columns_in_any_order(modes, weights_on_device):
+    """slos_xmodel on a plan whose photons are not sorted by column (the Python kernels sort them), and with
+    the weights on the GPU: the mixture does not depend on the photons' order."""
+    n, m, x = 4, 6, 0.6
+    U = haar_unitary(m, 5).to(torch.complex64).to(DEV).unsqueeze(0).contiguous()
+    w = [x ** (n - L) * (1 - x) ** L for L in range(n + 1)]
+    w.append(n * w[n - 1] + w[n])
+    res = []
+    for cols in (modes, sorted(modes)):
+        p = Plan(n, m, "fock", cols)
+        b = ctypes.c_size_t()
+        nat.check(p._lib.slos_xmodel_workspace(p._h, 1, n, 0, ctypes.byref(b)), "workspace")
+        ws = torch.empty(b.value, dtype=torch.uint8, device=DEV)
+        out = torch.empty(1, p.sizes[n], device=DEV)
+        wd = torch.tensor(w, dtype=torch.float32, device=DEV)
+        wh = (ctypes.c_float * len(w))(*w)
+        nat.check(p._lib.slos_xmodel(p._h, nat.ptr(U), 1, n, nat.ptr(wd) if weights_on_device else wh, weights_on_device,
+                                     nat.ptr(out), 0, nat.ptr(ws), b.value, nat.stream_handle(U.device)), "slos_xmodel")
+        res.append(out)
+    assert abs(float(res[1].double().sum()) - 1) < 1e-5
+    # (another order of the same float32 sums: a few tens of roundings of terms of at most the value)
+    assert ((res[0] - res[1]).abs() <= 64 * 2.0 ** -24 * (res[1] + 1e-3)).all()
