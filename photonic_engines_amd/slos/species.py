@@ -201,14 +201,14 @@ def _raise_rows(kernel, q: torch.Tensor, k: int, W: torch.Tensor) -> torch.Tenso
 _NATIVE_SETS, _NATIVE_PHOTONS = 1 << 20, 24
 
 
-def _weights(x: torch.Tensor, n: int, b_max: int) -> torch.Tensor:
-    """float64 [n + 2] (and x's own shape): x^(n-L) (1-x)^L, the weight of each set of L distinguishable photons, for L = 0..n,
-    then the weight of all sets of n - 1 and n photons that b_max admits together. Differentiable in x."""
-    L = torch.arange(n + 1, dtype=torch.float64, device=x.device).reshape(-1, *([1] * x.dim()))
-    xd = x.double()
-    w = xd ** (n - L) * (1 - xd) ** L
-    top = sum(math.comb(n, k) * w[k] for k in (n, n - 1) if 0 <= k <= b_max)
-    return torch.cat([w, torch.as_tensor(top, dtype=w.dtype, device=x.device).expand(1, *x.shape)])
+def _weights(x: torch.Tensor | float, n: int, b_max: int) -> list:
+    """x^(n-L) (1-x)^L, the weight of each set of L distinguishable photons, for L = 0..n, then the weight of
+    all sets of n - 1 and n photons that b_max admits together: n + 2 of them, in FP64. Differentiable in a
+    tensor x, also twice and at 0 and 1 (whole exponents: torch's power of a tensor by a tensor is not)."""
+    if isinstance(x, torch.Tensor):
+        x = x.double()
+    w = [x ** (n - L) * (1 - x) ** L for L in range(n + 1)]
+    return [*w, sum(math.comb(n, k) * w[k] for k in (n, n - 1) if 0 <= k <= b_max)]
 
 
 def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, value: float, b_max: int) -> torch.Tensor | None:
@@ -220,8 +220,8 @@ def _native_x(kernel, Ub: torch.Tensor, x: torch.Tensor, value: float, b_max: in
             or not 3 <= n <= min(_NATIVE_PHOTONS, Ub.shape[-1]) or not 1 <= Ub.shape[0] <= MAX_ROWS
             or sum(math.comb(n, L) for L in range(min(b_max, n - 2) + 2)) > _NATIVE_SETS):
         return None
-    w = _weights(torch.tensor(value, dtype=x.dtype), n, b_max)
-    return kernel._plan.xmodel(Ub, b_max, w.tolist(), nat.FLAG_COMPENSATED if kernel.compensated else 0)
+    w = _weights(float(np.float32(value)), n, b_max)
+    return kernel._plan.xmodel(Ub, b_max, w, nat.FLAG_COMPENSATED if kernel.compensated else 0)
 
 
 def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torch.Tensor:
@@ -252,7 +252,7 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
     native = _native_x(kernel, Ub, x, d.x, b_max)
     if native is not None:
         return kernel._out(native, batched)
-    weights = _weights(x, n, b_max).to(dtype=rdt, device=Ub.device)
+    weights = [torch.as_tensor(w).to(dtype=rdt, device=Ub.device) for w in _weights(x, n, b_max)]
     B, m = Ub.shape[0], Ub.shape[-1]
     dev = Ub.device
     per = max(1, (2 << 30) // (rdt.itemsize * kernel.layers.size(n) * max(B, 1)))

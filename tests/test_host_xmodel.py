@@ -3,6 +3,7 @@ import ctypes
 import math
 from types import SimpleNamespace
 
+import numpy as np
 import torch
 
 from photonic_engines_amd import _native as nat
@@ -42,3 +43,16 @@ def test_more_photons_than_modes_are_refused():
     for m in (2, 3):
         native = species._native_x(kernel, torch.zeros(1, m, m, dtype=torch.complex64), torch.tensor(0.7), 0.7, 1)
         assert (native is None) == (m == 2)
+
+
+def test_weights_differentiate_twice_at_the_ends():
+    """d^2/dx^2 of x^(n-L) (1-x)^L, also where x or 1 - x is zero."""
+    n = 4
+    for x0 in (0.0, 0.3, 1.0):
+        x = torch.tensor(x0, dtype=torch.float64, requires_grad=True)
+        w = list(species._weights(x, n, n))[:n + 1]
+        for L in range(n + 1):
+            g, = torch.autograd.grad(w[L], x, create_graph=True)
+            h, = torch.autograd.grad(g, x, retain_graph=True)
+            p = np.polynomial.Polynomial([0, 1]) ** (n - L) * np.polynomial.Polynomial([1, -1]) ** L
+            assert abs(g.item() - p.deriv()(x0)) < 1e-12 and abs(h.item() - p.deriv(2)(x0)) < 1e-12, (x0, L)
