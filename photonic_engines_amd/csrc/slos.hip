@@ -197,6 +197,16 @@ int device_tables(const slos_plan* cp, DevTables* out) {
   return SLOS_OK;
 }
 
+// Allocations in its scope neither fail for nor end a graph capture of another thread (whose mode may
+// forbid them to every thread).
+struct BesideCaptures {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  BesideCaptures(const BesideCaptures&) = delete;
+  BesideCaptures& operator=(const BesideCaptures&) = delete;
+};
+
 bool has_insert_table(const slos_plan* p) {
   return p->multiset && !p->tuples.empty() && p->n >= 5 && p->size(5) <= slos::kInsertTuples &&
          p->tuples.size() * (uint64_t)p->me <= slos::kInsertWords;
@@ -222,6 +232,7 @@ int insert_table(const slos_plan* cp, hipStream_t st, const uint32_t** out) {
         HIP_TRY(hipStreamIsCapturing(st, &cap));
         if (cap != hipStreamCaptureStatusNone) return SLOS_OK;
         uint32_t* ins = nullptr;
+        const BesideCaptures guard;
         HIP_TRY(hipMalloc(&ins, words * sizeof(uint32_t)));
         hipLaunchKernelGGL(k_insert_table, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, t.cg, t.tuples, p->me,
                            (uint32_t)n4, (uint32_t)words, ins);
@@ -2410,7 +2421,7 @@ const XRows* xmodel_host_rows(const slos_plan* cp, int levels) {
 }
 
 // the same on the current GPU
-int xmodel_tables(const slos_plan* cp, int levels, const XRows& x, const uint32_t** out) {
+int xmodel_tables(const slos_plan* cp, int levels, const XRows& x, hipStream_t st, const uint32_t** out) {
   slos_plan* p = const_cast<slos_plan*>(cp);
   int d = 0;
   HIP_TRY(hipGetDevice(&d));
@@ -2418,9 +2429,15 @@ int xmodel_tables(const slos_plan* cp, int levels, const XRows& x, const uint32_
   for (auto& t : p->dev)
     if (t.device == d) {
       if (!t.xm[levels]) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cap));
+        if (cap != hipStreamCaptureStatusNone)
+          return fail(SLOS_EINVAL, "the plan's first x-model call cannot be captured: run it once before");
         uint32_t* dev = nullptr;
+        const BesideCaptures guard;
         HIP_TRY(hipMalloc(&dev, x.words.size() * sizeof(uint32_t)));
-        const hipError_t e = hipMemcpy(dev, x.words.data(), x.words.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
+        hipError_t e = hipMemcpyAsync(dev, x.words.data(), x.words.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);  // other streams may read it from here on
         if (e != hipSuccess) {
           (void)hipFree(dev);
           HIP_TRY(e);
@@ -2507,7 +2524,7 @@ int slos_xmodel(const slos_plan* p, const void* U, int64_t batch, int order, con
   rc = device_tables(p, &dt);
   if (rc) return rc;
   const uint32_t* tab = nullptr;
-  rc = xmodel_tables(p, x.levels, *x.rows, &tab);
+  rc = xmodel_tables(p, x.levels, *x.rows, reinterpret_cast<hipStream_t>(stream), &tab);
   if (rc) return rc;
   const int n = p->n;
   const int B = (int)batch;
