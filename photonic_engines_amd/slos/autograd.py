@@ -88,11 +88,22 @@ def _sparse(grad_p: torch.Tensor) -> bool:
     return int(torch.count_nonzero(sample)) * SPARSE_READOUT <= sample.numel()
 
 
-# A forward keeps every layer below the last while these take at most KEEP_BYTES (and the kernel was not
-# asked for checkpointing): forward and backward are then one native call each, and no layer is
-# recomputed but the last, in the pass that applies the readout's adjoint. Above it the even layers are
-# kept and the odd ones recomputed, layer by layer.
+# A forward keeps every layer below the last while these take at most KEEP_BYTES and a KEEP_SHARE-th of the
+# free memory (and the kernel was not asked for checkpointing): forward and backward are then one native
+# call each, and no layer is recomputed but the last, in the pass that applies the readout's adjoint. Else the
+# even layers are kept, half to three quarters of the bytes, and the odd ones recomputed, layer by layer. The
+# free memory is asked for from KEEP_LOOK bytes on (6 us, beside a forward of a few hundred).
 KEEP_BYTES = 1 << 30
+KEEP_SHARE = 16
+KEEP_LOOK = 1 << 25
+
+
+def _free_bytes(dev: torch.device, enough: int) -> int:
+    """Free bytes of the device, and those that torch's cache holds unused if the former are not `enough`."""
+    free = int(torch.cuda.mem_get_info(dev)[0])
+    if free < enough:
+        free += int(torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev))
+    return free
 
 
 def _kept_bytes(kernel, Ug: torch.Tensor, layer: int, cf: int) -> int | None:
@@ -103,7 +114,24 @@ def _kept_bytes(kernel, Ug: torch.Tensor, layer: int, cf: int) -> int | None:
     if getattr(kernel, "gradient_checkpointing", False):  # (superposition kernels have no such option)
         return None
     n = kernel._plan.saved_bytes(Ug.shape[0], layer)
-    return n if n <= KEEP_BYTES else None
+    if n > KEEP_BYTES:
+        return None
+    if n >= KEEP_LOOK and not (Ug.is_cuda and torch.cuda.is_current_stream_capturing()):
+        if n * KEEP_SHARE > _free_bytes(Ug.device, n * KEEP_SHARE):
+            return None
+    return n
+
+
+def _forward_kept(kernel, Ug: torch.Tensor, modes, layer: int, cf: int, probs: bool, scale: float):
+    """(output, the kept layers) of a forward whose backward is the native one, or None where that does not
+    apply or its layers find no memory."""
+    kept = _kept_bytes(kernel, Ug, layer, cf)
+    if kept is None:
+        return None
+    try:
+        return kernel._plan.forward_saved(Ug, modes, layer, probs, scale, kept)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def _user_grad(gU: torch.Tensor, ctx) -> torch.Tensor:
@@ -118,9 +146,9 @@ class SLOSProbs(torch.autograd.Function):
         cf = _layer_flags(kernel)                        # every layer as in the forward without grad
         ctx.kernel, ctx.Ug, ctx.cf = kernel, Ug, cf
         ctx.user_shape, ctx.user_dtype, ctx.user_device = U_user.shape, U_user.dtype, U_user.device
-        kept = _kept_bytes(kernel, Ug, n, cf)
+        kept = _forward_kept(kernel, Ug, modes, n, cf, True, kernel._input_norm)
         if kept is not None:
-            p, ctx.saved = plan.forward_saved(Ug, modes, n, True, kernel._input_norm, kept)
+            p, ctx.saved = kept
             return p
         ctx.saved, psi = _checkpointed_forward(plan, Ug, modes, n, cf)
         return plan.layer_step(Ug, n, modes[n - 1], psi, nat.OUT_PROBS, scale=kernel._input_norm, flags=cf)
@@ -159,9 +187,9 @@ class SLOSRaw(torch.autograd.Function):
         cf = _layer_flags(kernel)
         ctx.kernel, ctx.Ug, ctx.cf, ctx.modes, ctx.layer = kernel, Ug, cf, modes, layer
         ctx.user_shape, ctx.user_dtype, ctx.user_device = U_user.shape, U_user.dtype, U_user.device
-        kept = _kept_bytes(kernel, Ug, layer, cf)
+        kept = _forward_kept(kernel, Ug, modes, layer, cf, False, 1.0)
         if kept is not None:
-            out, ctx.saved = plan.forward_saved(Ug, modes, layer, False, 1.0, kept)
+            out, ctx.saved = kept
             return out
         ctx.saved, psi = _checkpointed_forward(plan, Ug, modes, layer, cf)
         return _hi(plan.layer_step(Ug, layer, modes[layer - 1], psi, nat.OUT_RAW, flags=cf))
