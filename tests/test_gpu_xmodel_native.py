@@ -9,7 +9,7 @@ import torch
 from helpers import haar_unitary
 
 from photonic_engines_amd import _native as nat
-from photonic_engines_amd.slos import FockSLOSKernel
+from photonic_engines_amd.slos import FockSLOSKernel, species
 from photonic_engines_amd.slos._plan import Plan
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +75,23 @@ def test_columns_in_any_order(modes, weights_on_device):
     assert abs(float(res[1].double().sum()) - 1) < 1e-5
     # (another order of the same float32 sums: a few tens of roundings of terms of at most the value)
     assert ((res[0] - res[1]).abs() <= 64 * 2.0 ** -24 * (res[1] + 1e-3)).all()
+
+
+@pytest.mark.parametrize("occ,mask,rows,order", [
+    ([1, 1, 1, 0, 0], "fock", 0, None), ([1] * 4 + [0] * 6, "fock", 2, 1), ([2, 0, 1, 1, 0, 1, 0], "fock", 0, None),
+    ([1] * 6 + [0] * 4, "fock", 0, 3), ([3, 2, 1, 0, 0, 0, 0], "fock", 3, 5), ([1] * 8 + [0] * 4, "fock", 0, None),
+    ([1] * 9 + [0], "fock", 0, 2), ([1, 0] * 5, "dual_rail", 0, None), ([1, 0, 1, 1, 0, 1, 1, 0], "unbunched", 2, None),
+    ([1, 0, 0, 0] * 3, "sparse_1in4", 0, None), ([1] * 5 + [0] * 4, "tail_empty", 0, 4), ([1] * 7 + [0] * 9, "fock", 0, 2)])
+@pytest.mark.parametrize("compensated", [False, True])
+def test_one_call_has_the_bits_of_the_layer_by_layer_form(monkeypatch, occ, mask, rows, order, compensated):
+    n, m = sum(occ), len(occ)
+    k = FockSLOSKernel(n, m, occ, mask=mask, device=DEV, compensated=compensated)
+    U = haar_unitary(m, n + m).to(torch.complex64).to(DEV)
+    if rows:
+        U = torch.stack([haar_unitary(m, n + m + b).to(torch.complex64).to(DEV) for b in range(rows)])
+    for x in (0.0, 0.37, 0.999):
+        one = k.probs(U, indist=x, order=order)
+        with monkeypatch.context() as mp:
+            mp.setattr(species, "_native_x", lambda *a: None)
+            many = k.probs(U, indist=x, order=order)
+        assert torch.equal(one, many), x
