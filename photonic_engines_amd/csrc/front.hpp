@@ -7,8 +7,8 @@
 // launches as long as layer kf-1 has at most kFrontStates states and the work groups of all rows
 // together do not fill the chip (see front_layers in slos.hip). A launch takes about 10 us (where the
 // tuple words do not give the positions they are searched for, see k_front); it replaces the fill and 3 to 6
-// launches of 5 us or more: probs(U) at n = 4, m = 12 34.8 -> 21.5 us, n = 6, m = 18 42.6 -> 24.3 us
-// (both now a matter of host time), n = 8, m = 24 126 -> 107 us.
+// launches of 5 us or more: probs(U) at n = 4, m = 12 34.8 -> 21.5 us, n = 6, m = 18 42.6 -> 24.3 us,
+// n = 8, m = 24 126 -> 107 us (with the host's part of then, 20 us of the first two).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

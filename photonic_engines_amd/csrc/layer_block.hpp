@@ -242,8 +242,8 @@ __device__ __forceinline__ void suffix_edges(const ChunkCtx<MAXD, SUF>& cx, Tupl
 // for every j: it is past the parents of the block only where a = (x, m-1, .., m-1) drops x < m - 1,
 // and then another block follows. Per step and block this takes 5 loads of 16 bytes and a masked one
 // in place of 10 of 8 bytes (whose lanes the cache serves at half its rate): the last layer at n = 11,
-// m = 32 25.9 -> 23.9 ms, of 170 instances (8, 20) 1.57 -> 1.46 ms. Compensated sums, which are bound
-// by their arithmetic, keep the 10 loads: the selects cost 2 % there (n = 9, m = 22, 339 -> 346 us).
+// m = 32 25.9 -> 23.9 ms, of 170 instances (8, 20) 1.57 -> 1.46 ms. So with compensated sums (n = 9, m = 22, layer
+// 9 173 -> 152 us; as two-sums in FP32 these were bound by their arithmetic, and the selects cost 2 %).
 template <int SUF>
 struct PairOffsets {
   uint32_t a[SUF], b[SUF];  // suffix parents of the two children (bytes)

@@ -30,8 +30,10 @@ __device__ __forceinline__ void cmac64(double2& a, double2 u, double2 v) {
   a.y = fma(u.y, v.x, a.y);
 }
 
-// KIND 0: raw complex128, 1: float64 probabilities, 2: scaled complex128 amplitudes; f: prod t_j!
-// (whole numbers below 2^24 for the prefixes of at most 8 positions, exact in float)
+// KIND 0: raw complex128, 1: float64 probabilities, 2: scaled complex128 amplitudes; f: prod t_j!, which
+// divides K!. Up to 13 photons every such number and every product on the way to it is exact in float: the odd
+// part of 13! is 6,081,075 < 2^24 (that of 14! is not below it).
+constexpr int kExactFactorials = 13;
 template <int KIND>
 __device__ __forceinline__ void store64(void* out, uint64_t i, double2 v, float f, double scale, unsigned flags) {
   if constexpr (KIND == 0) {
@@ -101,6 +103,7 @@ template <int KIND, int MAXD, int SUF>
 __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_layer_block_f64(
     const uint64_t* __restrict__ cg_t, const int* __restrict__ lo_t, const void* __restrict__ tuples, int me, int stride,
     int multiset, const double2* __restrict__ par_all, void* __restrict__ out_all, BlockLayerF64 p) {
+  static_assert(MAXD + SUF <= kExactFactorials, "store64 takes prod t_j! in float");
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SufRow64 rows[kSufRows];
   __shared__ float rn[kNormRows * kNormCodes];

@@ -835,7 +835,7 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
 }
 
 // one complex128 layer on the block or group-order kernel; -1 where they do not apply (layers of
-// fewer than 5 photons, prefixes of more than 8 positions, spaces without tuple words)
+// fewer than 5 photons, prefixes of more than 8 positions, spaces without tuple words, and by use_blocks)
 int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, slos::MatrixStride us, int64_t B, const void* par,
                      uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
   if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
@@ -875,8 +875,9 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   return SLOS_OK;
 }
 
-// one complex128 layer (thread-per-state, FP64): kind 0 raw complex128, 1 float64 probabilities,
-// 2 scaled complex128 amplitudes (SLOS_FLAG_IMMEDIATE: times sqrt(prod t!))
+// one complex128 layer, on the block or group-order kernel where launch_block_f64 takes it, else thread per
+// state: kind 0 raw complex128, 1 float64 probabilities, 2 scaled complex128 amplitudes (SLOS_FLAG_IMMEDIATE:
+// times sqrt(prod t!))
 int launch_layer_f64(const slos_plan* p, const DevTables& dt, int K, int col, const void* U, slos::MatrixStride us, int64_t B, const void* par,
                      uint64_t S_par, void* out, uint64_t S, int kind, double scale, unsigned flags, hipStream_t st) {
   if (!(flags & SLOS_FLAG_SIMPLE)) {
@@ -2245,8 +2246,9 @@ bool insert_walk(const slos_plan* p, int dp, uint64_t Sp, int64_t batch) {
 }
 
 // Parents per wave of the insert-table kernels: few, so that the waves in flight read near one
-// another (descents, us, with 64 / 128 / 256 / 512, measured without the merged blocks: 2.0M parents 57
-// / 65 / 73 / 93, 7.9M 157 / 147 / 157 / 202, 28M 588 / 467 / 460 / 555, 1.1G - / 20500 / 19100 / 19800).
+// another (descents, us, with 64 / 128 / 256 / 512: 0.66M parents 17.5 / 20.0 / 21.6 / 27.9, 2.0M 39 / 41 / 40 / 41, 7.9M
+// 127 / 111 / 108 / 135, 28M 492 / 383 / 383 / 445, 62M 1212 / 1042 / 1096 / 1203, 93M 1699 / 1257 / 1168 / 1258, 1.1G 23400 /
+// 18900 / 18900 / 19900).
 uint64_t insert_per_wave(uint64_t Sp) { return Sp < (1ull << 22) ? 64 : Sp < (1ull << 24) ? 128 : 256; }
 
 }  // namespace

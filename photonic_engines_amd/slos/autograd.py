@@ -2,7 +2,7 @@
 
 Replaces autograd through gather / mul / scatter_add_ (photonic_engines/slos/kernel.py:216-257)
 and the opt-in recomputing layer (_CheckpointedLayer, kernel.py:40-80). A forward keeps the layers below
-the last where they are small (KEEP_BYTES), else every other layer (the even ones), and the backward
+the last where they are small and memory is plenty (KEEP_BYTES), else every other layer (the even ones), and the backward
 then recomputes each odd layer once from the even layer below it; it runs the recurrence backwards with
 the adjoint kernels:
 
