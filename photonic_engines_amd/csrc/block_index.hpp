@@ -347,15 +347,19 @@ constexpr uint32_t kGroupItemChildren = 2048, kGroupItemWidth = 128;
 constexpr uint32_t kGroupFineChildren = 1024, kGroupFineWidth = 64;
 
 // the work items of layer K (prefix length d = K - 5 >= 2), 4 words each (r, u_b, u_e, 0): ranges of
-// about `children` children of the group, a multiple of `least` suffix positions
+// about `children` children of the group, a multiple of `least` suffix positions (multiset spaces)
 template <class Vec>
 inline void group_items(const SpaceView& sv, int K, Vec& out, uint32_t children = kGroupItemChildren,
                         uint32_t least = kGroupItemWidth) {
   const int d = K - 5;
   const uint64_t nR = sv.C(d - 1, 0);
-  int R[64];
+  int R[64] = {};
   for (uint64_t r = 0; r < nR; ++r) {
-    sv.unrank(r, d - 1, R);
+    if (r) {  // the next sorted tuple: the last position below me - 1 steps up, those after it follow
+      int i = d - 2;
+      while (R[i] == sv.me - 1) --i;
+      for (int x = R[i] + 1; i <= d - 2; ++i) R[i] = x;
+    }
     const uint32_t L = (uint32_t)sv.C(5, sv.lo[R[d - 2]]);
     uint32_t w = (children / (uint32_t)(R[0] + 1)) & ~(least - 1u);
     if (w < least) w = least;
