@@ -92,10 +92,10 @@ def _sparse(grad_p: torch.Tensor) -> bool:
 # free memory (and the kernel was not asked for checkpointing): forward and backward are then one native
 # call each, and no layer is recomputed but the last, in the pass that applies the readout's adjoint. Else the
 # even layers are kept, half to three quarters of the bytes, and the odd ones recomputed, layer by layer. The
-# free memory is asked for from KEEP_LOOK bytes on (6 us, beside a forward of a few hundred).
+# free memory is asked for from KEEP_LOOK bytes on (6 to 20 us of the host, beside a step of 1 ms or more).
 KEEP_BYTES = 1 << 30
 KEEP_SHARE = 16
-KEEP_LOOK = 1 << 25
+KEEP_LOOK = 1 << 26
 
 
 def _free_bytes(dev: torch.device, enough: int) -> int:

@@ -17,7 +17,7 @@ def test_all_layers_are_kept_where_memory_is_plenty(monkeypatch):
         return autograd._kept_bytes(SimpleNamespace(_plan=SimpleNamespace(saved_bytes=lambda B, layer: nbytes)), U, 3, 0)
 
     for nbytes, have, ok in ((1 << 20, 0, True), (1 << 30, 1 << 34, True), (1 << 30, (1 << 34) - 1, False),
-                             ((1 << 30) + 1, 1 << 38, False), (1 << 25, 1 << 28, False)):
+                             ((1 << 30) + 1, 1 << 38, False), (1 << 26, 1 << 29, False)):
         free[0] = have
         assert kept(nbytes) == (nbytes if ok else None), (nbytes, have)
 
