@@ -2328,8 +2328,11 @@ int run_descend(const slos_plan* p, const DevTables& dt, int k, const float* q_k
   return SLOS_OK;
 }
 
-// the layer k from which one launch takes every step down (descend_tail.hpp), or 0
-int tail_top(const slos_plan* p) {
+// The layer k from which one launch takes every step down (descend_tail.hpp), or 0: with more rows than CUs its work
+// groups of 1,024 threads take turns, and a launch a step is the shorter way (us, so / a launch a step: n = 5, m = 9, 1
+// row 18 / 28, 256 19 / 29, 512 30 / 29, 2048 102 / 33, 20000 958 / 136; n = 6, m = 12, 256 40 / 44, 512 66 / 59).
+int tail_top(const slos_plan* p, int64_t batch) {
+  if (batch > 256) return 0;
   int top = 0;
   for (int k = 1; k <= std::min(p->n, slos::kTailTop); ++k) {
     const uint64_t Sp = p->size(k - 1);
@@ -2362,7 +2365,7 @@ int slos_loss_thin(const slos_plan* p, const float* q, float* const* out, const 
   int rc = device_tables(p, &dt);
   if (rc) return rc;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int top = tail_top(p);
+  const int top = tail_top(p, batch);
   for (int k = p->n; k > top; --k) {
     rc = run_descend(p, dt, k, k == p->n ? q : out[k], out[k - 1], batch, 0u, scale[k - 1], st);
     if (rc) return rc;
