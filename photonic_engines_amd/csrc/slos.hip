@@ -650,12 +650,15 @@ struct ReduceArgs {
   int col[kMaxPhotons];
   int layers;
 };
-constexpr int kReduceAllThreads = 1024;
+// Work groups of 1,024 threads, or of 128 where there are many (1024 / 256 / 128 / 64 threads, us of a whole backward: 20,000
+// rows of n = 5, m = 10, dual rail, 1374 / 614 / 538 / 530, 2,000 of n = 2, m = 22 186 / 69 / 54 / 55, 100 of n = 6, m = 12 68 / 64 /
+// 63 / 65; one row of n = 8, m = 24 226 / 223 / 229 / 241, n = 5, m = 64 314 / 309 / 326 / 395).
+constexpr int kReduceAllThreads = 1024, kReduceManyThreads = 128;
 constexpr uint32_t kFew = 512;  // partials of a layer that one wave sums
 __global__ __launch_bounds__(kReduceAllThreads) void k_reduce_all(ReduceArgs a, const double2* __restrict__ partial, int me,
                                                                   int m, float2* __restrict__ gU) {
-  constexpr int kW = kReduceAllThreads / 64;
-  __shared__ double2 wave[kMaxPhotons][kW];
+  const int kW = (int)blockDim.x / 64;
+  __shared__ double2 wave[kMaxPhotons][kReduceAllThreads / 64];
   __shared__ float2 sum[kMaxPhotons];
   const int64_t b = blockIdx.y;
   const int j = blockIdx.x;
@@ -668,7 +671,7 @@ __global__ __launch_bounds__(kReduceAllThreads) void k_reduce_all(ReduceArgs a, 
       double sr = 0, si = 0;
       if (!few || l % kW == w) {
         const double2* src = partial + a.part[l] + (size_t)b * nblk * me + j;
-        for (uint32_t r = few ? threadIdx.x & 63u : threadIdx.x; r < nblk; r += few ? 64u : (uint32_t)kReduceAllThreads) {
+        for (uint32_t r = few ? threadIdx.x & 63u : threadIdx.x; r < nblk; r += few ? 64u : blockDim.x) {
           const double2 v = src[(size_t)r * me];
           sr += v.x;
           si += v.y;
@@ -2228,7 +2231,8 @@ int slos_backward(const slos_plan* p, const void* U, int64_t batch, const int32_
     gk = gout;
     next ^= 1;
   }
-  hipLaunchKernelGGL(k_reduce_all, dim3((unsigned)p->m, (unsigned)batch), dim3(kReduceAllThreads), 0, st, ra,
+  const int threads = (int64_t)p->m * batch > 1024 ? kReduceManyThreads : kReduceAllThreads;
+  hipLaunchKernelGGL(k_reduce_all, dim3((unsigned)p->m, (unsigned)batch), dim3((unsigned)threads), 0, st, ra,
                      reinterpret_cast<const double2*>(base), p->me, p->m, static_cast<float2*>(grad_U));
   HIP_TRY(hipGetLastError());
   return SLOS_OK;

@@ -252,7 +252,8 @@ def x_mixture(kernel, U: torch.Tensor, indist, order: int | None = None) -> torc
     native = _native_x(kernel, Ub, x, d.x, b_max)
     if native is not None:
         return kernel._out(native, batched)
-    weights = [torch.as_tensor(w).to(dtype=rdt, device=Ub.device) for w in _weights(x, n, b_max)]
+    weights = torch.stack([torch.as_tensor(w, dtype=torch.float64, device=x.device).expand(x.shape)
+                           for w in _weights(x, n, b_max)]).to(dtype=rdt, device=Ub.device)
     B, m = Ub.shape[0], Ub.shape[-1]
     dev = Ub.device
     per = max(1, (2 << 30) // (rdt.itemsize * kernel.layers.size(n) * max(B, 1)))
