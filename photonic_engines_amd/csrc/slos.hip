@@ -721,7 +721,10 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
 // state, where both can. The block kernels share index work between states but wait on their own
 // set-up, and a block must be long enough to fill waves; the two give the same bits. Measured (us, block
 // or group order against thread):
-//   group order: 347k states 21 / 14, 2.0M 28 / 29, 7.9M 56 / 94; compensated 490k 44 / 17;
+//   group order: 347k states 21 / 14, 2.0M 28 / 29, 7.9M 56 / 94; compensated 490k 44 / 17; where a group, the
+//   states of one (K - 6)-position prefix, is short (many rows of few modes), 20,000 rows of 364 states (6 a group)
+//   1904 / 137, 1,000 of 6,435 (179) 81 / 75, 3,000 of 1,716 (245) 54 / 53, 300 of 24,310 (442) 60 / 82, complex128 one of 2.5M
+//   (291) 50 / 43;
 //   blocks, multiset: 98k states 18.4 / 13.8, 475k 18.9 / 14.9, 2.3M (72,000 a block) 33 / 30, 9.3M (3,400 a
 //   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
 //   blocks, collision-free: 126k 41 / 15, 3.1M (209 a block) 101 / 55, 2.0M (4,680 a block) 39 / 32, 54.6M
@@ -746,7 +749,7 @@ bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool 
   if (f64 && K > 12 && S < (1ull << 32)) return S * (uint64_t)B >= (1ull << 25);
   if (K > 12 || S >= (1ull << 32)) return true;
   if (S * (uint64_t)B < (1ull << 21)) return false;
-  if (suf == 5 && !p->items[K].empty()) return true;
+  if (suf == 5 && !p->items[K].empty()) return S >= 320 * p->size(K - 6);
   const double per = (double)S / (double)p->size(K - suf), states = (double)S * (double)B;
   if (per >= (p->multiset ? 256.0 : 8192.0)) return true;
   return states * per >= (double)(p->multiset ? 1ull << 33 : S < (1ull << 20) ? 1ull << 32 : 1ull << 34);
