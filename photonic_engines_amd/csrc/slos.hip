@@ -1953,10 +1953,16 @@ bool adjoint_walk(const slos_plan* p, int k) {
 // child's index anew: the one for few parents, and for many modes, where the thread-per-state kernel has
 // few waves (its sums' LDS). Adjoint layers with their sums, us, lane a mode / walk: 98k parents in all (24
 // modes) 31 / 35, 171k (14) 35 / 29, 377k (32) 68 / 57; lane a mode / thread per state: 17k (24) 26 / 38, 119k (14)
-// 30 / 34, 273k (12) 54 / 42, 886k (20) 100 / 116, 209k (32) 44 / 92, 766k (64) 234 / 592, 1.1M (40) 268 / 417.
+// 30 / 34, 273k (12) 54 / 42, 886k (20) 100 / 116, 209k (32) 44 / 92, 766k (64) 234 / 592, 1.1M (40) 268 / 417. In set
+// masks most modes have no child: sparse_1in4, 2.6M (20) 335 / 152, 1.2M (24) 129 / 102, 1.1M (32) 132 / 202; dual rail,
+// 672k (20) 73 / 62, 253k (24) 36 / 46; collision-free 1.6M (20) 165 / 171. Where the thread-per-state forms are
+// exact (parents of at most 3 photons), and in sparse_1in4, it must fill its 32 or 64 lanes to four fifths: 3 photons, 78k
+// (24) 29 / 28, 520k (24) 99 / 89, 598k (32) 123 / 176, 574k (40) 239 / 191, 915k (64) 503 / 696; sparse_1in4 1.9M (36) 363 / 332.
 bool adjoint_modes(const slos_plan* p, int k, int64_t batch) {
   if (k - 1 > slos::kModesPhotons || p->me > 64 || p->size(k) >= (1ull << 31)) return false;
-  return p->size(k - 1) <= (1ull << 17) / (uint64_t)batch || (!adjoint_walk(p, k) && p->me >= 20);
+  return p->size(k - 1) <= (k - 1 <= 3 ? 1ull << 16 : 1ull << 17) / (uint64_t)batch ||
+         (!adjoint_walk(p, k) && p->me >= 20 + 4 * p->shift &&
+          ((k - 1 > 3 && p->shift < 2) || 5 * p->me >= 4 * slos::modes_lanes(p->me)));
 }
 
 // modes: the kernel with a lane a mode, else the walk or the thread-per-state kernel
