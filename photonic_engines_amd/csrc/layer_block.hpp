@@ -609,14 +609,15 @@ __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTab
   const uint64_t g_end = (g + a.per_wave < a.S) ? g + a.per_wave : a.S;
   const int d = K - SUF;
 
-  // the block holding g: its prefix rank r and g's offset inside it (scalar path)
-  uint64_t r, u0;
-  {
-    int q[MAXD];
-    u0 = unrank_prefix<MAXD>(tg, K, d, g, q);
-    r = prefix_rank<MAXD>(tg, d, q);
-  }
+  uint64_t r = 0, u0 = 0;
+  bool seek = true;
   while (g < g_end) {
+    if (seek) {  // the block holding g: its prefix rank r and g's offset inside it (scalar path)
+      int q[MAXD];
+      u0 = unrank_prefix<MAXD>(tg, K, d, g, q);
+      r = prefix_rank<MAXD>(tg, d, q);
+    }
+    const uint64_t g0 = g;
     if (r >= a.S_pre) break;  // cannot happen while g < S; keeps the loop bounded regardless
     fill_block_table<MAXD, SUF>(tl, K, d, r, a.S_pre, tbl, lane);
     const int nb = (int)((a.S_pre - r < kBlockBatch) ? a.S_pre - r : kBlockBatch);
@@ -658,6 +659,9 @@ __device__ __forceinline__ void block_wave(const BlockTables& tg, const BlockTab
       u0 = 0;
     }
     r += kBlockBatch;
+    // 64 prefixes without a child: a set mask's, whose runs of them are thousands long. On to the next child's
+    // block.
+    seek = g == g0;
   }
 }
 

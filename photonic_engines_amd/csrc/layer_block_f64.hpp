@@ -132,13 +132,15 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
   void* out = static_cast<char*>(out_all) + (size_t)b * a.S * (KIND == 1 ? 8 : 16);
   const auto* words = static_cast<const TupleWordT<SUF>*>(tuples);
   const uint32_t C0 = (uint32_t)cg_t[(SUF - 1) * stride];
-  uint64_t r, u0;
-  {
-    int q[MAXD];
-    u0 = unrank_prefix<MAXD>(tg, K, d, g, q);
-    r = prefix_rank<MAXD>(tg, d, q);
-  }
+  uint64_t r = 0, u0 = 0;
+  bool seek = true;
   while (g < g_end) {
+    if (seek) {
+      int q[MAXD];
+      u0 = unrank_prefix<MAXD>(tg, K, d, g, q);
+      r = prefix_rank<MAXD>(tg, d, q);
+    }
+    const uint64_t g0 = g;
     if (r >= a.S_pre) break;  // cannot happen while g < S; keeps the loop bounded regardless
     fill_block_table<MAXD, SUF>(tl, K, d, r, a.S_pre, tbl, lane);
     const int nb = (int)((a.S_pre - r < kBlockBatch) ? a.S_pre - r : kBlockBatch);
@@ -164,6 +166,9 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3
       u0 = 0;
     }
     r += kBlockBatch;
+    // 64 prefixes without a child: a set mask's, whose runs of them are thousands long. On to the next child's
+    // block.
+    seek = g == g0;
   }
 }
 
