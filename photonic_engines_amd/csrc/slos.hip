@@ -717,6 +717,15 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
   return (dt.tuples5 && K - 5 >= 1 && K - 5 <= 8 && block_lds_fit(K, p->me, 5)) ? 5 : slos::kSuf;
 }
 
+// (K - suf)-position prefixes of layer K that have children: those that end at or below the last mode with suf admissible
+// positions behind it, as many as tuples of as many modes from the other end
+uint64_t full_blocks(const slos_plan* p, int K, int suf) {
+  const uint64_t* rest = p->cg.data() + (size_t)suf * (p->me + 1);
+  int x = p->me - 1;
+  while (x > 0 && rest[p->lo[x]] == 0) --x;
+  return std::max<uint64_t>(1, p->cg[(size_t)(K - suf) * (p->me + 1) + (p->me - 1 - x)]);
+}
+
 // Whether layer K (S states, B rows) runs on the block or group-order kernel rather than one thread a
 // state, where both can. The block kernels share index work between states but wait on their own
 // set-up, and a block must be long enough to fill waves; the two give the same bits. Measured (us, block
@@ -727,17 +736,19 @@ int block_suffix(const slos_plan* p, const DevTables& dt, int K) {
 //   (291) 50 / 43;
 //   blocks, multiset: 98k states 18.4 / 13.8, 475k 18.9 / 14.9, 2.3M (72,000 a block) 33 / 30, 9.3M (3,400 a
 //   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
-//   blocks, collision-free: 126k 41 / 15, 3.1M (209 a block) 101 / 55, 2.0M (4,680 a block) 39 / 32, 54.6M
-//   (92 a block) 1266 / 898, 7.6M (119,000 a block) 57 / 118.
-// Shorter blocks pay where the layer is large: a state costs 6 us / 10^6 in blocks and 13 to 19 by threads, a
-// block some 2.6 us / 1000 besides, and the launch some 40 us of waves that wait on their first blocks. So
-// the line is one of states times states a block, 2^34 for set masks, on layers of less than 2^20 states
-// (rows of a batch, whose parents stay in the L2) 2^32:
-//   8.4e9 (5.9M states, 1,441 a block) 93 / 81, 2.2e10 (10.5M, 2,120) 119 / 141, 7.5e9 (14.3M, 522) 227 / 206, 2.2e10 (28M,
-//   780) 348 / 397, 6e9 (30M, 210) 586 / 464, 2.1e10 (64.5M, 320) 973 / 1027, 1.8e10 (129M, 142) 2158 / 2331, 8.2e11
-//   (273M, 2,992) 1996 / 4186; rows: 2.7e9 (10 of 735k, 363) 107 / 94, 6.3e9 (200 of 78k, 408) 131 / 152, 1.3e10 (50 of 735k,
-//   363) 351 / 439, 1.4e10 (20 of 143k, 4,750) 24 / 35.
-// and 2^33 for the multiset layers that have no group order: 12 photons, 1.8e9 (17.4M, 101) 364 / 268, 7.7e9 (52M, 149)
+//   blocks, collision-free: 126k 41 / 15, 3.1M (522 a block) 93 / 47, 54.6M (308 a block) 1235 / 970, 7.6M (119,000 a
+//   block) 57 / 118.
+// Shorter blocks pay where the layer is large: a state costs 6 us / 10^6 in blocks and 13 to 25 by threads, a
+// block some 2 us / 1000 besides, and the launch some 40 us of waves that wait on their first blocks. So
+// the line of set masks is one of states times states a block that has any (full_blocks): collision-free 3e10, dual rail
+// 1.4e10, sparse_1in4, whose threads take longest, 4e9; at most 1e10 on layers of less than 2^20 states (rows of a
+// batch, whose parents stay in the L2):
+//   collision-free, 1.5e10 (5.9M states) 93 / 81, 3.8e10 (10.5M) 121 / 130, 1.6e10 (14.3M) 230 / 188, 4.5e10 (28M) 355 / 364, 1.7e10
+//   (30M) 585 / 421, 5.2e10 (64.5M) 867 / 949, 5.6e10 (129M) 1836 / 2348, 2.8e11 (94M) 803 / 1285;
+//   dual rail, 8e9 (3.3M) 55 / 47, 4.5e9 (8.2M) 130 / 120, 1.5e10 (70M) 1387 / 2474, 2.6e10 (76M) 1116 / 1507, 5.5e10 (11M) 107 / 138;
+//   sparse_1in4, 1.1e9 (1.0M) 21 / 22, 4.3e9 (4.2M) 62 / 78, 1.4e10 (2.9M) 39 / 41, 1.7e10 (16.8M) 178 / 402, 2.2e11 (69M) 534 / 1119;
+//   rows, 5.6e9 (10 of 735k) 107 / 94, 4e9 (60 of 647k) 777 / 600, 1.1e10 (200 of 78k) 131 / 152, 2.8e10 (50 of 735k) 351 / 439.
+// and 2^33 for the multiset layers that have no group order: 12 photons, 1.8e9 (17.4M, 101 a block) 364 / 268, 7.7e9 (52M, 149)
 //   768 / 790 (compensated 1607 / 1334, complex128 948 / 917), 3e10 (141M, 214) 1482 / 2317.
 // The thread kernel's exact forms are those of at most 12 photons and 2^32 states. The line holds for
 // compensated sums (8 photons, 1.1M states 27 / 24, 2.2M 33 / 45, 9 photons, 3.1M 46 / 63; collision-free 3.1M (209 a
@@ -750,9 +761,10 @@ bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool 
   if (K > 12 || S >= (1ull << 32)) return true;
   if (S * (uint64_t)B < (1ull << 21)) return false;
   if (suf == 5 && !p->items[K].empty()) return S >= 320 * p->size(K - 6);
-  const double per = (double)S / (double)p->size(K - suf), states = (double)S * (double)B;
-  if (per >= (p->multiset ? 256.0 : 8192.0)) return true;
-  return states * per >= (double)(p->multiset ? 1ull << 33 : S < (1ull << 20) ? 1ull << 32 : 1ull << 34);
+  const double per = (double)S / (double)full_blocks(p, K, suf), states = (double)S * (double)B;
+  if (p->multiset) return per >= 256.0 || states * per >= (double)(1ull << 33);
+  const double line = p->shift == 0 ? 3e10 : p->shift == 1 ? 1.4e10 : 4e9;
+  return states * per >= (S < (1ull << 20) ? std::min(line, 1e10) : line);
 }
 
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
