@@ -740,14 +740,17 @@ uint64_t full_blocks(const slos_plan* p, int K, int suf) {
 //   block) 57 / 118.
 // Shorter blocks pay where the layer is large: a state costs 6 us / 10^6 in blocks and 13 to 25 by threads, a
 // block some 2 us / 1000 besides, and the launch some 40 us of waves that wait on their first blocks. So
-// the line of set masks is one of states times states a block that has any (full_blocks): collision-free 3e10, dual rail
-// 1.4e10, sparse_1in4, whose threads take longest, 4e9; at most 1e10 on layers of less than 2^20 states (rows of a
-// batch, whose parents stay in the L2):
+// the line of set masks is one of states times states a block that has any (full_blocks): collision-free 3e10 (complex128,
+// whose blocks gain least, 4e10), dual rail 1.4e10, sparse_1in4, whose threads take longest, 4e9; lower for three
+// rows or more, whose blocks hide one another's set-up: collision-free 1.7e10, dual rail 4e9:
 //   collision-free, 1.5e10 (5.9M states) 93 / 81, 3.8e10 (10.5M) 121 / 130, 1.6e10 (14.3M) 230 / 188, 4.5e10 (28M) 355 / 364, 1.7e10
 //   (30M) 585 / 421, 5.2e10 (64.5M) 867 / 949, 5.6e10 (129M) 1836 / 2348, 2.8e11 (94M) 803 / 1285;
 //   dual rail, 8e9 (3.3M) 55 / 47, 4.5e9 (8.2M) 130 / 120, 1.5e10 (70M) 1387 / 2474, 2.6e10 (76M) 1116 / 1507, 5.5e10 (11M) 107 / 138;
 //   sparse_1in4, 1.1e9 (1.0M) 21 / 22, 4.3e9 (4.2M) 62 / 78, 1.4e10 (2.9M) 39 / 41, 1.7e10 (16.8M) 178 / 402, 2.2e11 (69M) 534 / 1119;
-//   rows, 5.6e9 (10 of 735k) 107 / 94, 4e9 (60 of 647k) 777 / 600, 1.1e10 (200 of 78k) 131 / 152, 2.8e10 (50 of 735k) 351 / 439.
+//   rows, collision-free, 5.6e9 (10 of 735k) 107 / 94, 9.9e9 (9 of 7.7M) 1307 / 1191, 1.5e10 (3 of 13.1M) 653 / 565, 2.1e10 (9 of
+//   13.0M) 1885 / 2008, 2.8e10 (3 of 20.0M) 723 / 855, compensated 1.2e10 (9 of 5.3M) 1184 / 1301, 1.4e10 (3 of 21.5M) 2114 / 1956,
+//   2.8e10 1276 / 1634, complex128 2.1e10 (200 of 500k) 1558 / 1454, 2.8e10 1114 / 1114, 4.8e10 (9 of 6.9M) 900 / 988; dual rail, 9e8
+//   (9 of 750k) 126 / 115, 4.5e9 (200 of 115k) 271 / 323, 1e10 (40 of 1.0M) 513 / 616, complex128 3.9e9 (3 of 7.4M) 556 / 546, 1e10 702 / 754.
 // and 2^33 for the multiset layers that have no group order: 12 photons, 1.8e9 (17.4M, 101 a block) 364 / 268, 7.7e9 (52M, 149)
 //   768 / 790 (compensated 1607 / 1334, complex128 948 / 917), 3e10 (141M, 214) 1482 / 2317.
 // The thread kernel's exact forms are those of at most 12 photons and 2^32 states. The line holds for
@@ -763,8 +766,8 @@ bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool 
   if (suf == 5 && !p->items[K].empty()) return S >= 320 * p->size(K - 6);
   const double per = (double)S / (double)full_blocks(p, K, suf), states = (double)S * (double)B;
   if (p->multiset) return per >= 256.0 || states * per >= (double)(1ull << 33);
-  const double line = p->shift == 0 ? 3e10 : p->shift == 1 ? 1.4e10 : 4e9;
-  return states * per >= (S < (1ull << 20) ? std::min(line, 1e10) : line);
+  if (p->shift == 0) return states * per >= (f64 ? 4e10 : B > 2 ? 1.7e10 : 3e10);
+  return states * per >= (p->shift == 1 && B <= 2 ? 1.4e10 : 4e9);
 }
 
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
