@@ -771,10 +771,15 @@ bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool 
 }
 
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
-// there is one for every XCD and the grid's thread count stays below 2^32, else a row per grid y.
-dim3 batch_grid(uint64_t wgs, int64_t B, slos::BlockLayer* L) {
+// there is one for every XCD and the grid's thread count stays below 2^32, else a row per grid y. A row's
+// parent layer (par_bytes) is of use to the one XCD it is read into while a fair part of it stays in the L2;
+// rows far larger only crowd one another out of the 256 MB behind it. Last layer, us, 1-D against 2-D: 5 MiB of
+// parents (32 rows of (8, 20)) 344 / 355, 12 MiB (9 of (9, 26), collision-free) 330 / 341, 24 MiB (9 of (9, 28)) 571 / 569, 29
+// MiB (sparse_1in4's layer 7 of 12) 604 / 569, 58 MiB (9 of (6, 60)) 3663 / 2719, 109 MiB (9 of (10, 30)) 2557 / 2327; complex128
+// 10 MiB 661 / 704, 22 MiB (dual rail's layer 8 of 16) 410 / 443, 25 MiB (9 of (7, 30)) 675 / 665, 127 MiB 3283 / 3179.
+dim3 batch_grid(uint64_t wgs, int64_t B, uint64_t par_bytes, slos::BlockLayer* L) {
   L->row_wgs = (uint32_t)wgs;
-  const bool flat = B >= 8 && wgs * (uint64_t)B < (1ull << 32) / slos::kBlockThreads;
+  const bool flat = B >= 8 && par_bytes <= (24ull << 20) && wgs * (uint64_t)B < (1ull << 32) / slos::kBlockThreads;
   L->rows = flat ? (uint32_t)B : 1u;
   return flat ? dim3((unsigned)(wgs * (uint64_t)B)) : dim3((unsigned)wgs, (unsigned)B);
 }
@@ -797,6 +802,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs&
   const uint64_t wgs = (waves + slos::kWaves - 1) / slos::kWaves;
   if (wgs > 0x7fffffffull) return fail(SLOS_ERANGE, "layer too large for one launch");
   if (a.B > 65535) return fail(SLOS_ERANGE, "batch > 65535");
+  const uint64_t par_bytes = a.S_par * sizeof(float2) * (a.par_lo ? 2 : 1);
   // layers in group order where their work items exist (plain or compensated sums; probabilities or
   // complex64)
   if (suf == 5 && kind != 2 && dt.items[a.K]) {
@@ -805,7 +811,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs&
     const uint64_t gwgs = ((uint64_t)gn + slos::kWaves - 1) / slos::kWaves;
     if (shg + slos::kBlockStaticLds <= lds_limit() && gwgs <= 0x7fffffffull) {
       L.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
-      const slos::BlockGrid bg{batch_grid(gwgs, a.B, &L), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
+      const slos::BlockGrid bg{batch_grid(gwgs, a.B, par_bytes, &L), shg, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
       slos::launch_layer_group(a.K - suf, kind, comp, bg, a.par, a.out, L, gitems, gn);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
@@ -813,7 +819,7 @@ int launch_block(const slos_plan* p, const DevTables& dt, const slos::LayerArgs&
   }
   const size_t sh = block_lds_fit(a.K, p->me, suf);
   if (!sh) return fail(SLOS_ERANGE, "block kernel LDS exceeds the GPU's LDS");
-  const slos::BlockGrid bg{batch_grid(wgs, a.B, &L), sh, st, dt.cg, dt.lo,
+  const slos::BlockGrid bg{batch_grid(wgs, a.B, par_bytes, &L), sh, st, dt.cg, dt.lo,
                            suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
   if (kind == 0) slos::launch_layer_block<0>(comp, a.K - suf, suf, bg, a.par, a.out, L);
   else if (kind == 1) slos::launch_layer_block<1>(comp, a.K - suf, suf, bg, a.par, a.out, L);
@@ -878,7 +884,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
     const uint64_t wgs = ((uint64_t)n_items + slos::kWaves - 1) / slos::kWaves;
     if (sh + slos::kBlockStaticLds64 <= lds_limit() && wgs <= 0x7fffffffull) {
       L.l.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * slos::kGroupItemChildren));
-      const slos::BlockGrid bg{batch_grid(wgs, B, &L.l), sh, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
+      const slos::BlockGrid bg{batch_grid(wgs, B, S_par * sizeof(double2), &L.l), sh, st, dt.cg, dt.lo, dt.tuples5, p->me, p->multiset};
       slos::launch_layer_group_f64(d, kind, bg, static_cast<const double2*>(par), out, L, items, n_items);
       HIP_TRY(hipGetLastError());
       return SLOS_OK;
@@ -892,7 +898,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   L.l.xcd_chunk = (uint32_t)std::max<uint64_t>(1, (1ull << 20) / ((uint64_t)slos::kWaves * L.l.per_wave));
   const uint64_t wgs = ((S + L.l.per_wave - 1) / L.l.per_wave + slos::kWaves - 1) / slos::kWaves;
   if (wgs > 0x7fffffffull) return -1;
-  const slos::BlockGrid bg{batch_grid(wgs, B, &L.l), sh, st, dt.cg, dt.lo,
+  const slos::BlockGrid bg{batch_grid(wgs, B, S_par * sizeof(double2), &L.l), sh, st, dt.cg, dt.lo,
                            suf == 5 ? static_cast<const void*>(dt.tuples5) : dt.tuples, p->me, p->multiset};
   slos::launch_layer_block_f64(kind, d, suf, bg, static_cast<const double2*>(par), out, L);
   HIP_TRY(hipGetLastError());

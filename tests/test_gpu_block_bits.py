@@ -110,3 +110,14 @@ def test_long_runs_of_prefixes_without_children():
             a = k._plan.forward(U, layer=layer, modes=k.input_modes[:layer], flags=flags | nat.FLAG_BLOCK)
             b = k._plan.forward(U, layer=layer, modes=k.input_modes[:layer], flags=flags | nat.FLAG_SIMPLE)
             assert torch.equal(a, b), (layer, flags)
+
+
+@pytest.mark.parametrize("n,m,mask,dtype", [(8, 26, "fock", torch.complex64), (9, 29, "unbunched", torch.complex64), (8, 24, "fock", torch.complex128)])
+def test_rows_of_wide_layers_equal_single_matrices(n, m, mask, dtype):
+    """9 rows whose last layers' parents are above the 24 MiB a row up to which whole rows go to one XCD,
+    and whose first layers' are below it."""
+    k = _kernel(n, m, mask, dtype=dtype)
+    U = _matrices(m, 9, dtype)
+    p = k._plan.forward(U, out_kind=nat.OUT_PROBS, flags=nat.FLAG_BLOCK)
+    for b in (0, 7, 8):
+        assert torch.equal(p[b], k._plan.forward(U[b:b + 1], out_kind=nat.OUT_PROBS, flags=nat.FLAG_BLOCK)[0]), b
