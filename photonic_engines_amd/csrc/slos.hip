@@ -732,25 +732,31 @@ uint64_t full_blocks(const slos_plan* p, int K, int suf) {
 // or group order against thread):
 //   group order: 347k states 21 / 14, 2.0M 28 / 29, 7.9M 56 / 94; compensated 490k 44 / 17; where a group, the
 //   states of one (K - 6)-position prefix, is short (many rows of few modes), 20,000 rows of 364 states (6 a group)
-//   1904 / 137, 1,000 of 6,435 (179) 81 / 75, 3,000 of 1,716 (245) 54 / 53, 300 of 24,310 (442) 60 / 82, complex128 one of 2.5M
-//   (291) 50 / 43;
+//   1904 / 137, 1,000 of 6,435 (179) 81 / 75, 3,000 of 1,716 (245) 54 / 53, 800 of 12,870 (286) 116 / 107, 300 of 92,378 (323) 285 / 301, of
+//   24,310 (442) 60 / 82; 2.5M states (291) 46 / 41, 30 rows of them 893 / 1045 (compensated 1673 / 1757), 200 of 352,716 (258) 810 /
+//   845 (1622 / 1604); complex128 300 of 92,378 412 / 375, 9 of 646,646 (355) 82 / 76, one of 4.5M (383) 71 / 74;
 //   blocks, multiset: 98k states 18.4 / 13.8, 475k 18.9 / 14.9, 2.3M (72,000 a block) 33 / 30, 9.3M (3,400 a
 //   block) 74 / 78, 17.4M (102 a block, 12 photons) 368 / 274;
 //   blocks, collision-free: 126k 41 / 15, 3.1M (522 a block) 93 / 47, 54.6M (308 a block) 1235 / 970, 7.6M (119,000 a
 //   block) 57 / 118.
 // Shorter blocks pay where the layer is large: a state costs 6 us / 10^6 in blocks and 13 to 25 by threads, a
 // block some 2 us / 1000 besides, and the launch some 40 us of waves that wait on their first blocks. So
-// the line of set masks is one of states times states a block that has any (full_blocks): collision-free 3e10 (complex128,
-// whose blocks gain least, 4e10), dual rail 1.4e10, sparse_1in4, whose threads take longest, 4e9; lower for three
-// rows or more, whose blocks hide one another's set-up: collision-free 1.7e10, dual rail 4e9:
+// the line of set masks is one of states times states a block that has any (full_blocks), by mask, since their threads
+// take longer the fewer modes a photon may enter, by sums, since those in 64 bits gain most (compensated) and least (complex128),
+// and lower for rows of a batch, whose blocks hide one another's set-up (not on the smallest launches of dual rail):
 //   collision-free, 1.5e10 (5.9M states) 93 / 81, 3.8e10 (10.5M) 121 / 130, 1.6e10 (14.3M) 230 / 188, 4.5e10 (28M) 355 / 364, 1.7e10
-//   (30M) 585 / 421, 5.2e10 (64.5M) 867 / 949, 5.6e10 (129M) 1836 / 2348, 2.8e11 (94M) 803 / 1285;
-//   dual rail, 8e9 (3.3M) 55 / 47, 4.5e9 (8.2M) 130 / 120, 1.5e10 (70M) 1387 / 2474, 2.6e10 (76M) 1116 / 1507, 5.5e10 (11M) 107 / 138;
-//   sparse_1in4, 1.1e9 (1.0M) 21 / 22, 4.3e9 (4.2M) 62 / 78, 1.4e10 (2.9M) 39 / 41, 1.7e10 (16.8M) 178 / 402, 2.2e11 (69M) 534 / 1119;
-//   rows, collision-free, 5.6e9 (10 of 735k) 107 / 94, 9.9e9 (9 of 7.7M) 1307 / 1191, 1.5e10 (3 of 13.1M) 653 / 565, 2.1e10 (9 of
+//   (30M) 585 / 421, 5.2e10 (64.5M) 867 / 949, 5.6e10 (129M) 1836 / 2348, 2.8e11 (94M) 803 / 1285; compensated 1.7e10 928 / 841;
+//   rows 5.6e9 (10 of 735k) 107 / 94, 9.9e9 (9 of 7.7M) 1307 / 1191, 1.5e10 (3 of 13.1M) 653 / 565, 2.1e10 (9 of
 //   13.0M) 1885 / 2008, 2.8e10 (3 of 20.0M) 723 / 855, compensated 1.2e10 (9 of 5.3M) 1184 / 1301, 1.4e10 (3 of 21.5M) 2114 / 1956,
-//   2.8e10 1276 / 1634, complex128 2.1e10 (200 of 500k) 1558 / 1454, 2.8e10 1114 / 1114, 4.8e10 (9 of 6.9M) 900 / 988; dual rail, 9e8
-//   (9 of 750k) 126 / 115, 4.5e9 (200 of 115k) 271 / 323, 1e10 (40 of 1.0M) 513 / 616, complex128 3.9e9 (3 of 7.4M) 556 / 546, 1e10 702 / 754.
+//   2.8e10 1276 / 1634, complex128 2.1e10 (200 of 500k) 1558 / 1454, 2.8e10 1114 / 1114, 4.8e10 (9 of 6.9M) 900 / 988;
+//   dual rail, 8e9 (3.3M) 55 / 47, 6.3e9 (25M) 531 / 479, 1.1e10 436 / 439, 1.5e10 (70M) 1387 / 2474, 2.6e10 (76M) 1116 / 1507, 5.5e10
+//   (11M) 107 / 138, compensated 1.3e9 (7.5M) 243 / 229, 2.7e9 (8.9M) 249 / 252, 4.5e9 193 / 212, complex128 1.6e10 (20M) 421 / 383,
+//   2e10 (12M) 192 / 217; rows 1.4e9 (200 of 68k) 219 / 197, 2.1e9 (20 of 745k) 248 / 249, 4.5e9 (200 of 113k) 271 / 323, 3.7e9 (3M states in
+//   all) 39 / 34, 1.2e10 (4M) 45 / 43, 1.3e10 (7M) 62 / 65, compensated 4.3e8 (5M) 157 / 138, 6.6e8 (10M) 296 / 317, 1.1e9 (3M) 83 / 84, 3.3e9
+//   (23M) 475 / 611, complex128 2.1e9 326 / 320, 4.5e9 362 / 382;
+//   sparse_1in4, 1.1e9 (1.0M) 21 / 22, 4.3e9 (4.2M) 62 / 78, 1.4e10 (2.9M) 39 / 41, 1.7e10 (16.8M) 178 / 402, 2.2e11 (69M) 534 / 1119; rows
+//   2.4e9 (9 of 262k) 33 / 37, compensated 50 / 59; complex128 by states alone, 2.6M 52 / 45, 5.4M 76 / 67, 3 rows of 2.9M 134 / 119, 9
+//   of 1.0M 188 / 199, 10.8M 145 / 152, 16.8M 342 / 460;
 // and 2^33 for the multiset layers that have no group order: 12 photons, 1.8e9 (17.4M, 101 a block) 364 / 268, 7.7e9 (52M, 149)
 //   768 / 790 (compensated 1607 / 1334, complex128 948 / 917), 3e10 (141M, 214) 1482 / 2317.
 // The thread kernel's exact forms are those of at most 12 photons and 2^32 states. The line holds for
@@ -759,15 +765,19 @@ uint64_t full_blocks(const slos_plan* p, int K, int suf) {
 // block) 101 / 54, 10.7M 80 / 117). At 13 photons, the most the complex128 block kernel takes, its blocks of tens of
 // states lose to the thread kernel's 16-photon form up to some ten million: 203k states 96 / 15, 5.2M 229 / 172,
 // 10.4M 350 / 336 (raw layers 424 / 296), 37M 959 / 1220 (1113 / 1096), 120M 2209 / 3978.
-bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool f64) {
+bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool comp, bool f64) {
+  const double states = (double)S * (double)B;
   if (f64 && K > 12 && S < (1ull << 32)) return S * (uint64_t)B >= (1ull << 25);
   if (K > 12 || S >= (1ull << 32)) return true;
   if (S * (uint64_t)B < (1ull << 21)) return false;
-  if (suf == 5 && !p->items[K].empty()) return S >= 320 * p->size(K - 6);
-  const double per = (double)S / (double)full_blocks(p, K, suf), states = (double)S * (double)B;
+  if (suf == 5 && !p->items[K].empty())
+    return S >= (f64 ? 370 : S >= (1ull << 20) && states >= (double)(1ull << 23) ? 280 : 320) * p->size(K - 6);
+  const double per = (double)S / (double)full_blocks(p, K, suf);
   if (p->multiset) return per >= 256.0 || states * per >= (double)(1ull << 33);
-  if (p->shift == 0) return states * per >= (f64 ? 4e10 : B > 2 ? 1.7e10 : 3e10);
-  return states * per >= (p->shift == 1 && B <= 2 ? 1.4e10 : 4e9);
+  const bool rows = B > 1, large = states >= (double)(1ull << 23);
+  if (p->shift == 0) return states * per >= (f64 ? 4e10 : comp ? (rows ? 1.2e10 : 2.2e10) : rows ? 1.7e10 : 3e10);
+  if (p->shift == 1) return states * per >= (comp ? (rows && large ? 6e8 : 2.7e9) : rows ? (large ? 2.5e9 : 1.2e10) : f64 ? 2e10 : 1.4e10);
+  return f64 ? states >= 9e6 : states * per >= 2e9;
 }
 
 // The grid of `wgs` work groups a row (see slos::batch_item): 1-D over all rows from 8 rows on, where
@@ -853,7 +863,7 @@ int launch_layer(const slos_plan* p, const DevTables& dt, int K, int col, const 
   a.par_lo = (comp && par_hilo) ? B * (int64_t)S_par : 0;
   a.out_lo = (comp && out_hilo && kind == 0) ? B * (int64_t)S : 0;
   if (!(flags & SLOS_FLAG_SIMPLE) && dt.tuples && K > slos::kSuf && K - slos::kSuf <= 16 &&
-      block_lds_fit(K, p->me, slos::kSuf) && (flags & SLOS_FLAG_BLOCK || use_blocks(p, K, block_suffix(p, dt, K), S, B, false)))
+      block_lds_fit(K, p->me, slos::kSuf) && (flags & SLOS_FLAG_BLOCK || use_blocks(p, K, block_suffix(p, dt, K), S, B, comp, false)))
     return launch_block(p, dt, a, kind, comp, st);
   const size_t sh = (((size_t)(K + 1) * (p->me + 1) * 8 + p->me * 4 + 15) & ~(size_t)15) + (size_t)p->m * 8;
   if (sh > lds_limit()) return fail(SLOS_ERANGE, "counting table does not fit LDS");
@@ -871,7 +881,7 @@ int launch_block_f64(const slos_plan* p, const DevTables& dt, int K, int col, co
   if (!dt.tuples || K <= slos::kSuf || B > 65535) return -1;
   const int suf = dt.tuples5 && K > 5 ? 5 : slos::kSuf;
   const int d = K - suf;
-  if (d > 8 || !(flags & SLOS_FLAG_BLOCK || use_blocks(p, K, suf, S, B, true))) return -1;
+  if (d > 8 || !(flags & SLOS_FLAG_BLOCK || use_blocks(p, K, suf, S, B, false, true))) return -1;
   slos::BlockLayerF64 L{};
   L.l.K = K; L.l.m = p->m; L.l.col = col; L.l.S_par = S_par; L.l.S = S; L.l.S_pre = p->size(d);
   L.l.flags = flags;
