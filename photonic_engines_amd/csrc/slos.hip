@@ -764,11 +764,13 @@ uint64_t full_blocks(const slos_plan* p, int K, int suf) {
 // block) 115 / 72, 10.7M 106 / 153) and for complex128 (f64: 1.1M 26 / 18, 2.2M 28 / 32, 3.1M 39 / 45; 3.1M (209 a
 // block) 101 / 54, 10.7M 80 / 117). At 13 photons, the most the complex128 block kernel takes, its blocks of tens of
 // states lose to the thread kernel's 16-photon form up to some ten million: 203k states 96 / 15, 5.2M 229 / 172,
-// 10.4M 350 / 336 (raw layers 424 / 296), 37M 959 / 1220 (1113 / 1096), 120M 2209 / 3978.
+// 10.4M 350 / 336 (raw layers 424 / 296), 37M 959 / 1220 (1113 / 1096), 120M 2209 / 3978; and in rows of short blocks at
+// any size: 2,000 of (13, 7), 9 states a block, 4146 / 1721, 20 of (13, 12), 33, 1889 / 1581, 4 of (13, 14), 51, 1149 / 1338.
 bool use_blocks(const slos_plan* p, int K, int suf, uint64_t S, int64_t B, bool comp, bool f64) {
   const double states = (double)S * (double)B;
-  if (f64 && K > 12 && S < (1ull << 32)) return S * (uint64_t)B >= (1ull << 25);
-  if (K > 12 || S >= (1ull << 32)) return true;
+  if (S >= (1ull << 32) || (K > 12 && !f64)) return true;
+  if (K > 12 && p->multiset) return S * (uint64_t)B >= (1ull << 25) && S >= 48 * full_blocks(p, K, suf);
+  if (K > 12 && S * (uint64_t)B < (1ull << 25)) return false;
   if (S * (uint64_t)B < (1ull << 21)) return false;
   if (suf == 5 && !p->items[K].empty())
     return S >= (f64 ? 370 : S >= (1ull << 20) && states >= (double)(1ull << 23) ? 280 : 320) * p->size(K - 6);
